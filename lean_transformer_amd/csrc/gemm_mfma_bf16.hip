@@ -28,7 +28,7 @@ bool lt_gemm_mfma_supported(const GemmProblem& p, int kind) {
   // Tiles that stick out past N (and past M for an mn-major A) are the copy-based kernel's: it copies the last row or the
   // last 8 columns again and its epilogue skips what is outside, 8 columns at a time.
   if (p.N % tile_n != 0 || (!a_km && p.M % BM != 0)) {
-    if (p.N % 8 != 0 || (!a_km && p.M % 8 != 0) || !dma_selected(p, kind, LT_BF16)) return false;
+    if (p.N % 8 != 0 || (!a_km && p.M % 8 != 0) || !dma_selected(p, kind)) return false;
   }
   if ((int64_t)((p.M + BM - 1) / BM) * ((p.N + tile_n - 1) / tile_n) > 0x7fffffff) return false;
   // the epilogue moves 8 columns at a time
@@ -43,8 +43,7 @@ bool lt_gemm_mfma_supported(const GemmProblem& p, int kind) {
   for (int s = 0; s < p.nseg; s++) {
     if ((bool)p.A[s].kmajor != a_km || (bool)p.B[s].kmajor != b_km) return false;
     if (p.K[s] <= 0) return false;
-    // k-major operands are read in whole 64-element k-steps; mn-major ones are zero-filled past K
-    if ((a_km || b_km) && p.K[s] % BK != 0) return false;
+    if ((a_km || b_km) && p.K[s] % 8 != 0) return false;
     if (p.A[s].ld % 8 != 0 || p.B[s].ld % 8 != 0) return false;
     if (!lt_aligned(p.A[s].ptr, 16) || !lt_aligned(p.B[s].ptr, 16)) return false;
   }
@@ -56,7 +55,7 @@ bool lt_sparse_mfma_supported(const GemmProblem& p, int kind);
 int lt_gemm_colsum_rows(const GemmProblem& p, int dtype, int io_dtype) {
   if (dtype != LT_BF16 || p.epi.ld_pre % 8 != 0) return 0;
   if (p.sp.mode == SPARSE_NONE)
-    return lt_gemm_mfma_supported(p, EPI_ACT_BWD) && dma_selected(p, EPI_ACT_BWD, io_dtype) ? 128 : 0;
+    return lt_gemm_mfma_supported(p, EPI_ACT_BWD) && dma_selected(p, EPI_ACT_BWD) ? 128 : 0;
   // the walk's straight-line strips keep the sums: every tile must take them
   return p.sp.mode == SPARSE_DX && lt_sparse_mfma_supported(p, EPI_ACT_BWD) && p.M % 256 == 0 &&
                  p.epi.act == LT_ACT_GELU_FUSED && p.epi.hid
@@ -134,7 +133,7 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
   const bool a_km = p.A[0].kmajor, b_km = p.B[0].kmajor;
   const EpiParams& e = p.epi;
   bool ok = dtype == LT_BF16 && p.nseg == 1 && p.sp.mode == SPARSE_NONE && p.M > 0 && p.N > 0 && p.N % 128 == 0 &&
-            !(!a_km && b_km) && (a_km || p.M % 128 == 0) && ((!a_km && !b_km) || p.K[0] % BK == 0) && p.K[0] > 0 &&
+            !(!a_km && b_km) && (a_km || p.M % 128 == 0) && ((!a_km && !b_km) || p.K[0] % 8 == 0) && p.K[0] > 0 &&
             p.A[0].ld % 8 == 0 && p.B[0].ld % 8 == 0 && lt_aligned(p.A[0].ptr, 16) && lt_aligned(p.B[0].ptr, 16) &&
             e.ldo == p.N && lt_aligned(e.out, 16) && (!e.bias || lt_aligned(e.bias, 16));
   const int64_t tiles = ((p.M + 127) / 128) * (p.N / 128);
@@ -145,8 +144,7 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
     // 256 x 256 tiles fit: the copy-based kernel, its reduction split when the tiles alone leave CUs idle
     const int slices = p.nseg == 1 ? splitk_slices(p.M, p.N, p.K[0]) : 1;
     const size_t need = (size_t)slices * (size_t)p.M * (size_t)p.N * sizeof(float);
-    if (slices > 1 && workspace && workspace_bytes >= need && p.variant != 1 && p.K[0] % 64 == 0 && e.ldo == p.N &&
-        dma_offsets_fit(p, EPI_STORE)) {
+    if (slices > 1 && workspace && workspace_bytes >= need && dma_selected(p, EPI_STORE) && e.ldo == p.N) {
       GemmProblem q = p;
       q.ksplit = slices;
       q.split_stride = p.M * p.N;
@@ -242,9 +240,8 @@ int lt_launch_gemm_out(const GemmProblem& p, int dtype, int io_dtype, void* work
     q.epi.ldo = p.N;
     q.epi.out_dtype = LT_F32;
     const size_t slice = (size_t)p.M * (size_t)p.N * sizeof(float);
-    // the tiled kernel where it takes the problem (a k-major reduction splits in blocks of 64), else the any-shape kernel
-    const bool tiled = dtype == LT_BF16 && p.variant != 1 && p.K[0] % 64 == 0 && lt_gemm_mfma_supported(q, EPI_STORE) &&
-                       dma_offsets_fit(q, EPI_STORE);
+    // the tiled kernel where it takes the problem, else the any-shape kernel
+    const bool tiled = dtype == LT_BF16 && lt_gemm_mfma_supported(q, EPI_STORE) && dma_selected(q, EPI_STORE);
     const bool tiled_unsplit = dtype == LT_BF16 && lt_gemm_mfma_supported(p, EPI_OUT);
     const int wanted = tiled ? splitk_slices(p.M, p.N, p.K[0]) : tiled_unsplit ? 1 : generic_splitk_slices(p.M, p.N, p.K[0]);
     const int slices = (int)std::min<size_t>((size_t)wanted, workspace_bytes / slice);
@@ -281,7 +278,7 @@ bool lt_sparse_mfma_supported(const GemmProblem& p, int kind) {
   }
   if (!lt_aligned(sp.weight, 16)) return false;
   if (p.nseg > 1) {
-    if (p.K[1] <= 0 || p.K[1] % BK != 0 || p.A[1].ld % 8 != 0 || p.B[1].ld % 8 != 0 || !lt_aligned(p.A[1].ptr, 16) ||
+    if (p.K[1] <= 0 || p.K[1] % 8 != 0 || p.A[1].ld % 8 != 0 || p.B[1].ld % 8 != 0 || !lt_aligned(p.A[1].ptr, 16) ||
         !lt_aligned(p.B[1].ptr, 16))
       return false;
   }
@@ -302,10 +299,10 @@ bool lt_sparse_forward_grouped(const GemmProblem& p, int kind) {
   if (sp.out_group < 4 || sp.out_group % 4 != 0 || sp.out_stride > 1 || p.N % 256 != 0) return false;
   // the list travels in one register: at most 64 entries, input block and flat position in 16 bits each
   if (sp.blocks_per_out > 64 || sp.ld_act / 64 * sp.blocks_per_in > 65535) return false;
-  if (p.nseg > 1 && p.K[1] % 64 != 0) return false;
+  if (p.nseg > 1 && p.K[1] % 64 != 0) return false;  // (this form copies whole k-blocks only)
   // 32-bit byte offsets inside a tile
-  if (256 * sp.ld_act * 2 >= (int64_t)1 << 32) return false;
-  if (p.nseg > 1 && (256 * p.A[1].ld * 2 >= (int64_t)1 << 32 || 256 * p.B[1].ld * 2 >= (int64_t)1 << 32)) return false;
+  if (257 * sp.ld_act * 2 + 1024 >= (int64_t)1 << 32) return false;
+  if (p.nseg > 1 && (257 * p.A[1].ld * 2 + 1024 >= (int64_t)1 << 32 || 257 * p.B[1].ld * 2 + 1024 >= (int64_t)1 << 32)) return false;
   return true;
 }
 
@@ -314,8 +311,7 @@ bool lt_sparse_dw_out_grouped(const GemmProblem& p) {
   const int64_t out_features = sp.ld_act;
   if (sp.out_stride > 1 && (int64_t)sp.out_group * sp.out_stride * 64 != out_features) return false;  // runs must tile the blocks
   return sp.mode == SPARSE_DW && sp.out_group >= 4 && sp.out_group % 4 == 0 && sp.forward_indices && out_features % 256 == 0 &&
-         sp.tokens % DK == 0 && sp.tokens > 0 && 32 * sp.ld_act * 2 + out_features * 2 < (int64_t)1 << 32 &&
-         32 * sp.ld_act2 * 2 + p.N * 2 < (int64_t)1 << 32;
+         sp.tokens > 0 && 33 * sp.ld_act * 2 + 1024 < (int64_t)1 << 32 && 33 * sp.ld_act2 * 2 + 1024 < (int64_t)1 << 32;
 }
 
 int lt_sparse_dw_in_grouped_slices(const GemmProblem& p) {
@@ -324,8 +320,8 @@ int lt_sparse_dw_in_grouped_slices(const GemmProblem& p) {
   if (sp.mode != SPARSE_DW || !lt_sparse_mfma_supported(p, EPI_STORE) || lt_sparse_dw_out_grouped(p)) return 0;
   if (sp.in_group < 4 || sp.in_group % 4 != 0 || !sp.backward_indices || in_features % 256 != 0) return 0;
   if (sp.in_stride > 1 && (int64_t)sp.in_group * sp.in_stride * 64 != in_features) return 0;  // runs must tile the blocks
-  if (sp.tokens <= 0 || sp.tokens % DK != 0) return 0;
-  if (32 * sp.ld_act * 2 + out_features * 2 >= (int64_t)1 << 32 || 32 * sp.ld_act2 * 2 + in_features * 2 >= (int64_t)1 << 32) return 0;
+  if (sp.tokens <= 0) return 0;
+  if (33 * sp.ld_act * 2 + 1024 >= (int64_t)1 << 32 || 33 * sp.ld_act2 * 2 + 1024 >= (int64_t)1 << 32) return 0;
   // enough workgroups for the 256 CUs, each slice at least 32 k-steps long
   const int64_t tiles = (int64_t)((sp.blocks_per_in + 3) / 4) * (in_features / 256);
   if (tiles >= 192) return 1;

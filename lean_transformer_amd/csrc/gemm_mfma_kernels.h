@@ -194,7 +194,10 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
     return (t % runs) * sp.walk_run + t / runs;
   };
   // global -> registers for k-step kt (ph: 0 = the tile's own block column, 1 = the matching linear block column)
-  auto load_tiles = [&](int kt, int ph, u32x4 (&ra)[A_CHUNKS], u32x4 (&rb)[B_CHUNKS]) __attribute__((always_inline)) {
+  // TAIL: the step may reach past the end of its reduction; pieces of a k-major operand past it repeat the last piece (and are
+  // zeroed by store_tiles)
+  auto load_tiles = [&](auto TAIL, int kt, int ph, u32x4 (&ra)[A_CHUNKS], u32x4 (&rb)[B_CHUNKS]) __attribute__((always_inline)) {
+    constexpr bool tail = decltype(TAIL)::value;
     const int seg = kt >= kt_seg0;
     int64_t k0 = (int64_t)(seg ? kt - kt_seg0 : kt) * BK;
     int64_t K = p.K[seg];
@@ -229,7 +232,7 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
       if constexpr (A_KM) {
         const int row = q >> 3, c = q & 7;
         const int64_t gm = min(m0 + row, p.M - 1);  // rows past M are clamped (their results are never stored)
-        ra[i] = *reinterpret_cast<const u32x4*>(A + gm * lda + k0 + c * 8);
+        ra[i] = *reinterpret_cast<const u32x4*>(A + gm * lda + (tail ? min(k0 + c * 8, K - 8) : k0 + c * 8));
       } else {
         // rows past K: the last row again, zeroed on the way into LDS (store_tiles) -- a load under a branch would make
         // every later wait on the memory counter a wait for all of them, and no load could stay in flight across a step
@@ -253,8 +256,8 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
           gn = b_row0 + row;
         }
         // a sparse FWD weight block holds its own 64 k: its columns start at 0, not at the gathered k0
-        const int64_t bk0 = (SP == SPARSE_FWD && !seg) ? 0 : k0;
-        rb[i] = *reinterpret_cast<const u32x4*>(B + gn * ldb + bk0 + c * 8);
+        const int64_t bk = (SP == SPARSE_FWD && !seg) ? c * 8 : tail ? min(k0 + c * 8, K - 8) : k0 + c * 8;
+        rb[i] = *reinterpret_cast<const u32x4*>(B + gn * ldb + bk);
       } else {
         const int kr = q / (BN / 8), c = q % (BN / 8);
         const int64_t gk = min(k0 + kr, K - 1);
@@ -262,7 +265,7 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
       }
     }
   };
-  // how many of the BK k-rows of step kt exist; mn-major operand tiles are zero-filled past them
+  // how many of the BK k of step kt exist (a multiple of 8 where an operand is k-major); operand tiles are zero-filled past them
   auto k_rows = [&](int kt) -> int {
     const int seg = kt >= kt_seg0;
     if ((SP == SPARSE_FWD || SP == SPARSE_DX) && !seg) return BK;
@@ -271,13 +274,14 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
     return (int)min((int64_t)BK, K - k0);
   };
   // registers -> LDS stage s
-  auto store_tiles = [&](int s, int rows, const u32x4 (&ra)[A_CHUNKS], const u32x4 (&rb)[B_CHUNKS]) __attribute__((always_inline)) {
+  auto store_tiles = [&](auto TAIL, int s, int rows, const u32x4 (&ra)[A_CHUNKS], const u32x4 (&rb)[B_CHUNKS]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < A_CHUNKS; i++) {
       const int q = tid + i * NT;
       if constexpr (A_KM) {
         const int row = q >> 3, c = q & 7;
-        *reinterpret_cast<u32x4*>(&lds_a[s][(row * 8 + (c ^ swz_km(row))) * 8]) = (PF == 1 || rows > 0) ? ra[i] : u32x4{0u, 0u, 0u, 0u};
+        *reinterpret_cast<u32x4*>(&lds_a[s][(row * 8 + (c ^ swz_km(row))) * 8]) =
+            !decltype(TAIL)::value || c * 8 < rows ? ra[i] : u32x4{0u, 0u, 0u, 0u};
       } else {
         const int kr = q / (BM / 8), c = q % (BM / 8);
         *reinterpret_cast<u32x4*>(&lds_a[s][kr * BM + ((c ^ swz_mn_cols<BM>(kr)) << 3)]) = kr < rows ? ra[i] : u32x4{0u, 0u, 0u, 0u};
@@ -288,7 +292,8 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
       const int q = tid + i * NT;
       if constexpr (B_KM) {
         const int row = q >> 3, c = q & 7;
-        *reinterpret_cast<u32x4*>(&lds_b[s][(row * 8 + (c ^ swz_km(row))) * 8]) = (PF == 1 || rows > 0) ? rb[i] : u32x4{0u, 0u, 0u, 0u};
+        *reinterpret_cast<u32x4*>(&lds_b[s][(row * 8 + (c ^ swz_km(row))) * 8]) =
+            !decltype(TAIL)::value || c * 8 < rows ? rb[i] : u32x4{0u, 0u, 0u, 0u};
       } else {
         const int kr = q / (BN / 8), c = q % (BN / 8);
         *reinterpret_cast<u32x4*>(&lds_b[s][kr * BN + ((c ^ swz_mn_cols<BN>(kr)) << 3)]) = kr < rows ? rb[i] : u32x4{0u, 0u, 0u, 0u};
@@ -357,17 +362,29 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
   if constexpr (PF == 1) {
     lt_static_for<PH>([&](auto PHASE) __attribute__((always_inline)) {
       constexpr int ph = decltype(PHASE)::value;
+      using Whole = std::false_type;
+      using Tail = std::true_type;
       if (kt_begin < kt_end) {
-        load_tiles(kt_begin, ph, ra_set[0], rb_set[0]);
-        store_tiles(kt_begin & 1, k_rows(kt_begin), ra_set[0], rb_set[0]);
+        load_tiles(Tail{}, kt_begin, ph, ra_set[0], rb_set[0]);
+        store_tiles(Tail{}, kt_begin & 1, k_rows(kt_begin), ra_set[0], rb_set[0]);
       }
       __syncthreads();
-      for (int kt = kt_begin; kt < kt_end; kt++) {
-        const int s = kt & 1;
+      // steps whose next step has whole k-major tiles, then the rest: with the test for a ragged end in every step the
+      // input-gradient walk of a PixelFly layer (hidden 4096) takes 244 us instead of 206
+      const int seg_last = kt_total > kt_seg0;
+      const int kt_whole = SP == SPARSE_DW || p.K[seg_last] % BK == 0 ? kt_end : min(kt_end, kt_total - 1);
+      int kt = kt_begin;
+      for (; kt + 1 < kt_whole; kt++) {
+        load_tiles(Whole{}, kt + 1, ph, ra_set[0], rb_set[0]);
+        multiply_stage(kt & 1, PHASE);
+        store_tiles(Whole{}, (kt & 1) ^ 1, k_rows(kt + 1), ra_set[0], rb_set[0]);
+        __syncthreads();
+      }
+      for (; kt < kt_end; kt++) {
         const bool has_next = kt + 1 < kt_end;
-        if (has_next) load_tiles(kt + 1, ph, ra_set[0], rb_set[0]);
-        multiply_stage(s, PHASE);
-        if (has_next) store_tiles(s ^ 1, k_rows(kt + 1), ra_set[0], rb_set[0]);
+        if (has_next) load_tiles(Tail{}, kt + 1, ph, ra_set[0], rb_set[0]);
+        multiply_stage(kt & 1, PHASE);
+        if (has_next) store_tiles(Tail{}, (kt & 1) ^ 1, k_rows(kt + 1), ra_set[0], rb_set[0]);
         __syncthreads();
       }
     });
@@ -390,18 +407,18 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
       auto rows_of = [&](int i) { return i < steps ? k_rows(kt_of(i)) : 0; };
       lt_static_for<PF>([&](auto D) __attribute__((always_inline)) {
         constexpr int d = decltype(D)::value;
-        load_tiles(kt_of(d), 0, ra_set[d], rb_set[d]);
+        load_tiles(std::true_type{}, kt_of(d), 0, ra_set[d], rb_set[d]);
       });
-      store_tiles(0, rows_of(0), ra_set[0], rb_set[0]);
+      store_tiles(std::true_type{}, 0, rows_of(0), ra_set[0], rb_set[0]);
       __syncthreads();
       for (int i0 = 0; i0 < padded; i0 += PF) {
         lt_static_for<PF>([&](auto D) __attribute__((always_inline)) {
           constexpr int d = decltype(D)::value;
           const int i = i0 + d;
           const int s = i & 1;
-          load_tiles(kt_of(i + PF), 0, ra_set[d], rb_set[d]);
+          load_tiles(std::true_type{}, kt_of(i + PF), 0, ra_set[d], rb_set[d]);
           multiply_stage(s, std::integral_constant<int, 0>{});
-          store_tiles(s ^ 1, rows_of(i + 1), ra_set[(d + 1) % PF], rb_set[(d + 1) % PF]);
+          store_tiles(std::true_type{}, s ^ 1, rows_of(i + 1), ra_set[(d + 1) % PF], rb_set[(d + 1) % PF]);
           __syncthreads();
         });
       }
@@ -635,8 +652,6 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
 // so no LDS read latency is exposed after the barrier and copies have 1 to 2.5 k-steps to land.  The epilogue stages the
 // accumulators through LDS one 32-row strip at a time; whole tiles in the usual configurations take straight-line strips.
 // =====================================================================================================================
-__device__ const u32x4 lt_zero_chunk = {0u, 0u, 0u, 0u};  // source of the lanes past the end of a ragged reduction
-
 constexpr int DK = 32;  // k per step of the copy-based kernel
 
 // scheduling hint for one half k-step: READS LDS reads over the first READ_SPAN of MFMAS matrix instructions and COPIES
@@ -671,8 +686,11 @@ template <int N, bool WAIT_LDS = true> __device__ __forceinline__ void wait_copi
 // base that advances by `unit_bytes` per copy unit (k-major: a block of 64 k; mn-major: a k-step of 32 k).
 template <bool KM> struct DmaOperand {
   static constexpr int LOADS = KM ? 8 : 4;  // copy instructions per wavefront per unit (32 or 16 KiB / 4 wavefronts / 1 KiB)
+  // Descriptor size of every copy: the buffer unit returns zeros for a lane whose offset is not below it.  No real offset
+  // reaches it (dma_offsets_fit leaves the top KiB of the 32-bit range free); OUTSIDE does, and marks what lies past the end of
+  // a reduction.
+  static constexpr uint32_t RECORDS = 0xfffffc00u, OUTSIDE = 0xfffffe00u;
   uint32_t off[LOADS];
-  int krow[LOADS];  // mn-major: k-row inside the k-step (for the ragged-reduction test)
   const char* base;
   int64_t unit_bytes;
   int seg;
@@ -696,12 +714,10 @@ template <bool KM> struct DmaOperand {
         int64_t g = min(row0 + local, row_limit - 1) - row0;
         if (pair_rows > 0) g += ((row & 127) >> 6) * pair_rows;
         off[j] = (uint32_t)((g * ld + c * 8) * 2);
-        krow[j] = 0;
       } else {
         const int kr = q >> 5, c = (q & 31) ^ swz_mn(kr);
         const int64_t col = min(row0 + c * 8, row_limit - 8) - row0;
         off[j] = (uint32_t)((kr * ld + col) * 2);
-        krow[j] = kr;
       }
     }
     base = KM ? ptr + row0 * ld * 2 : ptr + row0 * 2;
@@ -721,37 +737,32 @@ template <bool KM> struct DmaOperand {
       const int slot = c >> 3;
       const int blk = slot == 0 ? blocks[0] : slot == 1 ? blocks[1] : slot == 2 ? blocks[2] : blocks[3];
       off[j] = (uint32_t)((kr * ld + (int64_t)blk * 64 + (c & 7) * 8) * 2);
-      krow[j] = kr;
     }
     base = reinterpret_cast<const char*>(op.ptr);
     unit_bytes = DK * ld * 2;
   }
 
-  // all copies of unit u (counted inside the k-segment) into `dst`; k_limit: reduction length for the ragged test
+  // all copies of unit u (counted inside the k-segment) into `dst`.  Buffer form: wavefront-uniform descriptor of the unit + the
+  // lane's 32-bit offset.  No vector address arithmetic, and unlike the global form the compiler does not count it as a FLAT
+  // access, after which it turns every wait for LDS data into a wait for all of it.
   // J0, J1: range of this wavefront's copy instructions (a k-major block can go out in two halves)
-  template <bool K_TAIL, int J0 = 0, int J1 = LOADS>
-  __device__ __forceinline__ void issue(int u, bf16* dst, int wave, int64_t k_limit) const {
-    if constexpr (!(K_TAIL && !KM)) {
-      // Buffer form: wavefront-uniform descriptor of the unit + the lane's 32-bit offset.  No vector address arithmetic,
-      // and unlike the global form the compiler does not count it as a FLAT access, after which it turns every wait for
-      // LDS data into a wait for all of it.
-      const __amdgpu_buffer_rsrc_t rsrc =
-          __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base + u * unit_bytes), 0, -1, 0x00020000);
-#pragma unroll
-      for (int j = J0; j < J1; j++)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(dst + (wave * LOADS + j) * 512),
-                                                 16, (int)off[j], 0, 0, 0);
-      return;
-    }
-    // ragged reduction over mn-major operands: lanes past the end read a chunk of zeros instead
+  // TAIL: the unit may reach past k_limit, the length of the reduction (a multiple of 8 for a k-major operand): the 16-byte
+  // pieces past it arrive as zeros.  A whole unit goes through the same code, so that nothing in it is conditional.
+  template <bool TAIL, int J0 = 0, int J1 = LOADS>
+  __device__ __forceinline__ void issue(int u, bf16* dst, int wave, int lane, int k_limit) const {
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base + u * unit_bytes), 0, (int)RECORDS, 0x00020000);
 #pragma unroll
     for (int j = J0; j < J1; j++) {
-      const char* g = base + u * unit_bytes + off[j];
-      if constexpr (K_TAIL && !KM) {
-        if ((int64_t)u * DK + krow[j] >= k_limit) g = reinterpret_cast<const char*>(&lt_zero_chunk);
+      uint32_t o = off[j];
+      if constexpr (TAIL) {
+        const int q = (wave * LOADS + j) * 64 + lane;
+        const int k = KM ? u * 64 + ((q & 7) ^ swz_km(q >> 3)) * 8 : u * DK + (q >> 5);
+        // OUTSIDE where k >= k_limit, formed without a lane mask: the kernel has no scalar register left for one per copy
+        o = max(o, (uint32_t)((k_limit - 1 - k) >> 31) & OUTSIDE);
       }
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
-                                       (__attribute__((address_space(3))) void*)(dst + (wave * LOADS + j) * 512), 16, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(dst + (wave * LOADS + j) * 512), 16,
+                                               (int)o, 0, 0, 0);
     }
   }
 };
@@ -1096,7 +1107,7 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
 //   ib_e) and so form one [256 rows][64 k] k-major matrix.  The list sits in one register (lane e: ib_e << 16 | flat
 //   position) and is read with v_readlane, so the k-loop issues no memory instruction for it.  A second k-segment (the
 //   low-rank term) is an ordinary one.
-template <bool A_KM, bool B_KM, int KIND, typename TX, bool K_TAIL, int GATHER = 0>
+template <bool A_KM, bool B_KM, int KIND, typename TX, int GATHER = 0>
 __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem, int tiles_m, int tiles_n) {
   // A workgroup may loop over tiles.  Whatever the compiler finds to be the same in every tile -- values loaded from the problem
   // description, the wavefront's LDS addresses, lane offsets -- it would compute once and keep in registers across the whole
@@ -1109,8 +1120,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
   typedef const __attribute__((address_space(4))) GemmProblem* KernargProblem;
   KernargProblem pk = (KernargProblem)__builtin_amdgcn_kernarg_segment_ptr();
 #define p (*pk)
-  static_assert((GATHER != 1 && GATHER != 3) || (!A_KM && !B_KM && KIND == EPI_STORE && !K_TAIL), "gathered columns: weight-gradient layout");
-  static_assert(GATHER != 2 || (A_KM && B_KM && !K_TAIL), "gathered k-blocks: forward layout");
+  static_assert((GATHER != 1 && GATHER != 3) || (!A_KM && !B_KM && KIND == EPI_STORE), "gathered columns: weight-gradient layout");
+  static_assert(GATHER != 2 || (A_KM && B_KM), "gathered k-blocks: forward layout");
   constexpr int BM = 256, BN = 256, WN = 2, WTM = 128, WTN = 128, FM = 4, FN = 4;
   constexpr int HALF = 4;  // copy instructions per wavefront for a mn-major k-step or half a k-major block
   constexpr int KM_ELEMS = 256 * 64, MN_ELEMS = DK * 256;
@@ -1156,7 +1167,9 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
   bool gated = false;
   auto k_steps = [&]() {
     gated = (KIND == EPI_ACT_FWD) && p.epi.gated;
-    kt_all = (int)((p.K[0] + DK - 1) / DK) + (p.nseg > 1 ? (int)((p.K[1] + DK - 1) / DK) : 0);
+    // (a second segment starts at a whole k-major block: the first is padded to one with zeros)
+    const int seg0 = (A_KM || B_KM) && p.nseg > 1 ? (int)((p.K[0] + 63) / 64) * 2 : (int)((p.K[0] + DK - 1) / DK);
+    kt_all = seg0 + (p.nseg > 1 ? (int)((p.K[1] + DK - 1) / DK) : 0);
     kt_begin = 0;
     kt_total = kt_all;
     if (p.ksplit > 1) {
@@ -1164,7 +1177,13 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
       kt_begin = min(kt_all, (int)blockIdx.y * per);
       kt_total = min(per, kt_all - kt_begin);
     }
-    kt_seg0 = p.nseg > 1 ? (int)((p.K[0] + DK - 1) / DK) : kt_total;
+    kt_seg0 = p.nseg > 1 ? seg0 : kt_total;
+  };
+  // first k-step (local to the slice) whose copies may reach past the end of k-segment `seg`: those are left to the code that
+  // tests for it
+  auto kt_whole = [&](int seg) {
+    const int whole = (A_KM || B_KM) ? (int)(p.K[seg] / 64) * 2 : (int)(p.K[seg] / DK);
+    return seg ? kt_seg0 + whole : whole - kt_begin;
   };
   k_steps();
 
@@ -1210,7 +1229,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
   // nothing to gain for mn-major ones.
   int rot = 0;
   auto set_rot = [&](int v) {
-    if (!K_TAIL && GATHER == 0 && p.nseg == 1 && (kt_all & 1) == 0 && p.krot) {
+    if (GATHER == 0 && p.nseg == 1 && (p.K[0] & 63) == 0 && p.krot) {
       const unsigned bx = (unsigned)v;
       // (inside an XCD the eight tile rows start 2 k-steps apart at most: tiles that share a B panel then read it within 14
       // k-steps of each other, inside what the XCD's L2 still holds; 8 apart, as a long reduction would otherwise give,
@@ -1309,7 +1328,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
     const int ks = rotated(seg ? t - kt_seg0 : t + kt_begin);
     int unit = A_KM ? ks >> 1 : ks;
     if (GATHER == 2 && seg == 0) unit = __builtin_amdgcn_readlane(list_entry, ks >> 1) >> 16;
-    ca.template issue<K_TAIL, decltype(J0)::value, decltype(J1)::value>(unit, a_buf(I), wave, p.K[seg]);
+    ca.template issue<!decltype(steady)::value && GATHER != 2, decltype(J0)::value, decltype(J1)::value>(
+        unit, a_buf(I), wave, lane, (int)p.K[seg]);
   };
   auto copy_b = [&](auto steady, auto I, int t, auto J0, auto J1) {
     int seg = cb.seg;
@@ -1320,7 +1340,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
     const int ks = rotated(seg ? t - kt_seg0 : t + kt_begin);
     int unit = B_KM ? ks >> 1 : ks;
     if (GATHER == 2 && seg == 0) unit = __builtin_amdgcn_readlane(list_entry, ks >> 1) & 0xffff;
-    cb.template issue<K_TAIL, decltype(J0)::value, decltype(J1)::value>(unit, b_buf(I), wave, p.K[seg]);
+    cb.template issue<!decltype(steady)::value && GATHER != 2, decltype(J0)::value, decltype(J1)::value>(
+        unit, b_buf(I), wave, lane, (int)p.K[seg]);
   };
 
   // ---- MFMA operand fragments: 8 k values of row / column lane % 32 of a 32-wide block
@@ -1519,7 +1540,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
     for (;;) {
       // copies issued by the steady loop reach k-step kt + 7: they must exist and lie in the k-segment both operands' copy
       // offsets are set up for
-      const int bound = (ca.seg == 0 && p.nseg > 1) ? kt_seg0 : kt_total;
+      const int bound = __builtin_amdgcn_readfirstlane(min((ca.seg == 0 && p.nseg > 1) ? kt_seg0 : kt_total, kt_whole(ca.seg)));
       if (ca.seg == cb.seg) {
         for (; kt + 7 < bound; kt += 4) {
 #ifdef LT_TILE_TIMING
@@ -1613,26 +1634,17 @@ int launch_dma(const GemmProblem& problem, int io_dtype, hipStream_t stream) {
   const bool gated = KIND == EPI_ACT_FWD && p.epi.gated;
   const int tiles_m = (int)((p.M + 255) / 256);
   const int tiles_n = (int)((p.N + (gated ? 127 : 255)) / (gated ? 128 : 256));
-  bool k_tail = false;
-  for (int s = 0; s < p.nseg; s++) k_tail = k_tail || (p.K[s] % DK != 0);
   dim3 grid(dma_grid(p, tiles_m * tiles_n), (unsigned)(p.ksplit > 1 ? p.ksplit : 1)), block(256);
   const bool bf16_io = KIND == EPI_OUT && io_dtype == LT_BF16;
-  if constexpr (!A_KM && !B_KM) {
-    if (k_tail) {
-      hipLaunchKernelGGL((gemm_bf16_dma_kernel<A_KM, B_KM, KIND, float, true>), grid, block, 0, stream, p, tiles_m, tiles_n);
-      LT_LAUNCH_CHECK();
-      return LT_OK;
-    }
-  }
   // the type of x / y only enters the EPI_OUT epilogue: the other kinds have one instantiation
   if constexpr (KIND == EPI_OUT) {
     if (bf16_io) {
-      hipLaunchKernelGGL((gemm_bf16_dma_kernel<A_KM, B_KM, KIND, bf16, false>), grid, block, 0, stream, p, tiles_m, tiles_n);
+      hipLaunchKernelGGL((gemm_bf16_dma_kernel<A_KM, B_KM, KIND, bf16>), grid, block, 0, stream, p, tiles_m, tiles_n);
       LT_LAUNCH_CHECK();
       return LT_OK;
     }
   }
-  hipLaunchKernelGGL((gemm_bf16_dma_kernel<A_KM, B_KM, KIND, float, false>), grid, block, 0, stream, p, tiles_m, tiles_n);
+  hipLaunchKernelGGL((gemm_bf16_dma_kernel<A_KM, B_KM, KIND, float>), grid, block, 0, stream, p, tiles_m, tiles_n);
   LT_LAUNCH_CHECK();
   return LT_OK;
 }
@@ -1679,7 +1691,7 @@ template <int KIND> int launch_sparse(const GemmProblem& problem, int io_dtype, 
         q.K[0] = (int64_t)sp.blocks_per_out * 64;
         q.ksplit = 0; q.krot = 0;
         const int tiles_n = (int)(p.N / 256);
-        hipLaunchKernelGGL((gemm_bf16_dma_kernel<true, true, KIND, float, false, 2>), dim3(dma_grid(q, tiles_m * tiles_n)), block, 0,
+        hipLaunchKernelGGL((gemm_bf16_dma_kernel<true, true, KIND, float, 2>), dim3(dma_grid(q, tiles_m * tiles_n)), block, 0,
                            stream, q, tiles_m, tiles_n);
         LT_LAUNCH_CHECK();
         return LT_OK;
@@ -1709,7 +1721,7 @@ template <int KIND> int launch_sparse(const GemmProblem& problem, int io_dtype, 
         q.A[0].ptr = sp.act; q.A[0].ld = sp.ld_act; q.A[0].kmajor = 0;
         q.B[0].ptr = sp.act2; q.B[0].ld = sp.ld_act2; q.B[0].kmajor = 0;
         q.ksplit = 0; q.krot = 0;
-        hipLaunchKernelGGL((gemm_bf16_dma_kernel<false, false, EPI_STORE, float, false, 1>), dim3(dma_grid(q, tiles_m * tiles_n)),
+        hipLaunchKernelGGL((gemm_bf16_dma_kernel<false, false, EPI_STORE, float, 1>), dim3(dma_grid(q, tiles_m * tiles_n)),
                            block, 0, stream, q, tiles_m, tiles_n);
         LT_LAUNCH_CHECK();
         return LT_OK;
@@ -1725,7 +1737,7 @@ template <int KIND> int launch_sparse(const GemmProblem& problem, int io_dtype, 
         q.A[0].ptr = sp.act; q.A[0].ld = sp.ld_act; q.A[0].kmajor = 0;
         q.B[0].ptr = sp.act2; q.B[0].ld = sp.ld_act2; q.B[0].kmajor = 0;
         q.ksplit = slices > 1 ? slices : 0; q.krot = 0;
-        hipLaunchKernelGGL((gemm_bf16_dma_kernel<false, false, EPI_STORE, float, false, 3>),
+        hipLaunchKernelGGL((gemm_bf16_dma_kernel<false, false, EPI_STORE, float, 3>),
                            dim3(dma_grid(q, tiles_m * tiles_n), (unsigned)slices), block, 0, stream, q, tiles_m, tiles_n);
         LT_LAUNCH_CHECK();
         return LT_OK;
@@ -1747,26 +1759,17 @@ bool dma_offsets_fit(const GemmProblem& p, int kind) {
   for (int s = 0; s < p.nseg; s++) {
     const int64_t a_span = p.A[s].kmajor ? 256 * p.A[s].ld : 64 * p.A[s].ld;
     const int64_t b_span = p.B[s].kmajor ? ((gated ? p.N : 0) + 256) * p.B[s].ld : 64 * p.B[s].ld;
-    if ((a_span + 512) * 2 >= (int64_t)1 << 32 || (b_span + 512) * 2 >= (int64_t)1 << 32) return false;
+    // (DmaOperand::RECORDS: the top KiB of the offsets is never reached; k-step numbers are 32-bit)
+    if ((a_span + 512) * 2 >= (int64_t)1 << 32 || (b_span + 512) * 2 >= (int64_t)1 << 32 || p.K[s] >= 0x7fffff00) return false;
   }
   return true;
 }
 
 // whether a problem the tiled kernels take goes to the copy-based one
-bool dma_selected(const GemmProblem& p, int kind, int io_dtype) {
-  const bool a_km = p.A[0].kmajor, b_km = p.B[0].kmajor;
-  bool k_tail = false, k_blocks = true;
-  for (int s = 0; s < p.nseg; s++) {
-    k_tail = k_tail || (p.K[s] % DK != 0);
-    k_blocks = k_blocks && (p.K[s] % 64 == 0);  // k-major operands are copied in whole blocks of 64 k
-  }
-  const bool dma_ok = dma_offsets_fit(p, kind) && !(k_tail && kind == EPI_OUT && io_dtype == LT_BF16) &&
-                      ((!a_km && !b_km) || k_blocks);
-  return p.variant != 1 && dma_ok;
-}
+bool dma_selected(const GemmProblem& p, int kind) { return p.variant != 1 && dma_offsets_fit(p, kind); }
 
 template <bool A_KM, bool B_KM, int KIND> int launch_tile(const GemmProblem& p, int io_dtype, hipStream_t stream) {
-  if (dma_selected(p, KIND, io_dtype)) return launch_dma<A_KM, B_KM, KIND>(p, io_dtype, stream);
+  if (dma_selected(p, KIND)) return launch_dma<A_KM, B_KM, KIND>(p, io_dtype, stream);
   return launch_cfg<256, 256, 2, 2, A_KM, B_KM, KIND>(p, io_dtype, stream);
 }
 
