@@ -470,7 +470,7 @@ __device__ __forceinline__ void epi_out8_loaded(const EpiParams& e, int64_t m, i
 // ---------------------------------------------------------------------------------------------------------------------
 // launchers (defined in gemm_generic.hip / gemm_mfma_bf16.hip)
 // ---------------------------------------------------------------------------------------------------------------------
-// any shape, fp32 or bf16 operands (dtype), fp32 MFMA arithmetic.  io_dtype: dtype of x / y for EPI_OUT.
+// any shape, fp32 or bf16 operands (dtype), fp32 accumulation.  io_dtype: dtype of x / y for EPI_OUT.
 int lt_launch_gemm_generic(const GemmProblem& p, int kind, int dtype, int io_dtype, hipStream_t stream);
 // true when the tiled bf16 kernel handles this problem (operand layouts, alignment, tile divisibility)
 bool lt_gemm_mfma_supported(const GemmProblem& p, int kind);

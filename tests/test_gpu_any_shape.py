@@ -1,0 +1,78 @@
+"""The any-shape GEMM kernel: fp32 operands as three bfloat16 planes, its tile heights (64 and 128 rows), vector and scalar fetches,
+whole and ragged k-steps, split reductions, block-sparse walks over odd block sizes.
+
+Bound on a result of fp32 operands: the six plane products are exact in fp32, so an element is a chain of at most 6 ceil(K / 16) + 4
+fp32 accumulations (4 for the sum of the slices), each off by at most 2^-23 of the magnitudes it adds, plus the dropped products, at
+most 2^-22 of |a| |b|:  |c - ref| <= (6 ceil(K / 16) + 6) 2^-23 (|a| |b|^T)."""
+import pytest
+import torch
+
+from conftest import rel_err
+from lean_transformer_amd import _native as nat
+from test_gpu_kernels import _gemm, _operands
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _check(c, a, b, k):
+    """a [m, k], b [n, k] on the GPU"""
+    ref = a.double() @ b.double().t()
+    bound = (6 * -(-k // 16) + 6) * 2.0**-23 * (a.double().abs() @ b.double().abs().t())
+    worst = ((c.double() - ref).abs() - bound).max().item()
+    assert worst <= 0.0, f"{worst:.3e} beyond the bound"
+    return ref
+
+
+@pytest.mark.parametrize("a_kmajor,b_kmajor", [(True, True), (True, False), (False, False), (False, True)])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (64, 128, 16), (65, 129, 17), (63, 127, 15), (130, 132, 48), (200, 260, 100),
+                                   (5000, 1700, 36), (4100, 2048, 64)])
+def test_fp32_any_shape_and_layout(a_kmajor, b_kmajor, m, n, k):
+    """the last two have enough workgroups for 128-row tiles"""
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    a, b = torch.randn(m, k, generator=g, device=DEV), torch.randn(n, k, generator=g, device=DEV)
+    c = _gemm(a if a_kmajor else a.t().contiguous(), b if b_kmajor else b.t().contiguous(), a_kmajor, b_kmajor, m, n, k,
+              torch.float32, 1)
+    _check(c, a, b, k)
+
+
+@pytest.mark.parametrize("scale", [1.0, 2.0**100, 2.0**-90])
+def test_fp32_split_is_exact(scale):
+    """times the identity: every element comes back bit for bit, from the largest finite value down"""
+    g = torch.Generator(device=DEV).manual_seed(1)
+    a = torch.randn(130, 96, generator=g, device=DEV) * scale
+    a[0, :4] = torch.tensor([torch.finfo(torch.float32).max, -torch.finfo(torch.float32).max, 0.0, 1 + 2.0**-23], device=DEV)
+    eye = torch.eye(96, device=DEV)
+    assert torch.equal(_gemm(a, eye, True, True, 130, 96, 96, torch.float32, 1), a)
+
+
+def test_fp32_errors_do_not_add_up_over_rows():
+    """a bias of the accumulation's rounding would grow with the number of rows in a column sum (a bias gradient): the sum of M
+    independent errors is sqrt(M) times one of them; 4 times that leaves room for a bias of 6 % of the rms error at M = 4096"""
+    g = torch.Generator(device=DEV).manual_seed(2)
+    m, n, k = 4096, 768, 1536
+    a, b = torch.randn(m, k, generator=g, device=DEV), torch.randn(n, k, generator=g, device=DEV)
+    err = _gemm(a, b.t().contiguous(), True, False, m, n, k, torch.float32, 1).double() - a.double() @ b.double().t()
+    assert err.sum(0).norm().item() <= 4 * err.norm().item()
+
+
+def test_fp32_view_that_is_not_16_byte_aligned():
+    """rows of an odd length behind an odd offset: element-wise fetches and stores"""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    m, n, k = 70, 45, 33
+    store = torch.randn(m * k + n * k + 2, generator=g, device=DEV)
+    a, b = store[1:1 + m * k].view(m, k), store[1 + m * k:1 + m * k + n * k].view(n, k)
+    out = torch.full((m * n + 9,), 7.0, device=DEV)
+    c = out[1:1 + m * n].view(m, n)
+    nat.check(nat.lib().lt_gemm(nat.LT_F32, m, n, k, a.data_ptr(), 1, b.data_ptr(), 1, nat.LT_F32, c.data_ptr(), 1,
+                                nat.current_stream(c.device)), "lt_gemm")
+    _check(c, a, b, k)
+    assert out[0].item() == 7.0 and bool((out[1 + m * n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("a_kmajor,b_kmajor", [(True, True), (True, False), (False, False), (False, True)])
+@pytest.mark.parametrize("m,n,k", [(70, 45, 33), (129, 127, 31), (64, 128, 96), (4100, 2100, 72)])
+def test_16_bit_operands(dtype, a_kmajor, b_kmajor, m, n, k):
+    a, b, ref = _operands(m, n, k, a_kmajor, b_kmajor, dtype, seed=m + n + k)
+    assert rel_err(_gemm(a, b, a_kmajor, b_kmajor, m, n, k, torch.float32, 1), ref) <= 1e-5
