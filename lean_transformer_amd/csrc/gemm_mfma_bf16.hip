@@ -25,6 +25,8 @@ bool lt_gemm_mfma_supported(const GemmProblem& p, int kind) {
   const int64_t tile_n = gated ? BN / 2 : BN;
   const bool a_km = p.A[0].kmajor, b_km = p.B[0].kmajor;
   if (!a_km && b_km) return false;
+  if ((kind == EPI_ACT_FWD || kind == EPI_OUT) && !(a_km && b_km)) return false;
+  if (kind == EPI_ACT_BWD && !(a_km && !b_km)) return false;
   // Tiles that stick out past N (and past M for an mn-major A) are the copy-based kernel's: it copies the last row or the
   // last 8 columns again and its epilogue skips what is outside, 8 columns at a time.
   if (p.N % tile_n != 0 || (!a_km && p.M % BM != 0)) {

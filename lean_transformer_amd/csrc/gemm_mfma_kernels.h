@@ -542,7 +542,7 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
     for (int it = 0; it < NIT; it++) {
       float v[8];
       read_staged(it, v);
-      epi_act_bwd8_gelu<GATED>(epi, lane_row(i) + it * ROWS_PER_IT, lane_n, v, rows[it], colsum);
+      epi_act_bwd8_fixed<GATED, LT_ACT_GELU_FUSED>(epi, lane_row(i) + it * ROWS_PER_IT, lane_n, v, rows[it], colsum);
     }
     __builtin_amdgcn_wave_barrier();
   };
@@ -582,7 +582,7 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
       }
     }
 #pragma unroll
-    for (int it = 0; it < NITF; it++) epi_act_fwd8_gelu<GATED>(epi, mlane + it * RPI, n, vg[it], vl[GATED ? it : 0]);
+    for (int it = 0; it < NITF; it++) epi_act_fwd8_fixed<GATED, LT_ACT_GELU_FUSED>(epi, mlane + it * RPI, n, vg[it], vl[GATED ? it : 0]);
     __builtin_amdgcn_wave_barrier();
   };
   const bool whole_tile = m_base + BM <= m_limit;
@@ -832,10 +832,12 @@ __device__ __forceinline__ int lt_run_member(int t, int j, int len, int stride) 
 // gradient, at the flat position the forward table names.  List entries past the end (the last column tile) are not stored.
 // SCATTER == 2: the tile is 4 entries of a list of output blocks (rows) x the run of 4 input blocks that shares the list
 // (columns); piece (entry a, input block ib) is block ib * blocks_per_in + a.
-template <int FM, int KIND, typename TX, int tile_rows, int tile_cols, int SCATTER = 0>
+// ACT: the activation of EPI_ACT_FWD / EPI_ACT_BWD, or -1: chosen per element from epi.act.
+template <int FM, int KIND, typename TX, int tile_rows, int tile_cols, int SCATTER = 0, int ACT = -1>
 __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const GemmProblem& p, float* stage, const int64_t m0,
                                                   const int64_t n0, const int wm, const int wn, const bool gated) {
   constexpr int FN = 4, WTN = 128, WTM = FM * 32;
+  constexpr bool STRAIGHT_ACT = ACT == LT_ACT_GELU_FUSED || ACT == LT_ACT_SILU;  // short enough to be unrolled
   // the lane index is formed anew rather than kept in a register across the main loop, through an asm statement so that a
   // workgroup that loops over tiles does not keep what is derived from it alive from one tile's epilogue to the next's either
   int lane;
@@ -855,7 +857,7 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
 #pragma unroll
   for (int e = 0; e < 16; e++) colsum[e] = 0.f;
   // accumulators of strip I -> this wavefront's staging buffer
-  auto stage_strip = [&](auto I) {
+  auto stage_strip = [&](auto I) __attribute__((always_inline)) {
     constexpr int i = decltype(I)::value;
 #pragma unroll
     for (int j = 0; j < FN; j++)
@@ -863,54 +865,82 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
       for (int r = 0; r < 16; r++) *staged(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), j * 32 + (lane & 31)) = acc[i][j][r];
     __builtin_amdgcn_wave_barrier();
   };
-  auto for_each_strip = [&](auto&& strip) { lt_static_for<FM>(strip); };
-  auto generic_strip = [&](auto I) {
+  auto for_each_strip = [&](auto&& strip) __attribute__((always_inline)) { lt_static_for<FM>(strip); };
+  // Any activation, tiles that stick out past the last row or column.  What a strip reads from memory is requested four rows
+  // ahead, the first four before it is staged (rows and columns outside read the last row or column 0 again); the
+  // loop over the rows is rolled.  With loads one row after another behind the stores of the row before, and the activation
+  // chosen per element, the epilogues of [3333, 6400] in SiLU cost more than their main loops.
+  // (a lane number of its own per strip: what is derived from it would otherwise be computed once, before the choice among the
+  // strips, and take registers from all of them)
+  auto strip_lane = []() __attribute__((always_inline)) {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+  };
+  auto general_strip = [&](auto I) __attribute__((always_inline)) {
     constexpr int i = decltype(I)::value;
-    stage_strip(I);
+    const int lane = strip_lane();
     const int64_t mrow0 = m0 + wm * WTM + i * 32;
-    if (pair) {
-      // columns [0, WTN/2) of the sub-tile are gate columns, [WTN/2, WTN) the matching linear columns
-      constexpr int LANES_PER_ROW = WTN / 2 / 8, ROWS_PER_IT = 64 / LANES_PER_ROW;
-      for (int it = 0; it < 32 / ROWS_PER_IT; it++) {
-        const int row = it * ROWS_PER_IT + lane / LANES_PER_ROW, c = (lane % LANES_PER_ROW) * 8;
-        const int64_t m = mrow0 + row;
-        float vg[8], vl[8];
-        const float* sg = staged(row, c);
-        const float* sl = staged(row, WTN / 2 + c);
+    auto read8 = [&](int row, int c, float (&v)[8]) {
+      const float* sv = staged(row, c);
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(sv), hi = *reinterpret_cast<const f32x4*>(sv + 4);
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-          vg[e] = sg[e];
-          vl[e] = sl[e];
-        }
+      for (int e = 0; e < 4; e++) {
+        v[e] = lo[e];
+        v[4 + e] = hi[e];
+      }
+    };
+    if (pair) {
+      if constexpr (KIND == EPI_ACT_FWD) {
+        // columns [0, WTN/2) of the sub-tile are gate columns, [WTN/2, WTN) the matching linear columns
+        constexpr int LANES_PER_ROW = WTN / 2 / 8, ROWS_PER_IT = 64 / LANES_PER_ROW;
+        const int c = (lane % LANES_PER_ROW) * 8;
         const int64_t n = n0 + wn * (WTN / 2) + c;
-        if (m < p.M && n < p.N) epi_act_fwd_gated8(epi, m, n, vg, vl);
+        stage_strip(I);
+#pragma unroll 1
+        for (int it = 0; it < 32 / ROWS_PER_IT; it++) {
+          const int row = it * ROWS_PER_IT + lane / LANES_PER_ROW;
+          float vg[8], vl[8];
+          read8(row, c, vg);
+          read8(row, WTN / 2 + c, vl);
+          if (mrow0 + row < p.M && n < p.N) epi_act_fwd_gated8<ACT>(epi, mrow0 + row, n, vg, vl);
+        }
       }
     } else {
       constexpr int LANES_PER_ROW = WTN / 8, ROWS_PER_IT = 64 / LANES_PER_ROW, NIT = 32 / ROWS_PER_IT;
       const int c = (lane % LANES_PER_ROW) * 8;
       const int64_t n = n0 + wn * WTN + c;
       const bool in_n = n < p.N;  // N is a multiple of 8: the lane's 8 columns are all inside or all outside
-      const int64_t mlane = mrow0 + lane / LANES_PER_ROW;  // this lane's row in iteration 0
-      // global reads of the epilogue run two iterations ahead of their use
-      EpiLoad l0 = epi_load8<KIND, TX>(epi, mlane, n, in_n && mlane < p.M);
-      EpiLoad l1 = epi_load8<KIND, TX>(epi, mlane + ROWS_PER_IT, n, in_n && mlane + ROWS_PER_IT < p.M);
+      constexpr int AHEAD = 4;  // rows of reads in flight
+      EpiLoad in[AHEAD];
+      auto request = [&](int it) __attribute__((always_inline)) {
+        return epi_load8<KIND, TX>(epi, min(mrow0 + it * ROWS_PER_IT + lane / LANES_PER_ROW, p.M - 1), in_n ? n : 0, true);
+      };
+      constexpr bool READS = KIND == EPI_ACT_BWD || KIND == EPI_OUT;
+      if constexpr (READS) {
+#pragma unroll
+        for (int it = 0; it < AHEAD; it++) in[it] = request(it);
+      }
+      stage_strip(I);
+#pragma unroll 1
       for (int it = 0; it < NIT; it++) {
         const int row = it * ROWS_PER_IT + lane / LANES_PER_ROW;
         const int64_t m = mrow0 + row;
-        const int64_t m2 = m + 2 * ROWS_PER_IT;
-        const EpiLoad l2 = epi_load8<KIND, TX>(epi, m2, n, in_n && it + 2 < NIT && m2 < p.M);
         float v[8];
-        const float* sv = staged(row, c);
-#pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = sv[e];
+        read8(row, c, v);
+        EpiLoad next;
+        if constexpr (READS) next = request(min(it + AHEAD, NIT - 1));
         if (in_n && m < p.M) {
           if constexpr (KIND == EPI_STORE) epi_store8(epi, m, n, v);
-          else if constexpr (KIND == EPI_ACT_FWD) epi_act_fwd8(epi, m, n, v);
-          else if constexpr (KIND == EPI_ACT_BWD) epi_act_bwd8_loaded(epi, m, n, v, l0, colsum);
-          else epi_out8_loaded<TX>(epi, m, n, v, l0);
+          else if constexpr (KIND == EPI_ACT_FWD) epi_act_fwd8<ACT>(epi, m, n, v);
+          else if constexpr (KIND == EPI_ACT_BWD) epi_act_bwd8_loaded<ACT>(epi, m, n, v, in[0], colsum);
+          else epi_out8_loaded<TX>(epi, m, n, v, in[0]);
         }
-        l0 = l1;
-        l1 = l2;
+        if constexpr (READS) {
+#pragma unroll
+          for (int k = 0; k + 1 < AHEAD; k++) in[k] = in[k + 1];  // (registers cannot be indexed)
+          in[AHEAD - 1] = next;
+        }
       }
     }
     __builtin_amdgcn_wave_barrier();
@@ -932,7 +962,7 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
 #pragma unroll
       for (int e = 0; e < 8; e++) v[it][e] = raw[it][e >> 2][e & 3];
   };
-  // EPI_ACT_BWD, the usual case (whole tile in range, tanh GELU, h wanted): straight-line strips.  The pre-activation reads
+  // EPI_ACT_BWD, the usual case (whole tile in range, tanh GELU or SiLU, h wanted): straight-line strips.  The pre-activation reads
   // of ACT_WINDOW rows are in flight at any time -- the first window goes out before the strip is staged -- and, with no
   // branches in between, each row waits only for its own reads.
   constexpr int ACT_WINDOW = 3;
@@ -951,12 +981,12 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
     read_staged_rows(std::integral_constant<int, NIT>{}, std::integral_constant<int, ROWS_PER_IT>{}, LANES_PER_ROW, c, v);
 #pragma unroll
     for (int it = 0; it < NIT; it++) {
-      epi_act_bwd8_gelu<GATED>(epi, mlane + it * ROWS_PER_IT, n, v[it], win[it % ACT_WINDOW], colsum);
+      epi_act_bwd8_fixed<GATED, ACT>(epi, mlane + it * ROWS_PER_IT, n, v[it], win[it % ACT_WINDOW], colsum);
       if (it + ACT_WINDOW < NIT) win[it % ACT_WINDOW] = epi_load_pre8<GATED>(epi, mlane + (it + ACT_WINDOW) * ROWS_PER_IT, n);
     }
     __builtin_amdgcn_wave_barrier();
   };
-  // The other kinds, same idea: whole tile in range, tanh GELU, no dropout, residual present.
+  // The other kinds, same idea: whole tile in range, tanh GELU or SiLU, no dropout, residual present.
   const bool whole_tile = m0 + tile_rows <= p.M && n0 + (gated ? tile_cols / 2 : tile_cols) <= p.N;
   auto act_fwd_strip = [&](auto I, auto G) {
     constexpr int i = decltype(I)::value;
@@ -971,7 +1001,7 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
     if constexpr (GATED)
       read_staged_rows(std::integral_constant<int, NIT>{}, std::integral_constant<int, ROWS_PER_IT>{}, LANES_PER_ROW, WTN / 2 + c, v1);
 #pragma unroll
-    for (int it = 0; it < NIT; it++) epi_act_fwd8_gelu<GATED>(epi, mlane + it * ROWS_PER_IT, n, v0[it], v1[GATED ? it : 0]);
+    for (int it = 0; it < NIT; it++) epi_act_fwd8_fixed<GATED, ACT>(epi, mlane + it * ROWS_PER_IT, n, v0[it], v1[GATED ? it : 0]);
     __builtin_amdgcn_wave_barrier();
   };
   auto store_strip = [&](auto I, auto out_type) {
@@ -1041,26 +1071,29 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
     if (epi.out_dtype == LT_F32) for_each_strip([&](auto I) { scatter_strip(I, float{}); });
     else for_each_strip([&](auto I) { scatter_strip(I, bf16{}); });
   } else if constexpr (KIND == EPI_ACT_BWD) {
-    const bool straight = whole_tile && epi.act == LT_ACT_GELU_FUSED && epi.hid != nullptr;
-    if (straight && epi.gated) for_each_strip([&](auto I) { act_bwd_strip(I, std::true_type{}); });
-    else if (straight) for_each_strip([&](auto I) { act_bwd_strip(I, std::false_type{}); });
-    else for_each_strip(generic_strip);
+    const bool straight = whole_tile && epi.hid != nullptr;
+    if constexpr (STRAIGHT_ACT) {
+      if (straight && epi.gated) for_each_strip([&](auto I) { act_bwd_strip(I, std::true_type{}); });
+      else if (straight) for_each_strip([&](auto I) { act_bwd_strip(I, std::false_type{}); });
+    }
+    if (!STRAIGHT_ACT || !straight) for_each_strip(general_strip);
   } else if constexpr (KIND == EPI_ACT_FWD) {
-    const bool straight = whole_tile && epi.act == LT_ACT_GELU_FUSED;
-    if (straight && pair) for_each_strip([&](auto I) { act_fwd_strip(I, std::true_type{}); });
-    else if (straight) for_each_strip([&](auto I) { act_fwd_strip(I, std::false_type{}); });
-    else for_each_strip(generic_strip);
+    if constexpr (STRAIGHT_ACT) {
+      if (whole_tile && pair) for_each_strip([&](auto I) { act_fwd_strip(I, std::true_type{}); });
+      else if (whole_tile) for_each_strip([&](auto I) { act_fwd_strip(I, std::false_type{}); });
+    }
+    if (!STRAIGHT_ACT || !whole_tile) for_each_strip(general_strip);
   } else if constexpr (KIND == EPI_STORE) {
     if (whole_tile && epi.out_dtype == LT_F32) for_each_strip([&](auto I) { store_strip(I, float{}); });
     else if (whole_tile) for_each_strip([&](auto I) { store_strip(I, bf16{}); });
-    else for_each_strip(generic_strip);
+    else for_each_strip(general_strip);
   } else {
     if (whole_tile && epi.x && epi.drop.p == 0.f) {
       for_each_strip([&](auto I) { out_strip(I, std::false_type{}); });
     } else if (whole_tile && epi.x) {
       for_each_strip([&](auto I) { out_strip(I, std::true_type{}); });
     } else {
-      for_each_strip(generic_strip);
+      for_each_strip(general_strip);
     }
   }
   if constexpr (KIND == EPI_ACT_BWD) {
@@ -1107,7 +1140,7 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
 //   ib_e) and so form one [256 rows][64 k] k-major matrix.  The list sits in one register (lane e: ib_e << 16 | flat
 //   position) and is read with v_readlane, so the k-loop issues no memory instruction for it.  A second k-segment (the
 //   low-rank term) is an ordinary one.
-template <bool A_KM, bool B_KM, int KIND, typename TX, int GATHER = 0>
+template <bool A_KM, bool B_KM, int KIND, typename TX, int GATHER = 0, int ACT = -1>
 __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem, int tiles_m, int tiles_n) {
   // A workgroup may loop over tiles.  Whatever the compiler finds to be the same in every tile -- values loaded from the problem
   // description, the wavefront's LDS addresses, lane offsets -- it would compute once and keep in registers across the whole
@@ -1586,7 +1619,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
                             : wave == 1 ? (A_KM ? a_d1 + KM_ELEMS / 2 : a_s3)
                             : wave == 2 ? (B_KM ? b_d1 : b_s2)
                                         : (B_KM ? b_d1 + KM_ELEMS / 2 : b_s3);
-    dma_tile_epilogue<FM, KIND, TX, BM, BN, GATHER == 1 ? 1 : GATHER == 3 ? 2 : 0>(acc, *(const GemmProblem*)pk, reinterpret_cast<float*>(stage_buf), epi_m0,
+    dma_tile_epilogue<FM, KIND, TX, BM, BN, GATHER == 1 ? 1 : GATHER == 3 ? 2 : 0, ACT>(acc, *(const GemmProblem*)pk, reinterpret_cast<float*>(stage_buf), epi_m0,
                                                           epi_n0, wm, wn, gated);
     LT_TILE_STAMP(3);
     LT_TILE_STAMP_REALTIME(5);
@@ -1621,6 +1654,18 @@ inline unsigned dma_grid(const GemmProblem& p, int tiles) {
   return (n > 0 && tiles > n) ? (unsigned)n : (unsigned)tiles;
 }
 
+// launch(std::integral_constant<int, ACT>) with the activation the kernel is compiled for: kinds in frequent use have an
+// instantiation each, the rest share one that chooses per element.  (One kernel that chose among them per tile ran out of
+// registers: accumulators in scratch memory.)  The epilogues without an activation have one.
+template <int KIND, typename F> void with_activation(const GemmProblem& p, F&& launch) {
+  if constexpr (KIND == EPI_ACT_FWD || KIND == EPI_ACT_BWD) {
+    if (p.epi.act == LT_ACT_GELU_FUSED) return launch(std::integral_constant<int, LT_ACT_GELU_FUSED>{});
+    if (p.epi.act == LT_ACT_SILU) return launch(std::integral_constant<int, LT_ACT_SILU>{});
+    if (p.epi.act == LT_ACT_GELU) return launch(std::integral_constant<int, LT_ACT_GELU>{});
+  }
+  launch(std::integral_constant<int, -1>{});
+}
+
 template <bool A_KM, bool B_KM, int KIND>
 int launch_dma(const GemmProblem& problem, int io_dtype, hipStream_t stream) {
   GemmProblem p = problem;
@@ -1644,7 +1689,10 @@ int launch_dma(const GemmProblem& problem, int io_dtype, hipStream_t stream) {
       return LT_OK;
     }
   }
-  hipLaunchKernelGGL((gemm_bf16_dma_kernel<A_KM, B_KM, KIND, float>), grid, block, 0, stream, p, tiles_m, tiles_n);
+  with_activation<KIND>(p, [&](auto ACT) {
+    hipLaunchKernelGGL((gemm_bf16_dma_kernel<A_KM, B_KM, KIND, float, 0, decltype(ACT)::value>), grid, block, 0, stream, p, tiles_m,
+                       tiles_n);
+  });
   LT_LAUNCH_CHECK();
   return LT_OK;
 }
@@ -1691,8 +1739,10 @@ template <int KIND> int launch_sparse(const GemmProblem& problem, int io_dtype, 
         q.K[0] = (int64_t)sp.blocks_per_out * 64;
         q.ksplit = 0; q.krot = 0;
         const int tiles_n = (int)(p.N / 256);
-        hipLaunchKernelGGL((gemm_bf16_dma_kernel<true, true, KIND, float, 2>), dim3(dma_grid(q, tiles_m * tiles_n)), block, 0,
-                           stream, q, tiles_m, tiles_n);
+        with_activation<KIND>(q, [&](auto ACT) {
+          hipLaunchKernelGGL((gemm_bf16_dma_kernel<true, true, KIND, float, 2, decltype(ACT)::value>),
+                             dim3(dma_grid(q, tiles_m * tiles_n)), block, 0, stream, q, tiles_m, tiles_n);
+        });
         LT_LAUNCH_CHECK();
         return LT_OK;
       }
@@ -1773,12 +1823,17 @@ template <bool A_KM, bool B_KM, int KIND> int launch_tile(const GemmProblem& p, 
   return launch_cfg<256, 256, 2, 2, A_KM, B_KM, KIND>(p, io_dtype, stream);
 }
 
+// The fused epilogues occur in one layout each: the projections' (both operands k-major) and, for EPI_ACT_BWD, the input gradient's
+// (B mn-major); lt_gemm_mfma_supported refuses the others.
 template <int KIND> int launch_layout(const GemmProblem& p, int io_dtype, hipStream_t stream) {
   const bool a_km = p.A[0].kmajor, b_km = p.B[0].kmajor;
-  if (a_km && b_km) return launch_tile<true, true, KIND>(p, io_dtype, stream);
-  if (a_km && !b_km) return launch_tile<true, false, KIND>(p, io_dtype, stream);
-  if (!a_km && !b_km) return launch_tile<false, false, KIND>(p, io_dtype, stream);
-  LT_FAIL(LT_ERR_UNSUPPORTED, "tiled bf16 gemm: layout A mn-major x B k-major is not instantiated");
+  if constexpr (KIND != EPI_ACT_BWD)
+    if (a_km && b_km) return launch_tile<true, true, KIND>(p, io_dtype, stream);
+  if constexpr (KIND == EPI_STORE || KIND == EPI_ACT_BWD)
+    if (a_km && !b_km) return launch_tile<true, false, KIND>(p, io_dtype, stream);
+  if constexpr (KIND == EPI_STORE)
+    if (!a_km && !b_km) return launch_tile<false, false, KIND>(p, io_dtype, stream);
+  LT_FAIL(LT_ERR_UNSUPPORTED, "tiled bf16 gemm: epilogue %d is not instantiated for this operand layout", KIND);
 }
 
 }  // namespace

@@ -181,19 +181,24 @@ __device__ __forceinline__ void epi_store8(const EpiParams& e, int64_t m, int64_
   else store8(reinterpret_cast<bf16*>(e.out) + m * e.ldo + n, v);
 }
 
+// ACT: activation kind fixed at compile time, or -1 for e.act
+template <int ACT = -1>
 __device__ __forceinline__ void epi_act_fwd8(const EpiParams& e, int64_t m, int64_t n, float (&v)[8]) {
+  const int act = ACT >= 0 ? ACT : e.act;
   add_bias8(e.bias, n, v);
   float h[8];
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     v[i] = to_f32((bf16)v[i]);  // the activation sees the stored (rounded) pre-activation, as backward will
-    h[i] = act_value<false>(e.act, v[i]);
+    h[i] = act_value<false>(act, v[i]);
   }
   store8(reinterpret_cast<bf16*>(e.pre) + m * e.ld_pre + n, v);
   store8(reinterpret_cast<bf16*>(e.hid) + m * e.ld_hid + n, h);
 }
 
+template <int ACT = -1>
 __device__ __forceinline__ void epi_act_fwd_gated8(const EpiParams& e, int64_t m, int64_t n, float (&vg)[8], float (&vl)[8]) {
+  const int act = ACT >= 0 ? ACT : e.act;
   add_bias8(e.bias, n, vg);
   add_bias8(e.bias, e.inter + n, vl);
   float h[8];
@@ -201,7 +206,7 @@ __device__ __forceinline__ void epi_act_fwd_gated8(const EpiParams& e, int64_t m
   for (int i = 0; i < 8; i++) {
     vg[i] = to_f32((bf16)vg[i]);
     vl[i] = to_f32((bf16)vl[i]);
-    h[i] = act_value<false>(e.act, vg[i]) * vl[i];
+    h[i] = act_value<false>(act, vg[i]) * vl[i];
   }
   bf16* pre = reinterpret_cast<bf16*>(e.pre) + m * e.ld_pre + n;
   store8(pre, vg);
@@ -295,13 +300,15 @@ __device__ __forceinline__ void unpack_bf16x8(const lt_u32x4& raw, float (&v)[8]
 }
 
 // cs: running column sums of the 8 gate-side (and, gated, 8 linear-side at cs + 8) dpre values this lane has written
+template <int ACT = -1>
 __device__ __forceinline__ void epi_act_bwd8_loaded(const EpiParams& e, int64_t m, int64_t n, const float (&dh)[8],
                                                     const EpiLoad& l, float (&cs)[16]) {
+  const int act = ACT >= 0 ? ACT : e.act;
   bf16* dpre = reinterpret_cast<bf16*>(e.dpre) + m * e.ld_pre + n;
   float pg[8], a[8], da[8], o[8];
   unpack_bf16x8(l.a, pg);
 #pragma unroll
-  for (int i = 0; i < 8; i++) act_eval<false>(e.act, pg[i], a[i], da[i]);
+  for (int i = 0; i < 8; i++) act_eval<false>(act, pg[i], a[i], da[i]);
   if (e.gated) {
     float pl[8];
     unpack_bf16x8(l.b, pl);
@@ -330,14 +337,14 @@ __device__ __forceinline__ void epi_act_bwd8_loaded(const EpiParams& e, int64_t 
 // Straight-line epilogue bodies for the usual cases (whole tile in range, bias present, no dropout): the run-time choices of
 // the general functions above are made once per tile by the caller, not once per row; bias values of a lane's 8 columns
 // are loaded once per tile and passed in.
-// forward activation with the tanh GELU fixed (bias already in the accumulators)
-template <bool GATED>
-__device__ __forceinline__ void epi_act_fwd8_gelu(const EpiParams& e, int64_t m, int64_t n, float (&vg)[8], float (&vl)[8]) {
+// forward activation with its kind fixed (bias already in the accumulators)
+template <bool GATED, int ACT>
+__device__ __forceinline__ void epi_act_fwd8_fixed(const EpiParams& e, int64_t m, int64_t n, float (&vg)[8], float (&vl)[8]) {
   float h[8];
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     vg[i] = to_f32((bf16)vg[i]);  // the activation sees the stored (rounded) pre-activation, as backward will
-    h[i] = act_value<false>(LT_ACT_GELU_FUSED, vg[i]);
+    h[i] = act_value<false>(ACT, vg[i]);
     if constexpr (GATED) {
       vl[i] = to_f32((bf16)vl[i]);
       h[i] *= vl[i];
@@ -392,7 +399,7 @@ __device__ __forceinline__ void epi_out8_residual(const EpiParams& e, int64_t m,
   store8(reinterpret_cast<TX*>(e.y) + m * e.ldy + n, v);
 }
 
-// EPI_ACT_BWD without run-time choices -- tanh-approximated GELU, gating fixed at compile time, h always written, rows known to
+// EPI_ACT_BWD without run-time choices -- activation and gating fixed at compile time, h always written, rows known to
 // be in range: straight-line code, so the compiler can count exactly which of the reads in flight a row waits for
 template <bool GATED> __device__ __forceinline__ EpiLoad epi_load_pre8(const EpiParams& e, int64_t m, int64_t n) {
   EpiLoad l;
@@ -403,14 +410,14 @@ template <bool GATED> __device__ __forceinline__ EpiLoad epi_load_pre8(const Epi
   return l;
 }
 
-template <bool GATED>
-__device__ __forceinline__ void epi_act_bwd8_gelu(const EpiParams& e, int64_t m, int64_t n, const float (&dh)[8],
-                                                  const EpiLoad& l, float (&cs)[16]) {
+template <bool GATED, int ACT>
+__device__ __forceinline__ void epi_act_bwd8_fixed(const EpiParams& e, int64_t m, int64_t n, const float (&dh)[8],
+                                                   const EpiLoad& l, float (&cs)[16]) {
   bf16* dpre = reinterpret_cast<bf16*>(e.dpre) + m * e.ld_pre + n;
   float pg[8], a[8], da[8], o[8];
   unpack_bf16x8(l.a, pg);
 #pragma unroll
-  for (int i = 0; i < 8; i++) act_eval<false>(LT_ACT_GELU_FUSED, pg[i], a[i], da[i]);
+  for (int i = 0; i < 8; i++) act_eval<false>(ACT, pg[i], a[i], da[i]);
   if constexpr (GATED) {
     float pl[8];
     unpack_bf16x8(l.b, pl);

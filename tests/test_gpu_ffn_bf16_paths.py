@@ -39,8 +39,8 @@ OTHER_ACTS = [(a, g, t) for a in ("gelu", "relu", "silu") for g in (False, True)
 
 @pytest.mark.parametrize("act,gated,tokens", OTHER_ACTS)
 def test_bf16_other_activations_take_the_general_epilogue_strips(act, gated, tokens):
-    """the straight-line strips are compiled for the tanh GELU; every other activation goes through the strips that choose
-    per row (forward activation epilogue, backward d-activation epilogue with its fused column sums).  Every closed-form
+    """the straight-line strips are compiled for the tanh GELU and SiLU; every other activation goes through the general strips
+    (forward activation epilogue, backward d-activation epilogue with its fused column sums).  Every closed-form
     entry of the Hugging Face table has a row.  The derivative of relu (and of relu6, leaky_relu, hardswish)
     jumps at 0, so its gradients depend on the sign of the pre-activation as stored (bf16): the oracle is asked to round
     where the bf16 path stores (LayerNorm output, pre-activation, activation output), which is what the reference does
