@@ -150,6 +150,7 @@ size_t lt_gemm_generic_splitk_workspace(int64_t M, int64_t N, int64_t K) {
 
 int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
                           hipStream_t stream) {
+  if (lt_gemm_stream_supported(p, EPI_STORE, dtype, io_dtype)) return lt_launch_gemm_stream(p, EPI_STORE, dtype, io_dtype, stream);
   const bool a_km = p.A[0].kmajor, b_km = p.B[0].kmajor;
   const EpiParams& e = p.epi;
   bool ok = dtype == LT_BF16 && p.nseg == 1 && p.sp.mode == SPARSE_NONE && p.M > 0 && p.N > 0 && p.N % 128 == 0 &&
@@ -251,6 +252,7 @@ size_t lt_gemm_out_splitk_workspace(int64_t M, int64_t N, int64_t K, size_t cap_
 int lt_launch_gemm_out(const GemmProblem& p, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
                        hipStream_t stream) {
   const EpiParams& e = p.epi;
+  if (lt_gemm_stream_supported(p, EPI_OUT, dtype, io_dtype)) return lt_launch_gemm_stream(p, EPI_OUT, dtype, io_dtype, stream);
   if (p.nseg == 1 && p.sp.mode == SPARSE_NONE && workspace && lt_aligned(workspace, 16) && p.M > 0 && p.N > 0 &&
       p.N % 8 == 0 && e.ldy % 8 == 0 && lt_aligned(e.y, 16) && (!e.x || lt_aligned(e.x, 16)) &&
       (!e.bias || lt_aligned(e.bias, 16))) {
@@ -376,6 +378,7 @@ int lt_launch_gemm_sparse(const GemmProblem& p, int kind, int dtype, int io_dtyp
 }
 
 int lt_launch_gemm(const GemmProblem& p, int kind, int dtype, int io_dtype, hipStream_t stream) {
+  if (lt_gemm_stream_supported(p, kind, dtype, io_dtype)) return lt_launch_gemm_stream(p, kind, dtype, io_dtype, stream);
   if (dtype == LT_BF16 && lt_gemm_mfma_supported(p, kind)) return lt_launch_gemm_mfma(p, kind, io_dtype, stream);
   return lt_launch_gemm_generic(p, kind, dtype, io_dtype, stream);
 }

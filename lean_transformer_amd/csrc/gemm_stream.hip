@@ -1,0 +1,258 @@
+// Products of up to 64 rows with a weight matrix (token-by-token generation):  C[m, n] = sum_k A[m, k] W[n, k], both operands k-major,
+// fp32 or 16-bit, with the forward epilogues fused.
+//
+// What bounds it: the weights, which are read once (403 MB per token at hidden 4096, gated: 70 us at 5.8 TB/s); a 256 x 256 tile
+// spends all its time on a few rows, and leaves most CUs without a tile (hidden 4096, one token: 220 us for the block; 101 now, its two
+// products 53 and 31 us = 5.1 and 4.4 TB/s).  So the reduction
+// is split over the wavefronts of a workgroup: a workgroup owns 16 NT rows of W (gated up-projection: half of them gate rows, half
+// the matching linear rows), wavefront w takes the 128-byte k-blocks w, w + W, ... of all of them, and the partial sums meet in
+// LDS at the end, in wavefront order, so that a result is the same at every run.  A block is fetched 128 contiguous bytes per 8 lanes
+// into registers, DEPTH blocks ahead, and goes through a buffer in LDS that belongs to the wavefront alone (no barrier in the loop)
+// into the layout of v_mfma_f32_16x16x32 (fp32: v_mfma_f32_16x16x4, plain fp32 arithmetic), W as the first operand, so that a
+// lane ends up with 4 consecutive columns of one row.  Blocks past the end of the reduction arrive as zeros.
+#include <algorithm>
+
+#include "lt_gemm.h"
+
+namespace {
+
+template <typename TI> struct StreamMfma {  // 16-bit
+  static __device__ __forceinline__ f32x4 run(const lt_u32x4& a, const lt_u32x4& b, f32x4 c) {
+    return LT_MFMA_16X16X32(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c);
+  }
+};
+template <> struct StreamMfma<float> {
+  static __device__ __forceinline__ f32x4 run(const lt_u32x4& a, const lt_u32x4& b, f32x4 c) {
+    const f32x4 fa = __builtin_bit_cast(f32x4, a), fb = __builtin_bit_cast(f32x4, b);
+#pragma unroll
+    for (int e = 0; e < 4; e++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], fb[e], c, 0, 0, 0);
+    return c;
+  }
+};
+
+// MT: 16-row tiles of A (M <= 16 MT), NT: 16-row tiles of W per workgroup, WAVES: wavefronts per workgroup
+template <typename TI, int KIND, typename TX, int MT, int NT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void gemm_stream_kernel(GemmProblem p) {
+  constexpr int TILES = NT + MT, LOADS = 2 * TILES;      // per block and wavefront, 1 KiB each
+  constexpr int DEPTH = LOADS <= 10 ? 3 : 2;             // blocks in flight (registers)
+  constexpr int STAGE = TILES * 16 * 8;                  // 16-byte words: TILES * 16 rows of 128 bytes
+  constexpr int PAIRS = NT * MT;                         // 16 x 16 results
+  static_assert(PAIRS * 64 <= STAGE, "the partial sums take the place of the staged blocks");
+  __shared__ lt_u32x4 smem[WAVES * STAGE];
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const bool gated = KIND == EPI_ACT_FWD && p.epi.gated;
+  const int M = (int)p.M;
+  const int64_t N = p.N;  // gated: gate columns
+  const int own = gated ? NT / 2 : NT;  // tiles of output columns
+  const int64_t n0 = (int64_t)blockIdx.x * own * 16;
+
+  // 16-byte piece j of a block: row j * 8 + lane / 8 of [W tiles, A tiles], piece lane % 8 of its 128 bytes.  Rows past the last one
+  // read the last one again; they only feed results that are not stored.
+  const int row_in = lane >> 3;
+  const uint32_t k_bytes = (uint32_t)(p.K[0] * sizeof(TI));
+  const char* const w_base = reinterpret_cast<const char*>(p.B[0].ptr) + n0 * p.B[0].ld * (int64_t)sizeof(TI);
+  const char* const w_base2 = w_base + (gated ? N * p.B[0].ld * (int64_t)sizeof(TI) : 0);  // the linear half
+  const char* const a_base = reinterpret_cast<const char*>(p.A[0].ptr);
+  uint32_t off[LOADS];
+#pragma unroll
+  for (int j = 0; j < LOADS; j++) {
+    if (j < 2 * NT) {
+      const int tile = j >> 1, t = gated && tile >= NT / 2 ? tile - NT / 2 : tile;
+      const int64_t n = min(n0 + t * 16 + (j & 1) * 8 + row_in, N - 1) - n0;
+      off[j] = (uint32_t)(n * p.B[0].ld * (int64_t)sizeof(TI));
+    } else {
+      off[j] = (uint32_t)(min((j - 2 * NT) * 8 + row_in, M - 1) * p.A[0].ld * (int64_t)sizeof(TI));
+    }
+  }
+  const uint32_t my_k = (uint32_t)(lane & 7) * 16;
+  auto fetch = [&](uint32_t block, lt_u32x4 (&r)[LOADS]) __attribute__((always_inline)) {
+    const uint32_t k = min(block * 128 + my_k, k_bytes - 16);
+#pragma unroll
+    for (int j = 0; j < LOADS; j++) {
+      const char* base = j >= 2 * NT ? a_base : (NT > 1 && j >= NT) ? w_base2 : w_base;
+      r[j] = *reinterpret_cast<const lt_u32x4*>(base + (size_t)(off[j] + k));
+    }
+  };
+
+  f32x4 acc[NT][MT];
+#pragma unroll
+  for (int i = 0; i < NT; i++)
+#pragma unroll
+    for (int j = 0; j < MT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  lt_u32x4* const stage = smem + wave * STAGE;
+  // row r keeps its 16-byte piece c in slot c ^ (r / 2) % 8: the 16 rows a quarter of the wavefront reads cover all 64 banks
+  auto slot = [](int r, int c) { return r * 8 + (c ^ ((r >> 1) & 7)); };
+  auto consume = [&](uint32_t block, const lt_u32x4 (&r)[LOADS]) __attribute__((always_inline)) {
+    const bool inside = block * 128 + my_k < k_bytes;
+#pragma unroll
+    for (int j = 0; j < LOADS; j++) {
+      lt_u32x4 v = r[j];
+#pragma unroll
+      for (int e = 0; e < 4; e++) v[e] = inside ? v[e] : 0u;
+      stage[slot(j * 8 + row_in, lane & 7)] = v;
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const int c = (lane >> 4) + 4 * s;
+      lt_u32x4 w[NT], a[MT];
+#pragma unroll
+      for (int i = 0; i < NT; i++) w[i] = stage[slot(i * 16 + (lane & 15), c)];
+#pragma unroll
+      for (int j = 0; j < MT; j++) a[j] = stage[slot((NT + j) * 16 + (lane & 15), c)];
+#pragma unroll
+      for (int i = 0; i < NT; i++)
+#pragma unroll
+        for (int j = 0; j < MT; j++) acc[i][j] = StreamMfma<TI>::run(w[i], a[j], acc[i][j]);
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+
+  lt_u32x4 regs[DEPTH][LOADS];
+  const uint32_t blocks = (k_bytes + 127) / 128;
+#pragma unroll
+  for (int d = 0; d < DEPTH; d++) fetch(wave + d * WAVES, regs[d]);
+  for (uint32_t b = wave; b < blocks; b += DEPTH * WAVES) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) {
+      consume(b + d * WAVES, regs[d]);
+      fetch(b + (d + DEPTH) * WAVES, regs[d]);
+    }
+  }
+
+  // ---- partial sums of the wavefronts, then the epilogue: lane = row lane % 16 of A's tile, columns 4 (lane / 16) .. + 3 of W's
+  __syncthreads();
+  f32x4* const sums = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+  for (int i = 0; i < NT; i++)
+#pragma unroll
+    for (int j = 0; j < MT; j++) sums[(wave * PAIRS + i * MT + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  auto total = [&](int pair, float (&v)[4]) __attribute__((always_inline)) {
+    f32x4 t = sums[pair * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < WAVES; w++) t += sums[(w * PAIRS + pair) * 64 + lane];
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = t[e];
+  };
+  constexpr bool PRECISE = sizeof(TI) == 4;
+  const EpiParams& e = p.epi;
+  for (int q = wave; q < own * MT; q += WAVES) {
+    const int64_t m = (q % MT) * 16 + (lane & 15), n = n0 + (q / MT) * 16 + (lane >> 4) * 4;
+    if (m >= M || n >= N) continue;  // (N is a multiple of 4)
+    float v[4], bias[4] = {0.f, 0.f, 0.f, 0.f};
+    total(q, v);
+    if (e.bias) load4(e.bias + n, bias);
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] += bias[i];
+    if constexpr (KIND == EPI_STORE) {
+      if (e.out_dtype == LT_F32) store4(reinterpret_cast<float*>(e.out) + m * e.ldo + n, v);
+      else store4(reinterpret_cast<bf16*>(e.out) + m * e.ldo + n, v);
+    } else if constexpr (KIND == EPI_ACT_FWD) {
+      TI* pre = reinterpret_cast<TI*>(e.pre) + m * e.ld_pre + n;
+      float h[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        v[i] = to_f32(from_f32<TI>(v[i]));  // the activation sees the stored (rounded) pre-activation, as backward will
+        h[i] = act_value<PRECISE>(e.act, v[i]);
+      }
+      store4(pre, v);
+      if (gated) {
+        float l[4], lb[4] = {0.f, 0.f, 0.f, 0.f};
+        total(q + own * MT, l);
+        if (e.bias) load4(e.bias + e.inter + n, lb);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          l[i] = to_f32(from_f32<TI>(l[i] + lb[i]));
+          h[i] *= l[i];
+        }
+        store4(pre + e.inter, l);
+      }
+      store4(reinterpret_cast<TI*>(e.hid) + m * e.ld_hid + n, h);
+    } else {
+      const int64_t idx = m * e.ldy + n;
+      if (e.drop.p > 0.f) {
+        bool keep[4];
+        dropout_keep4(e.drop, idx, keep);
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = keep[i] ? v[i] * e.drop.scale : 0.f;
+      }
+      if (e.x) {
+        float r[4];
+        load4(reinterpret_cast<const TX*>(e.x) + idx, r);
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] += r[i];
+      }
+      store4(reinterpret_cast<TX*>(e.y) + idx, v);
+    }
+  }
+}
+
+template <typename TI, int KIND, typename TX, int MT, int NT, int WAVES>
+int launch(const GemmProblem& p, bool gated, hipStream_t stream) {
+  const int64_t cols = 16 * (gated ? NT / 2 : NT);
+  hipLaunchKernelGGL((gemm_stream_kernel<TI, KIND, TX, MT, NT, WAVES>), dim3((unsigned)((p.N + cols - 1) / cols)), dim3(64 * WAVES), 0,
+                     stream, p);
+  LT_LAUNCH_CHECK();
+  return LT_OK;
+}
+
+// Workgroup shape.  Many rows of W: four tiles of them per workgroup, which reads A once for 64 of them ([1, 4096] x [32768, 4096]:
+// 52.8 us = 5.1 TB/s, two tiles 61.3).  Few: one tile, and more wavefronts share its reduction ([24, 16384] x [4096, 16384]: 35.6 us
+// against 39.5 with two tiles, [48, 6400] x [1600, 6400]: 15.3 against 18.3).  Between: two, eight wavefronts ([24, 2048] x [8192,
+// 2048]: 8.7 us, 13.6 with one tile; [48, 2048]: 11.6, 18.8).
+template <typename TI, int KIND, typename TX> int launch_shape(const GemmProblem& p, hipStream_t stream) {
+  const bool gated = KIND == EPI_ACT_FWD && p.epi.gated;
+  const int64_t rows = gated ? 2 * p.N : p.N;
+  const bool many = rows >= 512 * 64, few = rows <= 4096 && !gated;  // (a gated workgroup pairs two tiles)
+  if (p.M <= 16) {
+    if (many) return launch<TI, KIND, TX, 1, 4, 4>(p, gated, stream);
+    if (few) return launch<TI, KIND, TX, 1, 1, 16>(p, gated, stream);
+    return launch<TI, KIND, TX, 1, 2, 8>(p, gated, stream);
+  }
+  if (p.M <= 32) {
+    if (many) return launch<TI, KIND, TX, 2, 4, 4>(p, gated, stream);
+    if (few) return launch<TI, KIND, TX, 2, 1, 16>(p, gated, stream);
+    return launch<TI, KIND, TX, 2, 2, 8>(p, gated, stream);
+  }
+  if (many) return launch<TI, KIND, TX, 4, 4, 4>(p, gated, stream);
+  if (few) return launch<TI, KIND, TX, 4, 1, 8>(p, gated, stream);
+  return launch<TI, KIND, TX, 4, 2, 8>(p, gated, stream);
+}
+
+template <typename TI> int launch_kind(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream) {
+  if (kind == EPI_STORE) return launch_shape<TI, EPI_STORE, float>(p, stream);
+  if (kind == EPI_ACT_FWD) return launch_shape<TI, EPI_ACT_FWD, float>(p, stream);
+  if constexpr (sizeof(TI) == 2)
+    if (io_dtype == LT_BF16) return launch_shape<TI, EPI_OUT, bf16>(p, stream);
+  return launch_shape<TI, EPI_OUT, float>(p, stream);
+}
+
+}  // namespace
+
+bool lt_gemm_stream_supported(const GemmProblem& p, int kind, int dtype, int io_dtype) {
+  const EpiParams& e = p.epi;
+  const int64_t piece = dtype == LT_F32 ? 4 : 8, bytes = dtype == LT_F32 ? 4 : 2;  // elements per 16 bytes
+  if (p.sp.mode != SPARSE_NONE || p.nseg != 1 || p.ksplit > 1 || p.variant || kind == EPI_ACT_BWD) return false;
+  if (p.M < 1 || p.M > 64 || p.N < 1 || p.K[0] < 1 || !p.A[0].kmajor || !p.B[0].kmajor) return false;
+  if (dtype == LT_F32 && kind == EPI_OUT && io_dtype != LT_F32) return false;
+  // 16-byte pieces of every row, 4 columns per store
+  if (p.N % 4 || p.K[0] % piece || p.A[0].ld % piece || p.B[0].ld % piece || !lt_aligned(p.A[0].ptr, 16) || !lt_aligned(p.B[0].ptr, 16))
+    return false;
+  // 32-bit byte offsets inside a workgroup's rows and along k (which runs up to 3 x 16 x 128 bytes past the end)
+  if (64 * std::max(p.A[0].ld, p.B[0].ld) * bytes >= (int64_t)1 << 31) return false;
+  if ((p.N + 7) / 8 > 0x7fffffff) return false;
+  if (e.bias && !lt_aligned(e.bias, 16)) return false;
+  if (kind == EPI_STORE) return e.ldo % 4 == 0 && lt_aligned(e.out, 16);
+  if (kind == EPI_ACT_FWD)
+    return e.ld_pre % 4 == 0 && e.ld_hid % 4 == 0 && e.inter % 4 == 0 && (!e.gated || e.inter == p.N) && e.hid &&
+           lt_aligned(e.pre, 16) && lt_aligned(e.hid, 16);
+  return e.ldy % 4 == 0 && lt_aligned(e.y, 16) && (!e.x || lt_aligned(e.x, 16));
+}
+
+int lt_launch_gemm_stream(const GemmProblem& p, int kind, int dtype, int io_dtype, hipStream_t stream) {
+  LT_REQUIRE(lt_gemm_stream_supported(p, kind, dtype, io_dtype), LT_ERR_UNSUPPORTED, "streaming gemm does not take this problem");
+  LtProfileScope scope("gemm_stream", lt_gemm_flops(p, kind), 0.0, stream);
+  return dtype == LT_F32 ? launch_kind<float>(p, kind, io_dtype, stream) : launch_kind<bf16>(p, kind, io_dtype, stream);
+}

@@ -16,10 +16,12 @@ typedef _Float16 bf16;
 #define LT_BF16 LT_F16
 #define LT_HALF_NAME "fp16"
 #define LT_MFMA_32X32X16(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0)
+#define LT_MFMA_16X16X32(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0)
 #else
 typedef __bf16 bf16;
 #define LT_HALF_NAME "bf16"
 #define LT_MFMA_32X32X16(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0)
+#define LT_MFMA_16X16X32(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0)
 #endif
 typedef __attribute__((__vector_size__(8 * sizeof(bf16)))) bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(short)))) short s16x4;
@@ -150,6 +152,7 @@ __device__ __forceinline__ float wave_sum(float v) {
 // ---------------------------------------------------------------------------------------------------------------------
 // activations and their derivatives, evaluated in fp32 registers.  PRECISE selects libm-grade tanh/exp for the fp32 path;
 // the bf16 path uses the hardware exp2 / reciprocal approximations (error far below one bf16 ulp).
+// gelu_fused follows lean_transformer/utils.py:24-38, including its truncated constants.
 // ---------------------------------------------------------------------------------------------------------------------
 // 1 / x in one instruction (v_rcp_f32, 1 ulp; 0 for infinity).  __fdividef is a full division here: ten instructions, which
 // were a third of an activation epilogue's arithmetic.

@@ -482,6 +482,9 @@ int lt_launch_gemm_generic(const GemmProblem& p, int kind, int dtype, int io_dty
 // true when the tiled bf16 kernel handles this problem (operand layouts, alignment, tile divisibility)
 bool lt_gemm_mfma_supported(const GemmProblem& p, int kind);
 int lt_launch_gemm_mfma(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream);
+// up to 64 rows against a k-major weight matrix, forward epilogues (gemm_stream.hip)
+bool lt_gemm_stream_supported(const GemmProblem& p, int kind, int dtype, int io_dtype);
+int lt_launch_gemm_stream(const GemmProblem& p, int kind, int dtype, int io_dtype, hipStream_t stream);
 // algorithmic flops of a dense problem: 2 * M * N * (K0 + K1)
 double lt_gemm_flops(const GemmProblem& p, int kind);
 // block-sparse walk: matrix-core kernel for 64 x 64 bf16 blocks, else the any-shape kernel
