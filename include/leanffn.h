@@ -230,7 +230,8 @@ int lt_dropout_mask(int64_t tokens, int32_t hidden, float p, uint64_t seed, uint
 /* ---- plain GEMM on the library's kernels (tests and benchmarks of the MFMA core) -------------------------------------- */
 /* C[M,N] = op(A) op(B): a_kmajor != 0: A is [M,K] row-major, else [K,M]; b_kmajor != 0: B is [N,K] row-major, else [K,N].
  * force_generic (low 4 bits): 0 the library's own choice; 1 the any-shape kernel even when a tiled bf16 kernel applies;
- * 2 the register-staged tiled kernel instead of the copy-based one.  Bits 4..7, when non-zero, choose how workgroups stagger
+ * 2 the register-staged tiled kernel instead of the copy-based one; 3 the copy-based kernel of 256 x 256 tiles where that of
+ * 128 x 128 tiles or the streaming kernel of few rows would be taken.  Bits 4..7, when non-zero, choose how workgroups stagger
  * their walk over k in the copy-based kernel (15: not at all) instead of the default for the layout.  Bit 8: one workgroup
  * per tile in the copy-based kernel even when there are more tiles than compute units (by default one workgroup per compute
  * unit then loops over its tiles; both give the same bits).  The choice travels with the call (no process-wide state): lt_gemm

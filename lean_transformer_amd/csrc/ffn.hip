@@ -238,8 +238,10 @@ void plan_linear_backward(const lt_linear& lin, int64_t T, int dtype, Bump& ws, 
   if (lin.block == 0) {  // dW (and dx) of a small dense layer: the reduction is split across workgroups
     s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_splitk_workspace(lin.out_features, lin.in_features, T));
     s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_generic_splitk_workspace(lin.out_features, lin.in_features, T));
-    if (lin.lowrank == 0)
+    if (lin.lowrank == 0) {
       s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_generic_splitk_workspace(T, lin.in_features, lin.out_features));
+      if (dtype == LT_BF16) s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_mid_splitk_workspace(T, lin.in_features, lin.out_features));
+    }
   }
   if (lin.block == 64 && dtype == LT_BF16)
     s.skinny_bytes = std::max(s.skinny_bytes,
@@ -385,9 +387,9 @@ void plan_forward(const lt_ffn_desc& d, Bump& ws, FwdScratch& s) {
   s.hid = ws.take((size_t)d.tokens * d.intermediate * e);
   const int r = d.i2h.lowrank > d.h2o.lowrank ? d.i2h.lowrank : d.h2o.lowrank;
   s.skinny_bytes = r > 0 ? lt_gemm_skinny_workspace(d.tokens, r) : 0;
-  // dense down-projection of a short batch: room to split its reduction, no more than the saved pre-activation takes
+  // dense down-projection of a short batch: room to split its reduction, no more than the saved pre-activation takes or 32 MiB
   if (d.h2o.block == 0 && d.h2o.lowrank == 0 && !d.post_ln_weight) {
-    const size_t cap = (size_t)d.tokens * (d.gated ? 2 : 1) * d.intermediate * e;
+    const size_t cap = std::max((size_t)d.tokens * (d.gated ? 2 : 1) * d.intermediate * e, (size_t)32 << 20);
     s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_out_splitk_workspace(d.tokens, d.hidden, d.intermediate, cap));
   }
   s.skinny = s.skinny_bytes ? ws.take(s.skinny_bytes) : nullptr;
@@ -704,6 +706,6 @@ extern "C" int lt_gemm(int32_t dtype, int64_t m, int64_t n, int64_t k, const voi
   p.tile_loop = (force_generic >> 8) & 1;
   force_generic &= 15;
   if (force_generic == 1) return lt_launch_gemm_generic(p, EPI_STORE, dtype, dtype, (hipStream_t)stream);
-  p.variant = force_generic == 2 ? 1 : 0;  // 2: the register-staged tiled kernel instead of the copy-based one
+  p.variant = force_generic == 2 ? 1 : force_generic == 3 ? 2 : 0;
   return lt_launch_gemm(p, EPI_STORE, dtype, dtype, (hipStream_t)stream);
 }

@@ -54,8 +54,40 @@ bool lt_gemm_mfma_supported(const GemmProblem& p, int kind) {
 
 bool lt_sparse_mfma_supported(const GemmProblem& p, int kind);
 
+namespace {
+int64_t mid_tiles(int64_t M, int64_t N) { return ((M + 127) / 128) * ((N + 127) / 128); }
+// 128 x 128 tiles where they all run at once, two workgroups per CU; 256 x 256 ones then fill half of the chip at most.  [1024, 8192]
+// over 2048 (512 of them): 37 us against 47; [1536, 6400] over 1600 (600): 51 against 44.
+bool mid_selected(const GemmProblem& p, int kind) {
+  const int64_t columns = kind == EPI_ACT_FWD && p.epi.gated ? 2 * p.N : p.N;
+  return mid_tiles(p.M, columns) <= 512 && lt_gemm_mid_supported(p, kind);
+}
+// Slices of such a product's reduction: the least estimated time.  64 k take a workgroup 0.45 us alone on its CU, two of them 0.95 us
+// (measured on [128 - 4096, 2048] over 8192: 53 - 69 us for up to 256 workgroups, 125 for 512); a slice costs a write and a read of
+// its fp32 partial result at 5 TB/s, the sum a launch.
+int mid_slices(int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = mid_tiles(M, N), stages = (K + 63) / 64;
+  int best = 1;
+  double best_us = 1e30;
+  for (int s = 1; s <= 16 && (s == 1 || (tiles * s <= 512 && stages / s >= 4)); s++) {
+    const double us = (double)((stages + s - 1) / s) * (tiles * s <= 256 ? 0.45 : 0.95) + (s > 1 ? s * (double)M * N * 8.0 / 5e6 + 4.0 : 0.0);
+    if (us < best_us * 0.97) {
+      best_us = us;
+      best = s;
+    }
+  }
+  return best;
+}
+}  // namespace
+
+size_t lt_gemm_mid_splitk_workspace(int64_t M, int64_t N, int64_t K) {
+  const int slices = mid_tiles(M, N) <= 512 ? mid_slices(M, N, K) : 1;
+  return slices > 1 ? lt_align_up((size_t)slices * (size_t)M * (size_t)N * sizeof(float), 256) : 0;
+}
+
 int lt_gemm_colsum_rows(const GemmProblem& p, int dtype, int io_dtype) {
   if (dtype != LT_BF16 || p.epi.ld_pre % 8 != 0) return 0;
+  if (mid_selected(p, EPI_ACT_BWD)) return 64;
   if (p.sp.mode == SPARSE_NONE)
     return lt_gemm_mfma_supported(p, EPI_ACT_BWD) && dma_selected(p, EPI_ACT_BWD) ? 128 : 0;
   // the walk's straight-line strips keep the sums: every tile must take them
@@ -82,6 +114,7 @@ double lt_gemm_flops(const GemmProblem& p, int kind) {
 int lt_launch_gemm_mfma(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream) {
   LT_REQUIRE(lt_gemm_mfma_supported(p, kind), LT_ERR_UNSUPPORTED, "tiled bf16 gemm does not take this problem");
   LtProfileScope scope(mfma_tag(p, kind), lt_gemm_flops(p, kind), 0.0, stream);
+  if (mid_selected(p, kind)) return lt_launch_gemm_mid(p, kind, io_dtype, stream);
   switch (kind) {
     case EPI_STORE: return lt_mfma_launch_dense_kind0(p, io_dtype, stream);
     case EPI_ACT_FWD: return lt_mfma_launch_dense_kind1(p, io_dtype, stream);
@@ -153,6 +186,20 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
   if (lt_gemm_stream_supported(p, EPI_STORE, dtype, io_dtype)) return lt_launch_gemm_stream(p, EPI_STORE, dtype, io_dtype, stream);
   const bool a_km = p.A[0].kmajor, b_km = p.B[0].kmajor;
   const EpiParams& e = p.epi;
+  if (dtype == LT_BF16 && mid_selected(p, EPI_STORE) && e.ldo == p.N) {
+    const size_t slice = (size_t)p.M * (size_t)p.N * sizeof(float);
+    const int slices = (int)std::min<size_t>((size_t)mid_slices(p.M, p.N, p.K[0]), workspace ? workspace_bytes / slice : 0);
+    if (slices <= 1) return lt_launch_gemm(p, EPI_STORE, dtype, io_dtype, stream);
+    GemmProblem q = p;
+    q.ksplit = slices;
+    q.split_stride = p.M * p.N;
+    q.epi = EpiParams{};
+    q.epi.out = workspace;
+    q.epi.ldo = p.N;
+    q.epi.out_dtype = LT_F32;
+    LT_TRY(lt_launch_gemm(q, EPI_STORE, dtype, io_dtype, stream));
+    return lt_splitk_reduce((const float*)workspace, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream);
+  }
   bool ok = dtype == LT_BF16 && p.nseg == 1 && p.sp.mode == SPARSE_NONE && p.M > 0 && p.N > 0 && p.N % 128 == 0 &&
             !(!a_km && b_km) && (a_km || p.M % 128 == 0) && ((!a_km && !b_km) || p.K[0] % 8 == 0) && p.K[0] > 0 &&
             p.A[0].ld % 8 == 0 && p.B[0].ld % 8 == 0 && lt_aligned(p.A[0].ptr, 16) && lt_aligned(p.B[0].ptr, 16) &&
@@ -243,7 +290,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_out_kernel(const float* __r
 }  // namespace
 
 size_t lt_gemm_out_splitk_workspace(int64_t M, int64_t N, int64_t K, size_t cap_bytes) {
-  const size_t full = std::max(lt_gemm_splitk_workspace(M, N, K), lt_gemm_generic_splitk_workspace(M, N, K));
+  const size_t full = std::max({lt_gemm_splitk_workspace(M, N, K), lt_gemm_generic_splitk_workspace(M, N, K),
+                                lt_gemm_mid_splitk_workspace(M, N, K)});
   const size_t slice = (size_t)M * (size_t)N * sizeof(float);
   if (full == 0 || cap_bytes < 2 * slice) return 0;
   return std::min(full, lt_align_up(cap_bytes / slice * slice, 256));
@@ -265,7 +313,8 @@ int lt_launch_gemm_out(const GemmProblem& p, int dtype, int io_dtype, void* work
     // the tiled kernel where it takes the problem, else the any-shape kernel
     const bool tiled = dtype == LT_BF16 && lt_gemm_mfma_supported(q, EPI_STORE) && dma_selected(q, EPI_STORE);
     const bool tiled_unsplit = dtype == LT_BF16 && lt_gemm_mfma_supported(p, EPI_OUT);
-    const int wanted = tiled ? splitk_slices(p.M, p.N, p.K[0]) : tiled_unsplit ? 1 : generic_splitk_slices(p.M, p.N, p.K[0]);
+    const int wanted = dtype == LT_BF16 && mid_selected(q, EPI_STORE) ? mid_slices(p.M, p.N, p.K[0])
+                       : tiled ? splitk_slices(p.M, p.N, p.K[0]) : tiled_unsplit ? 1 : generic_splitk_slices(p.M, p.N, p.K[0]);
     const int slices = (int)std::min<size_t>((size_t)wanted, workspace_bytes / slice);
     if (slices > 1) {
       q.ksplit = slices;

@@ -1,0 +1,297 @@
+// Tiled 16-bit products of a middling number of rows (65 to about a thousand: a prompt, a short training batch): 128 x 128 tiles, operands
+// copied global -> LDS, A k-major, B k-major or mn-major, the fused epilogues of the copy-based 256 x 256 kernel.
+//
+// What bounds it: 256 x 256 tiles of [512, 8192] are 64 workgroups for 256 CUs, each walking the whole reduction; four times as many
+// tiles fill the chip, at the price of LDS bandwidth: a wavefront's 64 x 64 sub-tile reads as many cycles of LDS as it has of
+// matrix instructions, so a chip full of 256 x 256 tiles is faster (the line: mid_selected in gemm_mfma_bf16.hip).  A grid of at most
+// one workgroup per CU keeps four 64-k stages of both operands in LDS (128 KiB), three of them on their way; a larger one two
+// stages, and two workgroups share a CU.  Measured, 256 x 256 tiles against these: [512, 8192] over 2048 43 us, 21 (805 TFLOP/s); [1024,
+// 4096] over 16384 276, 137 (1000 TFLOP/s); [768, 3072] over 768 22, 11.
+//
+// LDS layouts, swizzles and the transposing read of an mn-major operand are those of gemm_mfma_kernels.h.  Every copy tests for the
+// end of the reduction (the buffer unit returns zeros past the descriptor's size), so that whole, ragged and absent stages go through
+// the same straight-line code.
+#include "gemm_mfma_kernels.h"
+
+namespace {
+
+constexpr int MID = 128;  // tile rows and columns
+
+// copies of one operand: 64 k x 128 rows per stage, 4 per wavefront
+template <bool KM> struct MidOperand {
+  static constexpr int LOADS = 4;
+  static constexpr uint32_t RECORDS = 0xfffffc00u, OUTSIDE = 0xfffffe00u;
+  uint32_t off[LOADS];
+  const char* base;
+  int64_t unit_bytes;
+
+  // row0: first row (k-major) or column of the tile, of `limit`; past the end the last row / the last 8 columns are copied again.
+  // pair_rows > 0 (gated): tile row r is weight row row0 + 32 (r / 64) + r % 32, plus pair_rows where r % 64 >= 32.
+  __device__ __forceinline__ void setup(const GemmOperand& op, int64_t row0, int64_t limit, int64_t pair_rows, int wave, int lane) {
+    const int64_t ld = op.ld;
+    const char* ptr = reinterpret_cast<const char*>(op.ptr);
+#pragma unroll
+    for (int j = 0; j < LOADS; j++) {
+      const int q = (wave * LOADS + j) * 64 + lane;  // 16-byte slot of the stage
+      if constexpr (KM) {
+        const int row = q >> 3, c = (q & 7) ^ swz_km(row);
+        const int local = pair_rows > 0 ? (row >> 6) * 32 + (row & 31) : row;
+        int64_t g = min(row0 + local, limit - 1) - row0;
+        if (pair_rows > 0) g += ((row >> 5) & 1) * pair_rows;
+        off[j] = (uint32_t)((g * ld + c * 8) * 2);
+      } else {
+        const int kr = q >> 4, c = (q & 15) ^ swz_mn(kr);
+        off[j] = (uint32_t)((kr * ld + min(row0 + c * 8, limit - 8) - row0) * 2);
+      }
+    }
+    base = KM ? ptr + row0 * ld * 2 : ptr + row0 * 2;
+    unit_bytes = KM ? 64 * 2 : 64 * ld * 2;
+  }
+  // the 64 k from u * 64 on; pieces at or past k_limit arrive as zeros
+  __device__ __forceinline__ void issue(int u, bf16* dst, int wave, int lane, int k_limit) const {
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base + u * unit_bytes), 0, (int)RECORDS, 0x00020000);
+#pragma unroll
+    for (int j = 0; j < LOADS; j++) {
+      const int q = (wave * LOADS + j) * 64 + lane;
+      const int k = u * 64 + (KM ? ((q & 7) ^ swz_km(q >> 3)) * 8 : q >> 4);
+      const uint32_t o = k < k_limit ? off[j] : OUTSIDE;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(dst + (wave * LOADS + j) * 512), 16,
+                                               (int)o, 0, 0, 0);
+    }
+  }
+};
+
+template <bool B_KM, int KIND, typename TX, int ACT, int STAGES>
+__global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int tiles_m, int tiles_n) {
+  static_assert(STAGES == 2 || STAGES == 4, "stages");
+  constexpr int ELEMS = MID * 64;
+  // an array per stage and operand: the compiler can prove that copies and reads do not alias
+  __shared__ __attribute__((aligned(1024))) bf16 a0[ELEMS];
+  __shared__ __attribute__((aligned(1024))) bf16 a1[ELEMS];
+  __shared__ __attribute__((aligned(1024))) bf16 a2[ELEMS];
+  __shared__ __attribute__((aligned(1024))) bf16 a3[ELEMS];
+  __shared__ __attribute__((aligned(1024))) bf16 b0[ELEMS];
+  __shared__ __attribute__((aligned(1024))) bf16 b1[ELEMS];
+  __shared__ __attribute__((aligned(1024))) bf16 b2[ELEMS];
+  __shared__ __attribute__((aligned(1024))) bf16 b3[ELEMS];
+  auto a_buf = [&](auto S) -> bf16* {
+    constexpr int s = decltype(S)::value % STAGES;
+    return s == 0 ? a0 : s == 1 ? a1 : s == 2 ? a2 : a3;
+  };
+  auto b_buf = [&](auto S) -> bf16* {
+    constexpr int s = decltype(S)::value % STAGES;
+    return s == 0 ? b0 : s == 1 ? b1 : s == 2 ? b2 : b3;
+  };
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const bool gated = KIND == EPI_ACT_FWD && p.epi.gated;
+
+  // workgroup i runs on XCD i % 8; each XCD takes a contiguous range of tiles, GROUP_M tile rows at a time
+  const int num_pid = tiles_m * tiles_n;
+  int pid = blockIdx.x;
+  if ((num_pid & 7) == 0) pid = (pid & 7) * (num_pid >> 3) + (pid >> 3);
+  const int in_group = GROUP_M * tiles_n, first_m = pid / in_group * GROUP_M, group_m = min(tiles_m - first_m, GROUP_M);
+  const int64_t m0 = (int64_t)(first_m + pid % in_group % group_m) * MID;
+  const int64_t n0 = (int64_t)(pid % in_group / group_m) * (gated ? MID / 2 : MID);
+
+  // this workgroup's stages: first .. first + total of the reduction (slice blockIdx.y of them), walked from `rot` on and around:
+  // with a power-of-two leading dimension the rows of a k-major tile otherwise lie on the same memory channels, chip-wide
+  const int all = (int)((p.K[0] + 63) / 64);
+  int first = 0, total = all;
+  if (p.ksplit > 1) {
+    const int per = (all + p.ksplit - 1) / p.ksplit;
+    first = min(all, (int)blockIdx.y * per);
+    total = min(per, all - first);
+  }
+  const int rot = total > 0 ? (int)(((blockIdx.x & 7) * (unsigned)(total >> 3) + ((blockIdx.x >> 3) & 7)) % (unsigned)total) : 0;
+  const int k_limit = (int)p.K[0];
+  MidOperand<true> ca;
+  MidOperand<B_KM> cb;
+  ca.setup(p.A[0], m0, p.M, 0, wave, lane);
+  cb.setup(p.B[0], n0, p.N, gated ? p.N : 0, wave, lane);
+  auto copy = [&](auto S, int t) __attribute__((always_inline)) {
+    int u = t + rot;
+    if (u >= total) u -= total;
+    u = t < total ? first + u : all;  // (past the last stage: zeros)
+    ca.issue(u, a_buf(S), wave, lane, k_limit);
+    cb.issue(u, b_buf(S), wave, lane, k_limit);
+  };
+
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+  auto frag_km = [&](const bf16* buf, int base, int kk) -> bf16x8 {
+    const int row = base + (lane & 31);
+    return *reinterpret_cast<const bf16x8*>(&buf[(row * 8 + ((kk * 2 + (lane >> 5)) ^ swz_km(row))) * 8]);
+  };
+  auto frag_mn = [&](const bf16* tile, int base, int kk) -> bf16x8 {
+    union { bf16x8 v; s16x4 h[2]; } u;
+    const int i16 = lane & 15, col = base + ((lane >> 4) & 1) * 16 + 4 * (i16 & 3);
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const int kr = kk * 16 + 8 * (lane >> 5) + 4 * s + (i16 >> 2);
+      const bf16* src = &tile[kr * MID + ((((col >> 3) ^ swz_mn(kr)) << 3) | (col & 7))];
+      u.h[s] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(src));
+    }
+    return u.v;
+  };
+  auto multiply = [&](auto S) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) {
+      bf16x8 a[2], b[2];
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        a[i] = frag_km(a_buf(S), wm * 64 + i * 32, kk);
+        if constexpr (B_KM) b[i] = frag_km(b_buf(S), wn * 64 + i * 32, kk);
+        else b[i] = frag_mn(b_buf(S), wn * 64 + i * 32, kk);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = LT_MFMA_32X32X16(a[i], b[j], acc[i][j]);
+    }
+  };
+  // stage t: its copies have landed in every wavefront after the barrier, and every wavefront has read stage t - 1, whose buffer the
+  // copies of stage t + STAGES - 1 then take
+  constexpr int AHEAD = STAGES - 1;
+  lt_static_for<AHEAD>([&](auto S) __attribute__((always_inline)) { copy(S, decltype(S)::value); });
+  for (int t0 = 0; t0 < total; t0 += STAGES) {
+    lt_static_for<STAGES>([&](auto S) __attribute__((always_inline)) {
+      constexpr int s = decltype(S)::value;
+      wait_copies_and_barrier<(AHEAD - 1) * 8>();
+      copy(std::integral_constant<int, s + AHEAD>{}, t0 + s + AHEAD);
+      multiply(S);  // (zeros past the last stage)
+    });
+  }
+  wait_copies_and_barrier<0>();
+
+  // ---- epilogue: strips of 32 rows x 64 columns, transposed through 8 KiB of LDS of this wavefront's own and read back 8 columns per
+  //      lane; what a strip reads from memory is requested before it is staged.  Accumulator register r of a 32 x 32 block is row
+  //      8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32; columns of rows with bit 2 set are staged 32 further on (banks).
+  EpiParams epi = p.epi;
+  if (KIND == EPI_STORE && p.ksplit > 1) epi.out = reinterpret_cast<float*>(epi.out) + (int64_t)blockIdx.y * p.split_stride;
+  epi.bias = nullptr;
+  float* const stage = reinterpret_cast<float*>(wave == 0 ? a0 : wave == 1 ? a1 : wave == 2 ? b0 : b1);
+  auto staged = [&](int row, int col) -> float* { return &stage[row * 64 + (col ^ (((row >> 2) & 1) << 5))]; };
+  float colsum[16];  // EPI_ACT_BWD: column sums of the dpre values this lane writes
+#pragma unroll
+  for (int e = 0; e < 16; e++) colsum[e] = 0.f;
+  auto strips = [&](auto G) __attribute__((always_inline)) {
+    constexpr bool PAIR = decltype(G)::value;
+    constexpr int PER_ROW = PAIR ? 4 : 8, ROWS = 64 / PER_ROW, NIT = 32 / ROWS;
+    const int c = (lane % PER_ROW) * 8;
+    const int64_t n = n0 + wn * (PAIR ? 32 : 64) + c;
+    const bool in_n = n < p.N;  // N is a multiple of 8
+    float bias0[8], bias1[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) bias0[e] = bias1[e] = 0.f;
+    if (p.epi.bias && in_n) {
+      load8(p.epi.bias + n, bias0);
+      if constexpr (PAIR) load8(p.epi.bias + epi.inter + n, bias1);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int64_t mrow0 = m0 + wm * 64 + i * 32 + lane / PER_ROW;
+      EpiLoad in[NIT];
+      if constexpr (KIND == EPI_ACT_BWD || KIND == EPI_OUT) {
+#pragma unroll
+        for (int it = 0; it < NIT; it++)
+          in[it] = epi_load8<KIND, TX>(epi, min(mrow0 + it * ROWS, p.M - 1), in_n ? n : 0, true);
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) *staged(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), j * 32 + (lane & 31)) = acc[i][j][r];
+      __builtin_amdgcn_wave_barrier();
+      auto read8 = [&](int row, int col, const float (&bias)[8], float (&v)[8]) __attribute__((always_inline)) {
+        const float* sv = staged(row, col);
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(sv), hi = *reinterpret_cast<const f32x4*>(sv + 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          v[e] = lo[e] + bias[e];
+          v[4 + e] = hi[e] + bias[4 + e];
+        }
+      };
+#pragma unroll
+      for (int it = 0; it < NIT; it++) {
+        const int row = it * ROWS + lane / PER_ROW;
+        const int64_t m = mrow0 + it * ROWS;
+        float v[8];
+        read8(row, c, bias0, v);
+        if constexpr (PAIR) {
+          float vl[8];
+          read8(row, 32 + c, bias1, vl);
+          if (in_n && m < p.M) epi_act_fwd_gated8<ACT>(epi, m, n, v, vl);
+        } else if (in_n && m < p.M) {
+          if constexpr (KIND == EPI_STORE) epi_store8(epi, m, n, v);
+          else if constexpr (KIND == EPI_ACT_FWD) epi_act_fwd8<ACT>(epi, m, n, v);
+          else if constexpr (KIND == EPI_ACT_BWD) epi_act_bwd8_loaded<ACT>(epi, m, n, v, in[it], colsum);
+          else epi_out8_loaded<TX>(epi, m, n, v, in[it]);
+        }
+      }
+    }
+    if constexpr (KIND == EPI_ACT_BWD) {
+      if (epi.colsum) {  // lanes l, l + 8, ... hold the same columns; one partial row per 64 rows of the result
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+#pragma unroll
+          for (int mask = 8; mask < 64; mask <<= 1) colsum[e] += __shfl_xor(colsum[e], mask, 64);
+        if (lane < 8 && in_n && m0 + wm * 64 < p.M) {
+          float* dst = epi.colsum + ((m0 + wm * 64) / 64) * epi.ld_pre + n;
+          float lo[8], hi[8];
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            lo[e] = colsum[e];
+            hi[e] = colsum[8 + e];
+          }
+          store8(dst, lo);
+          if (epi.gated) store8(dst + epi.inter, hi);
+        }
+      }
+    }
+  };
+  if constexpr (KIND == EPI_ACT_FWD) {
+    if (gated) strips(std::true_type{});
+    else strips(std::false_type{});
+  } else {
+    strips(std::false_type{});
+  }
+}
+
+template <bool B_KM, int KIND, typename TX> int launch_mid(const GemmProblem& p, hipStream_t stream) {
+  const bool gated = KIND == EPI_ACT_FWD && p.epi.gated;
+  const int tiles_m = (int)((p.M + MID - 1) / MID), tiles_n = (int)((p.N + (gated ? 63 : 127)) / (gated ? 64 : 128));
+  const int slices = p.ksplit > 1 ? p.ksplit : 1;
+  const dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)slices), block(256);
+  with_activation<KIND>(p, [&](auto ACT) {
+    if (tiles_m * tiles_n * slices <= 256)
+      hipLaunchKernelGGL((gemm_bf16_mid_kernel<B_KM, KIND, TX, decltype(ACT)::value, 4>), grid, block, 0, stream, p, tiles_m, tiles_n);
+    else
+      hipLaunchKernelGGL((gemm_bf16_mid_kernel<B_KM, KIND, TX, decltype(ACT)::value, 2>), grid, block, 0, stream, p, tiles_m, tiles_n);
+  });
+  LT_LAUNCH_CHECK();
+  return LT_OK;
+}
+
+}  // namespace
+
+bool lt_gemm_mid_supported(const GemmProblem& p, int kind) {
+  return p.nseg == 1 && p.sp.mode == SPARSE_NONE && p.variant == 0 && p.A[0].kmajor && p.K[0] < (int64_t)1 << 30 &&
+         lt_gemm_mfma_supported(p, kind) && dma_offsets_fit(p, kind);
+}
+
+int lt_launch_gemm_mid(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream) {
+  LT_REQUIRE(lt_gemm_mid_supported(p, kind), LT_ERR_UNSUPPORTED, "128 x 128 gemm does not take this problem");
+  const bool b_km = p.B[0].kmajor;
+  if (kind == EPI_STORE) return b_km ? launch_mid<true, EPI_STORE, float>(p, stream) : launch_mid<false, EPI_STORE, float>(p, stream);
+  if (kind == EPI_ACT_FWD) return launch_mid<true, EPI_ACT_FWD, float>(p, stream);
+  if (kind == EPI_ACT_BWD) return launch_mid<false, EPI_ACT_BWD, float>(p, stream);
+  return io_dtype == LT_BF16 ? launch_mid<true, EPI_OUT, bf16>(p, stream) : launch_mid<true, EPI_OUT, float>(p, stream);
+}

@@ -97,7 +97,8 @@ struct GemmProblem {
   int ksplit;
   int64_t split_stride;
   int krot;  // copy-based kernel: how workgroups stagger their walk over k (0: all start at k = 0)
-  int variant;  // tiled bf16 kernels: 0 the launcher's choice, 1 the register-staged kernel where the copy-based one applies
+  int variant;  // 16-bit kernels: 0 the launcher's choice, 1 the register-staged kernel where a copy-based one applies, 2 the 256 x 256
+                // copy-based one where that of 128 x 128 tiles or the streaming one applies
   int tile_loop;  // copy-based kernel: 0 the launcher's choice (one workgroup per CU that loops over its tiles when there are
                   // more tiles than CUs), 1 one workgroup per tile
   unsigned long long* tile_stamps;  // instrumented build only (-DLT_TILE_TIMING): 8 words of clock stamps per tile; else null
@@ -485,6 +486,9 @@ int lt_launch_gemm_mfma(const GemmProblem& p, int kind, int io_dtype, hipStream_
 // up to 64 rows against a k-major weight matrix, forward epilogues (gemm_stream.hip)
 bool lt_gemm_stream_supported(const GemmProblem& p, int kind, int dtype, int io_dtype);
 int lt_launch_gemm_stream(const GemmProblem& p, int kind, int dtype, int io_dtype, hipStream_t stream);
+// 128 x 128 tiles for products too small to fill the chip with 256 x 256 ones (gemm_mid.hip)
+bool lt_gemm_mid_supported(const GemmProblem& p, int kind);
+int lt_launch_gemm_mid(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream);
 // algorithmic flops of a dense problem: 2 * M * N * (K0 + K1)
 double lt_gemm_flops(const GemmProblem& p, int kind);
 // block-sparse walk: matrix-core kernel for 64 x 64 bf16 blocks, else the any-shape kernel
@@ -507,6 +511,8 @@ int lt_launch_gemm_sparse(const GemmProblem& p, int kind, int dtype, int io_dtyp
 size_t lt_gemm_skinny_workspace(int64_t tokens, int64_t lowrank);
 // partial sums of a split [M, N] result on 256 x 256 tiles (0 when the tiles alone fill the chip)
 size_t lt_gemm_splitk_workspace(int64_t M, int64_t N, int64_t K);
+// same for 128 x 128 tiles
+size_t lt_gemm_mid_splitk_workspace(int64_t M, int64_t N, int64_t K);
 // same for the any-shape kernel (fp32 path, shapes the tiled kernels do not take)
 size_t lt_gemm_generic_splitk_workspace(int64_t M, int64_t N, int64_t K);
 // rows per partial row of EpiParams::colsum when lt_launch_gemm / lt_launch_gemm_sparse sends this EPI_ACT_BWD problem to a

@@ -1,0 +1,49 @@
+"""16-bit products on 128 x 128 tiles (gemm_mid.hip): rows and columns around the tile and its 64-wide sub-tiles, reductions around the
+8-element piece, the 64-k stage and the four stages in flight, one workgroup per CU and two (320 tiles), split reductions whose
+last slice is short or empty.
+
+Bound of test_gemm: fp32 accumulation of exact products, at most K + 16 additions each off by 2^-23 of the magnitudes it adds."""
+import pytest
+import torch
+
+import lean_transformer_amd as lt
+from conftest import assert_close
+from helpers import oracle_params, run_oracle
+from test_gpu_kernels import _gemm, _kernel_tags
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b_kmajor", [True, False])
+@pytest.mark.parametrize("m,n,k", [(65, 8, 8), (127, 72, 64), (128, 128, 72), (129, 136, 192), (300, 264, 256), (192, 520, 264),
+                                   (66, 64, 1000), (1000, 5000, 136)])
+def test_gemm(dtype, b_kmajor, m, n, k):
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    a, b = torch.randn(m, k, generator=g, device=DEV).to(dtype), torch.randn(n, k, generator=g, device=DEV).to(dtype)
+    c = _gemm(a, b if b_kmajor else b.t().contiguous(), True, b_kmajor, m, n, k, torch.float32, 0)
+    worst = (c.double() - a.double() @ b.double().t()).abs() - (k + 16) * 2.0**-23 * (a.double().abs() @ b.double().abs().t())
+    assert worst.max().item() <= 0.0
+
+
+@pytest.mark.parametrize("gated,dropout,post_ln", [(False, 0.0, False), (True, 0.0, True)])
+@pytest.mark.parametrize("tokens,hidden,inter", [(65, 136, 2056), (130, 264, 8200), (513, 128, 1000)])
+def test_split_reductions_of_a_training_step(gated, dropout, post_ln, tokens, hidden, inter):
+    """the down-projection (its reduction is `inter`) and du (twice that when gated), through their summing passes"""
+    torch.manual_seed(tokens)
+    ffn = lt.LeanFFN(hidden, inter, gated=gated, post_layer_norm=post_ln, layer_norm_eps=1e-5).to(DEV).to(torch.bfloat16)
+    x, dy = torch.randn(tokens, hidden), torch.randn(tokens, hidden)
+    y_ref, dx_ref, g_ref = run_oracle(oracle_params(ffn), x, dy)
+    xd = x.to(DEV).requires_grad_(True)
+
+    def step():
+        y = ffn(xd)
+        return y, torch.autograd.grad(y, [xd, ffn.i2h_proj.weight, ffn.i2h_proj.bias, ffn.h2o_proj.weight], dy.to(DEV))
+
+    (y, (dx, *grads)), tags = _kernel_tags(step)
+    assert any(t.startswith("splitk_reduce") for t in tags), tags
+    assert_close(y, y_ref, torch.bfloat16, "y")
+    assert_close(dx, dx_ref, torch.bfloat16, "dx")
+    for name, g, r in zip(("i2h.weight", "i2h.bias", "h2o.weight"), grads, g_ref[2:5]):
+        assert_close(g, r, torch.bfloat16, name)
