@@ -122,11 +122,13 @@ typedef struct lt_ffn_desc {
   int32_t compute_dtype; /* lt_dtype of weights, GEMM operands, the saved pre-activation and weight gradients */
   float ln_eps;
   float dropout_p;        /* 0 disables dropout (also pass 0 in eval mode) */
+  int32_t vector_dtype;   /* lt_dtype of the small vectors below (LayerNorm parameters, i2h.bias, h2o.bias): LT_F32, or
+                             compute_dtype: one kernel then widens them into the workspace.  Gradients of them are fp32 */
   uint64_t dropout_seed;  /* Philox key */
   uint64_t dropout_offset;/* Philox stream offset; forward and backward of one call must pass the same pair */
-  const float* ln_weight; /* [H] fp32 */
-  const float* ln_bias;   /* [H] fp32 */
-  const float* post_ln_weight; /* [H] fp32 or NULL: optional LayerNorm after the down-projection */
+  const float* ln_weight; /* [H] vector_dtype (as the next three) */
+  const float* ln_bias;   /* [H] */
+  const float* post_ln_weight; /* [H] or NULL: optional LayerNorm after the down-projection */
   const float* post_ln_bias;
   lt_linear i2h; /* H -> (gated ? 2I : I) */
   lt_linear h2o; /* I -> H */

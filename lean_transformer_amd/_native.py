@@ -48,7 +48,7 @@ class LtFfnDesc(ctypes.Structure):
     _fields_ = [
         ("tokens", c_int64), ("hidden", c_int32), ("intermediate", c_int32), ("gated", c_int32), ("act", c_int32),
         ("residual", c_int32), ("io_dtype", c_int32), ("compute_dtype", c_int32), ("ln_eps", c_float),
-        ("dropout_p", c_float), ("dropout_seed", c_uint64), ("dropout_offset", c_uint64),
+        ("dropout_p", c_float), ("vector_dtype", c_int32), ("dropout_seed", c_uint64), ("dropout_offset", c_uint64),
         ("ln_weight", c_void_p), ("ln_bias", c_void_p), ("post_ln_weight", c_void_p), ("post_ln_bias", c_void_p),
         ("i2h", LtLinear), ("h2o", LtLinear),
     ]

@@ -422,7 +422,7 @@ __global__ __launch_bounds__(256) void colreduce4_multi_kernel(ColReduceQueue q)
 static void launch_colreduce(int rows, int64_t stride, int cols, const float* partial, float* out, hipStream_t stream,
                              ColReduceQueue* defer = nullptr) {
   const bool vec = (cols & 3) == 0 && (stride & 3) == 0 && lt_aligned(partial, 16) && lt_aligned(out, 16);
-  if (vec && defer && defer->n < 4) {
+  if (vec && defer && defer->n < ColReduceQueue::MAX) {
     defer->job[defer->n++] = ColReduceJob{partial, out, rows, cols, stride};
     return;
   }
@@ -915,7 +915,7 @@ static int colsum_slices(int64_t rows) {
 size_t lt_colsum_workspace(int64_t rows, int cols) { return (size_t)colsum_slices(rows) * (size_t)cols * sizeof(float); }
 
 int lt_colsum(int64_t rows, int cols, int64_t ld, int dtype, const void* in, float* out, void* workspace,
-              size_t workspace_bytes, hipStream_t stream) {
+              size_t workspace_bytes, hipStream_t stream, ColReduceQueue* defer) {
   LT_REQUIRE(rows > 0 && cols > 0 && in && out, LT_ERR_BAD_ARG, "colsum: bad arguments");
   LT_REQUIRE(workspace && workspace_bytes >= lt_colsum_workspace(rows, cols), LT_ERR_WORKSPACE,
              "colsum: workspace of %zu bytes needed", lt_colsum_workspace(rows, cols));
@@ -936,7 +936,7 @@ int lt_colsum(int64_t rows, int cols, int64_t ld, int dtype, const void* in, flo
     else
       hipLaunchKernelGGL((colsum_partial_kernel<bf16>), grid, block, 0, stream, rows, cols, ld, (const bf16*)in, rps, partial);
   }
-  launch_colreduce(slices, (int64_t)cols, cols, partial, out, stream);
+  launch_colreduce(slices, (int64_t)cols, cols, partial, out, stream, defer);
   LT_LAUNCH_CHECK();
   return LT_OK;
 }
@@ -1007,7 +1007,7 @@ int lt_dropout_cast_colsum(int64_t rows, int cols, int in_dtype, const void* in,
              "dropout + column sums: workspace of %zu bytes needed", lt_colsum_workspace(rows, cols));
   if ((cols & 7) != 0 || !lt_aligned(in, 16) || !lt_aligned(out, 16) || !lt_aligned(workspace, 16)) {
     LT_TRY(lt_dropout_cast(rows * cols, in_dtype, in, out_dtype, out, drop, stream));
-    return lt_colsum(rows, cols, cols, out_dtype, out, colsum, workspace, workspace_bytes, stream);
+    return lt_colsum(rows, cols, cols, out_dtype, out, colsum, workspace, workspace_bytes, stream, defer);
   }
   LtProfileScope scope("dropout_replay_cast", 0.0, (double)rows * cols * (lt_dtype_size(in_dtype) + lt_dtype_size(out_dtype)),
                        stream);
@@ -1048,6 +1048,30 @@ int lt_splitk_reduce(const float* partial, int slices, int64_t stride, int64_t c
   return LT_OK;
 }
 
+namespace {
+// 4 elements per thread, blockIdx.y picks the vector.  A few ten kilobytes: bound by its launch, which is why it is one
+__global__ __launch_bounds__(256) void widen_kernel(WidenJobs jobs) {
+  const int j = blockIdx.y;
+  const bf16* in = reinterpret_cast<const bf16*>(jobs.in[j]);
+  const int base = blockIdx.x * 1024 + threadIdx.x;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const int i = base + e * 256;
+    if (i < jobs.count[j]) jobs.out[j][i] = (float)in[i];
+  }
+}
+}  // namespace
+
+int lt_widen(const WidenJobs& jobs, hipStream_t stream) {
+  if (jobs.n == 0) return LT_OK;
+  int most = 0;
+  for (int i = 0; i < jobs.n; i++) most = std::max(most, jobs.count[i]);
+  LtProfileScope scope("widen_vectors", 0.0, 6.0 * most * jobs.n, stream);
+  hipLaunchKernelGGL(widen_kernel, dim3((unsigned)((most + 1023) / 1024), (unsigned)jobs.n), dim3(256), 0, stream, jobs);
+  LT_LAUNCH_CHECK();
+  return LT_OK;
+}
+
 int lt_colreduce_flush(ColReduceQueue& queue, hipStream_t stream) {
   if (queue.n == 0) return LT_OK;
   int blocks = 1;
@@ -1066,7 +1090,7 @@ int lt_colreduce_flush(ColReduceQueue& queue, hipStream_t stream) {
 int lt_colreduce(int rows, int64_t stride, int cols, const float* partial, float* out, hipStream_t stream,
                  ColReduceQueue* defer) {
   LT_REQUIRE(rows > 0 && cols > 0 && partial && out, LT_ERR_BAD_ARG, "colreduce: bad arguments");
-  if (defer && defer->n < 4 && (cols & 3) == 0 && (stride & 3) == 0 && lt_aligned(partial, 16) && lt_aligned(out, 16)) {
+  if (defer && defer->n < ColReduceQueue::MAX && (cols & 3) == 0 && (stride & 3) == 0 && lt_aligned(partial, 16) && lt_aligned(out, 16)) {
     launch_colreduce(rows, stride, cols, partial, out, stream, defer);
     return LT_OK;
   }

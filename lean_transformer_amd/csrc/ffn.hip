@@ -258,7 +258,7 @@ void plan_linear_backward(const lt_linear& lin, int64_t T, int dtype, Bump& ws, 
 int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void* x_act, const void* dy,
                          const void* lowrank_hid, int kind_dx, const EpiParams& epi_dx, const lt_linear_grads& grads,
                          const LinearBwdScratch& s, int io_dtype, hipStream_t stream, float* act_colsum = nullptr,
-                         int* act_colsum_rows = nullptr) {
+                         int* act_colsum_rows = nullptr, ColReduceQueue* defer = nullptr) {
   const int64_t in = lin.in_features, out = lin.out_features, r = lin.lowrank;
   const bool need_dx = kind_dx >= 0;
   if (r > 0 && (need_dx || grads.lowrank_first)) {  // g_hid = dy L2  [T, r]
@@ -298,7 +298,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
       LT_TRY(lt_launch_gemm_sparse(p, kind_dx, dtype, io_dtype, stream));
     }
   }
-  if (grads.bias) LT_TRY(lt_colsum(T, (int)out, out, dtype, dy, grads.bias, s.colsum, s.colsum_bytes, stream));
+  if (grads.bias) LT_TRY(lt_colsum(T, (int)out, out, dtype, dy, grads.bias, s.colsum, s.colsum_bytes, stream, defer));
   if (grads.weight) {
     GemmProblem p = blank_problem();
     if (lin.block == 0) {  // dW[out, in] = dy^T x
@@ -360,6 +360,8 @@ int check_ffn_desc(const lt_ffn_desc* d) {
              (long long)d->tokens, d->hidden, d->intermediate);
   LT_TRY(check_dtype(d->io_dtype, "ffn io_dtype"));
   LT_TRY(check_dtype(d->compute_dtype, "ffn compute_dtype"));
+  LT_REQUIRE(d->vector_dtype == LT_F32 || d->vector_dtype == d->compute_dtype, LT_ERR_BAD_ARG,
+             "ffn vector_dtype: %d is neither fp32 nor the compute dtype", d->vector_dtype);
   LT_REQUIRE(d->act >= 0 && d->act < LT_ACT_COUNT, LT_ERR_UNSUPPORTED, "ffn: unknown activation %d", d->act);
   LT_REQUIRE(d->ln_weight && d->ln_bias, LT_ERR_BAD_ARG, "ffn: LayerNorm parameters missing");
   LT_REQUIRE((d->post_ln_weight == nullptr) == (d->post_ln_bias == nullptr), LT_ERR_BAD_ARG, "ffn: post-LN needs weight and bias");
@@ -379,7 +381,41 @@ struct FwdScratch {
   void* hid;     // [T, I] compute dtype: activation output
   void* skinny;  // split-k partial sums of the low-rank GEMMs
   size_t skinny_bytes;
+  float* vectors;  // 16-bit small vectors in fp32
 };
+
+// room for the small vectors of a call in fp32, where they are not (with_biases: the forward pass reads those too); each piece
+// starts at a multiple of 64 elements
+float* take_vectors(const lt_ffn_desc& d, Bump& ws, bool with_biases) {
+  if (d.vector_dtype == LT_F32) return nullptr;
+  size_t elements = lt_align_up(d.hidden, 64) * (d.post_ln_weight ? 4 : 2);
+  if (with_biases) elements += lt_align_up(d.i2h.out_features, 64) + lt_align_up(d.h2o.out_features, 64);
+  return (float*)ws.take(elements * sizeof(float));
+}
+
+// fills that room and points the descriptor at it
+int widen_vectors(lt_ffn_desc& d, float* room, bool with_biases, hipStream_t stream) {
+  if (d.vector_dtype == LT_F32) return LT_OK;
+  WidenJobs jobs;
+  jobs.n = 0;
+  auto widen = [&](const float*& vector, int count) {
+    if (!vector) return;
+    jobs.in[jobs.n] = vector;
+    jobs.out[jobs.n] = room;
+    jobs.count[jobs.n++] = count;
+    vector = room;
+    room += lt_align_up(count, 64);
+  };
+  widen(d.ln_weight, d.hidden);
+  widen(d.ln_bias, d.hidden);
+  widen(d.post_ln_weight, d.hidden);
+  widen(d.post_ln_bias, d.hidden);
+  if (with_biases) {
+    widen(d.i2h.bias, d.i2h.out_features);
+    widen(d.h2o.bias, d.h2o.out_features);
+  }
+  return lt_widen(jobs, stream);
+}
 
 void plan_forward(const lt_ffn_desc& d, Bump& ws, FwdScratch& s) {
   const size_t e = lt_dtype_size(d.compute_dtype);
@@ -393,6 +429,7 @@ void plan_forward(const lt_ffn_desc& d, Bump& ws, FwdScratch& s) {
     s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_out_splitk_workspace(d.tokens, d.hidden, d.intermediate, cap));
   }
   s.skinny = s.skinny_bytes ? ws.take(s.skinny_bytes) : nullptr;
+  s.vectors = take_vectors(d, ws, true);
 }
 
 struct BwdScratch {
@@ -405,6 +442,8 @@ struct BwdScratch {
   void* du;          // [T, H] compute dtype (as the reference's autocast matmul leaves it)
   void* ln_ws;
   size_t ln_ws_bytes;
+  void* post_ln_ws;   // the same, post-LN only (both wait for the end of the step)
+  float* vectors;     // 16-bit LayerNorm parameters in fp32
   float* act_colsum;  // [ceil(T / 64), N1]: partial column sums of dpre from the epilogue that writes it
   LinearBwdScratch h2o, i2h;
 };
@@ -422,6 +461,8 @@ void plan_backward(const lt_ffn_desc& d, Bump& ws, BwdScratch& s) {
   s.du = ws.take((size_t)T * d.hidden * e);
   s.ln_ws_bytes = lt_ln_backward_workspace(T, d.hidden);
   s.ln_ws = ws.take(s.ln_ws_bytes);
+  s.post_ln_ws = d.post_ln_weight ? ws.take(s.ln_ws_bytes) : nullptr;
+  s.vectors = take_vectors(d, ws, false);
   s.act_colsum = (float*)ws.take((size_t)((T + 63) / 64) * n1 * sizeof(float));
   plan_linear_backward(d.h2o, T, d.compute_dtype, ws, s.h2o);
   plan_linear_backward(d.i2h, T, d.compute_dtype, ws, s.i2h);
@@ -451,7 +492,7 @@ extern "C" size_t lt_ffn_backward_workspace_bytes(const lt_ffn_desc* desc) {
 extern "C" int lt_ffn_forward(const lt_ffn_desc* desc, const void* x, void* y, const lt_ffn_saved* saved, void* workspace,
                               size_t workspace_bytes, void* stream_) {
   LT_TRY(check_ffn_desc(desc));
-  const lt_ffn_desc& d = *desc;
+  lt_ffn_desc d = *desc;
   hipStream_t stream = (hipStream_t)stream_;
   LT_REQUIRE(x && y && saved && saved->pre_activation && saved->ln_stats, LT_ERR_BAD_ARG, "ffn forward: null tensor");
   LT_REQUIRE(!d.post_ln_weight || saved->post_ln_input, LT_ERR_BAD_ARG, "ffn forward: post_ln_input buffer missing");
@@ -461,6 +502,7 @@ extern "C" int lt_ffn_forward(const lt_ffn_desc* desc, const void* x, void* y, c
   Bump ws(workspace);
   FwdScratch s;
   plan_forward(d, ws, s);
+  LT_TRY(widen_vectors(d, s.vectors, true, stream));
   const int64_t T = d.tokens, H = d.hidden, I = d.intermediate, N1 = d.gated ? 2 * I : I;
   const int cdt = d.compute_dtype, io = d.io_dtype;
   const DropoutParams drop = make_dropout(d.dropout_p, d.dropout_seed, d.dropout_offset);
@@ -495,7 +537,7 @@ extern "C" int lt_ffn_forward(const lt_ffn_desc* desc, const void* x, void* y, c
 extern "C" int lt_ffn_backward(const lt_ffn_desc* desc, const void* x, const void* dy, const lt_ffn_saved* saved,
                                const lt_ffn_grads* grads, void* workspace, size_t workspace_bytes, void* stream_) {
   LT_TRY(check_ffn_desc(desc));
-  const lt_ffn_desc& d = *desc;
+  lt_ffn_desc d = *desc;
   hipStream_t stream = (hipStream_t)stream_;
   LT_REQUIRE(x && dy && saved && grads && saved->pre_activation && saved->ln_stats, LT_ERR_BAD_ARG, "ffn backward: null tensor");
   LT_REQUIRE(!d.post_ln_weight || saved->post_ln_input, LT_ERR_BAD_ARG, "ffn backward: post_ln_input missing");
@@ -507,6 +549,7 @@ extern "C" int lt_ffn_backward(const lt_ffn_desc* desc, const void* x, const voi
   Bump ws(workspace);
   BwdScratch s;
   plan_backward(d, ws, s);
+  LT_TRY(widen_vectors(d, s.vectors, false, stream));
   const int64_t T = d.tokens, H = d.hidden, I = d.intermediate, N1 = d.gated ? 2 * I : I;
   const int cdt = d.compute_dtype, io = d.io_dtype;
   const DropoutParams drop = make_dropout(d.dropout_p, d.dropout_seed, d.dropout_offset);
@@ -532,7 +575,7 @@ extern "C" int lt_ffn_backward(const lt_ffn_desc* desc, const void* x, const voi
     LT_TRY(lt_ln_forward(T, (int)H, d.ln_eps, cdt, saved->post_ln_input, nullptr, nullptr, cdt, nullptr, s.post_stats, cdt,
                          nullptr, nullptr, false, stream));
     LT_TRY(lt_ln_backward(T, (int)H, cdt, saved->post_ln_input, s.post_stats, d.post_ln_weight, cdt, g, cdt, nullptr,
-                          s.g_post, grads->post_ln_weight, grads->post_ln_bias, s.ln_ws, s.ln_ws_bytes, stream));
+                          s.g_post, grads->post_ln_weight, grads->post_ln_bias, s.post_ln_ws, s.ln_ws_bytes, stream, &reduces));
     g = s.g_post;
   }
 
@@ -544,7 +587,7 @@ extern "C" int lt_ffn_backward(const lt_ffn_desc* desc, const void* x, const voi
     e.pre = saved->pre_activation; e.ld_pre = N1; e.dpre = s.dpre; e.hid = s.hid; e.ld_hid = I;
     e.gated = d.gated; e.act = d.act; e.inter = I;
     LT_TRY(linear_backward_impl(d.h2o, T, cdt, s.hid, g, saved->h2o_lowrank_hid, EPI_ACT_BWD, e, h2o_grads, s.h2o, io,
-                                stream, grads->i2h.bias ? s.act_colsum : nullptr, &bias_rows));
+                                stream, grads->i2h.bias ? s.act_colsum : nullptr, &bias_rows, &reduces));
   }
   lt_linear_grads i2h_grads = grads->i2h;
   if (bias_rows > 0) {  // db1 = column sums of dP, already reduced to one row per bias_rows tokens
@@ -560,7 +603,7 @@ extern "C" int lt_ffn_backward(const lt_ffn_desc* desc, const void* x, const voi
   {
     EpiParams e = epi_store_params(s.du, H, cdt, nullptr);
     LT_TRY(linear_backward_impl(d.i2h, T, cdt, s.u, s.dpre, saved->i2h_lowrank_hid, need_du ? EPI_STORE : -1, e,
-                                i2h_grads, s.i2h, io, stream));
+                                i2h_grads, s.i2h, io, stream, nullptr, nullptr, &reduces));
   }
   if (need_du) {
     LT_TRY(lt_ln_backward(T, (int)H, io, x, saved->ln_stats, d.ln_weight, cdt, s.du, io, d.residual ? dy : nullptr,

@@ -528,7 +528,8 @@ struct ColReduceJob {
   int64_t stride;
 };
 struct ColReduceQueue {
-  ColReduceJob job[4];
+  static constexpr int MAX = 6;
+  ColReduceJob job[MAX];
   int n;
 };
 int lt_colreduce_flush(ColReduceQueue& queue, hipStream_t stream);

@@ -12,7 +12,15 @@ int lt_ln_backward(int64_t T, int H, int x_dtype, const void* x, const float* st
                    void* workspace, size_t workspace_bytes, hipStream_t stream, ColReduceQueue* defer = nullptr);
 size_t lt_colsum_workspace(int64_t rows, int cols);
 int lt_colsum(int64_t rows, int cols, int64_t ld, int dtype, const void* in, float* out, void* workspace,
-              size_t workspace_bytes, hipStream_t stream);
+              size_t workspace_bytes, hipStream_t stream, ColReduceQueue* defer = nullptr);
+// 16-bit vectors -> fp32, one launch
+struct WidenJobs {
+  const void* in[6];
+  float* out[6];
+  int count[6];
+  int n;
+};
+int lt_widen(const WidenJobs& jobs, hipStream_t stream);
 int lt_act_forward(int64_t T, int64_t I, int gated, int act, int dtype, const void* pre, void* hid, hipStream_t stream);
 int lt_act_backward(int64_t T, int64_t I, int gated, int act, int dtype, const void* pre, const void* dhid, void* dpre,
                     hipStream_t stream);

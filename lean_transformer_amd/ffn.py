@@ -205,10 +205,10 @@ class _LeanFFN(torch.autograd.Function):
             ctx, tokens, hidden, ln_weight, ln_bias, i2h_weight, i2h_bias, i2h_lowrank_first, i2h_lowrank_second,
             i2h_forward_indices, i2h_backward_indices, h2o_weight, h2o_bias, h2o_lowrank_first, h2o_lowrank_second,
             h2o_forward_indices, h2o_backward_indices, post_ln_weight, post_ln_bias, io)
-        # fp32 copies of the small vectors (LayerNorm parameters, biases): backward reuses them instead of converting again.
-        # The parameters themselves go through save_for_backward below, so an in-place update between forward and backward
-        # makes ctx.saved_tensors raise (autograd's version check) before these copies could be used stale.
-        ctx._small_fp32 = (keep[0], keep[1], keep[2], keep[3], keep[4][1], keep[5][1])
+        # Where this call made fp32 copies of the small vectors (LayerNorm parameters, biases), backward reuses them instead of
+        # converting again.  The parameters themselves go through save_for_backward below, so an in-place update between
+        # forward and backward makes ctx.saved_tensors raise (autograd's version check) before these copies could be used stale.
+        ctx._small = None if desc.vector_dtype == desc.compute_dtype else keep[:6]
         n1 = desc.i2h.out_features
         y = torch.empty_like(x)
         pre_activation = torch.empty(tokens, n1, dtype=cdt, device=device)
@@ -237,12 +237,17 @@ class _LeanFFN(torch.autograd.Function):
         """ctypes descriptor + the converted tensors it points into (which must outlive the call)"""
         act, gated, ln_eps, residual, cdt = ctx._cfg
         p, seed, offset = ctx._dropout
-        keep = [_as(ln_weight, torch.float32), _as(ln_bias, torch.float32), _as(post_ln_weight, torch.float32),
-                _as(post_ln_bias, torch.float32)]
+        # the small vectors: as they are where all are in a 16-bit compute dtype (the library widens them, one launch), else fp32
+        keep = [ln_weight, ln_bias, post_ln_weight, post_ln_bias, i2h_bias, h2o_bias]
+        vector_dtype = cdt
+        if cdt == torch.float32 or not all(v is None or (v.dtype == cdt and v.is_contiguous()) for v in keep):
+            vector_dtype = torch.float32
+            keep = [_as(v, torch.float32) for v in keep]
+        ln_weight, ln_bias, post_ln_weight, post_ln_bias, i2h_bias, h2o_bias = keep
         projections = []
         for w, b, l1, l2, fwd, bwd in ((i2h_weight, i2h_bias, i2h_l1, i2h_l2, i2h_fwd, i2h_bwd),
                                        (h2o_weight, h2o_bias, h2o_l1, h2o_l2, h2o_fwd, h2o_bwd)):
-            tensors = (_as(w, cdt), _as(b, torch.float32), _as(l1, cdt), _as(l2, cdt),
+            tensors = (_as(w, cdt), b, _as(l1, cdt), _as(l2, cdt),
                        None if fwd is None else fwd.to(torch.int32).contiguous(),
                        None if bwd is None else bwd.to(torch.int64).contiguous())
             keep.append(tensors)
@@ -253,8 +258,9 @@ class _LeanFFN(torch.autograd.Function):
         desc.gated, desc.act, desc.residual = int(gated), act, int(residual)
         desc.io_dtype, desc.compute_dtype = nat.dtype_code(io), nat.dtype_code(cdt)
         desc.ln_eps, desc.dropout_p, desc.dropout_seed, desc.dropout_offset = ln_eps, p, seed, offset
-        desc.ln_weight, desc.ln_bias = nat.ptr(keep[0]), nat.ptr(keep[1])
-        desc.post_ln_weight, desc.post_ln_bias = nat.ptr(keep[2]), nat.ptr(keep[3])
+        desc.vector_dtype = nat.dtype_code(vector_dtype)
+        desc.ln_weight, desc.ln_bias = nat.ptr(ln_weight), nat.ptr(ln_bias)
+        desc.post_ln_weight, desc.post_ln_bias = nat.ptr(post_ln_weight), nat.ptr(post_ln_bias)
         desc.i2h, desc.h2o = projections
         return desc, keep
 
@@ -273,10 +279,11 @@ class _LeanFFN(torch.autograd.Function):
         if dy.dtype != io:
             dy = dy.to(io)
         dy = dy.contiguous()
-        ln_w32, ln_b32, post_w32, post_b32, i2h_b32, h2o_b32 = ctx._small_fp32
+        ln_w, ln_b, post_w, post_b, i2h_b, h2o_b = ctx._small or (ln_weight, ln_bias, post_ln_weight, post_ln_bias, i2h_bias,
+                                                                  h2o_bias)
         desc, keep = _LeanFFN._describe(
-            ctx, tokens, hidden, ln_w32, ln_b32, i2h_weight, i2h_b32, i2h_l1, i2h_l2, i2h_fwd, i2h_bwd,
-            h2o_weight, h2o_b32, h2o_l1, h2o_l2, h2o_fwd, h2o_bwd, post_w32, post_b32, io)
+            ctx, tokens, hidden, ln_w, ln_b, i2h_weight, i2h_b, i2h_l1, i2h_l2, i2h_fwd, i2h_bwd,
+            h2o_weight, h2o_b, h2o_l1, h2o_l2, h2o_fwd, h2o_bwd, post_w, post_b, io)
         need = ctx.needs_input_grad
 
         def new(like_shape, dtype, wanted):
