@@ -14,7 +14,8 @@
 // what it aligns away towards minus infinity (a bias of 0.1 - 0.2 units in the last place per instruction, measured), which
 // sums over many rows of a result would collect (a bias gradient is one over all tokens); odd rows of A are therefore negated
 // on the way in and odd rows of the result on the way out, so that the bias alternates.
-// An infinity among the operands gives NaN (its second plane is inf - inf) where fp32 arithmetic gives infinity or NaN.
+// An infinity has no such planes (inf - inf) and gives NaN; an element that comes out as NaN is therefore computed again, in fp32
+// arithmetic from the operands in memory, as the epilogue takes it up (a NaN among the operands ends that at once).
 // What bounds it: at 4096^3 a full round of workgroups runs at 1.2 PFLOP/s of bfloat16 products, what the tiled 16-bit kernel
 // reaches on the same data (the clock under load); smaller products lose to a last round that is not full and to the start and
 // end of a tile.  4096^3: 1411 us with the fp32 instruction, 723 now; a training step of T = 4096, hidden 768: 2263 us, 1154 now;
@@ -167,7 +168,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
   }
   if (m0 >= M || n0 >= N) return;  // whole workgroup
 
-  auto segment = [&](int s) -> Segment<TI> {
+  auto segment = [&](int s) __attribute__((always_inline)) -> Segment<TI> {
     Segment<TI> g;
     if (sp.mode == SPARSE_NONE) {
       g.A = reinterpret_cast<const TI*>(p.A[s].ptr); g.lda = p.A[s].ld;
@@ -226,13 +227,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
   // the cursor: segment and k of the next step to be fetched
   int seg = 0;
   Segment<TI> g = segment(0);
-  int64_t k0 = 0;
+  int64_t k0 = 0, slice_k0 = 0, slice_k1 = g.K;
   if (sp.mode == SPARSE_NONE && p.ksplit > 1) {
     // split reduction (one k-segment, EPI_STORE): slice blockIdx.y walks a whole number of k-steps and stores fp32 partial
     // sums at epi.out + slice * split_stride
     const int64_t steps = (g.K + BK - 1) / BK, per = (steps + p.ksplit - 1) / p.ksplit * BK;
     k0 = min(g.K, (int64_t)blockIdx.y * per);
     g.K = min(g.K, k0 + per);
+    slice_k0 = k0;
+    slice_k1 = g.K;
     epi.out = reinterpret_cast<float*>(epi.out) + (int64_t)blockIdx.y * p.split_stride;
   }
   int total = 0;  // steps (an empty slice: one step of zeros)
@@ -440,6 +443,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
   if constexpr (KIND == EPI_OUT)
     vec = vec && (epi.ldy & 3) == 0 && ((reinterpret_cast<uintptr_t>(epi.x) | reinterpret_cast<uintptr_t>(epi.y)) & 15) == 0;
 
+  // element (row m of the tile's coordinates, row j of B) of fp32 operands, in fp32 arithmetic
+  auto element = [&](int64_t m, int64_t j) __attribute__((always_inline)) {
+    float sum = 0.f;
+    for (int s = 0; s < nseg; s++) {
+      const Segment<TI> q = segment(s);
+      const int64_t end = s ? q.K : min(slice_k1, q.K);
+      for (int64_t k = s ? 0 : slice_k0; k < end && sum == sum; k++)
+        sum = fmaf(to_f32(A_KM ? q.A[m * q.lda + k] : q.A[k * q.lda + m]), to_f32(B_KM ? q.B[j * q.ldb + k] : q.B[k * q.ldb + j]), sum);
+    }
+    return sum;
+  };
   auto unflipped = [&](float v, int row) { return PLANES > 1 && (row & 1) ? -v : v; };  // (fp32: odd rows are negated)
 #pragma unroll
   for (int i = 0; i < FM; i++) {
@@ -468,9 +482,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
         stage[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * STAGE_LD + j * 32 + (lane & 31)] = unflipped(acc[i][j][r], r);
     __builtin_amdgcn_wave_barrier();
     auto row_of = [&](int it) { return it * rows_per_it + lane_row; };
-    auto staged = [&](int row, int col, float (&v)[4]) {
+    auto staged = [&](int row, int col, float (&v)[4]) __attribute__((always_inline)) {
       const float4 t = *reinterpret_cast<const float4*>(&stage[row * STAGE_LD + col]);
       v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+      if constexpr (PLANES > 1) {
+        const float any = (v[0] + v[1]) + (v[2] + v[3]);
+        if (__builtin_expect(any != any, 0)) {
+#pragma unroll 1
+          for (int e = 0; e < count; e++) {
+            const float o = e == 0 ? v[0] : e == 1 ? v[1] : e == 2 ? v[2] : v[3];
+            if (o == o) continue;
+            const float f = element(mrow0 + row, (gated ? n0 + wn * 32 + (col >= 32 ? N : 0) + (col & 31) : n0 + wn * 64 + col) + e);
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[q] = q == e ? f : v[q];
+          }
+        }
+      }
     };
     if constexpr (KIND == EPI_ACT_BWD || KIND == EPI_OUT) {
       lt_rolled_rows<READS>([&](int it, float (&r0)[4], float (&r1)[4]) {

@@ -76,3 +76,22 @@ def test_fp32_view_that_is_not_16_byte_aligned():
 def test_16_bit_operands(dtype, a_kmajor, b_kmajor, m, n, k):
     a, b, ref = _operands(m, n, k, a_kmajor, b_kmajor, dtype, seed=m + n + k)
     assert rel_err(_gemm(a, b, a_kmajor, b_kmajor, m, n, k, torch.float32, 1), ref) <= 1e-5
+
+
+@pytest.mark.parametrize("a_kmajor,b_kmajor", [(True, True), (True, False), (False, False), (False, True)])
+@pytest.mark.parametrize("m,n,k", [(65, 129, 17), (4100, 2048, 64)])
+def test_fp32_infinities_and_nans(a_kmajor, b_kmajor, m, n, k):
+    """an infinity has no exact planes: the elements it reaches are computed again and come out as fp32 arithmetic gives them,
+    infinite with the right sign, NaN where infinities of both signs or a zero meet; their neighbours are untouched"""
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    a, b = torch.randn(m, k, generator=g, device=DEV), torch.randn(n, k, generator=g, device=DEV)
+    inf = float("inf")
+    a[3, 5], a[8, k - 1], a[m - 1, 0], a[7, 1], a[7, 9], a[9, 2] = inf, -inf, inf, inf, -inf, float("nan")
+    b[2, 5], b[n - 1, 5], b[4, 0] = 0.0, -inf, inf
+    c = _gemm(a if a_kmajor else a.t().contiguous(), b if b_kmajor else b.t().contiguous(), a_kmajor, b_kmajor, m, n, k,
+              torch.float32, 1)
+    ref = (a.cpu().double() @ b.cpu().double().t()).to(DEV)
+    assert torch.equal(c.isnan(), ref.isnan()) and torch.equal(c.isinf(), ref.isinf())
+    assert torch.equal(c[c.isinf()].sign(), ref[ref.isinf()].sign().float())
+    finite = ref.isfinite()
+    assert (c.double() - ref)[finite].abs().max().item() <= 1e-4
