@@ -237,6 +237,7 @@ void plan_linear_backward(const lt_linear& lin, int64_t T, int dtype, Bump& ws, 
   s.skinny_bytes = lin.lowrank > 0 ? lt_gemm_skinny_workspace(T, lin.lowrank) : 0;
   if (lin.block == 0) {  // dW (and dx) of a small dense layer: the reduction is split across workgroups
     s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_splitk_workspace(lin.out_features, lin.in_features, T));
+    if (dtype == LT_BF16) s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_mid_splitk_workspace(lin.out_features, lin.in_features, T));
     s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_generic_splitk_workspace(lin.out_features, lin.in_features, T));
     if (lin.lowrank == 0) {
       s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_generic_splitk_workspace(T, lin.in_features, lin.out_features));

@@ -56,27 +56,47 @@ bool lt_sparse_mfma_supported(const GemmProblem& p, int kind);
 
 namespace {
 int64_t mid_tiles(int64_t M, int64_t N) { return ((M + 127) / 128) * ((N + 127) / 128); }
-// 128 x 128 tiles where they all run at once, two workgroups per CU; 256 x 256 ones then fill half of the chip at most.  [1024, 8192]
-// over 2048 (512 of them): 37 us against 47; [1536, 6400] over 1600 (600): 51 against 44.
-bool mid_selected(const GemmProblem& p, int kind) {
-  const int64_t columns = kind == EPI_ACT_FWD && p.epi.gated ? 2 * p.N : p.N;
-  return mid_tiles(p.M, columns) <= 512 && lt_gemm_mid_supported(p, kind);
-}
-// Slices of such a product's reduction: the least estimated time.  64 k take a workgroup 0.45 us alone on its CU, two of them 0.95 us
-// (measured on [128 - 4096, 2048] over 8192: 53 - 69 us for up to 256 workgroups, 125 for 512); a slice costs a write and a read of
-// its fp32 partial result at 5 TB/s, the sum a launch.
-int mid_slices(int64_t M, int64_t N, int64_t K) {
-  const int64_t tiles = mid_tiles(M, N), stages = (K + 63) / 64;
-  int best = 1;
+
+// An unfused product's reduction over `stages` stages, split into the number of slices with the least estimated time; returns it in
+// us.  A round of `tiles` * slices workgroups takes stage_us(workgroups) per stage; a slice costs a write and a read of its fp32
+// partial result at 5 TB/s, the sum a launch.
+template <typename F> double best_slices(int64_t M, int64_t N, int64_t tiles, int64_t stages, int64_t max_workgroups, F&& stage_us, int& slices) {
   double best_us = 1e30;
-  for (int s = 1; s <= 16 && (s == 1 || (tiles * s <= 512 && stages / s >= 4)); s++) {
-    const double us = (double)((stages + s - 1) / s) * (tiles * s <= 256 ? 0.45 : 0.95) + (s > 1 ? s * (double)M * N * 8.0 / 5e6 + 4.0 : 0.0);
+  slices = 1;
+  for (int s = 1; s <= 16 && (s == 1 || (tiles * s <= max_workgroups && stages / s >= 4)); s++) {
+    const double us = (double)((stages + s - 1) / s) * stage_us(tiles * s) + (s > 1 ? s * (double)M * N * 8.0 / 5e6 + 4.0 : 0.0);
     if (us < best_us * 0.97) {
       best_us = us;
-      best = s;
+      slices = s;
     }
   }
-  return best;
+  return best_us;
+}
+// 128 x 128 tiles: 64 k take a workgroup 0.45 us alone on its CU, two of them 0.95 us (measured on [128 - 4096, 2048] over 8192: 53 - 69
+// us for up to 256 workgroups, 125 for 512)
+double mid_best(int64_t M, int64_t N, int64_t K, int& slices) {
+  return best_slices(M, N, mid_tiles(M, N), (K + 63) / 64, 512, [](int64_t w) { return w <= 256 ? 0.45 : 0.95; }, slices);
+}
+int mid_slices(int64_t M, int64_t N, int64_t K) {
+  int slices;
+  mid_best(M, N, K, slices);
+  return slices;
+}
+int splitk_slices(int64_t M, int64_t N, int64_t K);
+// 128 x 128 tiles where they all run at once, two workgroups per CU; 256 x 256 ones then fill half of the chip at most.  [1024, 8192]
+// over 2048 (512 of them): 37 us against 47; [1536, 6400] over 1600 (600): 51 against 44.  A weight gradient's reduction (both operands
+// mn-major) is long and split in either kernel, so there the estimates are compared: 64 k of a 256 x 256 tile take 1.2 us, and its
+// start and end 5 us more.
+bool mid_selected(const GemmProblem& p, int kind) {
+  const int64_t columns = kind == EPI_ACT_FWD && p.epi.gated ? 2 * p.N : p.N;
+  if (mid_tiles(p.M, columns) > 512 || !lt_gemm_mid_supported(p, kind)) return false;
+  if (p.A[0].kmajor) return true;
+  int slices;
+  const double mid_us = mid_best(p.M, p.N, p.K[0], slices);
+  const int64_t s = splitk_slices(p.M, p.N, p.K[0]), tiles = ((p.M + 255) / 256) * ((p.N + 255) / 256);
+  const double us = (double)((tiles * s + 255) / 256) * ((double)((p.K[0] + 63) / 64 + s - 1) / s * 1.2 + 5.0) +
+                    (s > 1 ? s * (double)p.M * p.N * 8.0 / 5e6 + 4.0 : 0.0);
+  return mid_us < us;
 }
 }  // namespace
 

@@ -1,5 +1,5 @@
-// Tiled 16-bit products of a middling number of rows (65 to about a thousand: a prompt, a short training batch): 128 x 128 tiles, operands
-// copied global -> LDS, A k-major, B k-major or mn-major, the fused epilogues of the copy-based 256 x 256 kernel.
+// Tiled 16-bit products of a middling number of rows (65 to about a thousand: a prompt, a short training batch; gradients of small
+// factors): 128 x 128 tiles, operands copied global -> LDS, the operand layouts and fused epilogues of the copy-based 256 x 256 kernel.
 //
 // What bounds it: 256 x 256 tiles of [512, 8192] are 64 workgroups for 256 CUs, each walking the whole reduction; four times as many
 // tiles fill the chip, at the price of LDS bandwidth: a wavefront's 64 x 64 sub-tile reads as many cycles of LDS as it has of
@@ -62,7 +62,7 @@ template <bool KM> struct MidOperand {
   }
 };
 
-template <bool B_KM, int KIND, typename TX, int ACT, int STAGES>
+template <bool A_KM, bool B_KM, int KIND, typename TX, int ACT, int STAGES>
 __global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int tiles_m, int tiles_n) {
   static_assert(STAGES == 2 || STAGES == 4, "stages");
   constexpr int ELEMS = MID * 64;
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int t
   }
   const int rot = total > 0 ? (int)(((blockIdx.x & 7) * (unsigned)(total >> 3) + ((blockIdx.x >> 3) & 7)) % (unsigned)total) : 0;
   const int k_limit = (int)p.K[0];
-  MidOperand<true> ca;
+  MidOperand<A_KM> ca;
   MidOperand<B_KM> cb;
   ca.setup(p.A[0], m0, p.M, 0, wave, lane);
   cb.setup(p.B[0], n0, p.N, gated ? p.N : 0, wave, lane);
@@ -147,7 +147,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int t
       bf16x8 a[2], b[2];
 #pragma unroll
       for (int i = 0; i < 2; i++) {
-        a[i] = frag_km(a_buf(S), wm * 64 + i * 32, kk);
+        if constexpr (A_KM) a[i] = frag_km(a_buf(S), wm * 64 + i * 32, kk);
+        else a[i] = frag_mn(a_buf(S), wm * 64 + i * 32, kk);
         if constexpr (B_KM) b[i] = frag_km(b_buf(S), wn * 64 + i * 32, kk);
         else b[i] = frag_mn(b_buf(S), wn * 64 + i * 32, kk);
       }
@@ -265,16 +266,16 @@ __global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int t
   }
 }
 
-template <bool B_KM, int KIND, typename TX> int launch_mid(const GemmProblem& p, hipStream_t stream) {
+template <bool A_KM, bool B_KM, int KIND, typename TX> int launch_mid(const GemmProblem& p, hipStream_t stream) {
   const bool gated = KIND == EPI_ACT_FWD && p.epi.gated;
   const int tiles_m = (int)((p.M + MID - 1) / MID), tiles_n = (int)((p.N + (gated ? 63 : 127)) / (gated ? 64 : 128));
   const int slices = p.ksplit > 1 ? p.ksplit : 1;
   const dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)slices), block(256);
   with_activation<KIND>(p, [&](auto ACT) {
     if (tiles_m * tiles_n * slices <= 256)
-      hipLaunchKernelGGL((gemm_bf16_mid_kernel<B_KM, KIND, TX, decltype(ACT)::value, 4>), grid, block, 0, stream, p, tiles_m, tiles_n);
+      hipLaunchKernelGGL((gemm_bf16_mid_kernel<A_KM, B_KM, KIND, TX, decltype(ACT)::value, 4>), grid, block, 0, stream, p, tiles_m, tiles_n);
     else
-      hipLaunchKernelGGL((gemm_bf16_mid_kernel<B_KM, KIND, TX, decltype(ACT)::value, 2>), grid, block, 0, stream, p, tiles_m, tiles_n);
+      hipLaunchKernelGGL((gemm_bf16_mid_kernel<A_KM, B_KM, KIND, TX, decltype(ACT)::value, 2>), grid, block, 0, stream, p, tiles_m, tiles_n);
   });
   LT_LAUNCH_CHECK();
   return LT_OK;
@@ -283,15 +284,16 @@ template <bool B_KM, int KIND, typename TX> int launch_mid(const GemmProblem& p,
 }  // namespace
 
 bool lt_gemm_mid_supported(const GemmProblem& p, int kind) {
-  return p.nseg == 1 && p.sp.mode == SPARSE_NONE && p.variant == 0 && p.A[0].kmajor && p.K[0] < (int64_t)1 << 30 &&
+  return p.nseg == 1 && p.sp.mode == SPARSE_NONE && p.variant == 0 && p.K[0] < (int64_t)1 << 30 &&
          lt_gemm_mfma_supported(p, kind) && dma_offsets_fit(p, kind);
 }
 
 int lt_launch_gemm_mid(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream) {
   LT_REQUIRE(lt_gemm_mid_supported(p, kind), LT_ERR_UNSUPPORTED, "128 x 128 gemm does not take this problem");
   const bool b_km = p.B[0].kmajor;
-  if (kind == EPI_STORE) return b_km ? launch_mid<true, EPI_STORE, float>(p, stream) : launch_mid<false, EPI_STORE, float>(p, stream);
-  if (kind == EPI_ACT_FWD) return launch_mid<true, EPI_ACT_FWD, float>(p, stream);
-  if (kind == EPI_ACT_BWD) return launch_mid<false, EPI_ACT_BWD, float>(p, stream);
-  return io_dtype == LT_BF16 ? launch_mid<true, EPI_OUT, bf16>(p, stream) : launch_mid<true, EPI_OUT, float>(p, stream);
+  if (kind == EPI_STORE && !p.A[0].kmajor) return launch_mid<false, false, EPI_STORE, float>(p, stream);
+  if (kind == EPI_STORE) return b_km ? launch_mid<true, true, EPI_STORE, float>(p, stream) : launch_mid<true, false, EPI_STORE, float>(p, stream);
+  if (kind == EPI_ACT_FWD) return launch_mid<true, true, EPI_ACT_FWD, float>(p, stream);
+  if (kind == EPI_ACT_BWD) return launch_mid<true, false, EPI_ACT_BWD, float>(p, stream);
+  return io_dtype == LT_BF16 ? launch_mid<true, true, EPI_OUT, bf16>(p, stream) : launch_mid<true, true, EPI_OUT, float>(p, stream);
 }

@@ -16,13 +16,16 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("b_kmajor", [True, False])
+@pytest.mark.parametrize("a_kmajor,b_kmajor", [(True, True), (True, False), (False, False)])
 @pytest.mark.parametrize("m,n,k", [(65, 8, 8), (127, 72, 64), (128, 128, 72), (129, 136, 192), (300, 264, 256), (192, 520, 264),
                                    (66, 64, 1000), (1000, 5000, 136)])
-def test_gemm(dtype, b_kmajor, m, n, k):
+def test_gemm(dtype, a_kmajor, b_kmajor, m, n, k):
     g = torch.Generator(device=DEV).manual_seed(m + n + k)
     a, b = torch.randn(m, k, generator=g, device=DEV).to(dtype), torch.randn(n, k, generator=g, device=DEV).to(dtype)
-    c = _gemm(a, b if b_kmajor else b.t().contiguous(), True, b_kmajor, m, n, k, torch.float32, 0)
+    m8 = m if a_kmajor else -(-m // 8) * 8  # (an mn-major A has rows of a multiple of 8 elements)
+    a = torch.cat([a, a[:m8 - m]])
+    c = _gemm(a if a_kmajor else a.t().contiguous(), b if b_kmajor else b.t().contiguous(), a_kmajor, b_kmajor, m8, n, k,
+              torch.float32, 0)
     worst = (c.double() - a.double() @ b.double().t()).abs() - (k + 16) * 2.0**-23 * (a.double().abs() @ b.double().abs().t())
     assert worst.max().item() <= 0.0
 
