@@ -724,6 +724,16 @@ template <bool KM> struct DmaOperand {
     unit_bytes = KM ? 64 * 2 : DK * ld * 2;
   }
 
+  // a tile of `columns` < 256: what the buffer holds past them is not fetched (the buffer unit returns zeros)
+  __device__ __forceinline__ void keep_columns(int columns, int wave, int lane) {
+#pragma unroll
+    for (int j = 0; j < LOADS; j++) {
+      const int q = (wave * LOADS + j) * 64 + lane;
+      const int column = KM ? q >> 3 : ((q & 31) ^ swz_mn(q >> 5)) * 8;
+      if (column >= columns) off[j] = OUTSIDE;
+    }
+  }
+
   // mn-major operand whose 256 tile columns are four 64-wide column blocks gathered from anywhere in the matrix: block j of
   // the tile is the operand's column block blocks[j]
   __device__ __forceinline__ void setup_gather(const GemmOperand& op, const int (&blocks)[4], int wave, int lane) {
@@ -823,8 +833,8 @@ __device__ __forceinline__ int lt_run_member(int t, int j, int len, int stride) 
   return t / quads + stride * ((t % quads) * 4 + j);
 }
 
-// Epilogue of one wavefront's (FM * 32) x 128 sub-tile of a copy-based kernel: acc[i][j] is the 32 x 32 block at rows
-// m0 + wm * WTM + 32 i, columns n0 + wn * 128 + 32 j of the result (gated forward: blocks 0, 1 gate columns, 2, 3 the
+// Epilogue of one wavefront's (FM * 32) x (FN * 32) sub-tile of a copy-based kernel: acc[i][j] is the 32 x 32 block at rows
+// m0 + wm * WTM + 32 i, columns n0 + wn * FN * 32 + 32 j of the result (gated forward: blocks 0, 1 gate columns, 2, 3 the
 // matching linear columns).  `stage` is 16 KiB of LDS that belongs to this wavefront alone; tile_rows x tile_cols is the
 // workgroup's tile (for the whole-tile test).  The bias is already in the accumulators.
 // SCATTER (EPI_STORE only; the grouped block-sparse weight gradient): the tile is 4 output blocks (rows) x 4 entries of
@@ -833,10 +843,12 @@ __device__ __forceinline__ int lt_run_member(int t, int j, int len, int stride) 
 // SCATTER == 2: the tile is 4 entries of a list of output blocks (rows) x the run of 4 input blocks that shares the list
 // (columns); piece (entry a, input block ib) is block ib * blocks_per_in + a.
 // ACT: the activation of EPI_ACT_FWD / EPI_ACT_BWD, or -1: chosen per element from epi.act.
-template <int FM, int KIND, typename TX, int tile_rows, int tile_cols, int SCATTER = 0, int ACT = -1>
-__device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const GemmProblem& p, float* stage, const int64_t m0,
+template <int FM, int KIND, typename TX, int tile_rows, int tile_cols, int SCATTER = 0, int ACT = -1, int FN>
+__device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][FN], const GemmProblem& p, float* stage, const int64_t m0,
                                                   const int64_t n0, const int wm, const int wn, const bool gated) {
-  constexpr int FN = 4, WTN = 128, WTM = FM * 32;
+  // (FN == 3: four of the 16 lanes of a row would have no columns; they repeat the last 8, reads and stores alike)
+  constexpr int WTN = FN * 32, WTM = FM * 32, PITCH = 128, ROW_LANES = PITCH / 8;
+  static_assert(FN == 4 || (FN == 3 && SCATTER == 0 && (KIND == EPI_STORE || KIND == EPI_OUT)), "narrow tiles: plain epilogues");
   constexpr bool STRAIGHT_ACT = ACT == LT_ACT_GELU_FUSED || ACT == LT_ACT_SILU;  // short enough to be unrolled
   // the lane index is formed anew rather than kept in a register across the main loop, through an asm statement so that a
   // workgroup that loops over tiles does not keep what is derived from it alive from one tile's epilogue to the next's either
@@ -851,7 +863,7 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
   EpiParams epi = p.epi;
   epi.bias = nullptr;  // already in the accumulators
   if (KIND == EPI_STORE && p.ksplit > 1) epi.out = reinterpret_cast<float*>(epi.out) + (int64_t)blockIdx.y * p.split_stride;
-  auto staged = [&](int row, int col) -> float* { return &stage[row * WTN + (col ^ (((row >> 2) & 1) << 5))]; };
+  auto staged = [&](int row, int col) -> float* { return &stage[row * PITCH + (col ^ (((row >> 2) & 1) << 5))]; };
   const bool pair = (KIND == EPI_ACT_FWD) && gated;
   float colsum[16];  // EPI_ACT_BWD: column sums of this lane's 8 (+ 8) dpre columns over the rows it writes
 #pragma unroll
@@ -907,8 +919,8 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
         }
       }
     } else {
-      constexpr int LANES_PER_ROW = WTN / 8, ROWS_PER_IT = 64 / LANES_PER_ROW, NIT = 32 / ROWS_PER_IT;
-      const int c = (lane % LANES_PER_ROW) * 8;
+      constexpr int LANES_PER_ROW = ROW_LANES, ROWS_PER_IT = 64 / LANES_PER_ROW, NIT = 32 / ROWS_PER_IT;
+      const int c = min((lane % LANES_PER_ROW) * 8, WTN - 8);
       const int64_t n = n0 + wn * WTN + c;
       const bool in_n = n < p.N;  // N is a multiple of 8: the lane's 8 columns are all inside or all outside
       constexpr int AHEAD = 4;  // rows of reads in flight
@@ -969,8 +981,8 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
   auto act_bwd_strip = [&](auto I, auto G) {
     constexpr int i = decltype(I)::value;
     constexpr bool GATED = decltype(G)::value;
-    constexpr int LANES_PER_ROW = WTN / 8, ROWS_PER_IT = 64 / LANES_PER_ROW, NIT = 32 / ROWS_PER_IT;
-    const int c = (lane % LANES_PER_ROW) * 8;
+    constexpr int LANES_PER_ROW = ROW_LANES, ROWS_PER_IT = 64 / LANES_PER_ROW, NIT = 32 / ROWS_PER_IT;
+    const int c = min((lane % LANES_PER_ROW) * 8, WTN - 8);
     const int64_t n = n0 + wn * WTN + c;
     const int64_t mlane = m0 + wm * WTM + i * 32 + lane / LANES_PER_ROW;
     EpiLoad win[ACT_WINDOW];
@@ -1007,8 +1019,8 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
   auto store_strip = [&](auto I, auto out_type) {
     using TO = decltype(out_type);
     constexpr int i = decltype(I)::value;
-    constexpr int LANES_PER_ROW = WTN / 8, ROWS_PER_IT = 64 / LANES_PER_ROW, NIT = 32 / ROWS_PER_IT;
-    const int c = (lane % LANES_PER_ROW) * 8;
+    constexpr int LANES_PER_ROW = ROW_LANES, ROWS_PER_IT = 64 / LANES_PER_ROW, NIT = 32 / ROWS_PER_IT;
+    const int c = min((lane % LANES_PER_ROW) * 8, WTN - 8);
     const int64_t n = n0 + wn * WTN + c;
     const int64_t mlane = m0 + wm * WTM + i * 32 + lane / LANES_PER_ROW;
     stage_strip(I);
@@ -1021,8 +1033,8 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
   auto out_strip = [&](auto I, auto D) {
     constexpr bool DROPOUT = decltype(D)::value;
     constexpr int i = decltype(I)::value;
-    constexpr int LANES_PER_ROW = WTN / 8, ROWS_PER_IT = 64 / LANES_PER_ROW, NIT = 32 / ROWS_PER_IT;
-    const int c = (lane % LANES_PER_ROW) * 8;
+    constexpr int LANES_PER_ROW = ROW_LANES, ROWS_PER_IT = 64 / LANES_PER_ROW, NIT = 32 / ROWS_PER_IT;
+    const int c = min((lane % LANES_PER_ROW) * 8, WTN - 8);
     const int64_t n = n0 + wn * WTN + c;
     const int64_t mlane = m0 + wm * WTM + i * 32 + lane / LANES_PER_ROW;
     EpiLoad win[ACT_WINDOW];
@@ -1041,8 +1053,8 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
   auto scatter_strip = [&](auto I, auto out_type) {
     using TO = decltype(out_type);
     constexpr int i = decltype(I)::value;
-    constexpr int LANES_PER_ROW = WTN / 8, ROWS_PER_IT = 64 / LANES_PER_ROW, NIT = 32 / ROWS_PER_IT;
-    const int c = (lane % LANES_PER_ROW) * 8;
+    constexpr int LANES_PER_ROW = ROW_LANES, ROWS_PER_IT = 64 / LANES_PER_ROW, NIT = 32 / ROWS_PER_IT;
+    const int c = min((lane % LANES_PER_ROW) * 8, WTN - 8);
     int per_out, entry;  // length of the list, position in it
     int64_t flat;
     if constexpr (SCATTER == 1) {
@@ -1140,7 +1152,10 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][4], const Ge
 //   ib_e) and so form one [256 rows][64 k] k-major matrix.  The list sits in one register (lane e: ib_e << 16 | flat
 //   position) and is read with v_readlane, so the k-loop issues no memory instruction for it.  A second k-segment (the
 //   low-rank term) is an ordinary one.
-template <bool A_KM, bool B_KM, int KIND, typename TX, int GATHER = 0, int ACT = -1>
+//
+// FN == 3: tiles of 256 x 192, plain epilogues only.  The buffers stay those of 256 columns; copies of the last 64 are not fetched.
+// Chosen in launch_dma.
+template <bool A_KM, bool B_KM, int KIND, typename TX, int GATHER = 0, int ACT = -1, int FN = 4>
 __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem, int tiles_m, int tiles_n) {
   // A workgroup may loop over tiles.  Whatever the compiler finds to be the same in every tile -- values loaded from the problem
   // description, the wavefront's LDS addresses, lane offsets -- it would compute once and keep in registers across the whole
@@ -1155,7 +1170,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
 #define p (*pk)
   static_assert((GATHER != 1 && GATHER != 3) || (!A_KM && !B_KM && KIND == EPI_STORE), "gathered columns: weight-gradient layout");
   static_assert(GATHER != 2 || (A_KM && B_KM), "gathered k-blocks: forward layout");
-  constexpr int BM = 256, BN = 256, WN = 2, WTM = 128, WTN = 128, FM = 4, FN = 4;
+  constexpr int BM = 256, BN = 64 * FN, WN = 2, WTM = 128, WTN = 32 * FN, FM = 4;
+  static_assert(FN == 4 || (FN == 3 && GATHER == 0), "tile width");
   constexpr int HALF = 4;  // copy instructions per wavefront for a mn-major k-step or half a k-major block
   constexpr int KM_ELEMS = 256 * 64, MN_ELEMS = DK * 256;
   // k-major operands use the two d buffers, mn-major ones the four s tiles; the unused set is never referenced and takes
@@ -1347,6 +1363,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
     } else {
       const GemmOperand b = {p.B[seg].ptr, p.B[seg].ld, p.B[seg].kmajor};
       cb.setup(b, seg, n0, p.N, (B_KM && gated) ? p.N : 0, wave, lane);
+      if constexpr (FN < 4) cb.keep_columns(BN, wave, lane);
     }
   };
   setup_a(0);
@@ -1400,22 +1417,22 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
     const bf16* ta = a_buf(I);
     const bf16* tb = b_buf(I);
     // pair (A block i, B block i) after pair i - 1: the order in which the matrix instructions below first need them
-    static_assert(FM == FN, "reads alternate between the operands");
 #pragma unroll
     for (int i = 0; i < FM; i++) {
       if constexpr (A_KM) a[i] = frag_km(ta, wm * WTM + i * 32, kk, half);
       else a[i] = frag_mn(ta, wm * WTM + i * 32, kk);
+      if (i >= FN) continue;
       if constexpr (B_KM) b[i] = frag_km(tb, wn * WTN + i * 32, kk, half);
       else b[i] = frag_mn(tb, wn * WTN + i * 32, kk);
     }
   };
-  // the 16 matrix instructions of a half-step, in the order in which their fragments arrive (pair 0 first, pair 3 last):
+  // the 16 matrix instructions of a half-step (FN == 3: the first 12), in the order in which their fragments arrive (pair 0 first, pair 3 last):
   // the wait before the first one then covers two LDS reads, not all eight
   auto mfma_half = [&](bf16x8 (&a)[FM], bf16x8 (&b)[FN]) {
     constexpr int ORDER[16][2] = {{0, 0}, {1, 0}, {0, 1}, {1, 1}, {2, 0}, {2, 1}, {0, 2}, {1, 2},
                                   {2, 2}, {3, 0}, {3, 1}, {3, 2}, {0, 3}, {1, 3}, {2, 3}, {3, 3}};
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
+    for (int q = 0; q < FM * FN; q++) {
       const int x = ORDER[q][0], y = ORDER[q][1];
       acc[x][y] = LT_MFMA_32X32X16(a[x], b[y], acc[x][y]);
     }
@@ -1633,7 +1650,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
     LT_TILE_STAMP_REALTIME(4);
     LT_TILE_STAMP(6);
   }
-  static_assert(32 * WTN * 4 <= MN_ELEMS * 2, "a 32-row strip must fit the smallest buffer");
+  static_assert(32 * 128 * 4 <= MN_ELEMS * 2, "a 32-row strip must fit the smallest buffer");
 #undef p
 }
 
@@ -1681,6 +1698,22 @@ int launch_dma(const GemmProblem& problem, int io_dtype, hipStream_t stream) {
   const int tiles_n = (int)((p.N + (gated ? 127 : 255)) / (gated ? 128 : 256));
   dim3 grid(dma_grid(p, tiles_m * tiles_n), (unsigned)(p.ksplit > 1 ? p.ksplit : 1)), block(256);
   const bool bf16_io = KIND == EPI_OUT && io_dtype == LT_BF16;
+  // Tiles of 192 columns where that takes no more rounds of up to 256 tiles: each round is then 3/4 as long in matrix instructions,
+  // though not in copies, which is why one more round is not worth it.  256 against 192 columns, T 16384: [T, 768] over 2304 (192 or
+  // 256 tiles) 66 us, 58; over 6144 176, 166; down-projection [T, 768] over 3072 103, 100; [T, 2304] over 768 (three rounds) 79, 75.
+  if constexpr (A_KM && (KIND == EPI_STORE || KIND == EPI_OUT)) {
+    const int narrow_n = (int)((p.N + 191) / 192);
+    const int64_t wide_rounds = ((int64_t)tiles_m * tiles_n + 255) / 256, narrow_rounds = ((int64_t)tiles_m * narrow_n + 255) / 256;
+    if (p.ksplit <= 1 && narrow_n > tiles_n && narrow_rounds == wide_rounds) {
+      grid.x = dma_grid(p, tiles_m * narrow_n);
+      if (KIND == EPI_OUT && bf16_io)
+        hipLaunchKernelGGL((gemm_bf16_dma_kernel<A_KM, B_KM, KIND, bf16, 0, -1, 3>), grid, block, 0, stream, p, tiles_m, narrow_n);
+      else
+        hipLaunchKernelGGL((gemm_bf16_dma_kernel<A_KM, B_KM, KIND, float, 0, -1, 3>), grid, block, 0, stream, p, tiles_m, narrow_n);
+      LT_LAUNCH_CHECK();
+      return LT_OK;
+    }
+  }
   // the type of x / y only enters the EPI_OUT epilogue: the other kinds have one instantiation
   if constexpr (KIND == EPI_OUT) {
     if (bf16_io) {
