@@ -240,6 +240,11 @@ int lt_dropout_mask(int64_t tokens, int32_t hidden, float p, uint64_t seed, uint
  * may run concurrently with every other entry point. */
 int lt_gemm(int32_t dtype, int64_t m, int64_t n, int64_t k, const void* a, int32_t a_kmajor, const void* b,
             int32_t b_kmajor, int32_t c_dtype, void* c, int32_t force_generic, void* stream);
+/* C = op(A0) op(B0) + op(A1) op(B1) in one launch, as a projection and its low-rank term are computed: lt_gemm with a second pair
+ * of operands of the same layouts and a reduction of k1. */
+int lt_gemm_two_segments(int32_t dtype, int64_t m, int64_t n, int64_t k0, const void* a0, const void* b0, int64_t k1,
+                         const void* a1, const void* b1, int32_t a_kmajor, int32_t b_kmajor, int32_t c_dtype, void* c,
+                         int32_t force_generic, void* stream);
 
 /* ---- per-kernel timing (no counterpart in the reference: measurement only) ----------------------------------------------
  * While enabled, every kernel launch of the library is bracketed by two HIP events recorded on the launch stream.

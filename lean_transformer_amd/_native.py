@@ -26,7 +26,7 @@ EXPORTED_SYMBOLS = (
     "lt_blocksparse_forward", "lt_blocksparse_backward",
     "lt_layernorm_forward", "lt_layernorm_backward_workspace_bytes", "lt_layernorm_backward",
     "lt_layernorm_backward_static_scratch_bytes", "lt_layernorm_backward_static",
-    "lt_activation_forward", "lt_activation_backward", "lt_dropout_mask", "lt_gemm",
+    "lt_activation_forward", "lt_activation_backward", "lt_dropout_mask", "lt_gemm", "lt_gemm_two_segments",
     "lt_profile_enable", "lt_profile_reset", "lt_profile_read",
 )
 
@@ -108,6 +108,8 @@ def _declare(lib):
     lib.lt_dropout_mask.argtypes = [c_int64, c_int32, c_float, c_uint64, c_uint64, c_void_p, c_void_p]
     lib.lt_gemm.argtypes = [c_int32, c_int64, c_int64, c_int64, c_void_p, c_int32, c_void_p, c_int32, c_int32, c_void_p,
                             c_int32, c_void_p]
+    lib.lt_gemm_two_segments.argtypes = [c_int32, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_void_p,
+                                         c_int32, c_int32, c_int32, c_void_p, c_int32, c_void_p]
     lib.lt_profile_enable.argtypes = [c_int32]
     lib.lt_profile_reset.argtypes = []
     lib.lt_profile_read.argtypes = [POINTER(LtProfileEntry), c_int32]

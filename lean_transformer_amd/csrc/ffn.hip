@@ -736,6 +736,18 @@ extern "C" int lt_dropout_mask(int64_t tokens, int32_t hidden, float p, uint64_t
   return lt_dropout_mask_launch(tokens * hidden, keep, make_dropout(p, seed, offset), (hipStream_t)stream);
 }
 
+namespace {
+int launch_plain_gemm(GemmProblem& p, int32_t dtype, int32_t c_dtype, void* c, int32_t flags, void* stream) {
+  p.epi = epi_store_params(c, p.N, c_dtype, nullptr);
+  p.krot = (flags >> 4) & 15;
+  p.tile_loop = (flags >> 8) & 1;
+  const int kernel = flags & 15;
+  if (kernel == 1) return lt_launch_gemm_generic(p, EPI_STORE, dtype, dtype, (hipStream_t)stream);
+  p.variant = kernel == 2 ? 1 : kernel == 3 ? 2 : 0;
+  return lt_launch_gemm(p, EPI_STORE, dtype, dtype, (hipStream_t)stream);
+}
+}  // namespace
+
 extern "C" int lt_gemm(int32_t dtype, int64_t m, int64_t n, int64_t k, const void* a, int32_t a_kmajor, const void* b,
                        int32_t b_kmajor, int32_t c_dtype, void* c, int32_t force_generic, void* stream) {
   LT_TRY(check_dtype(dtype, "gemm"));
@@ -745,11 +757,21 @@ extern "C" int lt_gemm(int32_t dtype, int64_t m, int64_t n, int64_t k, const voi
   p.M = m; p.N = n; p.K[0] = k;
   p.A[0] = operand(a, a_kmajor ? k : m, a_kmajor);
   p.B[0] = operand(b, b_kmajor ? k : n, b_kmajor);
-  p.epi = epi_store_params(c, n, c_dtype, nullptr);
-  p.krot = (force_generic >> 4) & 15;
-  p.tile_loop = (force_generic >> 8) & 1;
-  force_generic &= 15;
-  if (force_generic == 1) return lt_launch_gemm_generic(p, EPI_STORE, dtype, dtype, (hipStream_t)stream);
-  p.variant = force_generic == 2 ? 1 : force_generic == 3 ? 2 : 0;
-  return lt_launch_gemm(p, EPI_STORE, dtype, dtype, (hipStream_t)stream);
+  return launch_plain_gemm(p, dtype, c_dtype, c, force_generic, stream);
+}
+
+extern "C" int lt_gemm_two_segments(int32_t dtype, int64_t m, int64_t n, int64_t k0, const void* a0, const void* b0, int64_t k1,
+                                    const void* a1, const void* b1, int32_t a_kmajor, int32_t b_kmajor, int32_t c_dtype, void* c,
+                                    int32_t force_generic, void* stream) {
+  LT_TRY(check_dtype(dtype, "gemm"));
+  LT_TRY(check_dtype(c_dtype, "gemm output"));
+  LT_REQUIRE(a0 && b0 && a1 && b1 && c && m > 0 && n > 0 && k0 > 0 && k1 > 0, LT_ERR_BAD_ARG, "gemm: bad arguments");
+  GemmProblem p = blank_problem();
+  p.M = m; p.N = n; p.nseg = 2;
+  p.K[0] = k0; p.K[1] = k1;
+  p.A[0] = operand(a0, a_kmajor ? k0 : m, a_kmajor);
+  p.B[0] = operand(b0, b_kmajor ? k0 : n, b_kmajor);
+  p.A[1] = operand(a1, a_kmajor ? k1 : m, a_kmajor);
+  p.B[1] = operand(b1, b_kmajor ? k1 : n, b_kmajor);
+  return launch_plain_gemm(p, dtype, c_dtype, c, force_generic, stream);
 }

@@ -371,8 +371,9 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
       __syncthreads();
       // steps whose next step has whole k-major tiles, then the rest: with the test for a ragged end in every step the
       // input-gradient walk of a PixelFly layer (hidden 4096) takes 244 us instead of 206
-      const int seg_last = kt_total > kt_seg0;
-      const int kt_whole = SP == SPARSE_DW || p.K[seg_last] % BK == 0 ? kt_end : min(kt_end, kt_total - 1);
+      const int kt_whole = SP == SPARSE_DW ? kt_end
+                                           : min(kt_end, lt_leading_whole_steps(SP == SPARSE_NONE ? p.K[0] : (int64_t)kt_seg0 * BK,
+                                                                                kt_total > kt_seg0 ? p.K[1] : 0, BK));
       int kt = kt_begin;
       for (; kt + 1 < kt_whole; kt++) {
         load_tiles(Whole{}, kt + 1, ph, ra_set[0], rb_set[0]);
