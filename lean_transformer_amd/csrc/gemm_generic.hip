@@ -406,13 +406,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
   }
   __syncthreads();
   for (int t = 0; t < total;) {
-    if (vectors()) {
-      while (t + 3 < total && k0 + 2 * BK <= g.K) {
+    if (t + 3 < total && k0 + 2 * BK <= g.K && vectors()) {
+      const int s = seg;  // (the next segment has an alignment of its own)
+      do {
         step_whole(S0{});
         step_whole(S1{});
         t += 2;
         next_segment();
-      }
+      } while (seg == s && t + 3 < total && k0 + 2 * BK <= g.K);
+      if (seg != s) continue;
     }
     if (t < total) step_ragged(S0{}, t++);
     if (t < total) step_ragged(S1{}, t++);

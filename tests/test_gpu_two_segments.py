@@ -36,3 +36,16 @@ def test_tiled_kernels(a_kmajor, b_kmajor, k0, k1, force):
     (c, ref, mag), tags = _kernel_tags(lambda: two_segments(torch.bfloat16, 300, 512, k0, k1, a_kmajor, b_kmajor, force))
     assert all(t.startswith("gemm_bf16_n") for t in tags), tags
     assert ((c.double() - ref).abs() - (k0 + k1 + 16) * 2.0**-23 * mag).max().item() <= 0.0
+
+
+@pytest.mark.parametrize("a_kmajor,b_kmajor", [(True, True), (True, False), (False, False), (False, True)])
+@pytest.mark.parametrize("dtype,k0,k1", [(torch.float32, 768, 34), (torch.float32, 96, 33), (torch.float32, 33, 96),
+                                         (torch.bfloat16, 128, 65), (torch.bfloat16, 192, 97), (torch.bfloat16, 65, 192)])
+@pytest.mark.parametrize("m,n", [(70, 45), (4100, 2100)])
+def test_any_shape_kernel(dtype, k0, k1, a_kmajor, b_kmajor, m, n):
+    """whole steps run from the first segment into the second, whose rows are not 16-byte aligned (rank 34 in fp32, 65 in 16 bits):
+    it must be fetched element by element, and the other way round; both tile heights"""
+    c, ref, mag = two_segments(dtype, m, n, k0, k1, a_kmajor, b_kmajor, 1)
+    k = k0 + k1
+    bound = 2.0**-23 * ((6 * (-(-k // 16) + 1) + 6) if dtype == torch.float32 else k + 16)  # (fp32: see test_gpu_any_shape.py)
+    assert ((c.double() - ref).abs() - bound * mag).max().item() <= 0.0
