@@ -456,7 +456,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
     }
     return sum;
   };
-  auto unflipped = [&](float v, int row) { return PLANES > 1 && (row & 1) ? -v : v; };  // (fp32: odd rows are negated)
+  // (fp32: odd rows are negated; 0 - v and not -v, so that a sum of zeros is +0 in every row)
+  auto unflipped = [&](float v, int row) { return PLANES > 1 && (row & 1) ? 0.f - v : v; };
 #pragma unroll
   for (int i = 0; i < FM; i++) {
     const int64_t mrow0 = m0 + wm * 32 * FM + i * 32;

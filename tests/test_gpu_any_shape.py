@@ -95,3 +95,10 @@ def test_fp32_infinities_and_nans(a_kmajor, b_kmajor, m, n, k):
     assert torch.equal(c[c.isinf()].sign(), ref[ref.isinf()].sign().float())
     finite = ref.isfinite()
     assert (c.double() - ref)[finite].abs().max().item() <= 1e-4
+
+
+def test_fp32_sums_of_zeros_are_positive():
+    """odd rows are negated on their way through the matrix cores; their zeros come back as +0, as any sum from +0 does"""
+    zeros, b = torch.zeros(70, 40, device=DEV), torch.randn(45, 40, device=DEV)
+    c = _gemm(zeros, b, True, True, 70, 45, 40, torch.float32, 1)
+    assert not bool(c.signbit().any()) and bool((c == 0).all())
