@@ -15,7 +15,7 @@
 // sums over many rows of a result would collect (a bias gradient is one over all tokens); odd rows of A are therefore negated
 // on the way in and odd rows of the result on the way out, so that the bias alternates.
 // An infinity has no such planes (inf - inf) and gives NaN; an element that comes out as NaN is therefore computed again, in fp32
-// arithmetic from the operands in memory, as the epilogue takes it up (a NaN among the operands ends that at once).
+// arithmetic from the operands in memory, as the epilogue takes it up (a NaN among its operands ends that where it is met).
 // What bounds it: at 4096^3 a full round of workgroups runs at 1.2 PFLOP/s of bfloat16 products, what the tiled 16-bit kernel
 // reaches on the same data (the clock under load); smaller products lose to a last round that is not full and to the start and
 // end of a tile.  4096^3: 1411 us with the fp32 instruction, 723 now; a training step of T = 4096, hidden 768: 2263 us, 1154 now;
@@ -445,14 +445,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
   if constexpr (KIND == EPI_OUT)
     vec = vec && (epi.ldy & 3) == 0 && ((reinterpret_cast<uintptr_t>(epi.x) | reinterpret_cast<uintptr_t>(epi.y)) & 15) == 0;
 
-  // element (row m of the tile's coordinates, row j of B) of fp32 operands, in fp32 arithmetic
+  // element (row m of the tile's coordinates, row j of B) of fp32 operands, in fp32 arithmetic; 8 k at a time, so that their loads
+  // wait for memory together, up to the 8 that hold a NaN
   auto element = [&](int64_t m, int64_t j) __attribute__((always_inline)) {
     float sum = 0.f;
     for (int s = 0; s < nseg; s++) {
       const Segment<TI> q = segment(s);
-      const int64_t end = s ? q.K : min(slice_k1, q.K);
-      for (int64_t k = s ? 0 : slice_k0; k < end && sum == sum; k++)
-        sum = fmaf(to_f32(A_KM ? q.A[m * q.lda + k] : q.A[k * q.lda + m]), to_f32(B_KM ? q.B[j * q.ldb + k] : q.B[k * q.ldb + j]), sum);
+      const int64_t end = s ? q.K : min(slice_k1, q.K), step_a = A_KM ? 1 : q.lda, step_b = B_KM ? 1 : q.ldb;
+      const TI* const row_a = q.A + (A_KM ? m * q.lda : m);
+      const TI* const row_b = q.B + (B_KM ? j * q.ldb : j);
+      for (int64_t k = s ? 0 : slice_k0; k < end && sum == sum; k += 8) {
+        float x[8], y[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const int64_t i = min(k + e, end - 1);
+          x[e] = to_f32(row_a[i * step_a]);
+          y[e] = to_f32(row_b[i * step_b]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) sum = k + e < end ? fmaf(x[e], y[e], sum) : sum;
+      }
     }
     return sum;
   };
