@@ -241,7 +241,9 @@ void plan_linear_backward(const lt_linear& lin, int64_t T, int dtype, Bump& ws, 
     s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_generic_splitk_workspace(lin.out_features, lin.in_features, T));
     if (lin.lowrank == 0) {
       s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_generic_splitk_workspace(T, lin.in_features, lin.out_features));
-      if (dtype == LT_BF16) s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_mid_splitk_workspace(T, lin.in_features, lin.out_features));
+      if (dtype == LT_BF16)
+        s.skinny_bytes = std::max({s.skinny_bytes, lt_gemm_mid_splitk_workspace(T, lin.in_features, lin.out_features),
+                                   lt_gemm_splitk_workspace(T, lin.in_features, lin.out_features)});
     }
   }
   if (lin.block == 64 && dtype == LT_BF16)

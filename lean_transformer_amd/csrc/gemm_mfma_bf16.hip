@@ -74,8 +74,8 @@ template <typename F> double best_slices(int64_t M, int64_t N, int64_t tiles, in
 }
 // 128 x 128 tiles: 64 k take a workgroup 0.45 us alone on its CU, two of them 0.95 us (measured on [128 - 4096, 2048] over 8192: 53 - 69
 // us for up to 256 workgroups, 125 for 512)
-double mid_best(int64_t M, int64_t N, int64_t K, int& slices) {
-  return best_slices(M, N, mid_tiles(M, N), (K + 63) / 64, 512, [](int64_t w) { return w <= 256 ? 0.45 : 0.95; }, slices);
+double mid_best(int64_t M, int64_t N, int64_t K, int& slices, double one = 0.45, double two = 0.95) {
+  return best_slices(M, N, mid_tiles(M, N), (K + 63) / 64, 512, [=](int64_t w) { return w <= 256 ? one : two; }, slices);
 }
 int mid_slices(int64_t M, int64_t N, int64_t K) {
   int slices;
@@ -84,19 +84,28 @@ int mid_slices(int64_t M, int64_t N, int64_t K) {
 }
 int splitk_slices(int64_t M, int64_t N, int64_t K);
 // 128 x 128 tiles where they all run at once, two workgroups per CU; 256 x 256 ones then fill half of the chip at most.  [1024, 8192]
-// over 2048 (512 of them): 37 us against 47; [1536, 6400] over 1600 (600): 51 against 44.  A weight gradient's reduction (both operands
-// mn-major) is long and split in either kernel, so there the estimates are compared: 64 k of a 256 x 256 tile take 1.2 us, and its
-// start and end 5 us more.
-bool mid_selected(const GemmProblem& p, int kind) {
+// over 2048 (512 of them): 37 us against 47; [1536, 6400] over 1600 (600): 51 against 44.  Where the product is unfused, the 256 x 256
+// kernel can split its reduction into as many slices as `room` (bytes of workspace) holds, and the estimates are compared:
+//   k-major A: 64 k take 0.58 us (two workgroups on a CU 1.04) against 1.45, and a start and an end of 15 us.  Down-projection of hidden
+//     4096 over 16384, T 1025 and 1790: 260 and 269 us against 209 and 238 in two slices; its input gradient, T 1024 and 1200: 170 and
+//     271 against 141 and 172; T 2048 (128 tiles of 256 x 256, unsplit): 271 against 374.  A tenth is left to the 128 x 128 tiles,
+//     within which either was the faster one.
+//   weight gradients (both operands mn-major): 64 k of a 256 x 256 tile take 1.2 us, and its start and end 5 us more.
+bool mid_selected(const GemmProblem& p, int kind, size_t room = 0) {
   const int64_t columns = kind == EPI_ACT_FWD && p.epi.gated ? 2 * p.N : p.N;
   if (mid_tiles(p.M, columns) > 512 || !lt_gemm_mid_supported(p, kind)) return false;
-  if (p.A[0].kmajor) return true;
+  const int64_t tiles = ((p.M + 255) / 256) * ((p.N + 255) / 256), stages = (p.K[0] + 63) / 64;
+  const double partial_us = (double)p.M * p.N * 4.0 / 5e6;  // a pass over one slice's partial sums
   int slices;
-  const double mid_us = mid_best(p.M, p.N, p.K[0], slices);
-  const int64_t s = splitk_slices(p.M, p.N, p.K[0]), tiles = ((p.M + 255) / 256) * ((p.N + 255) / 256);
-  const double us = (double)((tiles * s + 255) / 256) * ((double)((p.K[0] + 63) / 64 + s - 1) / s * 1.2 + 5.0) +
-                    (s > 1 ? s * (double)p.M * p.N * 8.0 / 5e6 + 4.0 : 0.0);
-  return mid_us < us;
+  int64_t s = splitk_slices(p.M, p.N, p.K[0]);
+  if (p.A[0].kmajor) {
+    s = std::min<int64_t>(s, (int64_t)(room / ((size_t)p.M * (size_t)p.N * sizeof(float))));
+    if (s <= 1) return true;
+    const double us = (double)((stages + s - 1) / s) * 1.45 + 15.0 + s * partial_us + 4.0;
+    return mid_best(p.M, p.N, p.K[0], slices, 0.58, 1.04) < 1.1 * us;
+  }
+  const double us = (double)((tiles * s + 255) / 256) * ((double)(stages + s - 1) / s * 1.2 + 5.0) + (s > 1 ? 2 * s * partial_us + 4.0 : 0.0);
+  return mid_best(p.M, p.N, p.K[0], slices) < us;
 }
 }  // namespace
 
@@ -206,7 +215,7 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
   if (lt_gemm_stream_supported(p, EPI_STORE, dtype, io_dtype)) return lt_launch_gemm_stream(p, EPI_STORE, dtype, io_dtype, stream);
   const bool a_km = p.A[0].kmajor, b_km = p.B[0].kmajor;
   const EpiParams& e = p.epi;
-  if (dtype == LT_BF16 && mid_selected(p, EPI_STORE) && e.ldo == p.N) {
+  if (dtype == LT_BF16 && e.ldo == p.N && mid_selected(p, EPI_STORE, workspace ? workspace_bytes : 0)) {
     const size_t slice = (size_t)p.M * (size_t)p.N * sizeof(float);
     const int slices = (int)std::min<size_t>((size_t)mid_slices(p.M, p.N, p.K[0]), workspace ? workspace_bytes / slice : 0);
     if (slices <= 1) return lt_launch_gemm(p, EPI_STORE, dtype, io_dtype, stream);
@@ -235,6 +244,7 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
     if (slices > 1 && workspace && workspace_bytes >= need && dma_selected(p, EPI_STORE) && e.ldo == p.N) {
       GemmProblem q = p;
       q.ksplit = slices;
+      q.variant = 2;
       q.split_stride = p.M * p.N;
       q.epi.out = workspace;
       q.epi.ldo = p.N;
@@ -333,12 +343,14 @@ int lt_launch_gemm_out(const GemmProblem& p, int dtype, int io_dtype, void* work
     // the tiled kernel where it takes the problem, else the any-shape kernel
     const bool tiled = dtype == LT_BF16 && lt_gemm_mfma_supported(q, EPI_STORE) && dma_selected(q, EPI_STORE);
     const bool tiled_unsplit = dtype == LT_BF16 && lt_gemm_mfma_supported(p, EPI_OUT);
-    const int wanted = dtype == LT_BF16 && mid_selected(q, EPI_STORE) ? mid_slices(p.M, p.N, p.K[0])
+    const bool mid = dtype == LT_BF16 && mid_selected(q, EPI_STORE, workspace_bytes);
+    const int wanted = mid ? mid_slices(p.M, p.N, p.K[0])
                        : tiled ? splitk_slices(p.M, p.N, p.K[0]) : tiled_unsplit ? 1 : generic_splitk_slices(p.M, p.N, p.K[0]);
     const int slices = (int)std::min<size_t>((size_t)wanted, workspace_bytes / slice);
     if (slices > 1) {
       q.ksplit = slices;
       q.split_stride = p.M * p.N;
+      if (tiled && !mid) q.variant = 2;
       if (tiled) LT_TRY(lt_launch_gemm(q, EPI_STORE, dtype, io_dtype, stream));
       else LT_TRY(lt_launch_gemm_generic(q, EPI_STORE, dtype, io_dtype, stream));
       LtProfileScope scope("splitk_reduce_out", 0.0,

@@ -50,3 +50,26 @@ def test_split_reductions_of_a_training_step(gated, dropout, post_ln, tokens, hi
     assert_close(dx, dx_ref, torch.bfloat16, "dx")
     for name, g, r in zip(("i2h.weight", "i2h.bias", "h2o.weight"), grads, g_ref[2:5]):
         assert_close(g, r, torch.bfloat16, name)
+
+
+def test_long_reduction_of_many_tiles():
+    """[1100, 4096] over 16384: 288 tiles of 128 x 128 leave the second workgroup of most CUs out; the down-projection and its input
+    gradient run on 256 x 256 tiles in slices instead.  Against float32 products of the same 16-bit weights."""
+    torch.manual_seed(0)
+    tokens, hidden, inter = 1100, 4096, 16384
+    ffn = lt.LeanFFN(hidden, inter, activation=lt.ACT2FN["linear"], gated=False, layer_norm_eps=1e-5).to(DEV).to(torch.bfloat16)
+    x = torch.randn(tokens, hidden, device=DEV, requires_grad=True)
+    dy = torch.randn(tokens, hidden, device=DEV)
+
+    def step():
+        y = ffn(x)
+        return y.detach(), torch.autograd.grad(y, x, dy)[0]
+
+    (y, dx), tags = _kernel_tags(step)
+    assert {"splitk_reduce_out", "splitk_reduce"} <= tags, tags
+    w1, b1, w2, b2 = (p.detach().float() for p in (ffn.i2h_proj.weight, ffn.i2h_proj.bias, ffn.h2o_proj.weight, ffn.h2o_proj.bias))
+    u = torch.nn.functional.layer_norm(x, (hidden,), ffn.pre_layer_norm.weight.float(), ffn.pre_layer_norm.bias.float(), 1e-5)
+    ref = (u @ w1.t() + b1) @ w2.t() + b2 + x
+    ref_dx, = torch.autograd.grad(ref, x, dy)
+    assert_close(y, ref.detach(), torch.bfloat16, "y")
+    assert_close(dx, ref_dx, torch.bfloat16, "dx")
