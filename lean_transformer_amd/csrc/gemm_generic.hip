@@ -8,9 +8,12 @@
 // 8 and the same exponent range, so every operand element is split without error into three bfloat16 planes, x = x1 + x2 + x3:
 // x1 is x truncated, x2 the remainder (16 bits, exact in fp32) rounded, x3 the rest (8 bits, exact).  A product of two floats
 // is nine products of planes, each of them exact in fp32; the six with a weight of 2^-16 or more are accumulated
-// (x1 y1, x1 y2, x2 y1, x2 y2, x1 y3, x3 y1), smallest first.  What is left out, x2 y3 + x3 y2 + x3 y3, is at most
-// 2^-7 2^-16 2 = 2^-22 of |x y| and 2^-24.5 of it on average with random sign, the size of the one rounding that every
-// fp32 accumulation makes, and the matrix unit adds 16 products per such rounding instead of 2.  The 16-bit instruction rounds
+// (x1 y1, x1 y2, x2 y1, x2 y2, x1 y3, x3 y1), and all nine where the whole reduction is one step.  What is left out, x2 y3 + x3 y2 +
+// x3 y3, is at most 2^-7 2^-16 2 = 2^-22 of |x y| and 2^-24.5 of it on average with random sign, the size of the one rounding that
+// every fp32 accumulation makes, and the matrix unit adds 16 products per such rounding instead of 2.  x1 y1 has accumulators of its
+// own: added to the whole sum, 16 products of 2^-16 are less than half a unit in its last place once a reduction of one sign has
+// a few thousand terms, and are lost every time (|x| |y| of normal numbers over 8192: 89 x 2^-24 off, 24 with the fp32 instruction).
+// Below 2^-110 an element's last plane is subnormal and loses bits below 2^-133.  The 16-bit instruction rounds
 // what it aligns away towards minus infinity (a bias of 0.1 - 0.2 units in the last place per instruction, measured), which
 // sums over many rows of a result would collect (a bias gradient is one over all tokens); odd rows of A are therefore negated
 // on the way in and odd rows of the result on the way out, so that the bias alternates.
@@ -45,12 +48,13 @@ template <typename TI> struct Operand {  // 16-bit: as they are
   static constexpr int A_PLANE[1] = {0}, B_PLANE[1] = {0};
 };
 template <> struct Operand<float> {
-  static constexpr int PLANES = 3, BK = 16, PRODUCTS = 6;
+  static constexpr int PLANES = 3, BK = 16, PRODUCTS = 9;
   typedef bfloat8 Frag;
   static __device__ __forceinline__ f32x16 mfma(Frag a, Frag b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
   }
-  static constexpr int A_PLANE[6] = {2, 0, 1, 1, 0, 0}, B_PLANE[6] = {0, 2, 1, 0, 1, 0};
+  // smallest first; FEW: the first three belong to short reductions only
+  static constexpr int A_PLANE[9] = {2, 1, 2, 2, 0, 1, 1, 0, 0}, B_PLANE[9] = {2, 2, 1, 0, 2, 1, 0, 1, 0}, FEW = 3;
 };
 
 // 8 consecutive k of one row, as fetched
@@ -121,7 +125,7 @@ template <int N, typename F> __device__ __forceinline__ void lt_rolled_rows(F&& 
 
 // A_KM, B_KM: layout of the operands (of every k-segment).  A block-sparse walk has the layout of its mode.
 template <typename TI, bool A_KM, bool B_KM, int KIND, typename TC, typename TX, int FM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4 : 3))) void gemm_generic_kernel(GemmProblem p, int tiles_m, int tiles_n) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((FM == 1 ? 4 : 3) - (sizeof(TI) == 4)))) void gemm_generic_kernel(GemmProblem p, int tiles_m, int tiles_n) {
   typedef Operand<TI> Op;
   typedef typename Op::Frag Frag;
   constexpr int BM = 64 * FM, BN = 128, BK = Op::BK, CH = BK / 8, PLANES = Op::PLANES;
@@ -209,16 +213,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
     return g;
   };
 
-  f32x16 acc[FM][2];
+  f32x16 acc[FM][2], rest[FM][2];  // rest (fp32): the products of planes below the first
 #pragma unroll
   for (int i = 0; i < FM; i++)
 #pragma unroll
     for (int j = 0; j < 2; j++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+      for (int r = 0; r < 16; r++) acc[i][j][r] = rest[i][j][r] = 0.f;
 
   // ---- main loop.  Step t multiplies LDS buffer t & 1 while the fetches of step t + 2 are in flight into register set t & 1; then the
-  //      pieces of step t + 1 (set (t + 1) & 1) are split and written to the other buffer.  The three or four workgroups of a CU
+  //      pieces of step t + 1 (set (t + 1) & 1) are split and written to the other buffer.  The two to four workgroups of a CU
   //      overlap each other's matrix and vector work: placing the split between the matrix instructions of the same wavefront
   //      measured the same.
   constexpr int A_PIECES = (BM * CH + 255) / 256, B_PIECES = BN * CH / 256;  // per thread and step
@@ -350,7 +354,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
       for (int q = 0; q < PLANES; q++) tb[(q * CH + b_chunk(i)) * B_ROWS + b_row(i)] = w[q];
     }
   };
-  auto multiply = [&](int buf) {
+  // tail (fp32): the three smallest products of planes instead of the six others
+  auto multiply = [&](auto tail, int buf) {
     const lt_u32x4* const ta = a_tile(buf);
     const lt_u32x4* const tb = b_tile(buf);
 #pragma unroll
@@ -366,12 +371,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
         for (int j = 0; j < 2; j++)
           bb[j][q] = __builtin_bit_cast(Frag, tb[(q * CH + chunk) * B_ROWS + wn * 64 + j * 32 + (lane & 31)]);
       }
-#pragma unroll
-      for (int t = 0; t < Op::PRODUCTS; t++)
+      if constexpr (PLANES == 1) {
 #pragma unroll
         for (int i = 0; i < FM; i++)
 #pragma unroll
-          for (int j = 0; j < 2; j++) acc[i][j] = Op::mfma(a[i][Op::A_PLANE[t]], bb[j][Op::B_PLANE[t]], acc[i][j]);
+          for (int j = 0; j < 2; j++) acc[i][j] = Op::mfma(a[i][0], bb[j][0], acc[i][j]);
+      } else {
+        constexpr bool TAIL = decltype(tail)::value;
+        constexpr int FIRST = TAIL ? 0 : Op::FEW, LAST = TAIL ? Op::FEW : Op::PRODUCTS - 1;
+#pragma unroll
+        for (int t = FIRST; t < LAST; t++)
+#pragma unroll
+          for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) rest[i][j] = Op::mfma(a[i][Op::A_PLANE[t]], bb[j][Op::B_PLANE[t]], rest[i][j]);
+        if constexpr (!TAIL) {
+#pragma unroll
+          for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) acc[i][j] = Op::mfma(a[i][0], bb[j][0], acc[i][j]);
+        }
+      }
     }
   };
   // a step whose successors are whole: nothing in it is conditional, so that the wait for the older fetches leaves the younger
@@ -379,7 +399,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
   auto step_whole = [&](auto S) {
     constexpr int set = decltype(S)::value;
     fetch(Whole{}, S);
-    multiply(set);
+    multiply(std::false_type{}, set);
     stash(std::integral_constant<int, set ^ 1>{}, set ^ 1);
     __syncthreads();
   };
@@ -389,7 +409,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
       fetch(Ragged{}, S);
       next_segment();
     }
-    multiply(set);
+    multiply(std::false_type{}, set);
     if (t + 1 < total) stash(std::integral_constant<int, set ^ 1>{}, set ^ 1);
     __builtin_amdgcn_s_waitcnt(0xf70);  // vmcnt(0): the loop above then starts with nothing unaccounted for
     __syncthreads();
@@ -405,6 +425,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
     next_segment();
   }
   __syncthreads();
+  if constexpr (PLANES > 1)
+    if (total == 1) multiply(std::true_type{}, 0);
   for (int t = 0; t < total;) {
     if (t + 3 < total && k0 + 2 * BK <= g.K && vectors()) {
       const int s = seg;  // (the next segment has an alignment of its own)
@@ -418,6 +440,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FM == 1 ? 4
     }
     if (t < total) step_ragged(S0{}, t++);
     if (t < total) step_ragged(S1{}, t++);
+  }
+
+  if constexpr (PLANES > 1) {
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) acc[i][j] += rest[i][j];
   }
 
   // ---- epilogue (the loop ended with a barrier).  Accumulator register r of a 32 x 32 block is row 8 * (r / 4) + 4 * (lane / 32) + r % 4, column lane % 32; each

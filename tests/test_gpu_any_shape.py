@@ -102,3 +102,17 @@ def test_fp32_sums_of_zeros_are_positive():
     zeros, b = torch.zeros(70, 40, device=DEV), torch.randn(45, 40, device=DEV)
     c = _gemm(zeros, b, True, True, 70, 45, 40, torch.float32, 1)
     assert not bool(c.signbit().any()) and bool((c == 0).all())
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 16, 3072, 8192])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_fp32_sums_of_one_sign(k, sign):
+    """no products are lost beside a large sum: 2-norm error at most that of K / 2 roundings to nearest (0.29 units of 2^-23 of a sum that
+    grows evenly: sqrt(K / 2 / 3) of them), which is what adding two exact products at a time makes, and one rounding of the result"""
+    g = torch.Generator(device=DEV).manual_seed(k)
+    a, b = torch.randn(256, k, generator=g, device=DEV).abs(), sign * torch.randn(512, k, generator=g, device=DEV).abs()
+    ref = a.double() @ b.double().t()
+    err = _gemm(a, b, True, True, 256, 512, k, torch.float32, 1).double() - ref
+    assert (err.norm() / ref.norm()).item() <= 0.29 * 2.0**-23 * (1 + (k / 6) ** 0.5)
+    if k == 1:  # one rounding, of a sum that the planes give to 2^-30
+        assert (err.abs() / ref.abs()).max().item() <= 2.0**-24 * (1 + 2.0**-6)
