@@ -236,7 +236,7 @@ void plan_linear_backward(const lt_linear& lin, int64_t T, int dtype, Bump& ws, 
   s.colsum = ws.take(s.colsum_bytes);
   s.skinny_bytes = lin.lowrank > 0 ? lt_gemm_skinny_workspace(T, lin.lowrank) : 0;
   if (lin.block == 0) {  // dW (and dx) of a small dense layer: the reduction is split across workgroups
-    s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_splitk_workspace(lin.out_features, lin.in_features, T));
+    if (dtype == LT_BF16) s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_splitk_workspace(lin.out_features, lin.in_features, T));
     if (dtype == LT_BF16) s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_mid_splitk_workspace(lin.out_features, lin.in_features, T));
     s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_generic_splitk_workspace(lin.out_features, lin.in_features, T));
     if (lin.lowrank == 0) {
@@ -429,7 +429,7 @@ void plan_forward(const lt_ffn_desc& d, Bump& ws, FwdScratch& s) {
   // dense down-projection of a short batch: room to split its reduction, no more than the saved pre-activation takes or 32 MiB
   if (d.h2o.block == 0 && d.h2o.lowrank == 0 && !d.post_ln_weight) {
     const size_t cap = std::max((size_t)d.tokens * (d.gated ? 2 : 1) * d.intermediate * e, (size_t)32 << 20);
-    s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_out_splitk_workspace(d.tokens, d.hidden, d.intermediate, cap));
+    s.skinny_bytes = std::max(s.skinny_bytes, lt_gemm_out_splitk_workspace(d.compute_dtype, d.tokens, d.hidden, d.intermediate, cap));
   }
   s.skinny = s.skinny_bytes ? ws.take(s.skinny_bytes) : nullptr;
   s.vectors = take_vectors(d, ws, true);

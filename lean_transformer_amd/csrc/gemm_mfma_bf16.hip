@@ -319,9 +319,9 @@ __global__ __launch_bounds__(256) void splitk_reduce_out_kernel(const float* __r
 }
 }  // namespace
 
-size_t lt_gemm_out_splitk_workspace(int64_t M, int64_t N, int64_t K, size_t cap_bytes) {
-  const size_t full = std::max({lt_gemm_splitk_workspace(M, N, K), lt_gemm_generic_splitk_workspace(M, N, K),
-                                lt_gemm_mid_splitk_workspace(M, N, K)});
+size_t lt_gemm_out_splitk_workspace(int dtype, int64_t M, int64_t N, int64_t K, size_t cap_bytes) {
+  size_t full = lt_gemm_generic_splitk_workspace(M, N, K);
+  if (dtype == LT_BF16) full = std::max({full, lt_gemm_splitk_workspace(M, N, K), lt_gemm_mid_splitk_workspace(M, N, K)});
   const size_t slice = (size_t)M * (size_t)N * sizeof(float);
   if (full == 0 || cap_bytes < 2 * slice) return 0;
   return std::min(full, lt_align_up(cap_bytes / slice * slice, 256));
