@@ -125,13 +125,16 @@ int lt_gemm_colsum_rows(const GemmProblem& p, int dtype, int io_dtype) {
              ? 64 : 0;
 }
 
-static const char* mfma_tag(const GemmProblem& p, int kind) {
-  static const char* names[3][4] = {
-      {"gemm_bf16_nt_store", "gemm_bf16_nt_act_fwd", "gemm_bf16_nt_act_bwd", "gemm_bf16_nt_out"},
-      {"gemm_bf16_nn_store", "gemm_bf16_nn_act_fwd", "gemm_bf16_nn_act_bwd", "gemm_bf16_nn_out"},
-      {"gemm_bf16_tn_store", "gemm_bf16_tn_act_fwd", "gemm_bf16_tn_act_bwd", "gemm_bf16_tn_out"}};
+static const char* mfma_tag(const GemmProblem& p, int kind, bool mid) {
+  static const char* names[2][3][4] = {
+      {{"gemm_bf16_nt_store", "gemm_bf16_nt_act_fwd", "gemm_bf16_nt_act_bwd", "gemm_bf16_nt_out"},
+       {"gemm_bf16_nn_store", "gemm_bf16_nn_act_fwd", "gemm_bf16_nn_act_bwd", "gemm_bf16_nn_out"},
+       {"gemm_bf16_tn_store", "gemm_bf16_tn_act_fwd", "gemm_bf16_tn_act_bwd", "gemm_bf16_tn_out"}},
+      {{"gemm_mid_nt_store", "gemm_mid_nt_act_fwd", "gemm_mid_nt_act_bwd", "gemm_mid_nt_out"},
+       {"gemm_mid_nn_store", "gemm_mid_nn_act_fwd", "gemm_mid_nn_act_bwd", "gemm_mid_nn_out"},
+       {"gemm_mid_tn_store", "gemm_mid_tn_act_fwd", "gemm_mid_tn_act_bwd", "gemm_mid_tn_out"}}};
   const int layout = p.A[0].kmajor ? (p.B[0].kmajor ? 0 : 1) : 2;
-  return names[layout][kind];
+  return names[mid][layout][kind];
 }
 
 double lt_gemm_flops(const GemmProblem& p, int kind) {
@@ -142,8 +145,9 @@ double lt_gemm_flops(const GemmProblem& p, int kind) {
 
 int lt_launch_gemm_mfma(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream) {
   LT_REQUIRE(lt_gemm_mfma_supported(p, kind), LT_ERR_UNSUPPORTED, "tiled bf16 gemm does not take this problem");
-  LtProfileScope scope(mfma_tag(p, kind), lt_gemm_flops(p, kind), 0.0, stream);
-  if (mid_selected(p, kind)) return lt_launch_gemm_mid(p, kind, io_dtype, stream);
+  const bool mid = mid_selected(p, kind);
+  LtProfileScope scope(mfma_tag(p, kind, mid), lt_gemm_flops(p, kind), 0.0, stream);
+  if (mid) return lt_launch_gemm_mid(p, kind, io_dtype, stream);
   switch (kind) {
     case EPI_STORE: return lt_mfma_launch_dense_kind0(p, io_dtype, stream);
     case EPI_ACT_FWD: return lt_mfma_launch_dense_kind1(p, io_dtype, stream);

@@ -35,6 +35,8 @@ OTHER_ACTS = [(a, g, t) for a in ("gelu", "relu", "silu") for g in (False, True)
     (a, i % 2 == 0, 300 if i % 3 == 0 else 512) for i, a in enumerate(
         ("quick_gelu", "gelu_10", "relu6", "relu2", "leaky_relu", "mish", "sigmoid", "tanh", "linear", "hardswish", "laplace",
          "sqrtsoftplus", "gelu_accurate", "gelu_fast"))]
+# more than 512 tiles of 128 x 128, above which the 256 x 256 kernel takes a product: its own general strips
+OTHER_ACTS += [("relu", True, 4200), ("gelu", False, 8300), ("silu", True, 4200)]
 
 
 @pytest.mark.parametrize("act,gated,tokens", OTHER_ACTS)
@@ -54,10 +56,12 @@ def test_bf16_other_activations_take_the_general_epilogue_strips(act, gated, tok
 
 @pytest.mark.parametrize("io_dtype", [torch.float32, BF16])
 @pytest.mark.parametrize("dropout", [0.0, 0.1])
-def test_bf16_without_residual(io_dtype, dropout):
-    """residual=False (reversible stacks add the input themselves): the down-projection epilogue has nothing to read"""
+@pytest.mark.parametrize("tokens", [512, 16500])
+def test_bf16_without_residual(io_dtype, dropout, tokens):
+    """residual=False (reversible stacks add the input themselves): the down-projection epilogue has nothing to read;
+    16500 tokens are more than 512 tiles of 128 x 128, which the 256 x 256 kernel takes"""
     torch.manual_seed(19)
-    tokens, hidden = 512, 512
+    hidden = 512
     ffn = lt.LeanFFN(hidden, 1024, gated=True, residual=False, dropout=dropout, layer_norm_eps=1e-5)
     _randomise_small_vectors(ffn)
     ffn = ffn.to(DEV).to(BF16)
@@ -68,12 +72,11 @@ def test_bf16_without_residual(io_dtype, dropout):
     _compare(ffn, x, dy, BF16, mask=mask)
 
 
-@pytest.mark.parametrize("hidden,inter", [(512, 1024), (1024, 2048)])
+@pytest.mark.parametrize("tokens,hidden,inter", [(384, 512, 1024), (384, 1024, 2048), (16500, 512, 1024)])
 @pytest.mark.parametrize("gated", [False, True])
 @pytest.mark.parametrize("dropout", [0.0, 0.1])
-def test_bf16_post_layer_norm(hidden, inter, gated, dropout):
+def test_bf16_post_layer_norm(tokens, hidden, inter, gated, dropout):
     torch.manual_seed(23)
-    tokens = 384
     ffn = lt.LeanFFN(hidden, inter, gated=gated, post_layer_norm=True, dropout=dropout, layer_norm_eps=1e-5)
     _randomise_small_vectors(ffn)
     ffn = ffn.to(DEV).to(BF16)

@@ -51,9 +51,12 @@ def test_gemm_any_shape_kernel(dtype, a_kmajor, b_kmajor, m, n, k):
 @pytest.mark.parametrize("a_kmajor,b_kmajor", [(True, True), (True, False), (False, False)])
 @pytest.mark.parametrize("m,n,k", [(512, 512, 256), (256, 768, 64), (1024, 256, 1024)])
 @pytest.mark.parametrize("c_dtype", [torch.float32, torch.bfloat16])
-def test_gemm_tiled_bf16_kernel(a_kmajor, b_kmajor, m, n, k, c_dtype):
+@pytest.mark.parametrize("force", [0, 3])
+def test_gemm_tiled_bf16_kernel(a_kmajor, b_kmajor, m, n, k, c_dtype, force):
+    """0: the library's choice (128 x 128 tiles at these sizes where A is k-major); 3: 256 x 256 tiles"""
     a, b, ref = _operands(m, n, k, a_kmajor, b_kmajor, torch.bfloat16, seed=m + 2 * n + 3 * k)
-    c = _gemm(a, b, a_kmajor, b_kmajor, m, n, k, c_dtype, force_generic=False)
+    c, tags = _kernel_tags(lambda: _gemm(a, b, a_kmajor, b_kmajor, m, n, k, c_dtype, force))
+    assert all(t.startswith("gemm_bf16_" if force else ("gemm_bf16_", "gemm_mid_")) for t in tags), tags
     if c_dtype == torch.float32:
         assert rel_err(c, ref) <= 1e-5
     else:
@@ -63,17 +66,18 @@ def test_gemm_tiled_bf16_kernel(a_kmajor, b_kmajor, m, n, k, c_dtype):
     assert rel_err(c.float(), c2) <= (1e-5 if c_dtype == torch.float32 else 1e-2)
 
 
-def test_gemm_tiled_bf16_ragged_rows_and_reduction():
+@pytest.mark.parametrize("force", [0, 3])
+def test_gemm_tiled_bf16_ragged_rows_and_reduction(force):
     # k-major A with a ragged row count (rows past M are clamped on load, never stored)
     a, b, ref = _operands(300, 256, 128, True, True, torch.bfloat16, seed=1)
-    assert rel_err(_gemm(a, b, True, True, 300, 256, 128, torch.float32, False), ref) <= 1e-5
+    assert rel_err(_gemm(a, b, True, True, 300, 256, 128, torch.float32, force), ref) <= 1e-5
     a, b, ref = _operands(777, 512, 192, True, False, torch.bfloat16, seed=2)
-    assert rel_err(_gemm(a, b, True, False, 777, 512, 192, torch.float32, False), ref) <= 1e-5
+    assert rel_err(_gemm(a, b, True, False, 777, 512, 192, torch.float32, force), ref) <= 1e-5
     # both operands mn-major with a reduction length that is not a multiple of the 64-wide k-step (zero-filled tail)
     a, b, ref = _operands(256, 512, 200, False, False, torch.bfloat16, seed=3)
-    assert rel_err(_gemm(a, b, False, False, 256, 512, 200, torch.float32, False), ref) <= 1e-5
+    assert rel_err(_gemm(a, b, False, False, 256, 512, 200, torch.float32, force), ref) <= 1e-5
     a, b, ref = _operands(512, 256, 1000, False, False, torch.bfloat16, seed=4)
-    assert rel_err(_gemm(a, b, False, False, 512, 256, 1000, torch.float32, False), ref) <= 1e-5
+    assert rel_err(_gemm(a, b, False, False, 512, 256, 1000, torch.float32, force), ref) <= 1e-5
 
 
 def _kernel_tags(fn):
@@ -122,16 +126,18 @@ def test_gemm_tile_loop_gives_the_same_bits_as_one_workgroup_per_tile(a_kmajor, 
                                                    (False, False, "gemm_bf16_tn_store")])
 @pytest.mark.parametrize("m,n,k", [(512, 320, 128), (256, 8, 64), (328, 200, 192), (1600, 1608, 320), (264, 776, 448)])
 @pytest.mark.parametrize("c_dtype", [torch.float32, torch.bfloat16])
-def test_gemm_tiled_bf16_tiles_past_the_edge(a_kmajor, b_kmajor, tag, m, n, k, c_dtype):
+@pytest.mark.parametrize("force", [0, 3])
+def test_gemm_tiled_bf16_tiles_past_the_edge(a_kmajor, b_kmajor, tag, m, n, k, c_dtype, force):
     """N (and, for an mn-major A, M) a multiple of 8 but not of the 256-wide tile: the tiled kernel still takes the problem,
-    re-reads the last row / last 8 columns for the part of the tile that sticks out and writes nothing there"""
+    re-reads the last row / last 8 columns for the part of the tile that sticks out and writes nothing there.
+    0: the library's choice of tile; 3: 256 x 256"""
     a, b, ref = _operands(m, n, k, a_kmajor, b_kmajor, torch.bfloat16, seed=m + 2 * n + 3 * k)
     flat = torch.full((m * n + 4096,), 7.0, dtype=c_dtype, device=DEV)  # the result, then a guard nothing may write
     c = flat[:m * n].view(m, n)
     _, tags = _kernel_tags(lambda: nat.check(
         nat.lib().lt_gemm(nat.dtype_code(a.dtype), m, n, k, nat.ptr(a), int(a_kmajor), nat.ptr(b), int(b_kmajor),
-                          nat.dtype_code(c_dtype), nat.ptr(c), 0, nat.current_stream(c.device)), "lt_gemm"))
-    assert tag in tags, tags
+                          nat.dtype_code(c_dtype), nat.ptr(c), force, nat.current_stream(c.device)), "lt_gemm"))
+    assert tags == {tag} or (force == 0 and tags == {tag.replace("bf16", "mid")}), tags
     assert bool((flat[m * n:] == 7.0).all())
     if c_dtype == torch.float32:
         assert rel_err(c, ref) <= 1e-5

@@ -24,8 +24,11 @@ def test_gemm(dtype, a_kmajor, b_kmajor, m, n, k):
     a, b = torch.randn(m, k, generator=g, device=DEV).to(dtype), torch.randn(n, k, generator=g, device=DEV).to(dtype)
     m8 = m if a_kmajor else -(-m // 8) * 8  # (an mn-major A has rows of a multiple of 8 elements)
     a = torch.cat([a, a[:m8 - m]])
-    c = _gemm(a if a_kmajor else a.t().contiguous(), b if b_kmajor else b.t().contiguous(), a_kmajor, b_kmajor, m8, n, k,
-              torch.float32, 0)
+    c, tags = _kernel_tags(lambda: _gemm(a if a_kmajor else a.t().contiguous(), b if b_kmajor else b.t().contiguous(), a_kmajor,
+                                         b_kmajor, m8, n, k, torch.float32, 0))
+    # (the tags are the bfloat16 library's; two mn-major operands go where the estimated time is the shorter)
+    if dtype == torch.bfloat16 and a_kmajor:
+        assert tags == {"gemm_mid_nt_store" if b_kmajor else "gemm_mid_nn_store"}, tags
     worst = (c.double() - a.double() @ b.double().t()).abs() - (k + 16) * 2.0**-23 * (a.double().abs() @ b.double().abs().t())
     assert worst.max().item() <= 0.0
 
@@ -66,7 +69,7 @@ def test_long_reduction_of_many_tiles():
         return y.detach(), torch.autograd.grad(y, x, dy)[0]
 
     (y, dx), tags = _kernel_tags(step)
-    assert {"splitk_reduce_out", "splitk_reduce"} <= tags, tags
+    assert {"gemm_bf16_nt_store", "splitk_reduce_out", "gemm_bf16_nn_store", "splitk_reduce"} <= tags, tags
     w1, b1, w2, b2 = (p.detach().float() for p in (ffn.i2h_proj.weight, ffn.i2h_proj.bias, ffn.h2o_proj.weight, ffn.h2o_proj.bias))
     u = torch.nn.functional.layer_norm(x, (hidden,), ffn.pre_layer_norm.weight.float(), ffn.pre_layer_norm.bias.float(), 1e-5)
     ref = (u @ w1.t() + b1) @ w2.t() + b2 + x
