@@ -68,7 +68,8 @@ typedef enum lt_act {
 } lt_act;
 
 /* One projection in the reference's "generalized linear" form: main weight (dense or native block-sparse), optional bias,
- * optional low-rank pair.  Weights and low-rank factors are in the compute dtype; the bias is always fp32. */
+ * optional low-rank pair.  Weights and low-rank factors are in the compute dtype; the bias is fp32, except in an
+ * lt_ffn_desc whose vector_dtype says otherwise. */
 typedef struct lt_linear {
   const void* weight;              /* dense: [out_features, in_features]; sparse: [in_features, blocks_per_in, block] */
   const float* bias;               /* [out_features] or NULL */
@@ -123,7 +124,7 @@ typedef struct lt_ffn_desc {
   float ln_eps;
   float dropout_p;        /* 0 disables dropout (also pass 0 in eval mode) */
   int32_t vector_dtype;   /* lt_dtype of the small vectors below (LayerNorm parameters, i2h.bias, h2o.bias): LT_F32, or
-                             compute_dtype: one kernel then widens them into the workspace.  Gradients of them are fp32 */
+                             compute_dtype (the float pointers then hold 16-bit elements): one kernel widens them into the workspace.  Gradients of them are fp32 */
   uint64_t dropout_seed;  /* Philox key */
   uint64_t dropout_offset;/* Philox stream offset; forward and backward of one call must pass the same pair */
   const float* ln_weight; /* [H] vector_dtype (as the next three) */

@@ -697,7 +697,7 @@ int lt_launch_gemm_generic(const GemmProblem& p, int kind, int dtype, int io_dty
     groups = p.ksplit;
   }
   const int64_t tiles_n = (cols + (gated ? 64 : 128) - 1) / (gated ? 64 : 128);
-  // 64-row tiles where there are no more rows, or where 128-row ones leave workgroup slots (two per CU) empty
+  // 64-row tiles where there are no more rows, or where there are fewer than two 128-row ones per CU
   const bool half_tile = rows <= 64 || (rows + 127) / 128 * tiles_n * groups < 512;
   const int64_t tiles_m = (rows + (half_tile ? 63 : 127)) / (half_tile ? 64 : 128);
   LT_REQUIRE(tiles_m * tiles_n <= 0x7fffffff, LT_ERR_UNSUPPORTED, "gemm: M=%lld N=%lld exceed the grid limit", (long long)p.M,

@@ -184,9 +184,10 @@ size_t lt_gemm_splitk_workspace(int64_t M, int64_t N, int64_t K) {
 
 namespace {
 // Slices of an any-shape product's reduction: the number with the least estimated time.  A CU holds three 128 x 128 workgroups
-// (four of the 64 x 128 ones a small grid runs on), and with w of them resident a k-step of 16 takes about 0.35 + 0.6 w us (0.42 +
-// 0.32 w), measured in fp32 on 4096^3 and 321 x 7168 x 1792; a slice costs a write and a read of its fp32 partial result at
-// 5 TB/s.  [4096, 768] over 3072: 4 slices, one round of 768 workgroups, 142 us where 5 slices take 190; unsplit 330.
+// (four of the 64 x 128 ones a small grid runs on), in fp32, which has twice the accumulators, one less; with w of them resident a
+// k-step of 16 takes about 0.35 + 0.6 w us (0.42 + 0.32 w), measured in fp32 on 4096^3 and 321 x 7168 x 1792; a slice costs a write and
+// a read of its fp32 partial result at 5 TB/s.  Counting the one less in fp32 changes nothing (training step, T 4096, hidden 768: 1266 us
+// and 1277), so the rule is the same for both.
 int generic_splitk_slices(int64_t M, int64_t N, int64_t K) {
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), half_tiles = ((M + 63) / 64) * ((N + 127) / 128);
   if (tiles >= 3072) return 1;

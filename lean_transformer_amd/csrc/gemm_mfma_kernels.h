@@ -4,7 +4,7 @@
 // Two kernels share the LDS layouts and the epilogues:
 //   gemm_bf16_dma_kernel  256 x 256 tile, operands copied global -> LDS without passing through registers; the kernel of
 //                         the dense projections (second half of this file)
-//   gemm_bf16_kernel      BM x BN tile, operands staged through registers; ragged reductions, the 128 x 128 tile of the
+//   gemm_bf16_kernel      BM x BN tile, operands staged through registers; 32-bit offset overflow, the 128 x 128 tile of the
 //                         skinny low-rank GEMMs, and the block-sparse walks over 64 x 64 blocks
 //
 // gemm_bf16_kernel.  Tile: BM x BN outputs per workgroup, 64 k per step, WM x WN wavefronts each owning a (BM/WM) x (BN/WN)

@@ -240,7 +240,7 @@ bool lt_gemm_stream_supported(const GemmProblem& p, int kind, int dtype, int io_
   // 16-byte pieces of every row, 4 columns per store
   if (p.N % 4 || p.K[0] % piece || p.A[0].ld % piece || p.B[0].ld % piece || !lt_aligned(p.A[0].ptr, 16) || !lt_aligned(p.B[0].ptr, 16))
     return false;
-  // 32-bit byte offsets inside a workgroup's rows and along k (which runs up to 3 x 16 x 128 bytes past the end)
+  // 32-bit byte offsets inside a workgroup's rows and along k (the blocks asked for run up to 2 x 3 x 16 past the end before they are clamped)
   if (64 * std::max(p.A[0].ld, p.B[0].ld) * bytes >= (int64_t)1 << 31) return false;
   if ((p.N + 7) / 8 > 0x7fffffff) return false;
   if (e.bias && !lt_aligned(e.bias, 16)) return false;

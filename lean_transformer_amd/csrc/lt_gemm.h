@@ -43,7 +43,7 @@ struct EpiParams {
   DropoutParams drop;
 };
 
-// Block-sparse operand walk (any-shape kernel only).  Workgroups with the same blockIdx.z form one group:
+// Block-sparse operand walk (any-shape kernel only).  Workgroups with the same blockIdx.y form one group:
 //   SPARSE_FWD  group = output block ob:  Y[:, ob] = sum_k X[:, ib_k] W4[ib_k, a_k]^T,  forward_indices[ob, k] = ib_k * A + a_k
 //   SPARSE_DX   group = input block ib:   dX[:, ib] = sum_a dY[:, ob_a] W4[ib, a],       ob_a = backward_indices[ib, a]
 //   SPARSE_DW   group = weight block (ib, a): dW4[ib, a] = dY[:, ob_a]^T X[:, ib]
@@ -106,66 +106,7 @@ struct GemmProblem {
 };
 
 // ---------------------------------------------------------------------------------------------------------------------
-// per-element epilogues.  TC: compute dtype (pre-activation, hidden, gradients of them), TX: dtype of x / y.
-// ---------------------------------------------------------------------------------------------------------------------
-template <typename TO> __device__ __forceinline__ void epi_store(const EpiParams& e, int64_t m, int64_t n, float v) {
-  if (e.bias) v += e.bias[n];
-  stf(reinterpret_cast<TO*>(e.out), m * e.ldo + n, v);
-}
-
-template <typename TC> __device__ __forceinline__ void epi_act_fwd(const EpiParams& e, int64_t m, int64_t n, float v) {
-  constexpr bool PRECISE = sizeof(TC) == 4;
-  if (e.bias) v += e.bias[n];
-  TC pv = from_f32<TC>(v);
-  reinterpret_cast<TC*>(e.pre)[m * e.ld_pre + n] = pv;
-  stf(reinterpret_cast<TC*>(e.hid), m * e.ld_hid + n, act_value<PRECISE>(e.act, to_f32(pv)));
-}
-
-// gated: column n of the gate half pairs with column I + n of the linear half
-template <typename TC>
-__device__ __forceinline__ void epi_act_fwd_gated(const EpiParams& e, int64_t m, int64_t n, float vg, float vl) {
-  constexpr bool PRECISE = sizeof(TC) == 4;
-  if (e.bias) {
-    vg += e.bias[n];
-    vl += e.bias[e.inter + n];
-  }
-  TC pg = from_f32<TC>(vg), pl = from_f32<TC>(vl);
-  TC* pre = reinterpret_cast<TC*>(e.pre);
-  pre[m * e.ld_pre + n] = pg;
-  pre[m * e.ld_pre + e.inter + n] = pl;
-  stf(reinterpret_cast<TC*>(e.hid), m * e.ld_hid + n, act_value<PRECISE>(e.act, to_f32(pg)) * to_f32(pl));
-}
-
-template <typename TC> __device__ __forceinline__ void epi_act_bwd(const EpiParams& e, int64_t m, int64_t n, float dh) {
-  constexpr bool PRECISE = sizeof(TC) == 4;
-  const TC* pre = reinterpret_cast<const TC*>(e.pre);
-  TC* dpre = reinterpret_cast<TC*>(e.dpre);
-  TC* hid = reinterpret_cast<TC*>(e.hid);
-  float a, da;
-  if (e.gated) {
-    float pg = to_f32(pre[m * e.ld_pre + n]), pl = to_f32(pre[m * e.ld_pre + e.inter + n]);
-    act_eval<PRECISE>(e.act, pg, a, da);
-    stf(dpre, m * e.ld_pre + n, dh * pl * da);
-    stf(dpre, m * e.ld_pre + e.inter + n, dh * a);
-    if (hid) stf(hid, m * e.ld_hid + n, a * pl);
-  } else {
-    float p = to_f32(pre[m * e.ld_pre + n]);
-    act_eval<PRECISE>(e.act, p, a, da);
-    stf(dpre, m * e.ld_pre + n, dh * da);
-    if (hid) stf(hid, m * e.ld_hid + n, a);
-  }
-}
-
-template <typename TX> __device__ __forceinline__ void epi_out(const EpiParams& e, int64_t m, int64_t n, float v) {
-  if (e.bias) v += e.bias[n];
-  int64_t idx = m * e.ldy + n;
-  if (e.drop.p > 0.f) v = dropout_keep(e.drop, idx) ? v * e.drop.scale : 0.f;
-  if (e.x) v += ldf(reinterpret_cast<const TX*>(e.x), idx);
-  stf(reinterpret_cast<TX*>(e.y), idx, v);
-}
-
-// ---------------------------------------------------------------------------------------------------------------------
-// the same epilogues on 8 consecutive columns n .. n + 7 of row m (n a multiple of 8, all leading dimensions multiples
+// Epilogues on 8 consecutive columns n .. n + 7 of row m (n a multiple of 8, all leading dimensions multiples
 // of 8): 16-byte global accesses, one Philox block per 4 elements.  Used by the tiled bf16 kernel (TC = bf16).
 // ---------------------------------------------------------------------------------------------------------------------
 __device__ __forceinline__ void add_bias8(const float* bias, int64_t n, float (&v)[8]) {
