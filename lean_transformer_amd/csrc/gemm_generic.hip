@@ -21,8 +21,8 @@
 // arithmetic from the operands in memory, as the epilogue takes it up (a NaN among its operands ends that where it is met).
 // What bounds it: at 4096^3 a full round of workgroups runs at 1.2 PFLOP/s of bfloat16 products, what the tiled 16-bit kernel
 // reaches on the same data (the clock under load); smaller products lose to a last round that is not full and to the start and
-// end of a tile.  4096^3: 1411 us with the fp32 instruction, 723 now; a training step of T = 4096, hidden 768: 2263 us, 1154 now;
-// its gradients' 2-norm errors against float64 0.9 - 1.0e-6 before, 0.7 - 0.9e-6 now.  16-bit operands, 4096^3: 1591 us, 189.
+// end of a tile.  4096^3: 1411 us with the fp32 instruction, 752 with one set of accumulators, 763 with two; a training step of T = 4096,
+// hidden 768: 2263 us, 1150, 1266; 2-norm error of 4096^3 against float64 1.15e-6, 1.01e-6, 0.39e-6.  16-bit operands, 4096^3: 1591 us, 221.
 //
 // Work decomposition: 256 threads = 4 wavefronts in a 2 x 2 grid over a (64 FM) x 128 output tile; each wavefront owns FM x 2
 // MFMA blocks of 32 x 32.  Operand tiles of BK k-steps are staged in LDS as 16-byte pieces of 8 consecutive k, [plane][k / 8][row],
