@@ -1702,7 +1702,8 @@ int launch_dma(const GemmProblem& problem, int io_dtype, hipStream_t stream) {
   // Tiles of 192 columns where that takes no more rounds of up to 256 tiles: each round is then 3/4 as long in matrix instructions,
   // though not in copies, which is why one more round is not worth it.  256 against 192 columns, T 16384: [T, 768] over 2304 (192 or
   // 256 tiles) 66 us, 58; over 6144 176, 166; down-projection [T, 768] over 3072 103, 100; [T, 2304] over 768 (three rounds) 79, 75.
-  if constexpr (A_KM && (KIND == EPI_STORE || KIND == EPI_OUT)) {
+  // Weight gradients: [1600, 6400] over 3333 (175 tiles, 225 or 238) 86 us, 75 - 81.
+  if constexpr (KIND == EPI_STORE || KIND == EPI_OUT) {
     const int narrow_n = (int)((p.N + 191) / 192);
     const int64_t wide_rounds = ((int64_t)tiles_m * tiles_n + 255) / 256, narrow_rounds = ((int64_t)tiles_m * narrow_n + 255) / 256;
     if (p.ksplit <= 1 && narrow_n > tiles_n && narrow_rounds == wide_rounds) {

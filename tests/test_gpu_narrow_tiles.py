@@ -69,3 +69,14 @@ def test_second_segment():
         y = layer(xd)
     assert_close(y, (x.double() @ w.t() + layer.bias.double()).float().cpu(), torch.bfloat16, "y")
     assert_close(torch.autograd.grad(y, xd, dy.to(y.dtype))[0], (dy.double() @ w).float().cpu(), torch.bfloat16, "dx")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(256, 136, 32), (264, 776, 33), (1600, 1608, 333), (8, 328, 7), (6400, 1600, 129)])
+def test_weight_gradient(dtype, m, n, k):
+    """both operands mn-major; the bound of test_gemm"""
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    a, b = torch.randn(k, m, generator=g, device=DEV).to(dtype), torch.randn(k, n, generator=g, device=DEV).to(dtype)
+    c = _gemm(a, b, False, False, m, n, k, torch.float32, 3)
+    worst = (c.double() - a.double().t() @ b.double()).abs() - (k + 16) * 2.0**-23 * (a.double().abs().t() @ b.double().abs())
+    assert worst.max().item() <= 0.0
