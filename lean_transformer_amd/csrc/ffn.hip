@@ -248,7 +248,8 @@ void plan_linear_backward(const lt_linear& lin, int64_t T, int dtype, Bump& ws, 
   }
   if (lin.block == 64 && dtype == LT_BF16)
     s.skinny_bytes = std::max(s.skinny_bytes,
-                              lt_sparse_dw_split_workspace(lin.in_features, lin.blocks_per_in, group_length(lin.in_group), T));
+                              lt_sparse_dw_split_workspace(lin.in_features, lin.out_features, lin.blocks_per_in, lin.blocks_per_out,
+                                                           group_length(lin.in_group), group_length(lin.out_group), T));
   s.skinny = s.skinny_bytes ? ws.take(s.skinny_bytes) : nullptr;
 }
 
@@ -320,7 +321,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
       p.sp.out_group = lin.forward_indices ? group_length(lin.out_group) : 0; p.sp.out_stride = group_stride(lin.out_group);
       p.sp.in_group = group_length(lin.in_group); p.sp.in_stride = group_stride(lin.in_group);
       p.epi = epi_store_params(grads.weight, lin.block, dtype, nullptr);
-      const int slices = dtype == LT_BF16 ? lt_sparse_dw_in_grouped_slices(p) : 0;
+      const int slices = dtype == LT_BF16 ? lt_sparse_dw_slices(p) : 0;
       const size_t elements = (size_t)(in / lin.block) * lin.blocks_per_in * lin.block * lin.block;
       if (slices > 1 && s.skinny && s.skinny_bytes >= (size_t)slices * elements * sizeof(float)) {
         // the reduction over the tokens split over workgroups: fp32 partial gradients, summed into the parameter's dtype
@@ -332,7 +333,8 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
         LT_TRY(lt_splitk_reduce((const float*)s.skinny, slices, (int64_t)elements, (int64_t)elements, lin.block, nullptr, dtype,
                                 grads.weight, stream));
       } else {
-        if (slices > 1) p.sp.in_group = 0;  // no room for the partial sums: the walk
+        // no room for the partial sums: runs of output blocks unsplit, runs of input blocks as the walk
+        if (slices > 1 && !lt_sparse_dw_out_grouped(p)) p.sp.in_group = 0;
         LT_TRY(lt_launch_gemm_sparse(p, EPI_STORE, dtype, io_dtype, stream));
       }
     }

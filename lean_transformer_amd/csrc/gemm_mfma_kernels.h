@@ -1797,7 +1797,9 @@ template <int KIND> int launch_sparse(const GemmProblem& problem, int io_dtype, 
     if constexpr (KIND == EPI_STORE) {
       const int64_t out_features = sp.ld_act;
       if (lt_sparse_dw_out_grouped(p)) {
-        // grouped: a dense both-operands-mn-major product dY^T X per run of 4 output blocks, over their shared list
+        // grouped: a dense both-operands-mn-major product dY^T X per run of 4 output blocks, over their shared list.  The
+        // reduction is split only when the caller asked (p.ksplit slices, epi.out pointing at fp32 partial sums)
+        const int slices = p.ksplit > 1 ? p.ksplit : 1;
         GemmProblem q = p;
         q.M = out_features;
         const int tiles_m = (int)(out_features / 256), tiles_n = (sp.blocks_per_out + 3) / 4;
@@ -1805,15 +1807,14 @@ template <int KIND> int launch_sparse(const GemmProblem& problem, int io_dtype, 
         q.nseg = 1; q.K[0] = sp.tokens; q.K[1] = 0;
         q.A[0].ptr = sp.act; q.A[0].ld = sp.ld_act; q.A[0].kmajor = 0;
         q.B[0].ptr = sp.act2; q.B[0].ld = sp.ld_act2; q.B[0].kmajor = 0;
-        q.ksplit = 0; q.krot = 0;
-        hipLaunchKernelGGL((gemm_bf16_dma_kernel<false, false, EPI_STORE, float, 1>), dim3(dma_grid(q, tiles_m * tiles_n)),
-                           block, 0, stream, q, tiles_m, tiles_n);
+        q.ksplit = slices > 1 ? slices : 0; q.krot = 0;
+        hipLaunchKernelGGL((gemm_bf16_dma_kernel<false, false, EPI_STORE, float, 1>),
+                           dim3(dma_grid(q, tiles_m * tiles_n), (unsigned)slices), block, 0, stream, q, tiles_m, tiles_n);
         LT_LAUNCH_CHECK();
         return LT_OK;
       }
-      if (lt_sparse_dw_in_grouped_slices(p) > 0) {
-        // grouped on the input side: dY^T X per run of 4 input blocks, over their shared list of output blocks.  The
-        // reduction is split only when the caller asked (p.ksplit slices, epi.out pointing at fp32 partial sums)
+      if (lt_sparse_dw_in_grouped(p)) {
+        // grouped on the input side: dY^T X per run of 4 input blocks, over their shared list of output blocks, split alike
         const int slices = p.ksplit > 1 ? p.ksplit : 1;
         GemmProblem q = p;
         const int tiles_m = (sp.blocks_per_in + 3) / 4, tiles_n = (int)(p.N / 256);

@@ -439,11 +439,14 @@ double lt_gemm_flops(const GemmProblem& p, int kind);
 bool lt_sparse_forward_grouped(const GemmProblem& p, int kind);
 // whether a block-sparse weight-gradient problem (SPARSE_DW) runs as dense products per run of 4 output blocks (sp.out_group)
 bool lt_sparse_dw_out_grouped(const GemmProblem& p);
-// ... or per run of 4 input blocks (sp.in_group): 0 when not, else the number of slices its reduction over the tokens is
-// best split into (1: no split).  With more than one slice the caller sets p.ksplit = slices, p.split_stride = elements of the
-// weight gradient, and points epi.out at fp32 partial sums (lt_sparse_dw_split_workspace bytes) that it sums afterwards.
-int lt_sparse_dw_in_grouped_slices(const GemmProblem& p);
-size_t lt_sparse_dw_split_workspace(int64_t in_features, int blocks_per_in, int in_group, int64_t tokens);
+// ... or per run of 4 input blocks (sp.in_group)
+bool lt_sparse_dw_in_grouped(const GemmProblem& p);
+// 0 when it runs as neither, else the number of slices its reduction over the tokens is best split into (1: no split).  With more
+// than one slice the caller sets p.ksplit = slices, p.split_stride = elements of the weight gradient, and points epi.out at fp32
+// partial sums (lt_sparse_dw_split_workspace bytes) that it sums afterwards.
+int lt_sparse_dw_slices(const GemmProblem& p);
+size_t lt_sparse_dw_split_workspace(int64_t in_features, int64_t out_features, int blocks_per_in, int blocks_per_out, int in_group,
+                                    int out_group, int64_t tokens);
 // whether the bf16 matrix-core walk for 64 x 64 blocks takes this block-sparse problem with epilogue `kind`
 bool lt_sparse_mfma_supported(const GemmProblem& p, int kind);
 int lt_launch_gemm_sparse(const GemmProblem& p, int kind, int dtype, int io_dtype, hipStream_t stream);
