@@ -12,6 +12,8 @@
 // end of the reduction (the buffer unit returns zeros past the descriptor's size), so that whole, ragged and absent stages go through
 // the same straight-line code.
 #include "gemm_mfma_kernels.h"
+#include "gemm_staged.h"
+#include "gemm_strips.h"
 
 namespace {
 
@@ -47,12 +49,12 @@ template <bool KM> struct MidOperand {
     base = KM ? ptr + row0 * ld * 2 : ptr + row0 * 2;
     unit_bytes = KM ? 64 * 2 : 64 * ld * 2;
   }
-  // the 64 k from u * 64 on; pieces at or past k_limit arrive as zeros
-  __device__ __forceinline__ void issue(int u, bf16* dst, int wave, int lane, int k_limit) const {
+  // copies J0 .. J1 - 1 of the 64 k from u * 64 on; pieces at or past k_limit arrive as zeros
+  template <int J0, int J1> __device__ __forceinline__ void issue(int u, bf16* dst, int wave, int lane, int k_limit) const {
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base + u * unit_bytes), 0, (int)RECORDS, 0x00020000);
 #pragma unroll
-    for (int j = 0; j < LOADS; j++) {
+    for (int j = J0; j < J1; j++) {
       const int q = (wave * LOADS + j) * 64 + lane;
       const int k = u * 64 + (KM ? ((q & 7) ^ swz_km(q >> 3)) * 8 : q >> 4);
       const uint32_t o = k < k_limit ? off[j] : OUTSIDE;
@@ -111,12 +113,14 @@ __global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int t
   MidOperand<B_KM> cb;
   ca.setup(p.A[0], m0, p.M, 0, wave, lane);
   cb.setup(p.B[0], n0, p.N, gated ? p.N : 0, wave, lane);
-  auto copy = [&](auto S, int t) __attribute__((always_inline)) {
+  // copies J0 .. J1 - 1 (A's four, then B's) of step t
+  auto copy = [&](auto S, int t, auto J0_, auto J1_) __attribute__((always_inline)) {
+    constexpr int j0 = decltype(J0_)::value, j1 = decltype(J1_)::value;
     int u = t + rot;
     if (u >= total) u -= total;
-    u = t < total ? first + u : all;  // (past the last stage: zeros)
-    ca.issue(u, a_buf(S), wave, lane, k_limit);
-    cb.issue(u, b_buf(S), wave, lane, k_limit);
+    u = t < total ? first + u : all;  // (past the last step: zeros)
+    if constexpr (j0 < 4) ca.template issue<j0, (j1 < 4 ? j1 : 4)>(u, a_buf(S), wave, lane, k_limit);
+    if constexpr (j1 > 4) cb.template issue<(j0 > 4 ? j0 - 4 : 0), j1 - 4>(u, b_buf(S), wave, lane, k_limit);
   };
 
   f32x16 acc[2][2];
@@ -141,128 +145,36 @@ __global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int t
     }
     return u.v;
   };
-  auto multiply = [&](auto S) __attribute__((always_inline)) {
-#pragma unroll
-    for (int kk = 0; kk < 4; kk++) {
-      bf16x8 a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; i++) {
-        if constexpr (A_KM) a[i] = frag_km(a_buf(S), wm * 64 + i * 32, kk);
-        else a[i] = frag_mn(a_buf(S), wm * 64 + i * 32, kk);
-        if constexpr (B_KM) b[i] = frag_km(b_buf(S), wn * 64 + i * 32, kk);
-        else b[i] = frag_mn(b_buf(S), wn * 64 + i * 32, kk);
-      }
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = LT_MFMA_32X32X16(a[i], b[j], acc[i][j]);
-    }
-  };
-  // stage t: its copies have landed in every wavefront after the barrier, and every wavefront has read stage t - 1, whose buffer the
-  // copies of stage t + STAGES - 1 then take
-  constexpr int AHEAD = STAGES - 1;
-  lt_static_for<AHEAD>([&](auto S) __attribute__((always_inline)) { copy(S, decltype(S)::value); });
-  for (int t0 = 0; t0 < total; t0 += STAGES) {
-    lt_static_for<STAGES>([&](auto S) __attribute__((always_inline)) {
-      constexpr int s = decltype(S)::value;
-      wait_copies_and_barrier<(AHEAD - 1) * 8>();
-      copy(std::integral_constant<int, s + AHEAD>{}, t0 + s + AHEAD);
-      multiply(S);  // (zeros past the last stage)
-    });
-  }
-  wait_copies_and_barrier<0>();
-
-  // ---- epilogue: strips of 32 rows x 64 columns, transposed through 8 KiB of LDS of this wavefront's own and read back 8 columns per
-  //      lane; what a strip reads from memory is requested before it is staged.  Accumulator register r of a 32 x 32 block is row
-  //      8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32; columns of rows with bit 2 set are staged 32 further on (banks).
-  EpiParams epi = p.epi;
-  if (KIND == EPI_STORE && p.ksplit > 1) epi.out = reinterpret_cast<float*>(epi.out) + (int64_t)blockIdx.y * p.split_stride;
-  epi.bias = nullptr;
-  float* const stage = reinterpret_cast<float*>(wave == 0 ? a0 : wave == 1 ? a1 : wave == 2 ? b0 : b1);
-  auto staged = [&](int row, int col) -> float* { return &stage[row * 64 + (col ^ (((row >> 2) & 1) << 5))]; };
-  float colsum[16];  // EPI_ACT_BWD: column sums of the dpre values this lane writes
-#pragma unroll
-  for (int e = 0; e < 16; e++) colsum[e] = 0.f;
-  auto strips = [&](auto G) __attribute__((always_inline)) {
-    constexpr bool PAIR = decltype(G)::value;
-    constexpr int PER_ROW = PAIR ? 4 : 8, ROWS = 64 / PER_ROW, NIT = 32 / ROWS;
-    const int c = (lane % PER_ROW) * 8;
-    const int64_t n = n0 + wn * (PAIR ? 32 : 64) + c;
-    const bool in_n = n < p.N;  // N is a multiple of 8
-    float bias0[8], bias1[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) bias0[e] = bias1[e] = 0.f;
-    if (p.epi.bias && in_n) {
-      load8(p.epi.bias + n, bias0);
-      if constexpr (PAIR) load8(p.epi.bias + epi.inter + n, bias1);
-    }
+  bf16x8 fa[2][2], fb[2][2];
+  auto load = [&](auto S, auto KK, auto F) __attribute__((always_inline)) {
+    constexpr int kk = decltype(KK)::value, f = decltype(F)::value;
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      const int64_t mrow0 = m0 + wm * 64 + i * 32 + lane / PER_ROW;
-      EpiLoad in[NIT];
-      if constexpr (KIND == EPI_ACT_BWD || KIND == EPI_OUT) {
-#pragma unroll
-        for (int it = 0; it < NIT; it++)
-          in[it] = epi_load8<KIND, TX>(epi, min(mrow0 + it * ROWS, p.M - 1), in_n ? n : 0, true);
-      }
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int j = 0; j < 2; j++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) *staged(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), j * 32 + (lane & 31)) = acc[i][j][r];
-      __builtin_amdgcn_wave_barrier();
-      auto read8 = [&](int row, int col, const float (&bias)[8], float (&v)[8]) __attribute__((always_inline)) {
-        const float* sv = staged(row, col);
-        const f32x4 lo = *reinterpret_cast<const f32x4*>(sv), hi = *reinterpret_cast<const f32x4*>(sv + 4);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          v[e] = lo[e] + bias[e];
-          v[4 + e] = hi[e] + bias[4 + e];
-        }
-      };
-#pragma unroll
-      for (int it = 0; it < NIT; it++) {
-        const int row = it * ROWS + lane / PER_ROW;
-        const int64_t m = mrow0 + it * ROWS;
-        float v[8];
-        read8(row, c, bias0, v);
-        if constexpr (PAIR) {
-          float vl[8];
-          read8(row, 32 + c, bias1, vl);
-          if (in_n && m < p.M) epi_act_fwd_gated8<ACT>(epi, m, n, v, vl);
-        } else if (in_n && m < p.M) {
-          if constexpr (KIND == EPI_STORE) epi_store8(epi, m, n, v);
-          else if constexpr (KIND == EPI_ACT_FWD) epi_act_fwd8<ACT>(epi, m, n, v);
-          else if constexpr (KIND == EPI_ACT_BWD) epi_act_bwd8_loaded<ACT>(epi, m, n, v, in[it], colsum);
-          else epi_out8_loaded<TX>(epi, m, n, v, in[it]);
-        }
-      }
-    }
-    if constexpr (KIND == EPI_ACT_BWD) {
-      if (epi.colsum) {  // lanes l, l + 8, ... hold the same columns; one partial row per 64 rows of the result
-#pragma unroll
-        for (int e = 0; e < 16; e++)
-#pragma unroll
-          for (int mask = 8; mask < 64; mask <<= 1) colsum[e] += __shfl_xor(colsum[e], mask, 64);
-        if (lane < 8 && in_n && m0 + wm * 64 < p.M) {
-          float* dst = epi.colsum + ((m0 + wm * 64) / 64) * epi.ld_pre + n;
-          float lo[8], hi[8];
-#pragma unroll
-          for (int e = 0; e < 8; e++) {
-            lo[e] = colsum[e];
-            hi[e] = colsum[8 + e];
-          }
-          store8(dst, lo);
-          if (epi.gated) store8(dst + epi.inter, hi);
-        }
-      }
+      if constexpr (A_KM) fa[f][i] = frag_km(a_buf(S), wm * 64 + i * 32, kk);
+      else fa[f][i] = frag_mn(a_buf(S), wm * 64 + i * 32, kk);
+      if constexpr (B_KM) fb[f][i] = frag_km(b_buf(S), wn * 64 + i * 32, kk);
+      else fb[f][i] = frag_mn(b_buf(S), wn * 64 + i * 32, kk);
     }
   };
+  auto multiply = [&](auto F) __attribute__((always_inline)) {
+    constexpr int f = decltype(F)::value;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) acc[i][j] = LT_MFMA_32X32X16(fa[f][i], fb[f][j], acc[i][j]);
+  };
+  using Loop = StagedLoop<STAGES, 8, 2 * (A_KM ? 1 : 2) + 2 * (B_KM ? 1 : 2)>;
+  Loop::start(0, copy, load);
+  Loop::run(0, total, copy, load, multiply);
+  wait_copies_and_barrier<0>();
+
+  // ---- epilogue (strip_epilogue)
+  float* const stage = reinterpret_cast<float*>(wave == 0 ? a0 : wave == 1 ? a1 : wave == 2 ? b0 : b1);
   if constexpr (KIND == EPI_ACT_FWD) {
-    if (gated) strips(std::true_type{});
-    else strips(std::false_type{});
+    if (gated) strip_epilogue<KIND, TX, ACT, true>(acc, p, stage, m0 + wm * 64, n0 + wn * 32, lane);
+    else strip_epilogue<KIND, TX, ACT, false>(acc, p, stage, m0 + wm * 64, n0 + wn * 64, lane);
   } else {
-    strips(std::false_type{});
+    strip_epilogue<KIND, TX, ACT, false>(acc, p, stage, m0 + wm * 64, n0 + wn * 64, lane);
   }
 }
 
