@@ -14,7 +14,7 @@ from concurrent.futures import ThreadPoolExecutor
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_PATH = os.path.join(CSRC, "libleanffn.so")
 # the tiled GEMM kernels are instantiated per epilogue kind in four translation units so that they compile in parallel
-SOURCES = ["gemm_mfma_kind0.hip", "gemm_mfma_kind1.hip", "gemm_mfma_kind2.hip", "gemm_mfma_kind3.hip", "gemm_mid.hip",
+SOURCES = ["gemm_mfma_kind0.hip", "gemm_mfma_kind1.hip", "gemm_mfma_kind2.hip", "gemm_mfma_kind3.hip", "gemm_mid.hip", "gemm_walk.hip",
            "gemm_generic.hip", "gemm_stream.hip", "elementwise.hip", "ffn.hip", "gemm_mfma_bf16.hip", "profile.hip"]
 # -packed-fp32-ops is switched off: the compiler must not form v_pk_{add,mul,fma}_f32 from scalar float code
 # -pragma-unroll-threshold: the fused GEMM epilogues index the accumulator registers from fully unrolled loops; left rolled

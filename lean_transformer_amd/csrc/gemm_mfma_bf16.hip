@@ -10,10 +10,8 @@ int lt_mfma_launch_dense_kind0(const GemmProblem& p, int io_dtype, hipStream_t s
 int lt_mfma_launch_dense_kind1(const GemmProblem& p, int io_dtype, hipStream_t stream);
 int lt_mfma_launch_dense_kind2(const GemmProblem& p, int io_dtype, hipStream_t stream);
 int lt_mfma_launch_dense_kind3(const GemmProblem& p, int io_dtype, hipStream_t stream);
-int lt_mfma_launch_sparse_kind0(const GemmProblem& p, int io_dtype, hipStream_t stream);
-int lt_mfma_launch_sparse_kind1(const GemmProblem& p, int io_dtype, hipStream_t stream);
-int lt_mfma_launch_sparse_kind2(const GemmProblem& p, int io_dtype, hipStream_t stream);
-int lt_mfma_launch_sparse_kind3(const GemmProblem& p, int io_dtype, hipStream_t stream);
+int lt_mfma_launch_sparse_kind0(const GemmProblem& p, hipStream_t stream);
+int lt_mfma_launch_sparse_kind1(const GemmProblem& p, hipStream_t stream);
 // 128 x 128 tile, plain store, `slices` slices of the reduction (gemm_mfma_kind0.hip)
 int lt_mfma_launch_skinny(const GemmProblem& p, int slices, hipStream_t stream);
 
@@ -119,10 +117,7 @@ int lt_gemm_colsum_rows(const GemmProblem& p, int dtype, int io_dtype) {
   if (mid_selected(p, EPI_ACT_BWD)) return 64;
   if (p.sp.mode == SPARSE_NONE)
     return lt_gemm_mfma_supported(p, EPI_ACT_BWD) && dma_selected(p, EPI_ACT_BWD) ? 128 : 0;
-  // the walk's straight-line strips keep the sums: every tile must take them
-  return p.sp.mode == SPARSE_DX && lt_sparse_mfma_supported(p, EPI_ACT_BWD) && p.M % 256 == 0 &&
-                 p.epi.act == LT_ACT_GELU_FUSED && p.epi.hid
-             ? 64 : 0;
+  return p.sp.mode == SPARSE_DX && lt_sparse_mfma_supported(p, EPI_ACT_BWD) ? 64 : 0;
 }
 
 static const char* mfma_tag(const GemmProblem& p, int kind, bool mid) {
@@ -385,7 +380,10 @@ bool lt_sparse_mfma_supported(const GemmProblem& p, int kind) {
     return true;
   }
   if (!lt_aligned(sp.weight, 16)) return false;
+  // the walk addresses a tile's rows with 32-bit byte offsets
+  if (257 * sp.ld_act * 2 + 1024 >= (int64_t)1 << 32) return false;
   if (p.nseg > 1) {
+    if (257 * p.A[1].ld * 2 + 1024 >= (int64_t)1 << 32 || 65 * p.B[1].ld * 2 + 1024 >= (int64_t)1 << 32) return false;
     if (p.K[1] <= 0 || p.K[1] % 8 != 0 || p.A[1].ld % 8 != 0 || p.B[1].ld % 8 != 0 || !lt_aligned(p.A[1].ptr, 16) ||
         !lt_aligned(p.B[1].ptr, 16))
       return false;
@@ -467,13 +465,10 @@ int lt_launch_gemm_sparse(const GemmProblem& p, int kind, int dtype, int io_dtyp
   if (sp.mode == SPARSE_DW) flops = 2.0 * (double)sp.tokens * (double)(p.N / 64) * sp.blocks_per_in * 4096.0;
   static const char* tags[4] = {"", "blocksparse_fwd_bf16", "blocksparse_dx_bf16", "blocksparse_dw_bf16"};
   LtProfileScope scope(tags[sp.mode], flops, 0.0, stream);
-  switch (kind) {
-    case EPI_STORE: return lt_mfma_launch_sparse_kind0(p, io_dtype, stream);
-    case EPI_ACT_FWD: return lt_mfma_launch_sparse_kind1(p, io_dtype, stream);
-    case EPI_ACT_BWD: return lt_mfma_launch_sparse_kind2(p, io_dtype, stream);
-    case EPI_OUT: return lt_mfma_launch_sparse_kind3(p, io_dtype, stream);
-  }
-  LT_FAIL(LT_ERR_BAD_ARG, "unknown epilogue kind %d", kind);
+  if (sp.mode != SPARSE_DW && !lt_sparse_forward_grouped(p, kind)) return lt_launch_gemm_walk(p, kind, io_dtype, stream);
+  if (kind == EPI_STORE) return lt_mfma_launch_sparse_kind0(p, stream);
+  if (kind == EPI_ACT_FWD) return lt_mfma_launch_sparse_kind1(p, stream);
+  LT_FAIL(LT_ERR_BAD_ARG, "block-sparse product: unknown epilogue kind %d", kind);
 }
 
 int lt_launch_gemm(const GemmProblem& p, int kind, int dtype, int io_dtype, hipStream_t stream) {

@@ -5,7 +5,7 @@
 //   gemm_bf16_dma_kernel  256 x 256 tile, operands copied global -> LDS without passing through registers; the kernel of
 //                         the dense projections (second half of this file)
 //   gemm_bf16_kernel      BM x BN tile, operands staged through registers; 32-bit offset overflow, the 128 x 128 tile of the
-//                         skinny low-rank GEMMs, and the block-sparse walks over 64 x 64 blocks
+//                         skinny low-rank GEMMs, and the block-sparse weight-gradient walk over 64 x 64 blocks
 //
 // gemm_bf16_kernel.  Tile: BM x BN outputs per workgroup, 64 k per step, WM x WN wavefronts each owning a (BM/WM) x (BN/WN)
 // sub-tile as 32 x 32 MFMA blocks.  Operand tiles go global -> registers -> LDS (16-byte accesses) and are double-buffered
@@ -95,27 +95,19 @@ template <int N, typename F> __device__ __forceinline__ void lt_static_for(F&& f
   lt_static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// PH = 2 (block-sparse forward with the gated activation epilogue only): a workgroup owns gate block tn and the matching
-// linear block tn + N / 64, which have index lists of their own.  It walks the two lists one after the other (two phases
-// over the same LDS stages) into two sets of accumulators and pairs them in the epilogue, so the gated activation needs no
-// pass of its own over the pre-activations.
 // PF: how many k-steps ahead of the matrix instructions the operand tiles are requested (in registers; the LDS holds two
 // stages whatever PF is).  1 for the MFMA-bound uses; the rank-r products stream a large operand once against a small one and
 // are bound by how many bytes a CU has in flight, so they ask further ahead.
-template <int BM, int BN, int WM, int WN, bool A_KM, bool B_KM, int KIND, typename TX, int SP = SPARSE_NONE, int PH = 1, int PF = 1>
+template <int BM, int BN, int WM, int WN, bool A_KM, bool B_KM, int KIND, typename TX, int SP = SPARSE_NONE, int PF = 1>
 __global__ __launch_bounds__(WM * WN * 64)
-__attribute__((amdgpu_waves_per_eu((SP != SPARSE_NONE || PF > 1) ? 2 : 1)))  // block-sparse walks, rank-r products: two workgroups per CU
+__attribute__((amdgpu_waves_per_eu((SP != SPARSE_NONE || PF > 1) ? 2 : 1)))  // block-sparse walk, rank-r products: two workgroups per CU
 void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
   constexpr int NT = WM * WN * 64;
-  static_assert(PF == 1 || (SP == SPARSE_NONE && PH == 1), "deeper prefetch: dense single-phase only");
-  static_assert(PH == 1 || (PH == 2 && SP == SPARSE_FWD && KIND == EPI_ACT_FWD && WN == 1), "two phases: gated block-sparse forward");
-  static_assert(SP == SPARSE_NONE || (SP == SPARSE_FWD && A_KM && B_KM && BN == 64) ||
-                    (SP == SPARSE_DX && A_KM && !B_KM && BN == 64) ||
-                    (SP == SPARSE_DW && !A_KM && !B_KM && BM == 256 && BN == 64 && WM == 4 && WN == 1),
-                "operand layouts and tile shape of the block-sparse walks");
+  static_assert(PF == 1 || SP == SPARSE_NONE, "deeper prefetch: dense only");
+  static_assert(SP == SPARSE_NONE || (SP == SPARSE_DW && KIND == EPI_STORE && !A_KM && !B_KM && BM == 256 && BN == 64 && WM == 4 && WN == 1),
+                "operand layouts and tile shape of the block-sparse walk");
   constexpr int WTM = BM / WM;
-  constexpr int WTN_IN = BN / WN, FN_IN = WTN_IN / 32;  // columns / column blocks of a wavefront in one phase
-  constexpr int WTN = WTN_IN * PH, FN = FN_IN * PH;     // ... and of its output sub-tile
+  constexpr int WTN = BN / WN, FN = WTN / 32;
   constexpr int FM = WTM / 32;
   constexpr int A_CHUNKS = BM * BK / 8 / NT, B_CHUNKS = BN * BK / 8 / NT;  // 16-byte chunks per thread per stage
   static_assert(BM * BK / 8 % NT == 0 && BN * BK / 8 % NT == 0, "tile must divide over the threads");
@@ -133,28 +125,17 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
   const int wm = wave / WN, wn = wave % WN;
   const bool gated = (KIND == EPI_ACT_FWD) && p.epi.gated;
 
-#ifdef LT_TILE_TIMING
-  unsigned long long* const tile_stamps =
-      ((SP == SPARSE_FWD || SP == SPARSE_DX) && p.tile_stamps) ? p.tile_stamps + (size_t)blockIdx.x * 8 : nullptr;
-#endif
-  LT_TILE_STAMP(0);
-  LT_TILE_STAMP_REALTIME(4);
   // ---- tile assignment: XCD-contiguous, grouped along M
   int pid = blockIdx.x;
   const int num_pid = tiles_m * tiles_n;
   if ((num_pid & 7) == 0) pid = (pid & 7) * (num_pid >> 3) + (pid >> 3);
-  // Block-sparse FWD / DX: the workgroups of one token tile gather column blocks of the same 256 activation rows (a few MiB
-  // that stay in the XCD's L2) while every block column has a weight list of its own, so one XCD's concurrent workgroups
-  // take one token tile and consecutive block columns.
-  constexpr int GROUP_ROWS = (SP == SPARSE_FWD || SP == SPARSE_DX) ? 1 : GROUP_M;
-  const int group = GROUP_ROWS * tiles_n;
-  const int first_m = (pid / group) * GROUP_ROWS;
-  const int gsz = min(tiles_m - first_m, GROUP_ROWS);
+  const int group = GROUP_M * tiles_n;
+  const int first_m = (pid / group) * GROUP_M;
+  const int gsz = min(tiles_m - first_m, GROUP_M);
   const int tm = first_m + (pid % group) % gsz;
   const int tn = (pid % group) / gsz;
   const int64_t m0 = (int64_t)tm * BM;
-  // gated: in gate columns; sparse FWD / DX: tn = block index (two phases: the gate block)
-  const int64_t n0 = (int64_t)tn * ((gated && PH == 1) ? BN / 2 : BN);
+  const int64_t n0 = (int64_t)tn * (gated ? BN / 2 : BN);  // gated: in gate columns
 
   f32x16 acc[FM][FN];
 #pragma unroll
@@ -166,12 +147,9 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
 
   u32x4 ra_set[PF][A_CHUNKS], rb_set[PF][B_CHUNKS];
 
-  // k-steps: dense: segment 0 then segment 1; sparse FWD / DX: the active blocks of this group, then the low-rank segment
+  // k-steps: dense: segment 0 then segment 1
   const SparseWalk& sp = p.sp;
-  const int sp_steps = SP == SPARSE_FWD ? sp.blocks_per_out : sp.blocks_per_in;
-  const int kt_seg0 = SP == SPARSE_NONE ? (int)((p.K[0] + BK - 1) / BK)
-                      : SP == SPARSE_DW ? (int)((sp.tokens + BK - 1) / BK)
-                                        : sp_steps;
+  const int kt_seg0 = (int)(((SP == SPARSE_DW ? sp.tokens : p.K[0]) + BK - 1) / BK);
   const int kt_total = kt_seg0 + ((SP != SPARSE_DW && p.nseg > 1) ? (int)((p.K[1] + BK - 1) / BK) : 0);
   // sparse DW: group tn = (input block, quad of its active output blocks a0 .. a0 + 3); a short last quad repeats the last
   // block (computed, not stored)
@@ -187,16 +165,10 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
       dw_ob[j] = sp.backward_indices[(int64_t)dw_ib * sp.blocks_per_in + min(dw_a0 + j, sp.blocks_per_in - 1)];
   }
 
-  // position in the group's index list taken at step t of the walk (see SparseWalk::walk_run)
-  auto walk_entry = [&](int t) {
-    if (sp.walk_run <= 1) return t;
-    const int runs = sp_steps / sp.walk_run;
-    return (t % runs) * sp.walk_run + t / runs;
-  };
-  // global -> registers for k-step kt (ph: 0 = the tile's own block column, 1 = the matching linear block column)
+  // global -> registers for k-step kt
   // TAIL: the step may reach past the end of its reduction; pieces of a k-major operand past it repeat the last piece (and are
   // zeroed by store_tiles)
-  auto load_tiles = [&](auto TAIL, int kt, int ph, u32x4 (&ra)[A_CHUNKS], u32x4 (&rb)[B_CHUNKS]) __attribute__((always_inline)) {
+  auto load_tiles = [&](auto TAIL, int kt, u32x4 (&ra)[A_CHUNKS], u32x4 (&rb)[B_CHUNKS]) __attribute__((always_inline)) {
     constexpr bool tail = decltype(TAIL)::value;
     const int seg = kt >= kt_seg0;
     int64_t k0 = (int64_t)(seg ? kt - kt_seg0 : kt) * BK;
@@ -204,24 +176,8 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
     const bf16* A = reinterpret_cast<const bf16*>(p.A[seg].ptr);
     const bf16* B = reinterpret_cast<const bf16*>(p.B[seg].ptr);
     int64_t lda = p.A[seg].ld, ldb = p.B[seg].ld;
-    int64_t b_row0 = n0 + (PH == 2 ? ph * p.N : 0);  // first B row (k-major) / column (mn-major) of this tile
-    if constexpr (SP == SPARSE_FWD) {
-      if (!seg) {  // A: column block ib of X; B: weight block f, a [64 rows][64 k] matrix of its own
-        const int f = sp.forward_indices[(int64_t)(tn + (PH == 2 ? ph * tiles_n : 0)) * sp.blocks_per_out + walk_entry(kt)];
-        A = reinterpret_cast<const bf16*>(sp.act); lda = sp.ld_act; k0 = (int64_t)(f / sp.blocks_per_in) * 64;
-        B = reinterpret_cast<const bf16*>(sp.weight) + (int64_t)f * 4096; ldb = 64; b_row0 = 0;
-        K = k0 + 64;
-      }
-    } else if constexpr (SP == SPARSE_DX) {
-      if (!seg) {  // A: column block ob of dY; B: weight block (ib, a) read as [64 k = output row][64 n = input column]
-        const int a = walk_entry(kt);
-        const int64_t ob = sp.backward_indices[(int64_t)tn * sp.blocks_per_in + a];
-        A = reinterpret_cast<const bf16*>(sp.act); lda = sp.ld_act; k0 = ob * 64;
-        B = reinterpret_cast<const bf16*>(sp.weight) + ((int64_t)tn * sp.blocks_per_in + a) * 4096 - k0 * 64; ldb = 64;
-        b_row0 = 0;
-        K = k0 + 64;
-      }
-    } else if constexpr (SP == SPARSE_DW) {  // A: four gathered dY column blocks; B: X column block ib; k = tokens
+    int64_t b_row0 = n0;  // first B row (k-major) / column (mn-major) of this tile
+    if constexpr (SP == SPARSE_DW) {  // A: four gathered dY column blocks; B: X column block ib; k = tokens
       A = reinterpret_cast<const bf16*>(sp.act); lda = sp.ld_act;
       B = reinterpret_cast<const bf16*>(sp.act2) + (int64_t)dw_ib * 64; ldb = sp.ld_act2; b_row0 = 0;
       K = sp.tokens;
@@ -249,14 +205,13 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
       if constexpr (B_KM) {
         const int row = q >> 3, c = q & 7;
         int64_t gn;
-        if (gated && PH == 1) {
+        if (gated) {
           const int rr = row % WTN;
           gn = (rr / (WTN / 2)) * p.N + n0 + (row / WTN) * (WTN / 2) + rr % (WTN / 2);
         } else {
           gn = b_row0 + row;
         }
-        // a sparse FWD weight block holds its own 64 k: its columns start at 0, not at the gathered k0
-        const int64_t bk = (SP == SPARSE_FWD && !seg) ? c * 8 : tail ? min(k0 + c * 8, K - 8) : k0 + c * 8;
+        const int64_t bk = tail ? min(k0 + c * 8, K - 8) : k0 + c * 8;
         rb[i] = *reinterpret_cast<const u32x4*>(B + gn * ldb + bk);
       } else {
         const int kr = q / (BN / 8), c = q % (BN / 8);
@@ -268,7 +223,6 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
   // how many of the BK k of step kt exist (a multiple of 8 where an operand is k-major); operand tiles are zero-filled past them
   auto k_rows = [&](int kt) -> int {
     const int seg = kt >= kt_seg0;
-    if ((SP == SPARSE_FWD || SP == SPARSE_DX) && !seg) return BK;
     const int64_t k0 = (int64_t)(seg ? kt - kt_seg0 : kt) * BK;
     const int64_t K = SP == SPARSE_DW ? (int64_t)sp.tokens : p.K[seg];
     return (int)min((int64_t)BK, K - k0);
@@ -320,19 +274,19 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
     return u.v;
   };
 
-  auto load_frags = [&](int s, int kk, bf16x8 (&a)[FM], bf16x8 (&b)[FN_IN]) {
+  auto load_frags = [&](int s, int kk, bf16x8 (&a)[FM], bf16x8 (&b)[FN]) {
 #pragma unroll
     for (int i = 0; i < FM; i++) {
       if constexpr (A_KM) a[i] = frag_km(lds_a[s], wm * WTM + i * 32, kk);
       else a[i] = frag_mn(lds_a[s], std::integral_constant<int, BM>{}, wm * WTM + i * 32, kk);
     }
 #pragma unroll
-    for (int j = 0; j < FN_IN; j++) {
-      if constexpr (B_KM) b[j] = frag_km(lds_b[s], wn * WTN_IN + j * 32, kk);
-      else b[j] = frag_mn(lds_b[s], std::integral_constant<int, BN>{}, wn * WTN_IN + j * 32, kk);
+    for (int j = 0; j < FN; j++) {
+      if constexpr (B_KM) b[j] = frag_km(lds_b[s], wn * WTN + j * 32, kk);
+      else b[j] = frag_mn(lds_b[s], std::integral_constant<int, BN>{}, wn * WTN + j * 32, kk);
     }
   };
-  constexpr int FRAG_READS = FM * (A_KM ? 1 : 2) + FN_IN * (B_KM ? 1 : 2);  // LDS read instructions per k-substep
+  constexpr int FRAG_READS = FM * (A_KM ? 1 : 2) + FN * (B_KM ? 1 : 2);  // LDS read instructions per k-substep
 
   // split-k: this workgroup's slice of the k-steps
   int kt_begin = 0, kt_end = kt_total;
@@ -343,9 +297,8 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
   }
   // the matrix instructions of one k-step on LDS stage s.  Fragments are double-buffered in registers: the LDS reads of
   // k-substep kk + 1 are issued before, and interleaved with, the MFMAs of k-substep kk
-  auto multiply_stage = [&](int s, auto PHASE) __attribute__((always_inline)) {
-    constexpr int j0 = decltype(PHASE)::value * FN_IN;  // this phase's accumulator columns
-    bf16x8 af[2][FM], bfr[2][FN_IN];
+  auto multiply_stage = [&](int s) __attribute__((always_inline)) {
+    bf16x8 af[2][FM], bfr[2][FN];
     load_frags(s, 0, af[0], bfr[0]);
 #pragma unroll
     for (int kk = 0; kk < BK / 16; kk++) {
@@ -353,42 +306,36 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
 #pragma unroll
       for (int i = 0; i < FM; i++)
 #pragma unroll
-        for (int j = 0; j < FN_IN; j++)
-          acc[i][j0 + j] = LT_MFMA_32X32X16(af[kk & 1][i], bfr[kk & 1][j], acc[i][j0 + j]);
-      if (kk + 1 < BK / 16) SchedInterleave<FRAG_READS, FM * FN_IN>::run();
+        for (int j = 0; j < FN; j++)
+          acc[i][j] = LT_MFMA_32X32X16(af[kk & 1][i], bfr[kk & 1][j], acc[i][j]);
+      if (kk + 1 < BK / 16) SchedInterleave<FRAG_READS, FM * FN>::run();
     }
   };
-  LT_TILE_STAMP(1);
   if constexpr (PF == 1) {
-    lt_static_for<PH>([&](auto PHASE) __attribute__((always_inline)) {
-      constexpr int ph = decltype(PHASE)::value;
-      using Whole = std::false_type;
-      using Tail = std::true_type;
-      if (kt_begin < kt_end) {
-        load_tiles(Tail{}, kt_begin, ph, ra_set[0], rb_set[0]);
-        store_tiles(Tail{}, kt_begin & 1, k_rows(kt_begin), ra_set[0], rb_set[0]);
-      }
+    using Whole = std::false_type;
+    using Tail = std::true_type;
+    if (kt_begin < kt_end) {
+      load_tiles(Tail{}, kt_begin, ra_set[0], rb_set[0]);
+      store_tiles(Tail{}, kt_begin & 1, k_rows(kt_begin), ra_set[0], rb_set[0]);
+    }
+    __syncthreads();
+    // steps whose next step has whole k-major tiles, then the rest
+    const int kt_whole = SP == SPARSE_DW ? kt_end
+                                         : min(kt_end, lt_leading_whole_steps(p.K[0], kt_total > kt_seg0 ? p.K[1] : 0, BK));
+    int kt = kt_begin;
+    for (; kt + 1 < kt_whole; kt++) {
+      load_tiles(Whole{}, kt + 1, ra_set[0], rb_set[0]);
+      multiply_stage(kt & 1);
+      store_tiles(Whole{}, (kt & 1) ^ 1, k_rows(kt + 1), ra_set[0], rb_set[0]);
       __syncthreads();
-      // steps whose next step has whole k-major tiles, then the rest: with the test for a ragged end in every step the
-      // input-gradient walk of a PixelFly layer (hidden 4096) takes 244 us instead of 206
-      const int kt_whole = SP == SPARSE_DW ? kt_end
-                                           : min(kt_end, lt_leading_whole_steps(SP == SPARSE_NONE ? p.K[0] : (int64_t)kt_seg0 * BK,
-                                                                                kt_total > kt_seg0 ? p.K[1] : 0, BK));
-      int kt = kt_begin;
-      for (; kt + 1 < kt_whole; kt++) {
-        load_tiles(Whole{}, kt + 1, ph, ra_set[0], rb_set[0]);
-        multiply_stage(kt & 1, PHASE);
-        store_tiles(Whole{}, (kt & 1) ^ 1, k_rows(kt + 1), ra_set[0], rb_set[0]);
-        __syncthreads();
-      }
-      for (; kt < kt_end; kt++) {
-        const bool has_next = kt + 1 < kt_end;
-        if (has_next) load_tiles(Tail{}, kt + 1, ph, ra_set[0], rb_set[0]);
-        multiply_stage(kt & 1, PHASE);
-        if (has_next) store_tiles(Tail{}, (kt & 1) ^ 1, k_rows(kt + 1), ra_set[0], rb_set[0]);
-        __syncthreads();
-      }
-    });
+    }
+    for (; kt < kt_end; kt++) {
+      const bool has_next = kt + 1 < kt_end;
+      if (has_next) load_tiles(Tail{}, kt + 1, ra_set[0], rb_set[0]);
+      multiply_stage(kt & 1);
+      if (has_next) store_tiles(Tail{}, (kt & 1) ^ 1, k_rows(kt + 1), ra_set[0], rb_set[0]);
+      __syncthreads();
+    }
   } else {
     // Register set d holds step i with i % PF == d from its request until it is written to LDS stage i & 1 at the end of
     // step i - 1; the set is then free for step i + PF, requested at the start of step i.
@@ -408,7 +355,7 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
       auto rows_of = [&](int i) { return i < steps ? k_rows(kt_of(i)) : 0; };
       lt_static_for<PF>([&](auto D) __attribute__((always_inline)) {
         constexpr int d = decltype(D)::value;
-        load_tiles(std::true_type{}, kt_of(d), 0, ra_set[d], rb_set[d]);
+        load_tiles(std::true_type{}, kt_of(d), ra_set[d], rb_set[d]);
       });
       store_tiles(std::true_type{}, 0, rows_of(0), ra_set[0], rb_set[0]);
       __syncthreads();
@@ -417,15 +364,14 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
           constexpr int d = decltype(D)::value;
           const int i = i0 + d;
           const int s = i & 1;
-          load_tiles(std::true_type{}, kt_of(i + PF), 0, ra_set[d], rb_set[d]);
-          multiply_stage(s, std::integral_constant<int, 0>{});
+          load_tiles(std::true_type{}, kt_of(i + PF), ra_set[d], rb_set[d]);
+          multiply_stage(s);
           store_tiles(std::true_type{}, s ^ 1, rows_of(i + 1), ra_set[(d + 1) % PF], rb_set[(d + 1) % PF]);
           __syncthreads();
         });
       }
     }
   }
-  LT_TILE_STAMP(2);
 
   // ---- epilogue.  The accumulators of a 32 x 32 block sit column-per-lane (register r = row 8 * (r / 4) + 4 * (lane / 32)
   //      + r % 4, column lane % 32); each wavefront transposes one 32-row strip of its sub-tile at a time through its own
@@ -529,107 +475,14 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
     }
     __builtin_amdgcn_wave_barrier();
   };
-  float colsum[16];  // EPI_ACT_BWD: column sums of this lane's 8 (+ 8) dpre columns over the rows it writes
-#pragma unroll
-  for (int e = 0; e < 16; e++) colsum[e] = 0.f;
-  auto act_bwd_strip = [&](auto I, auto G) __attribute__((always_inline)) {
-    constexpr int i = decltype(I)::value;
-    constexpr bool GATED = decltype(G)::value;
-    EpiLoad rows[NIT];
-#pragma unroll
-    for (int it = 0; it < NIT; it++) rows[it] = epi_load_pre8<GATED>(epi, lane_row(i) + it * ROWS_PER_IT, lane_n);
-    stage_strip(I);
-#pragma unroll
-    for (int it = 0; it < NIT; it++) {
-      float v[8];
-      read_staged(it, v);
-      epi_act_bwd8_fixed<GATED, LT_ACT_GELU_FUSED>(epi, lane_row(i) + it * ROWS_PER_IT, lane_n, v, rows[it], colsum);
-    }
-    __builtin_amdgcn_wave_barrier();
-  };
-  auto out_strip = [&](auto I) __attribute__((always_inline)) {
-    constexpr int i = decltype(I)::value;
-    EpiLoad rows[NIT];
-#pragma unroll
-    for (int it = 0; it < NIT; it++) rows[it] = epi_load_x8<TX>(epi, lane_row(i) + it * ROWS_PER_IT, lane_n);
-    stage_strip(I);
-#pragma unroll
-    for (int it = 0; it < NIT; it++) {
-      float v[8];
-      read_staged(it, v);
-      epi_out8_residual<TX>(epi, lane_row(i) + it * ROWS_PER_IT, lane_n, v, rows[it]);
-    }
-    __builtin_amdgcn_wave_barrier();
-  };
-  // forward activation, tanh GELU, h stored: the gate (or only) half and the linear half of a strip are read back from the
-  // stage with all LDS loads issued before the first value is used
-  auto act_fwd_strip = [&](auto I, auto G) __attribute__((always_inline)) {
-    constexpr int i = decltype(I)::value;
-    constexpr bool GATED = decltype(G)::value;
-    constexpr int LPR = (GATED ? WTN / 2 : WTN) / 8, RPI = 64 / LPR, NITF = 32 / RPI;
-    const int c = (lane % LPR) * 8;
-    const int64_t n = n0 + wn * (GATED ? WTN / 2 : WTN) + c;
-    const int64_t mlane = m_base + wm * WTM + i * 32 + lane / LPR;
-    stage_strip(I);
-    float vg[NITF][8], vl[GATED ? NITF : 1][8];
-#pragma unroll
-    for (int it = 0; it < NITF; it++) {
-      const float* sv = &stage[(it * RPI + lane / LPR) * STAGE_LD + c];
-#pragma unroll
-      for (int e = 0; e < 8; e++) vg[it][e] = sv[e];
-      if constexpr (GATED) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) vl[it][e] = sv[WTN / 2 + e];
-      }
-    }
-#pragma unroll
-    for (int it = 0; it < NITF; it++) epi_act_fwd8_fixed<GATED, LT_ACT_GELU_FUSED>(epi, mlane + it * RPI, n, vg[it], vl[GATED ? it : 0]);
-    __builtin_amdgcn_wave_barrier();
-  };
   const bool whole_tile = m_base + BM <= m_limit;
-  if constexpr (KIND == EPI_ACT_FWD && SP != SPARSE_NONE) {
-    const bool straight = whole_tile && epi.act == LT_ACT_GELU_FUSED && epi.hid != nullptr && epi.pre != nullptr;
-    if (straight && pair) lt_static_for<FM>([&](auto I) __attribute__((always_inline)) { act_fwd_strip(I, std::true_type{}); });
-    else if (straight) lt_static_for<FM>([&](auto I) __attribute__((always_inline)) { act_fwd_strip(I, std::false_type{}); });
-    else lt_static_for<FM>(generic_strip);
-  } else if constexpr (NIT <= 4 && KIND == EPI_STORE) {
+  if constexpr (NIT <= 4 && KIND == EPI_STORE) {
     if (whole_tile && epi.out_dtype == LT_F32) lt_static_for<FM>([&](auto I) __attribute__((always_inline)) { store_strip(I, float{}); });
     else if (whole_tile) lt_static_for<FM>([&](auto I) __attribute__((always_inline)) { store_strip(I, bf16{}); });
-    else lt_static_for<FM>(generic_strip);
-  } else if constexpr (NIT <= 4 && KIND == EPI_ACT_BWD) {
-    const bool straight = whole_tile && epi.act == LT_ACT_GELU_FUSED && epi.hid != nullptr;
-    if (straight && epi.gated) lt_static_for<FM>([&](auto I) __attribute__((always_inline)) { act_bwd_strip(I, std::true_type{}); });
-    else if (straight) lt_static_for<FM>([&](auto I) __attribute__((always_inline)) { act_bwd_strip(I, std::false_type{}); });
-    else lt_static_for<FM>(generic_strip);
-    if (straight && epi.colsum) {
-      // lanes with equal lane % LANES_PER_ROW hold the same columns for different rows of the wavefront's WTM-row sub-tile:
-      // one partial row per wavefront sub-tile
-      static_assert(WTM == 64 || KIND != EPI_ACT_BWD || NIT > 4, "the caller reduces one partial row per 64 output rows");
-#pragma unroll
-      for (int e = 0; e < 16; e++) {
-#pragma unroll
-        for (int d = LANES_PER_ROW; d < 64; d <<= 1) colsum[e] += __shfl_xor(colsum[e], d);
-      }
-      if (lane < LANES_PER_ROW) {
-        float* dst = epi.colsum + ((m_base + wm * WTM) / 64) * epi.ld_pre + lane_n;
-        float lo[8], hi[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-          lo[e] = colsum[e];
-          hi[e] = colsum[8 + e];
-        }
-        store8(dst, lo);
-        if (epi.gated) store8(dst + epi.inter, hi);
-      }
-    }
-  } else if constexpr (NIT <= 4 && KIND == EPI_OUT) {
-    if (whole_tile && epi.x && epi.drop.p == 0.f) lt_static_for<FM>(out_strip);
     else lt_static_for<FM>(generic_strip);
   } else {
     lt_static_for<FM>(generic_strip);
   }
-  LT_TILE_STAMP(3);
-  LT_TILE_STAMP_REALTIME(5);
 }
 
 // =====================================================================================================================
@@ -1751,48 +1604,21 @@ int launch_cfg(const GemmProblem& p, int io_dtype, hipStream_t stream) {
   return LT_OK;
 }
 
-template <int KIND> int launch_sparse(const GemmProblem& problem, int io_dtype, hipStream_t stream) {
-  GemmProblem p = problem;
-#ifdef LT_TILE_TIMING
-  // block-sparse FWD / DX launch number i of the process writes region i % 4 (8192 workgroups each) of its own buffer
-  if (const char* e = getenv("LT_TILE_TIMING_BUFFER_SPARSE")) {
-    if (p.sp.mode == SPARSE_FWD || p.sp.mode == SPARSE_DX)
-      p.tile_stamps = (unsigned long long*)(strtoull(e, nullptr, 0) + (size_t)(lt_tile_timing_launch_counter()++ % 4) * 8192 * 64);
-  }
-#endif
+// block-sparse problems that run on the kernels of this file: forward products over gathered k-blocks (lt_sparse_forward_grouped) and
+// weight gradients
+template <int KIND> int launch_sparse(const GemmProblem& p, hipStream_t stream) {
   const SparseWalk& sp = p.sp;
-  const bool bf16_io = KIND == EPI_OUT && io_dtype == LT_BF16;
   dim3 block(256);
-  if (sp.mode == SPARSE_FWD || sp.mode == SPARSE_DX) {
-    const int tiles_m = (int)((p.M + 255) / 256), groups = (int)(p.N / 64);
-    dim3 grid((unsigned)(tiles_m * groups));
-    using TXB = std::conditional_t<KIND == EPI_OUT, bf16, float>;  // only EPI_OUT touches x / y
-    if constexpr (KIND == EPI_STORE || KIND == EPI_ACT_FWD) {
-      if (lt_sparse_forward_grouped(p, KIND)) {
-        // runs of 4 output blocks share one list: a dense product over gathered k-blocks on 256 x 256 tiles
-        GemmProblem q = p;
-        q.K[0] = (int64_t)sp.blocks_per_out * 64;
-        q.ksplit = 0; q.krot = 0;
-        const int tiles_n = (int)(p.N / 256);
-        with_activation<KIND>(q, [&](auto ACT) {
-          hipLaunchKernelGGL((gemm_bf16_dma_kernel<true, true, KIND, float, 2, decltype(ACT)::value>),
-                             dim3(dma_grid(q, tiles_m * tiles_n)), block, 0, stream, q, tiles_m, tiles_n);
-        });
-        LT_LAUNCH_CHECK();
-        return LT_OK;
-      }
-    }
-    if (sp.mode == SPARSE_FWD && KIND == EPI_ACT_FWD && p.epi.gated) {
-      // p.N counts the gate columns: one workgroup per (token tile, gate block), paired with linear block tn + groups
-      if constexpr (KIND == EPI_ACT_FWD)
-        hipLaunchKernelGGL((gemm_bf16_kernel<256, 64, 4, 1, true, true, EPI_ACT_FWD, float, SPARSE_FWD, 2>), grid, block, 0, stream, p, tiles_m, groups);
-    } else if (sp.mode == SPARSE_FWD) {
-      if (bf16_io) hipLaunchKernelGGL((gemm_bf16_kernel<256, 64, 4, 1, true, true, KIND, TXB, SPARSE_FWD>), grid, block, 0, stream, p, tiles_m, groups);
-      else hipLaunchKernelGGL((gemm_bf16_kernel<256, 64, 4, 1, true, true, KIND, float, SPARSE_FWD>), grid, block, 0, stream, p, tiles_m, groups);
-    } else {
-      if (bf16_io) hipLaunchKernelGGL((gemm_bf16_kernel<256, 64, 4, 1, true, false, KIND, TXB, SPARSE_DX>), grid, block, 0, stream, p, tiles_m, groups);
-      else hipLaunchKernelGGL((gemm_bf16_kernel<256, 64, 4, 1, true, false, KIND, float, SPARSE_DX>), grid, block, 0, stream, p, tiles_m, groups);
-    }
+  if (sp.mode == SPARSE_FWD) {
+    // runs of 4 output blocks share one list: a dense product over gathered k-blocks on 256 x 256 tiles
+    GemmProblem q = p;
+    q.K[0] = (int64_t)sp.blocks_per_out * 64;
+    q.ksplit = 0; q.krot = 0;
+    const int tiles_m = (int)((p.M + 255) / 256), tiles_n = (int)(p.N / 256);
+    with_activation<KIND>(q, [&](auto ACT) {
+      hipLaunchKernelGGL((gemm_bf16_dma_kernel<true, true, KIND, float, 2, decltype(ACT)::value>),
+                         dim3(dma_grid(q, tiles_m * tiles_n)), block, 0, stream, q, tiles_m, tiles_n);
+    });
   } else {
     if constexpr (KIND == EPI_STORE) {
       const int64_t out_features = sp.ld_act;

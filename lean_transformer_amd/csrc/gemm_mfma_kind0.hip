@@ -5,8 +5,8 @@ int lt_mfma_launch_dense_kind0(const GemmProblem& p, int io_dtype, hipStream_t s
   return launch_layout<EPI_STORE>(p, io_dtype, stream);
 }
 
-int lt_mfma_launch_sparse_kind0(const GemmProblem& p, int io_dtype, hipStream_t stream) {
-  return launch_sparse<EPI_STORE>(p, io_dtype, stream);
+int lt_mfma_launch_sparse_kind0(const GemmProblem& p, hipStream_t stream) {
+  return launch_sparse<EPI_STORE>(p, stream);
 }
 
 namespace {
@@ -14,7 +14,7 @@ template <bool A_KM, bool B_KM> int launch_skinny(const GemmProblem& p, int slic
   const int tiles_m = (int)((p.M + 127) / 128), tiles_n = (int)(p.N / 128);
   dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)slices), block(256);
   // these products stream one large operand once against a small one: operand tiles are requested two k-steps ahead
-  hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, 2, 2, A_KM, B_KM, EPI_STORE, float, SPARSE_NONE, 1, 2>), grid, block, 0, stream, p, tiles_m, tiles_n);
+  hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, 2, 2, A_KM, B_KM, EPI_STORE, float, SPARSE_NONE, 2>), grid, block, 0, stream, p, tiles_m, tiles_n);
   LT_LAUNCH_CHECK();
   return LT_OK;
 }

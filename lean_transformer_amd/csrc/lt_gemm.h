@@ -431,6 +431,8 @@ int lt_launch_gemm_stream(const GemmProblem& p, int kind, int dtype, int io_dtyp
 // 128 x 128 tiles for products too small to fill the chip with 256 x 256 ones (gemm_mid.hip)
 bool lt_gemm_mid_supported(const GemmProblem& p, int kind);
 int lt_launch_gemm_mid(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream);
+// block-sparse forward product or input gradient that lt_sparse_mfma_supported takes (gemm_walk.hip)
+int lt_launch_gemm_walk(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream);
 // algorithmic flops of a dense problem: 2 * M * N * (K0 + K1)
 double lt_gemm_flops(const GemmProblem& p, int kind);
 // block-sparse walk: matrix-core kernel for 64 x 64 bf16 blocks, else the any-shape kernel
@@ -461,7 +463,7 @@ size_t lt_gemm_mid_splitk_workspace(int64_t M, int64_t N, int64_t K);
 // same for the any-shape kernel (fp32 path, shapes the tiled kernels do not take)
 size_t lt_gemm_generic_splitk_workspace(int64_t M, int64_t N, int64_t K);
 // rows per partial row of EpiParams::colsum when lt_launch_gemm / lt_launch_gemm_sparse sends this EPI_ACT_BWD problem to a
-// kernel that fills it (128: copy-based dense kernel; 64: block-sparse walk on whole tiles with the tanh GELU); 0: it will not
+// kernel that fills it (128: copy-based dense kernel; 64: 128 x 128 tiles, block-sparse walk); 0: it will not
 int lt_gemm_colsum_rows(const GemmProblem& p, int dtype, int io_dtype);
 // Column sums of partial rows that may wait: a caller that runs several passes with such a tail (the FFN backward: two bias
 // gradients and the LayerNorm parameter gradients) hands the same queue to each of them and flushes it once, one launch
