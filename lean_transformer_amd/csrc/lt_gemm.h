@@ -242,6 +242,24 @@ __device__ __forceinline__ void unpack_bf16x8(const lt_u32x4& raw, float (&v)[8]
   for (int i = 0; i < 8; i++) v[i] = (float)t.h[i];
 }
 
+// 8 values rounded to 16 bits and packed as they are stored; unpacking gives the rounded values back.  (The compiler does not see
+// through the packed words: it would round a second time, one by one, instead of unpacking, two instructions a value for one.)
+__device__ __forceinline__ lt_u32x4 round8(const float (&v)[8]) {
+  union { unsigned int w[4]; lt_u32x4 u; bf16 h[8]; } t;
+#pragma unroll
+  for (int i = 0; i < 8; i++) t.h[i] = (bf16)v[i];
+#pragma unroll
+  for (int i = 0; i < 4; i++) asm("" : "+v"(t.w[i]));
+  return t.u;
+}
+__device__ __forceinline__ void store8(bf16* p, const lt_u32x4& packed) { *reinterpret_cast<lt_u32x4*>(p) = packed; }
+__device__ __forceinline__ void add_rounded8(const lt_u32x4& packed, float* cs) {
+  float r[8];
+  unpack_bf16x8(packed, r);
+#pragma unroll
+  for (int i = 0; i < 8; i++) cs[i] += r[i];
+}
+
 // cs: running column sums of the 8 gate-side (and, gated, 8 linear-side at cs + 8) dpre values this lane has written
 template <int ACT = -1>
 __device__ __forceinline__ void epi_act_bwd8_loaded(const EpiParams& e, int64_t m, int64_t n, const float (&dh)[8],
@@ -257,22 +275,22 @@ __device__ __forceinline__ void epi_act_bwd8_loaded(const EpiParams& e, int64_t 
     unpack_bf16x8(l.b, pl);
 #pragma unroll
     for (int i = 0; i < 8; i++) o[i] = dh[i] * pl[i] * da[i];
-    store8(dpre, o);
-#pragma unroll
-    for (int i = 0; i < 8; i++) cs[i] += (float)(bf16)o[i];
+    lt_u32x4 packed = round8(o);
+    store8(dpre, packed);
+    add_rounded8(packed, cs);
 #pragma unroll
     for (int i = 0; i < 8; i++) o[i] = dh[i] * a[i];
-    store8(dpre + e.inter, o);
-#pragma unroll
-    for (int i = 0; i < 8; i++) cs[8 + i] += (float)(bf16)o[i];
+    packed = round8(o);
+    store8(dpre + e.inter, packed);
+    add_rounded8(packed, cs + 8);
 #pragma unroll
     for (int i = 0; i < 8; i++) a[i] *= pl[i];
   } else {
 #pragma unroll
     for (int i = 0; i < 8; i++) o[i] = dh[i] * da[i];
-    store8(dpre, o);
-#pragma unroll
-    for (int i = 0; i < 8; i++) cs[i] += (float)(bf16)o[i];
+    const lt_u32x4 packed = round8(o);
+    store8(dpre, packed);
+    add_rounded8(packed, cs);
   }
   if (e.hid) store8(reinterpret_cast<bf16*>(e.hid) + m * e.ld_hid + n, a);
 }
@@ -284,18 +302,19 @@ __device__ __forceinline__ void epi_act_bwd8_loaded(const EpiParams& e, int64_t 
 template <bool GATED, int ACT>
 __device__ __forceinline__ void epi_act_fwd8_fixed(const EpiParams& e, int64_t m, int64_t n, float (&vg)[8], float (&vl)[8]) {
   float h[8];
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    vg[i] = to_f32((bf16)vg[i]);  // the activation sees the stored (rounded) pre-activation, as backward will
-    h[i] = act_value<false>(ACT, vg[i]);
-    if constexpr (GATED) {
-      vl[i] = to_f32((bf16)vl[i]);
-      h[i] *= vl[i];
-    }
-  }
   bf16* pre = reinterpret_cast<bf16*>(e.pre) + m * e.ld_pre + n;
-  store8(pre, vg);
-  if constexpr (GATED) store8(pre + e.inter, vl);
+  lt_u32x4 packed = round8(vg);  // the activation sees the stored (rounded) pre-activation, as backward will
+  store8(pre, packed);
+  unpack_bf16x8(packed, vg);
+#pragma unroll
+  for (int i = 0; i < 8; i++) h[i] = act_value<false>(ACT, vg[i]);
+  if constexpr (GATED) {
+    packed = round8(vl);
+    store8(pre + e.inter, packed);
+    unpack_bf16x8(packed, vl);
+#pragma unroll
+    for (int i = 0; i < 8; i++) h[i] *= vl[i];
+  }
   store8(reinterpret_cast<bf16*>(e.hid) + m * e.ld_hid + n, h);
 }
 
@@ -366,22 +385,22 @@ __device__ __forceinline__ void epi_act_bwd8_fixed(const EpiParams& e, int64_t m
     unpack_bf16x8(l.b, pl);
 #pragma unroll
     for (int i = 0; i < 8; i++) o[i] = dh[i] * pl[i] * da[i];
-    store8(dpre, o);
-#pragma unroll
-    for (int i = 0; i < 8; i++) cs[i] += (float)(bf16)o[i];
+    lt_u32x4 packed = round8(o);
+    store8(dpre, packed);
+    add_rounded8(packed, cs);
 #pragma unroll
     for (int i = 0; i < 8; i++) o[i] = dh[i] * a[i];
-    store8(dpre + e.inter, o);
-#pragma unroll
-    for (int i = 0; i < 8; i++) cs[8 + i] += (float)(bf16)o[i];
+    packed = round8(o);
+    store8(dpre + e.inter, packed);
+    add_rounded8(packed, cs + 8);
 #pragma unroll
     for (int i = 0; i < 8; i++) a[i] *= pl[i];
   } else {
 #pragma unroll
     for (int i = 0; i < 8; i++) o[i] = dh[i] * da[i];
-    store8(dpre, o);
-#pragma unroll
-    for (int i = 0; i < 8; i++) cs[i] += (float)(bf16)o[i];
+    const lt_u32x4 packed = round8(o);
+    store8(dpre, packed);
+    add_rounded8(packed, cs);
   }
   store8(reinterpret_cast<bf16*>(e.hid) + m * e.ld_hid + n, a);
 }
