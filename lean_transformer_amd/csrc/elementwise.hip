@@ -346,6 +346,130 @@ __global__ __launch_bounds__(256) void ln_bwd_param_kernel(int64_t T, int H, con
   }
 }
 
+// Both halves in one pass for rows of up to 4096 elements: WPR wavefronts share a row (16 elements a lane), 16 / WPR rows are in a
+// workgroup at a time and up to 256 workgroups walk the rows, the next row's dy and x in flight while this one's sums go
+// through LDS; the column sums stay in registers and leave once, one partial row per workgroup.  Bound by memory: dy and x are
+// read once instead of twice.  Measured with fp32 x and residual, the two kernels against this: [4096, 4096] 72 us, 52; [16384, 768]
+// 48, 34.  Wider rows would need twice the partial rows or leave CUs idle, an fp32 dy more than the 128 registers of a wavefront:
+// both stay with the two kernels.
+template <typename TX, typename TDX, int WPR>
+__global__ __launch_bounds__(1024) void ln_bwd_rows_kernel(int64_t T, int H, const TX* __restrict__ x,
+                                                            const float* __restrict__ stats, const float* __restrict__ w,
+                                                            const bf16* __restrict__ dy, const TDX* __restrict__ residual_grad,
+                                                            TDX* __restrict__ dx, float* __restrict__ partial) {
+  constexpr int GROUPS = 16 / WPR;
+  typedef TX X4 __attribute__((ext_vector_type(4)));
+  typedef bf16 DY4 __attribute__((ext_vector_type(4)));
+  typedef TDX DX4 __attribute__((ext_vector_type(4)));
+  __shared__ __attribute__((aligned(16))) float w_lds[WPR * 1024];
+  __shared__ __attribute__((aligned(16))) float red[16][1024];
+  __shared__ float2 row_sums[2][16];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int group = wave / WPR, col0 = (wave % WPR) * 1024 + lane * 4;  // this lane's columns: col0 + 256 i .. + 3
+  for (int c = threadIdx.x; c < H; c += 1024) w_lds[c] = w[c];
+  __syncthreads();
+
+  X4 x_next[4];
+  DY4 dy_next[4];
+  auto request = [&](int64_t row) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int c = col0 + i * 256;
+      if (row < T && c < H) {
+        x_next[i] = *reinterpret_cast<const X4*>(x + row * H + c);
+        dy_next[i] = *reinterpret_cast<const DY4*>(dy + row * H + c);
+      }
+    }
+  };
+  float pw[4][4], pb[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) pw[i][e] = pb[i][e] = 0.f;
+  const float inv_h = 1.0f / (float)H;
+  const int64_t step = (int64_t)gridDim.x * GROUPS;
+  int buf = 0;
+  request((int64_t)blockIdx.x * GROUPS + group);
+  for (int64_t base = (int64_t)blockIdx.x * GROUPS; base < T; base += step, buf ^= 1) {  // (the same for the whole workgroup)
+    const int64_t row = base + group;
+    const bool live = row < T;
+    const float mean = live ? stats[row * 2] : 0.f, rstd = live ? stats[row * 2 + 1] : 0.f;
+    float xh[4][4];
+    DY4 g4[4];
+    DX4 res[4];
+    float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int c = col0 + i * 256;
+      if (live && c < H) {
+        if (residual_grad) res[i] = *reinterpret_cast<const DX4*>(residual_grad + row * H + c);
+        float wv[4];
+        load4(&w_lds[c], wv);
+        g4[i] = dy_next[i];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float g = (float)g4[i][e], dxh = g * wv[e];
+          xh[i][e] = ((float)x_next[i][e] - mean) * rstd;
+          s1 += dxh;
+          s2 += dxh * xh[i][e];
+          pw[i][e] += g * xh[i][e];
+          pb[i][e] += g;
+        }
+      }
+    }
+    request(row + step);
+    s1 = wave_sum(s1);
+    s2 = wave_sum(s2);
+    if constexpr (WPR > 1) {
+      if (lane == 0) row_sums[buf][wave] = make_float2(s1, s2);
+      // (not __syncthreads, which would wait for the loads in flight; two buffers: a wavefront writes one again only behind the
+      // barrier that all reads of it precede)
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      s1 = s2 = 0.f;
+#pragma unroll
+      for (int k = 0; k < WPR; k++) {
+        const float2 v = row_sums[buf][group * WPR + k];
+        s1 += v.x;
+        s2 += v.y;
+      }
+    }
+    const float c1 = s1 * inv_h, c2 = s2 * inv_h;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int c = col0 + i * 256;
+      if (live && c < H) {
+        float o[4], wv[4];
+        load4(&w_lds[c], wv);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          o[e] = rstd * ((float)g4[i][e] * wv[e] - c1 - xh[i][e] * c2);
+          if (residual_grad) o[e] += (float)res[i][e];
+        }
+        store4(dx + row * H + c, o);
+      }
+    }
+  }
+  // the groups' column sums, then one partial row per workgroup
+  auto fold = [&](const float (&sums)[4][4], float* out) __attribute__((always_inline)) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; i++) store4(&red[wave][i * 256 + lane * 4], sums[i]);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < WPR; k++) {
+      const int c = k * 1024 + (int)threadIdx.x;
+      if (c < H) {
+        float s = 0.f;
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++) s += red[g * WPR + k][threadIdx.x];
+        out[c] = s;
+      }
+    }
+  };
+  fold(pw, partial + (int64_t)blockIdx.x * 2 * H);
+  fold(pb, partial + ((int64_t)blockIdx.x * 2 + 1) * H);
+}
+
 // out[c] = sum_r partial[r * stride + c], one thread per column (rows are few)
 __global__ void colreduce_kernel(int rows, int64_t stride, int cols, const float* __restrict__ partial,
                                  float* __restrict__ out) {
@@ -713,7 +837,16 @@ static int ln_bwd_slices(int64_t T) {
   return (int)(s < 1 ? 1 : (s > 128 ? 128 : s));
 }
 
-// partial (dweight, dbias) rows: one pair per workgroup of the any-shape kernel or per row slice of the vectorised one
+// ln_bwd_rows_kernel: wavefronts per row, and workgroups (one per CU where there are rows enough: a pair of partial rows each, at
+// most 8 MiB, what the static scratch below holds)
+constexpr int LN_ROWS_MAX_H = 4096;
+static int ln_rows_wavefronts(int H) { return H <= 1024 ? 1 : H <= 2048 ? 2 : 4; }
+static int ln_bwd_rows_blocks(int64_t T, int H) {
+  const int64_t groups = 16 / ln_rows_wavefronts(H);
+  return (int)std::min<int64_t>(256, (T + groups - 1) / groups);
+}
+
+// partial (dweight, dbias) rows: one pair per workgroup of the one-pass and any-shape kernels or per row slice of the vectorised one
 size_t lt_ln_backward_workspace(int64_t T, int H) {
   const int rows = ln_bwd_blocks(T) > ln_bwd_slices(T) ? ln_bwd_blocks(T) : ln_bwd_slices(T);
   return (size_t)rows * 2 * (size_t)H * sizeof(float);
@@ -734,14 +867,39 @@ int lt_ln_backward(int64_t T, int H, int x_dtype, const void* x, const float* st
                    (!dx || lt_aligned(dx, 16)) && (!residual_grad || lt_aligned(residual_grad, 16)) &&
                    (!partial || lt_aligned(partial, 16));
   const bool wide = H > 256 * LNB_MAXC;  // wider than the register-resident kernels take
-  // partial (dweight, dbias) rows of the path taken: one pair per row slice (vectorised, wide) or per workgroup (any-shape)
-  int partial_rows = (vec || wide) ? ln_bwd_slices(T) : ln_bwd_blocks(T);
+  // both gradients of rows of up to 4096 elements, 16-bit dy: one pass over the inputs (ln_bwd_rows_kernel)
+  // (two kernels also where the caller's scratch holds only their fewer partial rows)
+  const bool one_pass = vec && dx && dweight && dy_dtype == LT_BF16 && H <= LN_ROWS_MAX_H &&
+                        workspace_bytes >= (size_t)ln_bwd_rows_blocks(T, H) * 2 * (size_t)H * sizeof(float);
+  // partial (dweight, dbias) rows of the path taken: one pair per row slice (vectorised, wide) or per workgroup (one pass, any-shape)
+  int partial_rows = one_pass ? ln_bwd_rows_blocks(T, H) : (vec || wide) ? ln_bwd_slices(T) : ln_bwd_blocks(T);
   if (dweight) {
     const size_t need = (size_t)partial_rows * 2 * (size_t)H * sizeof(float);
     LT_REQUIRE(workspace && workspace_bytes >= need, LT_ERR_WORKSPACE,
                "layernorm backward: %zu bytes of scratch needed for the parameter gradients, %zu given", need, workspace_bytes);
   }
-  if (vec) {
+  if (one_pass) {
+    dim3 grid((unsigned)partial_rows), block(1024);
+    const int wpr = ln_rows_wavefronts(H);
+#define LT_LNB_ROWS_W(TX, TDX, WPR)                                                                                             \
+  hipLaunchKernelGGL((ln_bwd_rows_kernel<TX, TDX, WPR>), grid, block, 0, stream, T, H, (const TX*)x, stats, w, (const bf16*)dy, \
+                     (const TDX*)residual_grad, (TDX*)dx, partial)
+#define LT_LNB_ROWS(TX, TDX)                      \
+  do {                                            \
+    if (wpr == 1) LT_LNB_ROWS_W(TX, TDX, 1);      \
+    else if (wpr == 2) LT_LNB_ROWS_W(TX, TDX, 2); \
+    else LT_LNB_ROWS_W(TX, TDX, 4);               \
+  } while (0)
+    switch (key) {  // (dy in 16 bits)
+      case 2: LT_LNB_ROWS(float, float); break;
+      case 3: LT_LNB_ROWS(float, bf16); break;
+      case 6: LT_LNB_ROWS(bf16, float); break;
+      default: LT_LNB_ROWS(bf16, bf16); break;
+    }
+#undef LT_LNB_ROWS
+#undef LT_LNB_ROWS_W
+    LT_LAUNCH_CHECK();
+  } else if (vec) {
     if (dx) {
       dim3 grid(blocks_for(T, 4)), block(256);
       const int maxv = ln_vectors_per_lane(H);
