@@ -207,11 +207,14 @@ int linear_forward_impl(const lt_linear& lin, int64_t T, int dtype, const void* 
   if (gated && !two_passes) {
     // Gate and linear output blocks have index lists of their own; the bf16 walk for 64 x 64 blocks pairs them inside one
     // workgroup.  Where the layout lets the product run on 256 x 256 tiles instead (runs of output blocks with a shared
-    // list), that and a separate activation pass are faster than the paired walk.
+    // list), that and a separate activation pass are faster than the paired walk for a large product: its 256 x 64 tiles read the
+    // operands more often, which costs more than the second pass once they no longer stay in the caches.  Stretched butterfly, the
+    // two passes and the walk, us: hidden 1024, T 4096 (pre-activation 64 MiB) 72 and 63; 2048, 4096 (128 MiB) 145 and 131; 4096,
+    // 2000 (125 MiB) 146 and 143; 4096, 4096 (256 MiB) 329 and 341.
     GemmProblem s = p;
     s.N = out;
     s.epi = epi_store_params(epi.pre, epi.ld_pre, dtype, epi.bias);
-    two_passes = lt_sparse_forward_grouped(s, EPI_STORE);
+    two_passes = T * out * 2 > ((int64_t)160 << 20) && lt_sparse_forward_grouped(s, EPI_STORE);
   }
   if (two_passes) {  // store the pre-activation, then the activation as a pass of its own
     p.N = out;

@@ -97,3 +97,25 @@ def test_forward_and_input_gradient(dtype, in_blocks, out_blocks, per_in, rank, 
         unit, tiny = UNIT[dtype], 2.0**-24 if dtype == torch.float16 else 0.0
         worst = (got.double() - ref).abs() - ((k + 16) * 2.0**-23 * magnitude + slack) * (1 + unit) - unit * ref.abs() - tiny
         assert worst.max().item() <= 0.0, worst.max().item()
+
+
+@pytest.mark.parametrize("tokens", [10240, 10248])
+def test_gated_up_projection_on_either_side_of_the_rule(tokens):
+    """a stretched butterfly of hidden 1024: up to 160 MiB of pre-activation the paired walk, above that 256 x 256 tiles and an activation
+    pass.  The normalised input, the pre-activation, the hidden activation and the weights' products of it are each off by at
+    most a unit (2^-8) relative to their own 2-norm."""
+    import oracle.ffn as offn
+    torch.manual_seed(3)
+    layout = "pixelfly(block_size=64, stretch=True)"
+    up, down = (lt.GeneralizedLinear(lt.GeneralizedMatrix(i, o, layout)) for i, o in ((1024, 8192), (4096, 1024)))
+    layer = lt.LeanFFN(1024, 4096, activation=lt.ACT2FN["gelu_fused"], gated=True, i2h_proj=up, h2o_proj=down)
+    layer = layer.to(DEV).to(torch.bfloat16).eval()
+    x = torch.randn(tokens, 1024, device=DEV)
+    with torch.no_grad():
+        y = layer(x) - x
+        rows = torch.cat([torch.arange(64), torch.arange(tokens - 64, tokens)]).to(DEV)
+        u = torch.nn.functional.layer_norm(x[rows].double(), (1024,))
+        pre = u @ dense_weight(up.weight, up.matrix.backward_indices, 8192).t()
+        hid = offn.apply_activation(pre, "gelu_fused", True)
+        ref = hid @ dense_weight(down.weight, down.matrix.backward_indices, 1024).t()
+    assert (y[rows].double() - ref).norm() <= 4 * 2.0**-8 * ref.norm()
