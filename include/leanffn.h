@@ -167,6 +167,9 @@ int lt_ffn_forward(const lt_ffn_desc* desc, const void* x, void* y, const lt_ffn
 /* gradients of the above given dy, recomputing LayerNorm output and activation from x and saved->pre_activation */
 int lt_ffn_backward(const lt_ffn_desc* desc, const void* x, const void* dy, const lt_ffn_saved* saved,
                     const lt_ffn_grads* grads, void* workspace, size_t workspace_bytes, void* stream);
+/* the same with the weight and low-rank gradients in grad_dtype: the compute dtype, or LT_F32 (then unrounded) */
+int lt_ffn_backward_to(const lt_ffn_desc* desc, const void* x, const void* dy, const lt_ffn_saved* saved,
+                       const lt_ffn_grads* grads, int32_t grad_dtype, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---- generalized linear: y = x W^T (+ bias) (+ (x L1^T) L2^T) ------------------------------------------------------- */
 size_t lt_linear_backward_workspace_bytes(const lt_linear* lin, int64_t tokens, int32_t dtype);
@@ -177,6 +180,10 @@ int lt_linear_forward(const lt_linear* lin, int64_t tokens, int32_t dtype, const
 int lt_linear_backward(const lt_linear* lin, int64_t tokens, int32_t dtype, const void* x, const void* dy,
                        const void* lowrank_hid, void* dx, const lt_linear_grads* grads, void* workspace,
                        size_t workspace_bytes, void* stream);
+/* the same with dx in dx_dtype and the weight and low-rank gradients in grad_dtype: each `dtype`, or LT_F32 (then unrounded) */
+int lt_linear_backward_to(const lt_linear* lin, int64_t tokens, int32_t dtype, const void* x, const void* dy,
+                          const void* lowrank_hid, int32_t dx_dtype, void* dx, const lt_linear_grads* grads, int32_t grad_dtype,
+                          void* workspace, size_t workspace_bytes, void* stream);
 
 /* Tests lin->out_group against lin->forward_indices on the device: writes 1 to *flag (device memory, 4 bytes) when every
  * aligned run of out_group output blocks shares one list of input blocks with adjacent weight blocks, else 0.  Asynchronous

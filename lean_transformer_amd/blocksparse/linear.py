@@ -139,6 +139,11 @@ def _as(t: Optional[torch.Tensor], dtype: torch.dtype) -> Optional[torch.Tensor]
     return t.contiguous()
 
 
+def _result_dtype(dtype: torch.dtype, *tensors: Optional[torch.Tensor]) -> torch.dtype:
+    """dtype the kernels write these tensors' gradients in: fp32 where all of them are, else the compute dtype"""
+    return torch.float32 if all(t is None or t.dtype == torch.float32 for t in tensors) else dtype
+
+
 def shared_list_run(forward_indices: torch.Tensor, blocks_per_in: int) -> int:
     """Largest power of two g such that every aligned run of g consecutive output blocks has the same list of input blocks
     (1 when neighbouring output blocks differ).  PixelFly with ``stretch=True`` on a matrix with more output than input
@@ -302,19 +307,22 @@ class _GeneralizedLinear(torch.autograd.Function):
         desc = linear_desc(w, None, l1, l2, fwd, bwd, forward_indices, backward_indices)
         tokens = x.shape[0]
         grads = nat.LtLinearGrads()
-        dx = torch.empty_like(x) if need[0] else None
-        dw = torch.empty_like(w) if need[1] else None
+        # straight in the type autograd hands on: fp32 from the accumulators where the tensors are fp32 (autocast)
+        dx_dtype, grad_dtype = _result_dtype(dtype, input), _result_dtype(dtype, main_weight, lowrank_first, lowrank_second)
+        dx = torch.empty(x.shape, dtype=dx_dtype, device=device) if need[0] else None
+        dw = torch.empty(w.shape, dtype=grad_dtype, device=device) if need[1] else None
         db = torch.empty(desc.out_features, dtype=torch.float32, device=device) if (ctx._has_bias and need[2]) else None
-        dl1 = torch.empty_like(l1) if (l1 is not None and need[3]) else None
-        dl2 = torch.empty_like(l2) if (l2 is not None and need[4]) else None
+        dl1 = torch.empty(l1.shape, dtype=grad_dtype, device=device) if (l1 is not None and need[3]) else None
+        dl2 = torch.empty(l2.shape, dtype=grad_dtype, device=device) if (l2 is not None and need[4]) else None
         grads.weight, grads.bias, grads.lowrank_first, grads.lowrank_second = (nat.ptr(dw), nat.ptr(db), nat.ptr(dl1),
                                                                                nat.ptr(dl2))
         if tokens > 0:
             lib = nat.lib(dtype)
             ws = nat.workspace(lib.lt_linear_backward_workspace_bytes(desc, tokens, nat.dtype_code(dtype)), device)
-            nat.check(lib.lt_linear_backward(desc, tokens, nat.dtype_code(dtype), nat.ptr(x), nat.ptr(dy), nat.ptr(hid),
-                                             nat.ptr(dx), grads, nat.ptr(ws), ws.numel(), nat.current_stream(device)),
-                      "lt_linear_backward", lib)
+            nat.check(lib.lt_linear_backward_to(desc, tokens, nat.dtype_code(dtype), nat.ptr(x), nat.ptr(dy), nat.ptr(hid),
+                                                nat.dtype_code(dx_dtype), nat.ptr(dx), grads, nat.dtype_code(grad_dtype),
+                                                nat.ptr(ws), ws.numel(), nat.current_stream(device)),
+                      "lt_linear_backward_to", lib)
         else:
             for g in (dw, db, dl1, dl2):
                 if g is not None:

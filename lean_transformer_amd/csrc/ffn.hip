@@ -259,12 +259,13 @@ void plan_linear_backward(const lt_linear& lin, int64_t T, int dtype, Bump& ws, 
 // gradient side of one generalized linear layer.  The input-gradient GEMM runs FIRST, through epilogue `kind_dx`
 // (EPI_ACT_BWD for the down-projection, whose epilogue also re-materialises this layer's own input `x_act`), then the
 // parameter gradients, which may therefore read x_act.  Pass kind_dx < 0 to skip the input gradient.
+// grad_dtype: type of the weight and low-rank gradients, the compute dtype or fp32 (what the accumulators hold)
 // act_colsum / act_colsum_rows: with an EPI_ACT_BWD input-gradient epilogue, room for the partial column sums of the dpre it
 // writes (one row of epi_dx.ld_pre floats per 64 tokens); *act_colsum_rows = tokens per partial row the kernel that ran
 // filled (0: it did not)
 int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void* x_act, const void* dy,
                          const void* lowrank_hid, int kind_dx, const EpiParams& epi_dx, const lt_linear_grads& grads,
-                         const LinearBwdScratch& s, int io_dtype, hipStream_t stream, float* act_colsum = nullptr,
+                         int grad_dtype, const LinearBwdScratch& s, int io_dtype, hipStream_t stream, float* act_colsum = nullptr,
                          int* act_colsum_rows = nullptr, ColReduceQueue* defer = nullptr) {
   const int64_t in = lin.in_features, out = lin.out_features, r = lin.lowrank;
   const bool need_dx = kind_dx >= 0;
@@ -312,7 +313,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
       p.M = out; p.N = in; p.K[0] = T;
       p.A[0] = operand(dy, out, false);
       p.B[0] = operand(x_act, in, false);
-      p.epi = epi_store_params(grads.weight, in, dtype, nullptr);
+      p.epi = epi_store_params(grads.weight, in, grad_dtype, nullptr);
       LT_TRY(lt_launch_gemm_skinny(p, dtype, io_dtype, s.skinny, s.skinny_bytes, stream));
     } else {
       p.M = lin.block; p.N = in; p.K[0] = T;
@@ -323,7 +324,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
       // (the grouped kernel reads the list from the forward table)
       p.sp.out_group = lin.forward_indices ? group_length(lin.out_group) : 0; p.sp.out_stride = group_stride(lin.out_group);
       p.sp.in_group = group_length(lin.in_group); p.sp.in_stride = group_stride(lin.in_group);
-      p.epi = epi_store_params(grads.weight, lin.block, dtype, nullptr);
+      p.epi = epi_store_params(grads.weight, lin.block, grad_dtype, nullptr);
       const int slices = dtype == LT_BF16 ? lt_sparse_dw_slices(p) : 0;
       const size_t elements = (size_t)(in / lin.block) * lin.blocks_per_in * lin.block * lin.block;
       if (slices > 1 && s.skinny && s.skinny_bytes >= (size_t)slices * elements * sizeof(float)) {
@@ -333,7 +334,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
         p.epi.out = s.skinny;
         p.epi.out_dtype = LT_F32;
         LT_TRY(lt_launch_gemm_sparse(p, EPI_STORE, dtype, io_dtype, stream));
-        LT_TRY(lt_splitk_reduce((const float*)s.skinny, slices, (int64_t)elements, (int64_t)elements, lin.block, nullptr, dtype,
+        LT_TRY(lt_splitk_reduce((const float*)s.skinny, slices, (int64_t)elements, (int64_t)elements, lin.block, nullptr, grad_dtype,
                                 grads.weight, stream));
       } else {
         // no room for the partial sums: runs of output blocks unsplit, runs of input blocks as the walk
@@ -348,7 +349,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
     q.M = out; q.N = r; q.K[0] = T;
     q.A[0] = operand(dy, out, false);
     q.B[0] = operand(lowrank_hid, r, false);
-    q.epi = epi_store_params(grads.lowrank_second, r, dtype, nullptr);
+    q.epi = epi_store_params(grads.lowrank_second, r, grad_dtype, nullptr);
     LT_TRY(lt_launch_gemm_skinny(q, dtype, io_dtype, s.skinny, s.skinny_bytes, stream));
   }
   if (r > 0 && grads.lowrank_first) {  // dL1[r, in] = g_hid^T x
@@ -356,7 +357,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
     q.M = r; q.N = in; q.K[0] = T;
     q.A[0] = operand(s.g_hid, r, false);
     q.B[0] = operand(x_act, in, false);
-    q.epi = epi_store_params(grads.lowrank_first, in, dtype, nullptr);
+    q.epi = epi_store_params(grads.lowrank_first, in, grad_dtype, nullptr);
     LT_TRY(lt_launch_gemm_skinny(q, dtype, io_dtype, s.skinny, s.skinny_bytes, stream));
   }
   return LT_OK;
@@ -543,10 +544,19 @@ extern "C" int lt_ffn_forward(const lt_ffn_desc* desc, const void* x, void* y, c
 }
 
 extern "C" int lt_ffn_backward(const lt_ffn_desc* desc, const void* x, const void* dy, const lt_ffn_saved* saved,
-                               const lt_ffn_grads* grads, void* workspace, size_t workspace_bytes, void* stream_) {
+                               const lt_ffn_grads* grads, void* workspace, size_t workspace_bytes, void* stream) {
+  LT_TRY(check_ffn_desc(desc));
+  return lt_ffn_backward_to(desc, x, dy, saved, grads, desc->compute_dtype, workspace, workspace_bytes, stream);
+}
+
+extern "C" int lt_ffn_backward_to(const lt_ffn_desc* desc, const void* x, const void* dy, const lt_ffn_saved* saved,
+                                  const lt_ffn_grads* grads, int32_t grad_dtype, void* workspace, size_t workspace_bytes,
+                                  void* stream_) {
   LT_TRY(check_ffn_desc(desc));
   lt_ffn_desc d = *desc;
   hipStream_t stream = (hipStream_t)stream_;
+  LT_REQUIRE(grad_dtype == LT_F32 || grad_dtype == d.compute_dtype, LT_ERR_BAD_ARG,
+             "ffn backward: weight gradients in dtype %d, neither fp32 nor the compute dtype", grad_dtype);
   LT_REQUIRE(x && dy && saved && grads && saved->pre_activation && saved->ln_stats, LT_ERR_BAD_ARG, "ffn backward: null tensor");
   LT_REQUIRE(!d.post_ln_weight || saved->post_ln_input, LT_ERR_BAD_ARG, "ffn backward: post_ln_input missing");
   LT_REQUIRE((grads->ln_weight == nullptr) == (grads->ln_bias == nullptr), LT_ERR_BAD_ARG, "ffn backward: pass both LayerNorm gradients or neither");
@@ -594,7 +604,7 @@ extern "C" int lt_ffn_backward(const lt_ffn_desc* desc, const void* x, const voi
     memset(&e, 0, sizeof(e));
     e.pre = saved->pre_activation; e.ld_pre = N1; e.dpre = s.dpre; e.hid = s.hid; e.ld_hid = I;
     e.gated = d.gated; e.act = d.act; e.inter = I;
-    LT_TRY(linear_backward_impl(d.h2o, T, cdt, s.hid, g, saved->h2o_lowrank_hid, EPI_ACT_BWD, e, h2o_grads, s.h2o, io,
+    LT_TRY(linear_backward_impl(d.h2o, T, cdt, s.hid, g, saved->h2o_lowrank_hid, EPI_ACT_BWD, e, h2o_grads, grad_dtype, s.h2o, io,
                                 stream, grads->i2h.bias ? s.act_colsum : nullptr, &bias_rows, &reduces));
   }
   lt_linear_grads i2h_grads = grads->i2h;
@@ -611,7 +621,7 @@ extern "C" int lt_ffn_backward(const lt_ffn_desc* desc, const void* x, const voi
   {
     EpiParams e = epi_store_params(s.du, H, cdt, nullptr);
     LT_TRY(linear_backward_impl(d.i2h, T, cdt, s.u, s.dpre, saved->i2h_lowrank_hid, need_du ? EPI_STORE : -1, e,
-                                i2h_grads, s.i2h, io, stream, nullptr, nullptr, &reduces));
+                                i2h_grads, grad_dtype, s.i2h, io, stream, nullptr, nullptr, &reduces));
   }
   if (need_du) {
     LT_TRY(lt_ln_backward(T, (int)H, io, x, saved->ln_stats, d.ln_weight, cdt, s.du, io, d.residual ? dy : nullptr,
@@ -643,8 +653,17 @@ extern "C" int lt_linear_forward(const lt_linear* lin, int64_t tokens, int32_t d
 extern "C" int lt_linear_backward(const lt_linear* lin, int64_t tokens, int32_t dtype, const void* x, const void* dy,
                                   const void* lowrank_hid, void* dx, const lt_linear_grads* grads, void* workspace,
                                   size_t workspace_bytes, void* stream) {
+  return lt_linear_backward_to(lin, tokens, dtype, x, dy, lowrank_hid, dtype, dx, grads, dtype, workspace, workspace_bytes, stream);
+}
+
+extern "C" int lt_linear_backward_to(const lt_linear* lin, int64_t tokens, int32_t dtype, const void* x, const void* dy,
+                                     const void* lowrank_hid, int32_t dx_dtype, void* dx, const lt_linear_grads* grads,
+                                     int32_t grad_dtype, void* workspace, size_t workspace_bytes, void* stream) {
   LT_REQUIRE(lin && x && dy && grads && tokens > 0, LT_ERR_BAD_ARG, "linear backward: bad arguments");
   LT_TRY(check_dtype(dtype, "linear backward"));
+  for (int result : {dx_dtype, grad_dtype})
+    LT_REQUIRE(result == LT_F32 || result == dtype, LT_ERR_BAD_ARG,
+               "linear backward: a result in dtype %d, neither fp32 nor the compute dtype", result);
   LT_TRY(check_linear(*lin, "linear", NEED_BWD_TABLE));
   LT_REQUIRE(workspace && lt_aligned(workspace, 256) &&
                  workspace_bytes >= lt_linear_backward_workspace_bytes(lin, tokens, dtype),
@@ -653,8 +672,8 @@ extern "C" int lt_linear_backward(const lt_linear* lin, int64_t tokens, int32_t 
   Bump ws(workspace);
   LinearBwdScratch s;
   plan_linear_backward(*lin, tokens, dtype, ws, s);
-  EpiParams e = epi_store_params(dx, lin->in_features, dtype, nullptr);
-  return linear_backward_impl(*lin, tokens, dtype, x, dy, lowrank_hid, dx ? EPI_STORE : -1, e, *grads, s, dtype,
+  EpiParams e = epi_store_params(dx, lin->in_features, dx_dtype, nullptr);
+  return linear_backward_impl(*lin, tokens, dtype, x, dy, lowrank_hid, dx ? EPI_STORE : -1, e, *grads, grad_dtype, s, dtype,
                               (hipStream_t)stream);
 }
 
@@ -691,7 +710,7 @@ extern "C" int lt_blocksparse_backward(const lt_linear* lin, int64_t tokens, int
   LinearBwdScratch s;
   memset(&s, 0, sizeof(s));
   EpiParams e = epi_store_params(dx, l.in_features, dtype, nullptr);
-  return linear_backward_impl(l, tokens, dtype, x, dy, nullptr, dx ? EPI_STORE : -1, e, grads, s, dtype,
+  return linear_backward_impl(l, tokens, dtype, x, dy, nullptr, dx ? EPI_STORE : -1, e, grads, dtype, s, dtype,
                               (hipStream_t)stream);
 }
 

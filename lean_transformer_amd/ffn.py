@@ -14,7 +14,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _native as nat
-from .blocksparse.linear import GeneralizedLinear, _as, compute_dtype_for, linear_desc
+from .blocksparse.linear import GeneralizedLinear, _as, _result_dtype, compute_dtype_for, linear_desc
 from .utils import ACT2FN, ACT_KINDS, activation_kind
 
 
@@ -307,12 +307,14 @@ class _LeanFFN(torch.autograd.Function):
             return buffer[small_offsets[i]:small_offsets[i] + small_sizes[i]] if small_sizes[i] else None
 
         d_ln_w, d_ln_b, d_post_w, d_post_b, d_i2h_b, d_h2o_b = (piece(small, i) for i in range(6))
-        d_i2h_w = new(i2h_weight.shape, cdt, need[3])
-        d_i2h_l1 = new(i2h_l1.shape, cdt, need[5]) if i2h_l1 is not None else None
-        d_i2h_l2 = new(i2h_l2.shape, cdt, need[6]) if i2h_l2 is not None else None
-        d_h2o_w = new(h2o_weight.shape, cdt, need[10])
-        d_h2o_l1 = new(h2o_l1.shape, cdt, need[12]) if h2o_l1 is not None else None
-        d_h2o_l2 = new(h2o_l2.shape, cdt, need[13]) if h2o_l2 is not None else None
+        # fp32 parameters (autocast): their gradients straight from the accumulators
+        grad_dtype = _result_dtype(cdt, i2h_weight, i2h_l1, i2h_l2, h2o_weight, h2o_l1, h2o_l2)
+        d_i2h_w = new(i2h_weight.shape, grad_dtype, need[3])
+        d_i2h_l1 = new(i2h_l1.shape, grad_dtype, need[5]) if i2h_l1 is not None else None
+        d_i2h_l2 = new(i2h_l2.shape, grad_dtype, need[6]) if i2h_l2 is not None else None
+        d_h2o_w = new(h2o_weight.shape, grad_dtype, need[10])
+        d_h2o_l1 = new(h2o_l1.shape, grad_dtype, need[12]) if h2o_l1 is not None else None
+        d_h2o_l2 = new(h2o_l2.shape, grad_dtype, need[13]) if h2o_l2 is not None else None
         outputs = (dx, d_ln_w, d_ln_b, d_post_w, d_post_b, d_i2h_w, d_i2h_b, d_i2h_l1, d_i2h_l2, d_h2o_w, d_h2o_b,
                    d_h2o_l1, d_h2o_l2)
         if tokens > 0:
@@ -325,8 +327,8 @@ class _LeanFFN(torch.autograd.Function):
                                    nat.ptr(h2o_hid))
             lib = nat.lib(cdt)
             ws = nat.workspace(lib.lt_ffn_backward_workspace_bytes(desc), device)
-            nat.check(lib.lt_ffn_backward(desc, nat.ptr(x), nat.ptr(dy), saved, grads, nat.ptr(ws), ws.numel(),
-                                          nat.current_stream(device)), "lt_ffn_backward", lib)
+            nat.check(lib.lt_ffn_backward_to(desc, nat.ptr(x), nat.ptr(dy), saved, grads, nat.dtype_code(grad_dtype), nat.ptr(ws),
+                                             ws.numel(), nat.current_stream(device)), "lt_ffn_backward_to", lib)
             del ws, keep
         else:
             for g in outputs[1:]:
