@@ -90,24 +90,23 @@ __global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int t
   const int wm = wave >> 1, wn = wave & 1;
   const bool gated = KIND == EPI_ACT_FWD && p.epi.gated;
 
-  // workgroup i runs on XCD i % 8; each XCD takes a contiguous range of tiles, GROUP_M tile rows at a time
-  const int num_pid = tiles_m * tiles_n;
-  int pid = blockIdx.x;
-  if ((num_pid & 7) == 0) pid = (pid & 7) * (num_pid >> 3) + (pid >> 3);
+  // each XCD takes a contiguous range of tiles, GROUP_M tile rows at a time
+  const int pid = p.ksplit > 1 ? split_tile() : xcd_order((int)blockIdx.x, tiles_m * tiles_n);
   const int in_group = GROUP_M * tiles_n, first_m = pid / in_group * GROUP_M, group_m = min(tiles_m - first_m, GROUP_M);
   const int64_t m0 = (int64_t)(first_m + pid % in_group % group_m) * MID;
   const int64_t n0 = (int64_t)(pid % in_group / group_m) * (gated ? MID / 2 : MID);
 
-  // this workgroup's stages: first .. first + total of the reduction (slice blockIdx.y of them), walked from `rot` on and around:
+  // this workgroup's stages: first .. first + total of the reduction (a slice of them), walked from `rot` on and around:
   // with a power-of-two leading dimension the rows of a k-major tile otherwise lie on the same memory channels, chip-wide
   const int all = (int)((p.K[0] + 63) / 64);
   int first = 0, total = all;
   if (p.ksplit > 1) {
     const int per = (all + p.ksplit - 1) / p.ksplit;
-    first = min(all, (int)blockIdx.y * per);
+    first = min(all, split_slice() * per);
     total = min(per, all - first);
   }
-  const int rot = total > 0 ? (int)(((blockIdx.x & 7) * (unsigned)(total >> 3) + ((blockIdx.x >> 3) & 7)) % (unsigned)total) : 0;
+  const unsigned v = blockIdx.y * gridDim.x + blockIdx.x;
+  const int rot = total > 0 ? (int)(((v & 7) * (unsigned)(total >> 3) + ((v >> 3) & 7)) % (unsigned)total) : 0;
   const int k_limit = (int)p.K[0];
   MidOperand<A_KM> ca;
   MidOperand<B_KM> cb;

@@ -13,7 +13,7 @@ template <int KIND, typename TX, int ACT, bool PAIR>
 __device__ __forceinline__ void strip_epilogue(const f32x16 (&acc)[2][2], const GemmProblem& p, float* stage, const int64_t m_first,
                                                const int64_t n_first, const int lane) {
   EpiParams epi = p.epi;
-  if (KIND == EPI_STORE && p.ksplit > 1) epi.out = reinterpret_cast<float*>(epi.out) + (int64_t)blockIdx.y * p.split_stride;
+  if (KIND == EPI_STORE && p.ksplit > 1) epi.out = reinterpret_cast<float*>(epi.out) + (int64_t)split_slice() * p.split_stride;
   epi.bias = nullptr;
   auto staged = [&](int row, int col) -> float* { return &stage[row * 64 + (col ^ (((row >> 2) & 1) << 5))]; };
   float colsum[16];  // EPI_ACT_BWD: column sums of the dpre values this lane writes
