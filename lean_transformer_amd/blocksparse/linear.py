@@ -141,7 +141,11 @@ def _as(t: Optional[torch.Tensor], dtype: torch.dtype) -> Optional[torch.Tensor]
 
 def _result_dtype(dtype: torch.dtype, *tensors: Optional[torch.Tensor]) -> torch.dtype:
     """dtype the kernels write these tensors' gradients in: fp32 where all of them are, else the compute dtype"""
-    return torch.float32 if all(t is None or t.dtype == torch.float32 for t in tensors) else dtype
+    if dtype != torch.float32:
+        for t in tensors:
+            if t is not None and t.dtype != torch.float32:
+                return dtype
+    return torch.float32
 
 
 def shared_list_run(forward_indices: torch.Tensor, blocks_per_in: int) -> int:
