@@ -380,10 +380,10 @@ bool lt_sparse_mfma_supported(const GemmProblem& p, int kind) {
     return true;
   }
   if (!lt_aligned(sp.weight, 16)) return false;
-  // the walk addresses a tile's rows with 32-bit byte offsets
+  // the walk addresses a tile's rows with 32-bit byte offsets, products of a row number and a pitch of at most 24 bits (2^32 / 257)
   if (257 * sp.ld_act * 2 + 1024 >= (int64_t)1 << 32) return false;
   if (p.nseg > 1) {
-    if (257 * p.A[1].ld * 2 + 1024 >= (int64_t)1 << 32 || 65 * p.B[1].ld * 2 + 1024 >= (int64_t)1 << 32) return false;
+    if (257 * p.A[1].ld * 2 + 1024 >= (int64_t)1 << 32 || 257 * p.B[1].ld * 2 + 1024 >= (int64_t)1 << 32) return false;
     if (p.K[1] <= 0 || p.K[1] % 8 != 0 || p.A[1].ld % 8 != 0 || p.B[1].ld % 8 != 0 || !lt_aligned(p.A[1].ptr, 16) ||
         !lt_aligned(p.B[1].ptr, 16))
       return false;
