@@ -298,23 +298,24 @@ __device__ __forceinline__ void epi_act_bwd8_loaded(const EpiParams& e, int64_t 
 // Straight-line epilogue bodies for the usual cases (whole tile in range, bias present, no dropout): the run-time choices of
 // the general functions above are made once per tile by the caller, not once per row; bias values of a lane's 8 columns
 // are loaded once per tile and passed in.
-// forward activation with its kind fixed (bias already in the accumulators)
+// forward activation with its kind fixed (bias already in the accumulators).  The values are rounded one by one, not through packed
+// words as in backward, where nothing else waits for them: GeGLU of [4096, 4096] x 16384 865 us, packed 873; SiLU of [3333, 1600] x 6400
+// 100.4, packed 101.6.
 template <bool GATED, int ACT>
 __device__ __forceinline__ void epi_act_fwd8_fixed(const EpiParams& e, int64_t m, int64_t n, float (&vg)[8], float (&vl)[8]) {
   float h[8];
-  bf16* pre = reinterpret_cast<bf16*>(e.pre) + m * e.ld_pre + n;
-  lt_u32x4 packed = round8(vg);  // the activation sees the stored (rounded) pre-activation, as backward will
-  store8(pre, packed);
-  unpack_bf16x8(packed, vg);
 #pragma unroll
-  for (int i = 0; i < 8; i++) h[i] = act_value<false>(ACT, vg[i]);
-  if constexpr (GATED) {
-    packed = round8(vl);
-    store8(pre + e.inter, packed);
-    unpack_bf16x8(packed, vl);
-#pragma unroll
-    for (int i = 0; i < 8; i++) h[i] *= vl[i];
+  for (int i = 0; i < 8; i++) {
+    vg[i] = to_f32((bf16)vg[i]);  // the activation sees the stored (rounded) pre-activation, as backward will
+    h[i] = act_value<false>(ACT, vg[i]);
+    if constexpr (GATED) {
+      vl[i] = to_f32((bf16)vl[i]);
+      h[i] *= vl[i];
+    }
   }
+  bf16* pre = reinterpret_cast<bf16*>(e.pre) + m * e.ld_pre + n;
+  store8(pre, vg);
+  if constexpr (GATED) store8(pre + e.inter, vl);
   store8(reinterpret_cast<bf16*>(e.hid) + m * e.ld_hid + n, h);
 }
 
