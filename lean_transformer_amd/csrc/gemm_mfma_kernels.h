@@ -60,25 +60,21 @@ namespace {
 
 constexpr int BK = 64;
 constexpr int GROUP_M = 8;
-// Workgroup v of a launch of n runs on XCD v % 8: the place it takes in an order in which the workgroups of one XCD follow each other
-__device__ __forceinline__ int xcd_order(int v, int n) {
-  const int each = n >> 3, more = n & 7, xcd = v & 7;
-  return xcd * each + min(xcd, more) + (v >> 3);
-}
-// The same for a split reduction (one workgroup per tile and slice: grid of tiles x slices), slice by slice: an XCD's workgroups are
+// A split reduction (one workgroup per tile and slice: grid of tiles x slices) in runs (lt_xcd_order), slice by slice: an XCD's workgroups are
 // neighbouring tiles of one slice or two and read the same rows of k through its L2.  Weight gradient [768, 3072] over 16384 (36 tiles,
 // 7 slices), tiles dealt to the XCDs in turn against this: 95 us, 85.
 __device__ __forceinline__ int split_place() {
-  return xcd_order((int)(blockIdx.y * gridDim.x + blockIdx.x), (int)(gridDim.x * gridDim.y));
+  return lt_xcd_order((int)(blockIdx.y * gridDim.x + blockIdx.x), (int)(gridDim.x * gridDim.y));
 }
 __device__ __forceinline__ int split_slice() { return __builtin_amdgcn_readfirstlane(split_place() / (int)gridDim.x); }
 __device__ __forceinline__ int split_tile() { return __builtin_amdgcn_readfirstlane(split_place() % (int)gridDim.x); }
-// Copy-based kernel: with a staggered walk over k (krot, two k-major operands) a slice's tiles are dealt to the XCDs on their own, each
-// XCD's walk an eighth of the reduction on.  [1537, 2880] over 11520 (84 tiles, 3 slices): 150 us in the order above, 137 in this.
+// Copy-based kernel, two k-major operands (krot): a slice's tiles are dealt to the XCDs on their own, in turn where 8 does not divide their
+// number.  [1537, 2880] over 11520 (84 tiles, 3 slices): 150 us in the order above, 137 in this; [1537, 2904] over 11616, where K is no
+// multiple of 64 and no walk is staggered: 174, 163.
 __device__ __forceinline__ int dma_split_slice(int krot) { return krot ? (int)blockIdx.y : split_slice(); }
 __device__ __forceinline__ int dma_split_tile(int krot, int tiles) {
   const int v = (int)blockIdx.x;
-  return !krot ? split_tile() : (tiles & 7) == 0 ? (v & 7) * (tiles >> 3) + (v >> 3) : v;
+  return !krot ? split_tile() : lt_turn_order(v, tiles);
 }
 typedef __attribute__((__vector_size__(4 * sizeof(unsigned int)))) unsigned int u32x4;
 
@@ -146,7 +142,7 @@ void gemm_bf16_kernel(GemmProblem p, int tiles_m, int tiles_n) {
   const bool gated = (KIND == EPI_ACT_FWD) && p.epi.gated;
 
   // ---- tile assignment: XCD-contiguous, grouped along M
-  const int pid = p.ksplit > 1 ? split_tile() : xcd_order((int)blockIdx.x, tiles_m * tiles_n);
+  const int pid = p.ksplit > 1 ? split_tile() : lt_xcd_order((int)blockIdx.x, tiles_m * tiles_n);
   const int group = GROUP_M * tiles_n;
   const int first_m = (pid / group) * GROUP_M;
   const int gsz = min(tiles_m - first_m, GROUP_M);
@@ -1117,7 +1113,10 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
   int tm = 0, tn = 0;
   int64_t m0 = 0, n0 = 0;
   auto place = [&](int v) {
-    const int pid = p.ksplit > 1 ? dma_split_tile(p.krot, num_pid) : xcd_order(v, num_pid);
+    int pid;
+    if (p.ksplit > 1) pid = dma_split_tile(p.krot, num_pid);
+    else if constexpr (GATHER == 0 && A_KM && B_KM) pid = lt_tile_order(v, tiles_m, tiles_n, lt_can_stagger(p.nseg, p.K[0]) && p.krot);
+    else pid = lt_xcd_order(v, num_pid);
     const int group = GROUP_M * tiles_n;
     const int first_m = (pid / group) * GROUP_M;
     const int gsz = min(tiles_m - first_m, GROUP_M);
@@ -1149,7 +1148,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
   // nothing to gain for mn-major ones.
   int rot = 0;
   auto set_rot = [&](int v) {
-    if (GATHER == 0 && p.nseg == 1 && (p.K[0] & 63) == 0 && p.krot) {
+    if (GATHER == 0 && lt_can_stagger(p.nseg, p.K[0]) && p.krot) {
       const unsigned bx = (unsigned)v;
       // (inside an XCD the eight tile rows start 2 k-steps apart at most: tiles that share a B panel then read it within 14
       // k-steps of each other, inside what the XCD's L2 still holds; 8 apart, as a long reduction would otherwise give,

@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int t
   const bool gated = KIND == EPI_ACT_FWD && p.epi.gated;
 
   // each XCD takes a contiguous range of tiles, GROUP_M tile rows at a time
-  const int pid = p.ksplit > 1 ? split_tile() : xcd_order((int)blockIdx.x, tiles_m * tiles_n);
+  const int pid = p.ksplit > 1 ? split_tile() : lt_xcd_order((int)blockIdx.x, tiles_m * tiles_n);
   const int in_group = GROUP_M * tiles_n, first_m = pid / in_group * GROUP_M, group_m = min(tiles_m - first_m, GROUP_M);
   const int64_t m0 = (int64_t)(first_m + pid % in_group % group_m) * MID;
   const int64_t n0 = (int64_t)(pid % in_group / group_m) * (gated ? MID / 2 : MID);

@@ -57,7 +57,7 @@ void gemm_walk_kernel(GemmProblem p, int tiles_m, int groups) {
   // while every block column has a weight list of its own, so one XCD's concurrent workgroups (workgroup i runs on XCD i % 8) take
   // one token tile and consecutive block columns.
   const int num_pid = tiles_m * groups;
-  const int pid = xcd_order((int)blockIdx.x, num_pid);
+  const int pid = lt_xcd_order((int)blockIdx.x, num_pid);
   const int tm = pid / groups, tn = pid % groups;
   const int64_t m0 = (int64_t)tm * 256, n0 = (int64_t)tn * 64;
 

@@ -1,6 +1,7 @@
 // GEMM problem description and fused epilogues shared by the any-shape kernel and the tiled bf16 MFMA kernel.
 #pragma once
 #include "lt_common.h"
+#include "lt_order.h"
 #include "lt_steps.h"
 
 // C[m, n] = sum over up to two K segments of  sum_k A_s(m, k) * B_s(n, k)   (fp32 accumulation), then one epilogue.
