@@ -60,14 +60,12 @@ namespace {
 
 constexpr int BK = 64;
 constexpr int GROUP_M = 8;
-// A split reduction (one workgroup per tile and slice: grid of tiles x slices) in runs (lt_xcd_order), slice by slice: an XCD's workgroups are
-// neighbouring tiles of one slice or two and read the same rows of k through its L2.  Weight gradient [768, 3072] over 16384 (36 tiles,
-// 7 slices), tiles dealt to the XCDs in turn against this: 95 us, 85.
-__device__ __forceinline__ int split_place() {
-  return lt_xcd_order((int)(blockIdx.y * gridDim.x + blockIdx.x), (int)(gridDim.x * gridDim.y));
+// Tile and slice of a workgroup of a split reduction (grid of tiles x slices), dealt slice by slice
+__device__ __forceinline__ lt_split_place split_place() {
+  return lt_split_by_slice((int)(blockIdx.y * gridDim.x + blockIdx.x), (int)gridDim.x, (int)gridDim.y);
 }
-__device__ __forceinline__ int split_slice() { return __builtin_amdgcn_readfirstlane(split_place() / (int)gridDim.x); }
-__device__ __forceinline__ int split_tile() { return __builtin_amdgcn_readfirstlane(split_place() % (int)gridDim.x); }
+__device__ __forceinline__ int split_slice() { return __builtin_amdgcn_readfirstlane(split_place().slice); }
+__device__ __forceinline__ int split_tile() { return __builtin_amdgcn_readfirstlane(split_place().tile); }
 // Copy-based kernel, two k-major operands (krot): a slice's tiles are dealt to the XCDs on their own, in turn where 8 does not divide their
 // number.  [1537, 2880] over 11520 (84 tiles, 3 slices): 150 us in the order above, 137 in this; [1537, 2904] over 11616, where K is no
 // multiple of 64 and no walk is staggered: 174, 163.

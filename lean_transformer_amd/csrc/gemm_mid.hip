@@ -91,7 +91,18 @@ __global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int t
   const bool gated = KIND == EPI_ACT_FWD && p.epi.gated;
 
   // each XCD takes a contiguous range of tiles, GROUP_M tile rows at a time
-  const int pid = p.ksplit > 1 ? split_tile() : lt_xcd_order((int)blockIdx.x, tiles_m * tiles_n);
+  const bool split = KIND == EPI_STORE && p.ksplit > 1;
+  const int v = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+  int pid, slice = 0, later = (v >> 3) & 7;  // (later: steps that a workgroup starts behind its neighbour on the XCD)
+  if (split) {
+    const bool tiles_first = A_KM && lt_split_tiles_first(p.M, p.N, p.K[0]);
+    const lt_split_place at = tiles_first ? lt_split_by_tile(v, tiles_m * tiles_n, p.ksplit) : lt_split_by_slice(v, tiles_m * tiles_n, p.ksplit);
+    pid = __builtin_amdgcn_readfirstlane(at.tile);
+    slice = __builtin_amdgcn_readfirstlane(at.slice);
+    if (tiles_first) later = pid & 7;
+  } else {
+    pid = lt_xcd_order(v, tiles_m * tiles_n);
+  }
   const int in_group = GROUP_M * tiles_n, first_m = pid / in_group * GROUP_M, group_m = min(tiles_m - first_m, GROUP_M);
   const int64_t m0 = (int64_t)(first_m + pid % in_group % group_m) * MID;
   const int64_t n0 = (int64_t)(pid % in_group / group_m) * (gated ? MID / 2 : MID);
@@ -100,13 +111,12 @@ __global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int t
   // with a power-of-two leading dimension the rows of a k-major tile otherwise lie on the same memory channels, chip-wide
   const int all = (int)((p.K[0] + 63) / 64);
   int first = 0, total = all;
-  if (p.ksplit > 1) {
+  if (split) {
     const int per = (all + p.ksplit - 1) / p.ksplit;
-    first = min(all, split_slice() * per);
+    first = min(all, slice * per);
     total = min(per, all - first);
   }
-  const unsigned v = blockIdx.y * gridDim.x + blockIdx.x;
-  const int rot = total > 0 ? (int)(((v & 7) * (unsigned)(total >> 3) + ((v >> 3) & 7)) % (unsigned)total) : 0;
+  const int rot = total > 0 ? (int)((unsigned)((v & 7) * (total >> 3) + later) % (unsigned)total) : 0;
   const int k_limit = (int)p.K[0];
   MidOperand<A_KM> ca;
   MidOperand<B_KM> cb;
@@ -170,10 +180,10 @@ __global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int t
   // ---- epilogue (strip_epilogue)
   float* const stage = reinterpret_cast<float*>(wave == 0 ? a0 : wave == 1 ? a1 : wave == 2 ? b0 : b1);
   if constexpr (KIND == EPI_ACT_FWD) {
-    if (gated) strip_epilogue<KIND, TX, ACT, true>(acc, p, stage, m0 + wm * 64, n0 + wn * 32, lane);
-    else strip_epilogue<KIND, TX, ACT, false>(acc, p, stage, m0 + wm * 64, n0 + wn * 64, lane);
+    if (gated) strip_epilogue<KIND, TX, ACT, true>(acc, p, slice, stage, m0 + wm * 64, n0 + wn * 32, lane);
+    else strip_epilogue<KIND, TX, ACT, false>(acc, p, slice, stage, m0 + wm * 64, n0 + wn * 64, lane);
   } else {
-    strip_epilogue<KIND, TX, ACT, false>(acc, p, stage, m0 + wm * 64, n0 + wn * 64, lane);
+    strip_epilogue<KIND, TX, ACT, false>(acc, p, slice, stage, m0 + wm * 64, n0 + wn * 64, lane);
   }
 }
 

@@ -8,12 +8,12 @@ namespace {
 // what a strip reads from memory is requested before it is staged.  Accumulator register r of a 32 x 32 block is row
 // 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32; columns of rows with bit 2 set are staged 32 further on (banks).
 // Rows m_first .. + 63, columns n_first .. + 63 of the result; PAIR (gated forward): acc[i][0] are gate columns n_first .. + 31,
-// acc[i][1] the matching linear ones.
+// acc[i][1] the matching linear ones.  slice: of a split reduction.
 template <int KIND, typename TX, int ACT, bool PAIR>
-__device__ __forceinline__ void strip_epilogue(const f32x16 (&acc)[2][2], const GemmProblem& p, float* stage, const int64_t m_first,
-                                               const int64_t n_first, const int lane) {
+__device__ __forceinline__ void strip_epilogue(const f32x16 (&acc)[2][2], const GemmProblem& p, const int slice, float* stage,
+                                               const int64_t m_first, const int64_t n_first, const int lane) {
   EpiParams epi = p.epi;
-  if (KIND == EPI_STORE && p.ksplit > 1) epi.out = reinterpret_cast<float*>(epi.out) + (int64_t)split_slice() * p.split_stride;
+  if (KIND == EPI_STORE && p.ksplit > 1) epi.out = reinterpret_cast<float*>(epi.out) + (int64_t)slice * p.split_stride;
   epi.bias = nullptr;
   auto staged = [&](int row, int col) -> float* { return &stage[row * 64 + (col ^ (((row >> 2) & 1) << 5))]; };
   float colsum[16];  // EPI_ACT_BWD: column sums of the dpre values this lane writes

@@ -232,10 +232,10 @@ void gemm_walk_kernel(GemmProblem p, int tiles_m, int groups) {
     lt_static_for<2>([&](auto J) __attribute__((always_inline)) {
       constexpr int j = decltype(J)::value;
       const f32x16 pair[2][2] = {{acc[0][j], acc2[0][j]}, {acc[1][j], acc2[1][j]}};
-      strip_epilogue<KIND, TX, ACT, true>(pair, p, stage, m0 + wave * 64, n0 + j * 32, lane);
+      strip_epilogue<KIND, TX, ACT, true>(pair, p, 0, stage, m0 + wave * 64, n0 + j * 32, lane);
     });
   } else {
-    strip_epilogue<KIND, TX, ACT, false>(acc, p, stage, m0 + wave * 64, n0, lane);
+    strip_epilogue<KIND, TX, ACT, false>(acc, p, 0, stage, m0 + wave * 64, n0, lane);
   }
   LT_TILE_STAMP(3);
   LT_TILE_STAMP_REALTIME(5);

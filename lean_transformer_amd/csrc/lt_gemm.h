@@ -94,7 +94,8 @@ struct GemmProblem {
   GemmOperand A[2], B[2];
   EpiParams epi;
   SparseWalk sp;  // sp.mode == SPARSE_NONE for a dense problem
-  // split-k (tiled kernel, EPI_STORE only): blockIdx.y = slice of the k-steps; slice s stores fp32 partial sums at
+  // split-k (EPI_STORE only): the k-steps are cut into this many slices, one workgroup per tile and slice (grid of tiles x slices; which
+  // of them a workgroup takes is its kernel's choice, lt_order.h: not blockIdx.y).  Slice s stores fp32 partial sums at
   // epi.out + s * split_stride elements, summed afterwards in slice order (deterministic)
   int ksplit;
   int64_t split_stride;

@@ -26,3 +26,28 @@ constexpr int LT_TURN_ROWS = 10;
 LT_HOST_DEVICE inline int lt_tile_order(int v, int tiles_m, int tiles_n, bool staggered) {
   return staggered && tiles_m <= LT_TURN_ROWS ? lt_turn_order(v, tiles_m * tiles_n) : lt_xcd_order(v, tiles_m * tiles_n);
 }
+
+struct lt_split_place { int tile, slice; };
+
+// A split reduction, slice by slice: an XCD's workgroups are neighbouring tiles of one slice or two and read the same rows of k through
+// its L2.  Weight gradient [768, 3072] over 16384 (36 tiles, 7 slices), tiles dealt to the XCDs in turn against this: 95 us, 85.
+LT_HOST_DEVICE inline lt_split_place lt_split_by_slice(int v, int tiles, int slices) {
+  const int place = lt_xcd_order(v, tiles * slices);
+  return {place % tiles, place / tiles};
+}
+
+// Tile by tile: an XCD's workgroups are the whole reductions of neighbouring tiles
+LT_HOST_DEVICE inline lt_split_place lt_split_by_tile(int v, int tiles, int slices) {
+  const int place = lt_xcd_order(v, tiles * slices);
+  return {place / slices, place % slices};
+}
+
+// 128 x 128 tiles, k-major A: tile by tile where one operand is streamed, with next to nothing of it used by two tiles (one tile column,
+// or two tile rows), and that operand is over 64 MiB.  By slices an XCD would read a narrow band of k of all its rows.  Slice by
+// slice and tile by tile: [4096, 128] over 16384 56 us, 50; [4096, 64] over 16384 57, 48; [129, 4096] over 32768 106, 94; [129, 4096] over
+// 16384 58, 54.  Below that size slice by slice is the faster one ([1000, 128] over 16384 16.8, 18.8), and by far where both operands are
+// used again ([4096, 256] over 16384 40, 52).
+LT_HOST_DEVICE inline bool lt_split_tiles_first(int64_t M, int64_t N, int64_t K) {
+  const bool thin = N <= 128 || M <= 256;
+  return thin && (M > N ? M : N) * K > (int64_t)1 << 25;
+}
