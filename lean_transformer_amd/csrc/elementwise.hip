@@ -350,7 +350,8 @@ __global__ __launch_bounds__(256) void ln_bwd_param_kernel(int64_t T, int H, con
 // workgroup at a time and up to 256 workgroups walk the rows, the next row's dy and x in flight while this one's sums go
 // through LDS; the column sums stay in registers and leave once, one partial row per workgroup.  Bound by memory: dy and x are
 // read once instead of twice.  Measured with fp32 x and residual, the two kernels against this: [4096, 4096] 72 us, 52; [16384, 768]
-// 48, 34.  Wider rows would need twice the partial rows or leave CUs idle, an fp32 dy more than the 128 registers of a wavefront:
+// 48, 34; with the sums of the partial rows and everything in the caches: [512, 2560] 16.6, 13.4; [4096, 256] 15.0, 12.6; [4096, 1536] 27.8,
+// 22.4; [4096, 2056] 39.6, 29.3.  Wider rows would need twice the partial rows or leave CUs idle, an fp32 dy more than the 128 registers of a wavefront:
 // both stay with the two kernels.
 template <typename TX, typename TDX, int WPR>
 __global__ __launch_bounds__(1024) void ln_bwd_rows_kernel(int64_t T, int H, const TX* __restrict__ x,
@@ -480,7 +481,9 @@ __global__ void colreduce_kernel(int rows, int64_t stride, int cols, const float
   out[c] = s;
 }
 
-// same, 16 row lanes x 16 column lanes of 4 columns per workgroup: short dependent chains, 16-byte loads
+// same, 16 row lanes x 16 column lanes of 4 columns per workgroup: short dependent chains, 16-byte loads, eight of them in flight (the
+// adds stay in row order).  Latency bounds it: with one load at a time the two sums of a LayerNorm backward's 256 partial rows took
+// longer than its two kernels' 64 had: [4096, 768] 23 us in all, 15 with eight in flight (two kernels and 64 rows: 21).
 __global__ __launch_bounds__(256) void colreduce4_kernel(int rows, int64_t stride, int cols, const float* __restrict__ partial,
                                                          float* __restrict__ out) {
   __shared__ float red[16][16][5];
@@ -488,6 +491,7 @@ __global__ __launch_bounds__(256) void colreduce4_kernel(int rows, int64_t strid
   const int c = (blockIdx.x * 16 + cl) * 4;
   float s[4] = {0.f, 0.f, 0.f, 0.f};
   if (c < cols) {
+#pragma unroll 8
     for (int r = rl; r < rows; r += 16) {
       float v[4];
       load4(partial + (int64_t)r * stride + c, v);
@@ -519,6 +523,7 @@ __global__ __launch_bounds__(256) void colreduce4_multi_kernel(ColReduceQueue q)
   if (blockIdx.x * 64 >= job.cols) return;  // (the whole workgroup)
   float s[4] = {0.f, 0.f, 0.f, 0.f};
   if (c < job.cols) {
+#pragma unroll 8
     for (int r = rl; r < job.rows; r += 16) {
       float v[4];
       load4(job.partial + (int64_t)r * job.stride + c, v);

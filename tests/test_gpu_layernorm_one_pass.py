@@ -65,6 +65,13 @@ def test_one_pass(tokens, hidden, x_dtype, dy_dtype, dx_dtype, with_residual):
     _check(x, dy, res, w, stats, _backward(x, dy, res, w, stats, dx_dtype))
 
 
+@pytest.mark.parametrize("partial_rows", [15, 17, 112, 127, 128, 129, 241])
+def test_sums_of_any_number_of_partial_rows(partial_rows):
+    """16 row lanes read eight partial rows ahead: around one turn of that, several, and a rest (68 columns: a column block and a bit)"""
+    tensors = _inputs(16 * partial_rows, 68, torch.float32, torch.bfloat16, torch.float32)
+    _check(*tensors, _backward(*tensors, torch.float32))
+
+
 def test_scratch_for_the_two_kernels_alone_is_still_enough():
     tensors = _inputs(640, 1024, torch.float32, torch.bfloat16, torch.float32)
     _check(*tensors, _backward(*tensors, torch.float32, workspace_rows=10))  # (the one pass would take 40)
