@@ -313,11 +313,11 @@ class _GeneralizedLinear(torch.autograd.Function):
         grads = nat.LtLinearGrads()
         # straight in the type autograd hands on: fp32 from the accumulators where the tensors are fp32 (autocast)
         dx_dtype, grad_dtype = _result_dtype(dtype, input), _result_dtype(dtype, main_weight, lowrank_first, lowrank_second)
-        dx = torch.empty(x.shape, dtype=dx_dtype, device=device) if need[0] else None
-        dw = torch.empty(w.shape, dtype=grad_dtype, device=device) if need[1] else None
+        dx = torch.empty_like(x, dtype=dx_dtype) if need[0] else None
+        dw = torch.empty_like(w, dtype=grad_dtype) if need[1] else None
         db = torch.empty(desc.out_features, dtype=torch.float32, device=device) if (ctx._has_bias and need[2]) else None
-        dl1 = torch.empty(l1.shape, dtype=grad_dtype, device=device) if (l1 is not None and need[3]) else None
-        dl2 = torch.empty(l2.shape, dtype=grad_dtype, device=device) if (l2 is not None and need[4]) else None
+        dl1 = torch.empty_like(l1, dtype=grad_dtype) if (l1 is not None and need[3]) else None
+        dl2 = torch.empty_like(l2, dtype=grad_dtype) if (l2 is not None and need[4]) else None
         grads.weight, grads.bias, grads.lowrank_first, grads.lowrank_second = (nat.ptr(dw), nat.ptr(db), nat.ptr(dl1),
                                                                                nat.ptr(dl2))
         if tokens > 0:
