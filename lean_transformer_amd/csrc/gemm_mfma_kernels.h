@@ -708,8 +708,8 @@ __device__ __forceinline__ int lt_run_member(int t, int j, int len, int stride) 
 // gradient, at the flat position the forward table names.  List entries past the end (the last column tile) are not stored.
 // SCATTER == 2: the tile is 4 entries of a list of output blocks (rows) x the run of 4 input blocks that shares the list
 // (columns); piece (entry a, input block ib) is block ib * blocks_per_in + a.
-// ACT: the activation of EPI_ACT_FWD / EPI_ACT_BWD, or -1: chosen per element from epi.act.
-template <int FM, int KIND, typename TX, int tile_rows, int tile_cols, int SCATTER = 0, int ACT = -1, int FN>
+// ACT: the activation of EPI_ACT_FWD / EPI_ACT_BWD, or -1: chosen per element from epi.act.  SPLITS: the reduction may be split.
+template <int FM, int KIND, typename TX, int tile_rows, int tile_cols, int SCATTER, int ACT, bool SPLITS, int FN>
 __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][FN], const GemmProblem& p, float* stage, const int64_t m0,
                                                   const int64_t n0, const int wm, const int wn, const bool gated) {
   // (FN == 3: four of the 16 lanes of a row would have no columns; they repeat the last 8, reads and stores alike)
@@ -728,7 +728,7 @@ __device__ __forceinline__ void dma_tile_epilogue(f32x16 (&acc)[FM][FN], const G
   //      r and r + 4, same columns) then hit different banks without padding the rows.
   EpiParams epi = p.epi;
   epi.bias = nullptr;  // already in the accumulators
-  if (KIND == EPI_STORE && p.ksplit > 1) epi.out = reinterpret_cast<float*>(epi.out) + (int64_t)dma_split_slice(p.krot) * p.split_stride;
+  if (SPLITS && p.ksplit > 1) epi.out = reinterpret_cast<float*>(epi.out) + (int64_t)dma_split_slice(p.krot) * p.split_stride;
   auto staged = [&](int row, int col) -> float* { return &stage[row * PITCH + (col ^ (((row >> 2) & 1) << 5))]; };
   const bool pair = (KIND == EPI_ACT_FWD) && gated;
   float colsum[16];  // EPI_ACT_BWD: column sums of this lane's 8 (+ 8) dpre columns over the rows it writes
@@ -1038,6 +1038,9 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
   static_assert(GATHER != 2 || (A_KM && B_KM), "gathered k-blocks: forward layout");
   constexpr int BM = 256, BN = 64 * FN, WN = 2, WTM = 128, WTN = 32 * FN, FM = 4;
   static_assert(FN == 4 || (FN == 3 && GATHER == 0), "tile width");
+  // split reductions: plain stores, tiles of full width (the code for them costs the launches that never split: gathered forward product
+  // of hidden 4096, T 4096 193 us with it, 191 without; SiLU of [3333, 1600] x 6400 101, 98)
+  constexpr bool SPLITS = KIND == EPI_STORE && GATHER != 2 && FN == 4;
   constexpr int HALF = 4;  // copy instructions per wavefront for a mn-major k-step or half a k-major block
   constexpr int KM_ELEMS = 256 * 64, MN_ELEMS = DK * 256;
   // k-major operands use the two d buffers, mn-major ones the four s tiles; the unused set is never referenced and takes
@@ -1087,7 +1090,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
     kt_all = seg0 + (p.nseg > 1 ? (int)((p.K[1] + DK - 1) / DK) : 0);
     kt_begin = 0;
     kt_total = kt_all;
-    if (p.ksplit > 1) {
+    if (SPLITS && p.ksplit > 1) {
       const int per = (((kt_all + p.ksplit - 1) / p.ksplit) + 1) & ~1;
       kt_begin = min(kt_all, dma_split_slice(p.krot) * per);
       kt_total = min(per, kt_all - kt_begin);
@@ -1112,7 +1115,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
   int64_t m0 = 0, n0 = 0;
   auto place = [&](int v) {
     int pid;
-    if (p.ksplit > 1) pid = dma_split_tile(p.krot, num_pid);
+    if (SPLITS && p.ksplit > 1) pid = dma_split_tile(p.krot, num_pid);
     else if constexpr (GATHER == 0 && A_KM && B_KM) pid = lt_tile_order(v, tiles_m, tiles_n, lt_can_stagger(p.nseg, p.K[0]) && p.krot);
     else pid = lt_xcd_order(v, num_pid);
     const int group = GROUP_M * tiles_n;
@@ -1505,7 +1508,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(GemmProblem problem,
                             : wave == 1 ? (A_KM ? a_d1 + KM_ELEMS / 2 : a_s3)
                             : wave == 2 ? (B_KM ? b_d1 : b_s2)
                                         : (B_KM ? b_d1 + KM_ELEMS / 2 : b_s3);
-    dma_tile_epilogue<FM, KIND, TX, BM, BN, GATHER == 1 ? 1 : GATHER == 3 ? 2 : 0, ACT>(acc, *(const GemmProblem*)pk, reinterpret_cast<float*>(stage_buf), epi_m0,
+    dma_tile_epilogue<FM, KIND, TX, BM, BN, GATHER == 1 ? 1 : GATHER == 3 ? 2 : 0, ACT, SPLITS>(acc, *(const GemmProblem*)pk, reinterpret_cast<float*>(stage_buf), epi_m0,
                                                           epi_n0, wm, wn, gated);
     LT_TILE_STAMP(3);
     LT_TILE_STAMP_REALTIME(5);
