@@ -334,7 +334,8 @@ def test_bf16_blocksparse_wide_layers_with_runs_on_the_input_side(tokens, fan_in
 @pytest.mark.parametrize("tokens", [512, 300])
 def test_bf16_ffn_with_blocksparse_projections_in_runs(gated, tokens):
     """LeanFFN whose up-projection is PixelFly stretched over a tall matrix (runs of output blocks with one list): plain GELU
-    takes the dense product's fused activation epilogue, GeGLU the product and the activation pass"""
+    takes the dense product's fused activation epilogue, GeGLU the paired walk (a pre-activation this small; the product and the
+    activation pass: test_gpu_sparse_paths.py)"""
     torch.manual_seed(tokens + gated)
     hidden, inter = 512, 2048
     layout = "pixelfly(block_size=64, stretch=True)"

@@ -8,6 +8,8 @@ import pytest
 import torch
 
 import lean_transformer_amd as lt
+from test_gpu_ffn import _compare
+from test_gpu_kernels import _kernel_tags
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -119,3 +121,38 @@ def test_gated_up_projection_on_either_side_of_the_rule(tokens):
         hid = offn.apply_activation(pre, "gelu_fused", True)
         ref = hid @ dense_weight(down.weight, down.matrix.backward_indices, 1024).t()
     assert (y[rows].double() - ref).norm() <= 4 * 2.0**-8 * ref.norm()
+
+
+@pytest.mark.parametrize("tokens,two_passes", [(20480, False), (20488, True)])
+def test_gated_up_projection_on_either_side_of_the_rule_with_gradients(tokens, two_passes):
+    """a stretched butterfly of hidden 512 with a low-rank term (of whole 64s, or the walk takes it in any case), 160 MiB of
+    pre-activation and a little more: outputs and all gradients
+    against the fp32 oracle at the bf16 bars, and which way the launch went"""
+    torch.manual_seed(tokens)
+    layout = "pixelfly(block_size=64, stretch=True)"
+    up, down = (lt.GeneralizedLinear(lt.GeneralizedMatrix(i, o, layout, 64)) for i, o in ((512, 4096), (2048, 512)))
+    layer = lt.LeanFFN(512, 2048, gated=True, layer_norm_eps=1e-5, i2h_proj=up, h2o_proj=down).to(DEV).to(torch.bfloat16)
+    x, dy = torch.randn(tokens, 512), torch.randn(tokens, 512)
+    _, tags = _kernel_tags(lambda: layer(x.to(DEV)))
+    assert ("activation_fwd" in tags) == two_passes, tags
+    _compare(layer, x, dy, torch.bfloat16, oracle_device=DEV)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_equal_rows_in_different_token_tiles(dtype):
+    """a walk starts its list at another entry in each 256-token tile, so that equal rows are summed in different orders and may differ
+    in their last bits: by no more than the two roundings and the two fp32 sums' bounds"""
+    torch.manual_seed(1)
+    layer = lt.GeneralizedLinear(lt.GeneralizedMatrix(1024, 1024, "scrambled(per_in=12)", 0), bias=False).to(DEV).to(dtype)
+    rows, dy_rows = torch.randn(256, 1024, device=DEV).to(dtype), torch.randn(256, 1024, device=DEV).to(dtype)
+    x, dy = rows.repeat(9, 1)[:2200].requires_grad_(True), dy_rows.repeat(9, 1)[:2200]
+    y = layer(x)
+    dx, = torch.autograd.grad(y, x, dy)
+    w = dense_weight(layer.weight, layer.matrix.backward_indices, 1024).abs()
+    unit, tiny = UNIT[dtype], 2.0**-24 if dtype == torch.float16 else 0.0
+    for got, magnitude in ((y.detach().double(), rows.double().abs() @ w.t()), (dx.double(), dy_rows.double().abs() @ w)):
+        bound = 2 * (1024 + 16) * 2.0**-23 * magnitude * (1 + unit) + 2 * tiny
+        for tile in range(1, 9):
+            part = got[256 * tile:256 * (tile + 1)]
+            worst = (part - got[:len(part)]).abs() - bound[:len(part)] - 2 * unit * got[:len(part)].abs() * (1 + unit)
+            assert worst.max().item() <= 0.0, (tile, worst.max().item())
