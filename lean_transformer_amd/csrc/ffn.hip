@@ -209,8 +209,9 @@ int linear_forward_impl(const lt_linear& lin, int64_t T, int dtype, const void* 
     // workgroup.  Where the layout lets the product run on 256 x 256 tiles instead (runs of output blocks with a shared
     // list), that and a separate activation pass are faster than the paired walk for a large product: its 256 x 64 tiles read the
     // operands more often, which costs more than the second pass once they no longer stay in the caches.  Stretched butterfly, the
-    // two passes and the walk, us: hidden 1024, T 4096 (pre-activation 64 MiB) 72 and 63; 2048, 4096 (128 MiB) 145 and 131; 4096,
-    // 2000 (125 MiB) 146 and 143; 4096, 4096 (256 MiB) 329 and 341.
+    // two passes and the walk, us: hidden 1024, T 4096 (pre-activation 64 MiB) 63 and 55; 2048, 4096 (128 MiB) 131 and 116; 4096,
+    // 2000 (125 MiB) 156 and 151; 4096, 2560 (160 MiB) 168 and 155; 4096, 4096 with rank 128 (256 MiB) 296 and 303.  Between the last
+    // two the walk is ahead up to some size (4096, 3072 (192 MiB) 198 and 189): the line is where it was drawn for a slower epilogue.
     GemmProblem s = p;
     s.N = out;
     s.epi = epi_store_params(epi.pre, epi.ld_pre, dtype, epi.bias);

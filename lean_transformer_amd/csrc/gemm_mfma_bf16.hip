@@ -71,7 +71,8 @@ template <typename F> double best_slices(int64_t M, int64_t N, int64_t tiles, in
   return best_us;
 }
 // 128 x 128 tiles: 64 k take a workgroup 0.45 us alone on its CU, two of them 0.95 us (measured on [128 - 4096, 2048] over 8192: 53 - 69
-// us for up to 256 workgroups, 125 for 512)
+// us for up to 256 workgroups, 125 for 512).  The main loop that copies between the matrix instructions takes 44 - 68 and 130 there; the
+// estimates, and those of mid_selected, are still the older loop's, which leave a product to the other kernel a little too soon.
 double mid_best(int64_t M, int64_t N, int64_t K, int& slices, double one = 0.45, double two = 0.95) {
   return best_slices(M, N, mid_tiles(M, N), (K + 63) / 64, 512, [=](int64_t w) { return w <= 256 ? one : two; }, slices);
 }

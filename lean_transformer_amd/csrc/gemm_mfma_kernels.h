@@ -96,11 +96,6 @@ template <int READS, int MFMAS, int G = 0> struct SchedInterleave {
   }
 };
 
-// SP != SPARSE_NONE: block-sparse walk with 64 x 64 blocks (see SparseWalk).  Each 64-wide k-step is one active block; its
-// operand tiles are fetched through the index tables, so nothing is gathered or scattered in HBM.  tiles_n then counts
-// groups: output blocks (FWD, tile 256 x 64), input blocks (DX, tile 256 x 64), or (input block, four of its active
-// output blocks) (DW, tile 256 x 64: four gathered dY column blocks against one X column block, reduced over tokens;
-// the four weight-gradient blocks are adjacent in the native [in_blocks, A, 64, 64] order).
 // f(std::integral_constant<int, 0>{}), ..., f(std::integral_constant<int, N - 1>{})
 template <typename F, int... Is> __device__ __forceinline__ void lt_static_for_impl(F& f, std::integer_sequence<int, Is...>) {
   (f(std::integral_constant<int, Is>{}), ...);
@@ -109,6 +104,9 @@ template <int N, typename F> __device__ __forceinline__ void lt_static_for(F&& f
   lt_static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+// SP == SPARSE_DW: block-sparse weight gradient with 64 x 64 blocks, reduced over the tokens.  tiles_n counts groups (input block, four of
+// its active output blocks): four gathered dY column blocks against one X column block, fetched through the index tables; the four
+// weight-gradient blocks are adjacent in the native [in_blocks, A, 64, 64] order.
 // PF: how many k-steps ahead of the matrix instructions the operand tiles are requested (in registers; the LDS holds two
 // stages whatever PF is).  1 for the MFMA-bound uses; the rank-r products stream a large operand once against a small one and
 // are bound by how many bytes a CU has in flight, so they ask further ahead.

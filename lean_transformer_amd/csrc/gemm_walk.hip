@@ -69,7 +69,10 @@ void gemm_walk_kernel(GemmProblem p, int tiles_m, int groups) {
 
   // Entry of the list taken at step t (SparseWalk::walk_run).  Token tiles start an eighth of the list apart: the rows of an activation
   // block lie a power of two apart, on few memory channels, and the tiles of one block column would ask for theirs at the same
-  // time.  hidden 4096, T 4096, all from the first entry against this: down-projection 108 us, 103; dh 248, 240; du 154, 150.
+  // time.  hidden 4096, T 4096, all from the first entry against this: down-projection 108 us, 103; dh 248, 240; du 154, 150; both products
+  // of a tiled butterfly's forward pass 434, 404.  The price: a row's terms are added in an order that depends on the tile it is in, so
+  // that equal rows may differ in their last bits from tile to tile (the dense kernels' staggered walks do the same).  Starts that go
+  // by the block column instead would not, and measured 459 for the 404.
   const int first = (tm & 7) * steps / 8;
   auto walk_entry = [&](int t) __attribute__((always_inline)) {
     t += first;

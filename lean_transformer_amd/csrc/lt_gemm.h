@@ -44,7 +44,8 @@ struct EpiParams {
   DropoutParams drop;
 };
 
-// Block-sparse operand walk (any-shape kernel only).  Workgroups with the same blockIdx.y form one group:
+// Block-sparse operands.  Any-shape kernel: workgroups with the same blockIdx.y form one group; the matrix-core kernels for 64 x 64 blocks
+// (gemm_walk.hip, launch_sparse) read the same tables.
 //   SPARSE_FWD  group = output block ob:  Y[:, ob] = sum_k X[:, ib_k] W4[ib_k, a_k]^T,  forward_indices[ob, k] = ib_k * A + a_k
 //   SPARSE_DX   group = input block ib:   dX[:, ib] = sum_a dY[:, ob_a] W4[ib, a],       ob_a = backward_indices[ib, a]
 //   SPARSE_DW   group = weight block (ib, a): dW4[ib, a] = dY[:, ob_a]^T X[:, ib]

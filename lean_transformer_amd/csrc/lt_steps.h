@@ -9,8 +9,7 @@
 #endif
 
 // Each segment takes ceil(k / step) k-steps of its own, the second's after the first's; the last of a segment is ragged where step
-// does not divide its length.  Number of leading steps that are whole (k1 == 0: one segment).  k0 counts as whole steps where a
-// block-sparse walk gives the first segment's, whose blocks are one step each.
+// does not divide its length.  Number of leading steps that are whole (k1 == 0: one segment).
 LT_HOST_DEVICE inline int lt_leading_whole_steps(int64_t k0, int64_t k1, int step) {
   const int first = (int)((k0 + step - 1) / step);
   if (k0 % step != 0) return first - 1;
