@@ -312,7 +312,8 @@ class _GeneralizedLinear(torch.autograd.Function):
         tokens = x.shape[0]
         grads = nat.LtLinearGrads()
         # straight in the type autograd hands on: fp32 from the accumulators where the tensors are fp32 (autocast)
-        dx_dtype, grad_dtype = _result_dtype(dtype, input), _result_dtype(dtype, main_weight, lowrank_first, lowrank_second)
+        dx_dtype = input.dtype if input.dtype == torch.float32 else dtype
+        grad_dtype = _result_dtype(dtype, main_weight, lowrank_first, lowrank_second)
         dx = torch.empty_like(x, dtype=dx_dtype) if need[0] else None
         dw = torch.empty_like(w, dtype=grad_dtype) if need[1] else None
         db = torch.empty(desc.out_features, dtype=torch.float32, device=device) if (ctx._has_bias and need[2]) else None
@@ -322,10 +323,12 @@ class _GeneralizedLinear(torch.autograd.Function):
                                                                                nat.ptr(dl2))
         if tokens > 0:
             lib = nat.lib(dtype)
-            ws = nat.workspace(lib.lt_linear_backward_workspace_bytes(desc, tokens, nat.dtype_code(dtype)), device)
-            nat.check(lib.lt_linear_backward_to(desc, tokens, nat.dtype_code(dtype), nat.ptr(x), nat.ptr(dy), nat.ptr(hid),
-                                                nat.dtype_code(dx_dtype), nat.ptr(dx), grads, nat.dtype_code(grad_dtype),
-                                                nat.ptr(ws), ws.numel(), nat.current_stream(device)),
+            code = nat.dtype_code(dtype)
+            ws = nat.workspace(lib.lt_linear_backward_workspace_bytes(desc, tokens, code), device)
+            nat.check(lib.lt_linear_backward_to(desc, tokens, code, nat.ptr(x), nat.ptr(dy), nat.ptr(hid),
+                                                code if dx_dtype == dtype else nat.LT_F32, nat.ptr(dx), grads,
+                                                code if grad_dtype == dtype else nat.LT_F32, nat.ptr(ws), ws.numel(),
+                                                nat.current_stream(device)),
                       "lt_linear_backward_to", lib)
         else:
             for g in (dw, db, dl1, dl2):
