@@ -484,43 +484,10 @@ __global__ void colreduce_kernel(int rows, int64_t stride, int cols, const float
 // same, 16 row lanes x 16 column lanes of 4 columns per workgroup: short dependent chains, 16-byte loads, eight of them in flight (the
 // adds stay in row order).  Latency bounds it: with one load at a time the two sums of a LayerNorm backward's 256 partial rows took
 // longer than its two kernels' 64 had: [4096, 768] 23 us in all, 15 with eight in flight (two kernels and 64 rows: 21).
-__global__ __launch_bounds__(256) void colreduce4_kernel(int rows, int64_t stride, int cols, const float* __restrict__ partial,
-                                                         float* __restrict__ out) {
+__device__ __forceinline__ void colreduce4_block(const ColReduceJob& job, unsigned block) {
   __shared__ float red[16][16][5];
   const int cl = threadIdx.x & 15, rl = threadIdx.x >> 4;
-  const int c = (blockIdx.x * 16 + cl) * 4;
-  float s[4] = {0.f, 0.f, 0.f, 0.f};
-  if (c < cols) {
-#pragma unroll 8
-    for (int r = rl; r < rows; r += 16) {
-      float v[4];
-      load4(partial + (int64_t)r * stride + c, v);
-#pragma unroll
-      for (int e = 0; e < 4; e++) s[e] += v[e];
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < 4; e++) red[rl][cl][e] = s[e];
-  __syncthreads();
-  if (rl == 0 && c < cols) {
-    float o[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      o[e] = 0.f;
-#pragma unroll
-      for (int q = 0; q < 16; q++) o[e] += red[q][cl][e];
-    }
-    store4(out + c, o);
-  }
-}
-
-// several such sums in one launch: blockIdx.y picks the job; the same arithmetic in the same order as colreduce4_kernel
-__global__ __launch_bounds__(256) void colreduce4_multi_kernel(ColReduceQueue q) {
-  __shared__ float red[16][16][5];
-  const ColReduceJob& job = q.job[blockIdx.y];
-  const int cl = threadIdx.x & 15, rl = threadIdx.x >> 4;
-  const int c = (blockIdx.x * 16 + cl) * 4;
-  if (blockIdx.x * 64 >= job.cols) return;  // (the whole workgroup)
+  const int c = (block * 16 + cl) * 4;
   float s[4] = {0.f, 0.f, 0.f, 0.f};
   if (c < job.cols) {
 #pragma unroll 8
@@ -540,10 +507,58 @@ __global__ __launch_bounds__(256) void colreduce4_multi_kernel(ColReduceQueue q)
     for (int e = 0; e < 4; e++) {
       o[e] = 0.f;
 #pragma unroll
-      for (int k = 0; k < 16; k++) o[e] += red[k][cl][e];
+      for (int q = 0; q < 16; q++) o[e] += red[q][cl][e];
     }
     store4(job.out + c, o);
   }
+}
+__global__ __launch_bounds__(256) void colreduce4_kernel(ColReduceJob job) { colreduce4_block(job, blockIdx.x); }
+
+// several such sums in one launch: blockIdx.y picks the job
+__global__ __launch_bounds__(256) void colreduce4_multi_kernel(ColReduceQueue q) {
+  const ColReduceJob& job = q.job[blockIdx.y];
+  if (blockIdx.x * 64 >= job.cols) return;  // (the whole workgroup)
+  colreduce4_block(job, blockIdx.x);
+}
+
+// sum of split-k partial results in slice order, 4 elements at i
+template <typename TO>
+__device__ __forceinline__ void splitk_sum4(const float* __restrict__ partial, int slices, int64_t stride, int64_t i, const float* __restrict__ bias,
+                                            int cols, TO* __restrict__ out) {
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int s = 0; s < slices; s++) {
+    float v[4];
+    load4(partial + (int64_t)s * stride + i, v);
+#pragma unroll
+    for (int e = 0; e < 4; e++) acc[e] += v[e];
+  }
+  if (bias) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) acc[e] += bias[(i + e) % cols];
+  }
+  store4(out + i, acc);
+}
+
+// Everything a queue holds in one launch, where it holds split reductions too: workgroups first[j] .. first[j + 1] - 1 work on job j, the
+// column sums (the longer chains) ahead of the split reductions; same sums in the same order as the kernels for one.  What bounds it: up to
+// a few MiB its launch and one trip to memory, 5 us whatever the job, which is why there is one for all.  Fused qkv with a rank-16 adapter,
+// four launches against one: 346 us, 332; tiled butterfly of hidden 1024, T 4000, rank 64, seven against two: 473, 455.
+struct SumBlocks { unsigned first[2 * ColReduceQueue::MAX]; };
+__global__ __launch_bounds__(256) void deferred_sums_kernel(ColReduceQueue q, SumBlocks blocks) {
+  int j = 0;  // (entries past the last job are the number of workgroups; all read at once, not one behind another)
+#pragma unroll
+  for (int k = 1; k < 2 * ColReduceQueue::MAX; k++) j += blockIdx.x >= blocks.first[k];
+  const unsigned block = blockIdx.x - blocks.first[j];
+  if (j < q.n) {
+    colreduce4_block(q.job[j], block);
+    return;
+  }
+  const SplitSumJob& job = q.split[j - q.n];
+  const int64_t i = ((int64_t)block * 256 + threadIdx.x) * 4;
+  if (i >= job.count) return;
+  if (job.out_dtype == LT_F32) splitk_sum4(job.partial, job.slices, job.stride, i, nullptr, 0, (float*)job.out);
+  else splitk_sum4(job.partial, job.slices, job.stride, i, nullptr, 0, (bf16*)job.out);
 }
 
 // out[c] = sum of `rows` rows of partial: picks the vector kernel when the layout allows; with a queue that has room, the
@@ -556,7 +571,7 @@ static void launch_colreduce(int rows, int64_t stride, int cols, const float* pa
     return;
   }
   if (vec)
-    hipLaunchKernelGGL(colreduce4_kernel, dim3((unsigned)((cols + 63) / 64)), dim3(256), 0, stream, rows, stride, cols, partial, out);
+    hipLaunchKernelGGL(colreduce4_kernel, dim3((unsigned)((cols + 63) / 64)), dim3(256), 0, stream, ColReduceJob{partial, out, rows, cols, stride});
   else
     hipLaunchKernelGGL(colreduce_kernel, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, stream, rows, stride, cols, partial, out);
 }
@@ -765,24 +780,12 @@ __global__ void dropout_mask_kernel(int64_t n, uint8_t* __restrict__ keep, Dropo
   keep[idx] = drop.p > 0.f ? (dropout_keep(drop, idx) ? 1 : 0) : 1;
 }
 
-// sum of split-k partial results in slice order, 4 elements per thread
+// 4 elements per thread
 template <typename TO>
 __global__ void splitk_reduce_kernel(const float* __restrict__ partial, int slices, int64_t stride, int64_t count, int cols,
                                      const float* __restrict__ bias, TO* __restrict__ out) {
   const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (i >= count) return;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < slices; s++) {
-    float v[4];
-    load4(partial + (int64_t)s * stride + i, v);
-#pragma unroll
-    for (int e = 0; e < 4; e++) acc[e] += v[e];
-  }
-  if (bias) {
-#pragma unroll
-    for (int e = 0; e < 4; e++) acc[e] += bias[(i + e) % cols];
-  }
-  store4(out + i, acc);
+  if (i < count) splitk_sum4(partial, slices, stride, i, bias, cols, out);
 }
 
 inline unsigned blocks_for(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
@@ -1197,10 +1200,26 @@ int lt_dropout_mask_launch(int64_t n, uint8_t* keep, const DropoutParams& drop, 
   return LT_OK;
 }
 
+float* lt_split_partials(void* workspace, size_t bytes, ColReduceQueue*& defer) {
+  bytes = lt_align_up(bytes, 256);
+  if (!defer || defer->n_split == ColReduceQueue::MAX || bytes > defer->room_bytes) {
+    defer = nullptr;
+    return (float*)workspace;
+  }
+  float* partial = (float*)defer->room;
+  defer->room += bytes;
+  defer->room_bytes -= bytes;
+  return partial;
+}
+
 int lt_splitk_reduce(const float* partial, int slices, int64_t stride, int64_t count, int cols, const float* bias,
-                     int out_dtype, void* out, hipStream_t stream) {
+                     int out_dtype, void* out, hipStream_t stream, ColReduceQueue* defer) {
   LT_REQUIRE(partial && out && slices > 0 && count > 0 && (count & 3) == 0 && (stride & 3) == 0, LT_ERR_BAD_ARG,
              "split-k reduce: bad arguments");
+  if (defer && !bias && defer->n_split < ColReduceQueue::MAX) {
+    defer->split[defer->n_split++] = SplitSumJob{partial, out, stride, count, slices, out_dtype};
+    return LT_OK;
+  }
   LtProfileScope scope("splitk_reduce", 0.0, (double)count * (4.0 * slices + lt_dtype_size(out_dtype)), stream);
   dim3 grid(blocks_for(count / 4, 256)), block(256);
   if (out_dtype == LT_F32)
@@ -1236,16 +1255,29 @@ int lt_widen(const WidenJobs& jobs, hipStream_t stream) {
 }
 
 int lt_colreduce_flush(ColReduceQueue& queue, hipStream_t stream) {
-  if (queue.n == 0) return LT_OK;
-  int blocks = 1;
+  if (queue.n + queue.n_split == 0) return LT_OK;
+  SumBlocks blocks;
+  unsigned total = 0, widest = 1;
   double bytes = 0.0;
+  int j = 0;
   for (int i = 0; i < queue.n; i++) {
-    blocks = std::max(blocks, (queue.job[i].cols + 63) / 64);
+    const unsigned n = (unsigned)((queue.job[i].cols + 63) / 64);
+    blocks.first[j++] = total;
+    total += n;
+    widest = std::max(widest, n);
     bytes += (double)queue.job[i].cols * 4.0 * (queue.job[i].rows + 1);
   }
-  LtProfileScope scope("colreduce", 0.0, bytes, stream);
-  hipLaunchKernelGGL(colreduce4_multi_kernel, dim3((unsigned)blocks, (unsigned)queue.n), dim3(256), 0, stream, queue);
-  queue.n = 0;
+  for (int i = 0; i < queue.n_split; i++) {
+    blocks.first[j++] = total;
+    total += blocks_for(queue.split[i].count / 4, 256);
+    bytes += (double)queue.split[i].count * (4.0 * queue.split[i].slices + lt_dtype_size(queue.split[i].out_dtype));
+  }
+  while (j < 2 * ColReduceQueue::MAX) blocks.first[j++] = total;
+  LtProfileScope scope(queue.n_split ? "splitk_reduce" : "colreduce", 0.0, bytes, stream);
+  // (column sums alone: a job per row of the grid, which saves a dependent read at the start of each workgroup, 5.5 us against 4.3)
+  if (queue.n_split) hipLaunchKernelGGL(deferred_sums_kernel, dim3(total), dim3(256), 0, stream, queue, blocks);
+  else hipLaunchKernelGGL(colreduce4_multi_kernel, dim3(widest, (unsigned)queue.n), dim3(256), 0, stream, queue);
+  queue.n = queue.n_split = 0;
   LT_LAUNCH_CHECK();
   return LT_OK;
 }

@@ -257,6 +257,25 @@ void plan_linear_backward(const lt_linear& lin, int64_t T, int dtype, Bump& ws, 
   s.skinny = s.skinny_bytes ? ws.take(s.skinny_bytes) : nullptr;
 }
 
+// Room for the partial results of the split weight and low-rank gradients of a layer, to be summed with others in one launch: at most
+// 32 MiB, an upper bound (up to 16 slices) where that is less.  Larger results gain nothing by waiting and are no longer in the caches then:
+// fused qkv over 16384 tokens with room for none 346 us, 8 MiB 337, 32 MiB 332, 128 MiB 336; tiled butterfly of hidden 1024 473, -, 455,
+// 455; GPT layer (57 and 66 MiB a result) 999, -, 999, 1003.
+constexpr size_t SUM_ROOM = (size_t)32 << 20;
+size_t deferred_sum_room(const lt_linear& lin, int64_t T, int dtype) {
+  const int64_t in = lin.in_features, out = lin.out_features;
+  size_t bytes = (size_t)16 * lin.lowrank * (in + out) * sizeof(float) + 3 * 256;
+  if (lin.block == 0) {
+    size_t dw = lt_gemm_generic_splitk_workspace(out, in, T);
+    if (dtype == LT_BF16) dw = std::max({dw, lt_gemm_splitk_workspace(out, in, T), lt_gemm_mid_splitk_workspace(out, in, T)});
+    bytes += dw;
+  } else if (lin.block == 64 && dtype == LT_BF16) {
+    bytes += lt_sparse_dw_split_workspace(in, out, lin.blocks_per_in, lin.blocks_per_out, group_length(lin.in_group),
+                                          group_length(lin.out_group), T);
+  }
+  return bytes > SUM_ROOM ? SUM_ROOM : bytes;
+}
+
 // gradient side of one generalized linear layer.  The input-gradient GEMM runs FIRST, through epilogue `kind_dx`
 // (EPI_ACT_BWD for the down-projection, whose epilogue also re-materialises this layer's own input `x_act`), then the
 // parameter gradients, which may therefore read x_act.  Pass kind_dx < 0 to skip the input gradient.
@@ -315,7 +334,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
       p.A[0] = operand(dy, out, false);
       p.B[0] = operand(x_act, in, false);
       p.epi = epi_store_params(grads.weight, in, grad_dtype, nullptr);
-      LT_TRY(lt_launch_gemm_skinny(p, dtype, io_dtype, s.skinny, s.skinny_bytes, stream));
+      LT_TRY(lt_launch_gemm_skinny(p, dtype, io_dtype, s.skinny, s.skinny_bytes, stream, defer));
     } else {
       p.M = lin.block; p.N = in; p.K[0] = T;
       p.sp.mode = SPARSE_DW; p.sp.block = lin.block; p.sp.blocks_per_out = lin.blocks_per_out;
@@ -332,11 +351,13 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
         // the reduction over the tokens split over workgroups: fp32 partial gradients, summed into the parameter's dtype
         p.ksplit = slices;
         p.split_stride = (int64_t)elements;
-        p.epi.out = s.skinny;
+        ColReduceQueue* later = defer;
+        float* const partial = lt_split_partials(s.skinny, (size_t)slices * elements * sizeof(float), later);
+        p.epi.out = partial;
         p.epi.out_dtype = LT_F32;
         LT_TRY(lt_launch_gemm_sparse(p, EPI_STORE, dtype, io_dtype, stream));
-        LT_TRY(lt_splitk_reduce((const float*)s.skinny, slices, (int64_t)elements, (int64_t)elements, lin.block, nullptr, grad_dtype,
-                                grads.weight, stream));
+        LT_TRY(lt_splitk_reduce(partial, slices, (int64_t)elements, (int64_t)elements, lin.block, nullptr, grad_dtype, grads.weight,
+                                stream, later));
       } else {
         // no room for the partial sums: runs of output blocks unsplit, runs of input blocks as the walk
         if (slices > 1 && !lt_sparse_dw_out_grouped(p)) p.sp.in_group = 0;
@@ -351,7 +372,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
     q.A[0] = operand(dy, out, false);
     q.B[0] = operand(lowrank_hid, r, false);
     q.epi = epi_store_params(grads.lowrank_second, r, grad_dtype, nullptr);
-    LT_TRY(lt_launch_gemm_skinny(q, dtype, io_dtype, s.skinny, s.skinny_bytes, stream));
+    LT_TRY(lt_launch_gemm_skinny(q, dtype, io_dtype, s.skinny, s.skinny_bytes, stream, defer));
   }
   if (r > 0 && grads.lowrank_first) {  // dL1[r, in] = g_hid^T x
     GemmProblem q = blank_problem();
@@ -359,7 +380,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
     q.A[0] = operand(s.g_hid, r, false);
     q.B[0] = operand(x_act, in, false);
     q.epi = epi_store_params(grads.lowrank_first, in, grad_dtype, nullptr);
-    LT_TRY(lt_launch_gemm_skinny(q, dtype, io_dtype, s.skinny, s.skinny_bytes, stream));
+    LT_TRY(lt_launch_gemm_skinny(q, dtype, io_dtype, s.skinny, s.skinny_bytes, stream, defer));
   }
   return LT_OK;
 }
@@ -456,6 +477,8 @@ struct BwdScratch {
   float* vectors;     // 16-bit LayerNorm parameters in fp32
   float* act_colsum;  // [ceil(T / 64), N1]: partial column sums of dpre from the epilogue that writes it
   LinearBwdScratch h2o, i2h;
+  void* sums;  // partial results of split gradients that are summed at the end of the step
+  size_t sum_bytes;
 };
 
 void plan_backward(const lt_ffn_desc& d, Bump& ws, BwdScratch& s) {
@@ -476,6 +499,8 @@ void plan_backward(const lt_ffn_desc& d, Bump& ws, BwdScratch& s) {
   s.act_colsum = (float*)ws.take((size_t)((T + 63) / 64) * n1 * sizeof(float));
   plan_linear_backward(d.h2o, T, d.compute_dtype, ws, s.h2o);
   plan_linear_backward(d.i2h, T, d.compute_dtype, ws, s.i2h);
+  s.sum_bytes = std::min(SUM_ROOM, deferred_sum_room(d.h2o, T, d.compute_dtype) + deferred_sum_room(d.i2h, T, d.compute_dtype));
+  s.sums = ws.take(s.sum_bytes);
 }
 
 }  // namespace
@@ -573,10 +598,11 @@ extern "C" int lt_ffn_backward_to(const lt_ffn_desc* desc, const void* x, const 
   const int cdt = d.compute_dtype, io = d.io_dtype;
   const DropoutParams drop = make_dropout(d.dropout_p, d.dropout_seed, d.dropout_offset);
 
-  // the small column sums at the end of three passes (two bias gradients, the LayerNorm parameter gradients) wait for one
-  // launch at the end of the step
+  // the sums at the end of several passes (bias, LayerNorm parameter, split weight and low-rank gradients) wait for one launch at the
+  // end of the step
   ColReduceQueue reduces;
-  reduces.n = 0;
+  reduces.room = (char*)s.sums;
+  reduces.room_bytes = s.sum_bytes;
   // gradient entering the down-projection: dropout replayed on dy, then (optionally) back through the post-LN
   const void* g = s.g;
   lt_linear_grads h2o_grads = grads->h2o;
@@ -639,6 +665,7 @@ extern "C" size_t lt_linear_backward_workspace_bytes(const lt_linear* lin, int64
   Bump ws(nullptr);
   LinearBwdScratch s;
   plan_linear_backward(*lin, tokens, dtype, ws, s);
+  ws.take(deferred_sum_room(*lin, tokens, dtype));
   return lt_align_up(ws.used, 256);
 }
 
@@ -673,9 +700,13 @@ extern "C" int lt_linear_backward_to(const lt_linear* lin, int64_t tokens, int32
   Bump ws(workspace);
   LinearBwdScratch s;
   plan_linear_backward(*lin, tokens, dtype, ws, s);
+  ColReduceQueue reduces;
+  reduces.room_bytes = deferred_sum_room(*lin, tokens, dtype);
+  reduces.room = (char*)ws.take(reduces.room_bytes);
   EpiParams e = epi_store_params(dx, lin->in_features, dx_dtype, nullptr);
-  return linear_backward_impl(*lin, tokens, dtype, x, dy, lowrank_hid, dx ? EPI_STORE : -1, e, *grads, grad_dtype, s, dtype,
-                              (hipStream_t)stream);
+  LT_TRY(linear_backward_impl(*lin, tokens, dtype, x, dy, lowrank_hid, dx ? EPI_STORE : -1, e, *grads, grad_dtype, s, dtype,
+                              (hipStream_t)stream, nullptr, nullptr, &reduces));
+  return lt_colreduce_flush(reduces, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------

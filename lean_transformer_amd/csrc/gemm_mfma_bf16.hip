@@ -212,23 +212,25 @@ size_t lt_gemm_generic_splitk_workspace(int64_t M, int64_t N, int64_t K) {
 }
 
 int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
-                          hipStream_t stream) {
+                          hipStream_t stream, ColReduceQueue* defer) {
   if (lt_gemm_stream_supported(p, EPI_STORE, dtype, io_dtype)) return lt_launch_gemm_stream(p, EPI_STORE, dtype, io_dtype, stream);
   const bool a_km = p.A[0].kmajor, b_km = p.B[0].kmajor;
   const EpiParams& e = p.epi;
+  if (e.bias) defer = nullptr;
+  const size_t slice = (size_t)p.M * (size_t)p.N * sizeof(float);
   if (dtype == LT_BF16 && e.ldo == p.N && mid_selected(p, EPI_STORE, workspace ? workspace_bytes : 0)) {
-    const size_t slice = (size_t)p.M * (size_t)p.N * sizeof(float);
     const int slices = (int)std::min<size_t>((size_t)mid_slices(p.M, p.N, p.K[0]), workspace ? workspace_bytes / slice : 0);
     if (slices <= 1) return lt_launch_gemm(p, EPI_STORE, dtype, io_dtype, stream);
     GemmProblem q = p;
     q.ksplit = slices;
     q.split_stride = p.M * p.N;
     q.epi = EpiParams{};
-    q.epi.out = workspace;
+    float* const partial = lt_split_partials(workspace, slices * slice, defer);
+    q.epi.out = partial;
     q.epi.ldo = p.N;
     q.epi.out_dtype = LT_F32;
     LT_TRY(lt_launch_gemm(q, EPI_STORE, dtype, io_dtype, stream));
-    return lt_splitk_reduce((const float*)workspace, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream);
+    return lt_splitk_reduce(partial, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream, defer);
   }
   bool ok = dtype == LT_BF16 && p.nseg == 1 && p.sp.mode == SPARSE_NONE && p.M > 0 && p.N > 0 && p.N % 128 == 0 &&
             !(!a_km && b_km) && (a_km || p.M % 128 == 0) && ((!a_km && !b_km) || p.K[0] % 8 == 0) && p.K[0] > 0 &&
@@ -241,18 +243,18 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
   if (!half_tiles && dtype == LT_BF16 && p.sp.mode == SPARSE_NONE && lt_gemm_mfma_supported(p, EPI_STORE)) {
     // 256 x 256 tiles fit: the copy-based kernel, its reduction split when the tiles alone leave CUs idle
     const int slices = p.nseg == 1 ? splitk_slices(p.M, p.N, p.K[0]) : 1;
-    const size_t need = (size_t)slices * (size_t)p.M * (size_t)p.N * sizeof(float);
-    if (slices > 1 && workspace && workspace_bytes >= need && dma_selected(p, EPI_STORE) && e.ldo == p.N) {
+    if (slices > 1 && workspace && workspace_bytes >= slices * slice && dma_selected(p, EPI_STORE) && e.ldo == p.N) {
       GemmProblem q = p;
       q.ksplit = slices;
       q.variant = 2;
       q.split_stride = p.M * p.N;
-      q.epi.out = workspace;
+      float* const partial = lt_split_partials(workspace, slices * slice, defer);
+      q.epi.out = partial;
       q.epi.ldo = p.N;
       q.epi.out_dtype = LT_F32;
       q.epi.bias = nullptr;
       LT_TRY(lt_launch_gemm(q, EPI_STORE, dtype, io_dtype, stream));
-      return lt_splitk_reduce((const float*)workspace, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream);
+      return lt_splitk_reduce(partial, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream, defer);
     }
     if (((p.M + 255) / 256) * ((p.N + 255) / 256) >= 64 || slices == 1) ok = false;
   }
@@ -262,15 +264,16 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
     const int slices = (!tiled && p.nseg == 1 && p.sp.mode == SPARSE_NONE && e.ldo == p.N && (p.N & 3) == 0 &&
                         lt_aligned(e.out, 16) && (!e.bias || lt_aligned(e.bias, 16)))
                            ? generic_splitk_slices(p.M, p.N, p.K[0]) : 1;
-    if (slices > 1 && workspace && workspace_bytes >= (size_t)slices * (size_t)p.M * (size_t)p.N * sizeof(float)) {
+    if (slices > 1 && workspace && workspace_bytes >= slices * slice) {
       GemmProblem q = p;
       q.ksplit = slices;
       q.split_stride = p.M * p.N;
-      q.epi.out = workspace;
+      float* const partial = lt_split_partials(workspace, slices * slice, defer);
+      q.epi.out = partial;
       q.epi.out_dtype = LT_F32;
       q.epi.bias = nullptr;
       LT_TRY(lt_launch_gemm_generic(q, EPI_STORE, dtype, io_dtype, stream));
-      return lt_splitk_reduce((const float*)workspace, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream);
+      return lt_splitk_reduce(partial, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream, defer);
     }
     return lt_launch_gemm(p, EPI_STORE, dtype, io_dtype, stream);
   }
@@ -282,14 +285,15 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
     // slices the partial sums cost more than the second workgroup hides -- measured on [4096, 128] results)
     const int64_t workgroups = tiles <= 64 ? 256 : 512;
     slices = (int)std::min<int64_t>(std::min<int64_t>(workgroups / tiles, kt_total / 4), SKINNY_MAX_SLICES);
-    const int64_t fit = (int64_t)(workspace_bytes / ((size_t)p.M * (size_t)p.N * sizeof(float)));
+    const int64_t fit = (int64_t)(workspace_bytes / slice);
     slices = (int)std::max<int64_t>(1, std::min<int64_t>(slices, fit));
   }
   GemmProblem q = p;
+  float* partial = nullptr;
   if (slices > 1) {
     q.ksplit = slices;
     q.split_stride = p.M * p.N;
-    q.epi.out = workspace;
+    q.epi.out = partial = lt_split_partials(workspace, slices * slice, defer);
     q.epi.out_dtype = LT_F32;
     q.epi.bias = nullptr;
   }
@@ -298,7 +302,7 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
     const int status = lt_mfma_launch_skinny(q, slices, stream);
     if (status != LT_OK || slices == 1) return status;
   }
-  return lt_splitk_reduce((const float*)workspace, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream);
+  return lt_splitk_reduce(partial, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream, defer);
 }
 
 namespace {

@@ -488,26 +488,39 @@ size_t lt_gemm_generic_splitk_workspace(int64_t M, int64_t N, int64_t K);
 // rows per partial row of EpiParams::colsum when lt_launch_gemm / lt_launch_gemm_sparse sends this EPI_ACT_BWD problem to a
 // kernel that fills it (128: copy-based dense kernel; 64: 128 x 128 tiles, block-sparse walk); 0: it will not
 int lt_gemm_colsum_rows(const GemmProblem& p, int dtype, int io_dtype);
-// Column sums of partial rows that may wait: a caller that runs several passes with such a tail (the FFN backward: two bias
-// gradients and the LayerNorm parameter gradients) hands the same queue to each of them and flushes it once, one launch
-// for all sums instead of one each.  The partial rows must stay untouched until the flush.
+// Sums that may wait: column sums of partial rows (bias and LayerNorm parameter gradients) and the partial results of split
+// reductions (weight and low-rank gradients).  A caller that runs several passes with such a tail (the backward of a layer or of the whole
+// block) hands the same queue to each of them and flushes it once: one launch for all sums instead of one each.  Partial rows and partial
+// results must stay untouched until the flush; the latter get their place from the queue's own `room`, what does not fit is summed at once.
 struct ColReduceJob {
   const float* partial;
   float* out;
   int rows, cols;
   int64_t stride;
 };
+struct SplitSumJob {
+  const float* partial;  // slice s at partial + s * stride
+  void* out;
+  int64_t stride, count;
+  int slices, out_dtype;
+};
 struct ColReduceQueue {
   static constexpr int MAX = 6;
   ColReduceJob job[MAX];
-  int n;
+  SplitSumJob split[MAX];
+  int n = 0, n_split = 0;
+  char* room = nullptr;  // 256-byte aligned
+  size_t room_bytes = 0;
 };
 int lt_colreduce_flush(ColReduceQueue& queue, hipStream_t stream);
 // out[c] = sum over `rows` partial rows of partial[r * stride + c] (now, or at the flush of `defer`)
 int lt_colreduce(int rows, int64_t stride, int cols, const float* partial, float* out, hipStream_t stream,
                  ColReduceQueue* defer = nullptr);
+// Where a split reduction of `bytes` leaves its partial results: in the room of `defer`, if that has it and a job left, else in
+// `workspace`; `defer` becomes null then.
+float* lt_split_partials(void* workspace, size_t bytes, ColReduceQueue*& defer);
 int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
-                          hipStream_t stream);
+                          hipStream_t stream, ColReduceQueue* defer = nullptr);
 // EPI_OUT problems with few output tiles and a long reduction (the down-projection of a short batch): the reduction split
 // over workgroups into fp32 partial sums in `workspace`, then one pass that sums them through the same epilogue.  Takes as
 // many slices as the workspace holds; falls back to lt_launch_gemm when the shape does not fit or one slice is enough.
@@ -515,8 +528,9 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
 size_t lt_gemm_out_splitk_workspace(int dtype, int64_t M, int64_t N, int64_t K, size_t cap_bytes);
 int lt_launch_gemm_out(const GemmProblem& p, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
                        hipStream_t stream);
-// out[i] = sum_s partial[s * stride + i] (+ bias[i % cols]) for i < count, cast to out_dtype
+// out[i] = sum_s partial[s * stride + i] (+ bias[i % cols]) for i < count, cast to out_dtype (now, or without a bias at the flush of
+// `defer`, which lt_split_partials took the partial results' place from)
 int lt_splitk_reduce(const float* partial, int slices, int64_t stride, int64_t count, int cols, const float* bias,
-                     int out_dtype, void* out, hipStream_t stream);
+                     int out_dtype, void* out, hipStream_t stream, ColReduceQueue* defer = nullptr);
 // picks the tiled kernel when it applies and dtype is bf16, else the any-shape kernel
 int lt_launch_gemm(const GemmProblem& p, int kind, int dtype, int io_dtype, hipStream_t stream);

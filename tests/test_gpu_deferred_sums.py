@@ -1,0 +1,51 @@
+"""Sums that wait for one launch at the end of a backward pass: split weight and low-rank gradients, bias gradients, in room for all of
+them, for some of them, and where nothing is split."""
+import pytest
+import torch
+
+import lean_transformer_amd as lt
+from lean_transformer_amd.blocksparse.linear import GeneralizedMatrix, GeneralizedLinear
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("tokens,fan_in,fan_out,rank,bias", [
+    (1, 8, 8, 0, True),          # nothing split, one column sum
+    (257, 64, 72, 8, True),      # one tile a product
+    (4099, 768, 320, 16, True),  # every gradient split, all in the room
+    (4099, 768, 320, 16, False),
+    (4096, 1536, 2048, 64, True),   # a weight gradient of more than the room, summed at once, beside low-rank ones that wait
+    (2051, 1003, 517, 5, True),     # sizes off every tile: the any-shape kernel's splits
+])
+@pytest.mark.parametrize("compute", ["autocast", "fp32"])
+def test_gradients_summed_at_the_end(tokens, fan_in, fan_out, rank, bias, compute):
+    torch.manual_seed(tokens + fan_in)
+    layer = GeneralizedLinear(GeneralizedMatrix(fan_in, fan_out), adapter_dim=rank, bias=bias).to(DEV)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.copy_(torch.randn_like(p).bfloat16() * 0.125)
+    x = torch.randn(tokens, fan_in, device=DEV).bfloat16().float().requires_grad_(True)
+    dy = torch.randn(tokens, fan_out, device=DEV).bfloat16().float()
+    half = compute == "autocast"
+    with torch.autocast("cuda", torch.bfloat16, enabled=half):
+        y = layer(x)
+    names, params = zip(*layer.named_parameters())
+    first = torch.autograd.grad(y, params, dy.to(y.dtype), retain_graph=True)
+    again = torch.autograd.grad(y, params, dy.to(y.dtype))
+    xd, dyd = x.detach().double(), dy.double()
+    for name, g, g2 in zip(names, first, again):
+        assert torch.equal(g, g2), name
+        if name.endswith("weight"):  # exact operands, fp32 sums: the worst case of a sum over the tokens
+            ref, room = dyd.t() @ xd, dyd.abs().t() @ xd.abs()
+        elif name == "bias":
+            ref, room = dyd.sum(0), dyd.abs().sum(0)
+        else:
+            r1, r2 = layer.adapter_first.detach().double(), layer.adapter_second.detach().double()
+            hid, g_hid = xd @ r1.t(), dyd @ r2
+            pair = (dyd, hid) if name == "adapter_second" else (g_hid, xd)
+            ref, room = pair[0].t() @ pair[1], pair[0].abs().t() @ pair[1].abs()
+            if half:  # the other factor was rounded to bfloat16 (2^-9 of each term)
+                assert ((g.double() - ref).abs() <= 2.0**-8 * room + 1e-30).all(), name
+                continue
+        assert ((g.double() - ref).abs() <= (tokens + fan_in + 64) * 2.0**-23 * room + 1e-30).all(), name
