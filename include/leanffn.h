@@ -124,7 +124,8 @@ typedef struct lt_ffn_desc {
   float ln_eps;
   float dropout_p;        /* 0 disables dropout (also pass 0 in eval mode) */
   int32_t vector_dtype;   /* lt_dtype of the small vectors below (LayerNorm parameters, i2h.bias, h2o.bias): LT_F32, or
-                             compute_dtype (the float pointers then hold 16-bit elements): one kernel widens them into the workspace.  Gradients of them are fp32 */
+                             compute_dtype (the float pointers then hold 16-bit elements): read as they are, or widened into the workspace.
+                             Gradients of them are fp32 unless lt_ffn_backward_typed is told otherwise */
   uint64_t dropout_seed;  /* Philox key */
   uint64_t dropout_offset;/* Philox stream offset; forward and backward of one call must pass the same pair */
   const float* ln_weight; /* [H] vector_dtype (as the next three) */
@@ -170,6 +171,11 @@ int lt_ffn_backward(const lt_ffn_desc* desc, const void* x, const void* dy, cons
 /* the same with the weight and low-rank gradients in grad_dtype: the compute dtype, or LT_F32 (then unrounded) */
 int lt_ffn_backward_to(const lt_ffn_desc* desc, const void* x, const void* dy, const lt_ffn_saved* saved,
                        const lt_ffn_grads* grads, int32_t grad_dtype, void* workspace, size_t workspace_bytes, void* stream);
+/* the same with the gradients of the small vectors (LayerNorm parameters, biases) in vector_grad_dtype: LT_F32, or the compute dtype (the
+ * float pointers then take 16-bit elements, the fp32 sums rounded once) */
+int lt_ffn_backward_typed(const lt_ffn_desc* desc, const void* x, const void* dy, const lt_ffn_saved* saved,
+                          const lt_ffn_grads* grads, int32_t grad_dtype, int32_t vector_grad_dtype, void* workspace,
+                          size_t workspace_bytes, void* stream);
 
 /* ---- generalized linear: y = x W^T (+ bias) (+ (x L1^T) L2^T) ------------------------------------------------------- */
 size_t lt_linear_backward_workspace_bytes(const lt_linear* lin, int64_t tokens, int32_t dtype);

@@ -23,7 +23,7 @@ EXPORTED_SYMBOLS = (
     "lt_version", "lt_last_error",
     "lt_ffn_forward_workspace_bytes", "lt_ffn_backward_workspace_bytes", "lt_ffn_forward", "lt_ffn_backward",
     "lt_linear_backward_workspace_bytes", "lt_linear_forward", "lt_linear_backward",
-    "lt_linear_backward_to", "lt_ffn_backward_to", "lt_linear_check_out_group", "lt_linear_check_in_group",
+    "lt_linear_backward_to", "lt_ffn_backward_to", "lt_ffn_backward_typed", "lt_linear_check_out_group", "lt_linear_check_in_group",
     "lt_blocksparse_forward", "lt_blocksparse_backward",
     "lt_layernorm_forward", "lt_layernorm_backward_workspace_bytes", "lt_layernorm_backward",
     "lt_layernorm_backward_static_scratch_bytes", "lt_layernorm_backward_static",
@@ -92,6 +92,8 @@ def _declare(lib):
                                        POINTER(LtLinearGrads), c_void_p, c_size_t, c_void_p]
     lib.lt_ffn_backward_to.argtypes = [POINTER(LtFfnDesc), c_void_p, c_void_p, POINTER(LtFfnSaved), POINTER(LtFfnGrads),
                                        c_int32, c_void_p, c_size_t, c_void_p]
+    lib.lt_ffn_backward_typed.argtypes = [POINTER(LtFfnDesc), c_void_p, c_void_p, POINTER(LtFfnSaved), POINTER(LtFfnGrads),
+                                          c_int32, c_int32, c_void_p, c_size_t, c_void_p]
     lib.lt_linear_backward_to.argtypes = [POINTER(LtLinear), c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_void_p,
                                           POINTER(LtLinearGrads), c_int32, c_void_p, c_size_t, c_void_p]
     lib.lt_blocksparse_forward.argtypes = [POINTER(LtLinear), c_int64, c_int32, c_void_p, c_void_p, c_void_p]

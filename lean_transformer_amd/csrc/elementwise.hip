@@ -14,13 +14,38 @@ static int ln_vectors_per_lane(int H) { return H <= 2048 ? 8 : H <= 4096 ? 16 : 
 // ---------------------------------------------------------------------------------------------------------------------
 // LayerNorm forward: one wavefront per row.  The row is read once into registers (when hidden % 4 == 0 and it fits), the
 // mean and the centred second moment are reduced across the 64 lanes with shuffles, and the normalised row is written in
-// the GEMM operand dtype.  TAIL fuses what follows a post-LayerNorm: dropout, then the residual add.
+// the GEMM operand dtype.  TAIL fuses what follows a post-LayerNorm: dropout, then the residual add.  Weight and bias come in TW, as the
+// module holds them, and workgroups behind those of the rows widen the biases of the products to come: a launch of their own for these few
+// kilobytes took 2.5 - 4 us and the host's time for it (with the trips to memory overlapped: eight tokens, hidden 768 44.6 us, 42.0; a prompt of 512, hidden 2048 63.5, 60.9).
 // ---------------------------------------------------------------------------------------------------------------------
-template <typename TX, typename TY, typename TR, bool TAIL, int MAXV>
+__device__ __forceinline__ void widen_block(const WidenJobs& jobs, int block) {
+  for (int j = 0; j < jobs.n; j++) {
+    const int blocks = (jobs.count[j] + 1023) / 1024;
+    if (block < blocks) {
+      const bf16* in = reinterpret_cast<const bf16*>(jobs.in[j]);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int i = block * 1024 + e * 256 + (int)threadIdx.x;
+        if (i < jobs.count[j]) jobs.out[j][i] = (float)in[i];
+      }
+      return;
+    }
+    block -= blocks;
+  }
+}
+
+template <typename TX, typename TY, typename TR, typename TW, bool TAIL, int MAXV>
 __global__ __launch_bounds__(256) void ln_fwd_kernel(int64_t T, int H, float eps, const TX* __restrict__ x,
-                                                      const float* __restrict__ w, const float* __restrict__ b,
+                                                      const TW* __restrict__ w, const TW* __restrict__ b,
                                                       TY* __restrict__ y, float* __restrict__ stats,
-                                                      const TR* __restrict__ residual, DropoutParams drop, int vec) {
+                                                      const TR* __restrict__ residual, DropoutParams drop, int vec, WidenJobs jobs) {
+  if (jobs.n > 0) {
+    const int64_t row_blocks = (T + 3) / 4;
+    if (blockIdx.x >= row_blocks) {
+      widen_block(jobs, (int)(blockIdx.x - row_blocks));
+      return;
+    }
+  }
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= T) return;
@@ -110,7 +135,7 @@ __global__ __launch_bounds__(256) void ln_fwd_kernel(int64_t T, int H, float eps
     rstd = 1.0f / sqrtf(wave_sum(q) * inv_h + eps);
     if (y) {
       for (int c = lane; c < H; c += 64) {
-        float o = (ldf(xr, c) - mean) * rstd * w[c] + b[c];
+        float o = (ldf(xr, c) - mean) * rstd * ldf(w, c) + ldf(b, c);
         if constexpr (TAIL) {
           if (drop.p > 0.f) o = dropout_keep(drop, row * H + c) ? o * drop.scale : 0.f;
           if (residual) o += ldf(residual, row * H + c);
@@ -355,7 +380,7 @@ __global__ __launch_bounds__(256) void ln_bwd_param_kernel(int64_t T, int H, con
 // both stay with the two kernels.
 template <typename TX, typename TDX, int WPR>
 __global__ __launch_bounds__(1024) void ln_bwd_rows_kernel(int64_t T, int H, const TX* __restrict__ x,
-                                                            const float* __restrict__ stats, const float* __restrict__ w,
+                                                            const float* __restrict__ stats, const void* __restrict__ w, int w_half,
                                                             const bf16* __restrict__ dy, const TDX* __restrict__ residual_grad,
                                                             TDX* __restrict__ dx, float* __restrict__ partial) {
   constexpr int GROUPS = 16 / WPR;
@@ -367,7 +392,7 @@ __global__ __launch_bounds__(1024) void ln_bwd_rows_kernel(int64_t T, int H, con
   __shared__ float2 row_sums[2][16];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int group = wave / WPR, col0 = (wave % WPR) * 1024 + lane * 4;  // this lane's columns: col0 + 256 i .. + 3
-  for (int c = threadIdx.x; c < H; c += 1024) w_lds[c] = w[c];
+  for (int c = threadIdx.x; c < H; c += 1024) w_lds[c] = w_half ? (float)reinterpret_cast<const bf16*>(w)[c] : reinterpret_cast<const float*>(w)[c];
   __syncthreads();
 
   X4 x_next[4];
@@ -472,13 +497,13 @@ __global__ __launch_bounds__(1024) void ln_bwd_rows_kernel(int64_t T, int H, con
 }
 
 // out[c] = sum_r partial[r * stride + c], one thread per column (rows are few)
-__global__ void colreduce_kernel(int rows, int64_t stride, int cols, const float* __restrict__ partial,
-                                 float* __restrict__ out) {
+__global__ void colreduce_kernel(ColReduceJob job) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
+  if (c >= job.cols) return;
   float s = 0.f;
-  for (int r = 0; r < rows; r++) s += partial[(int64_t)r * stride + c];
-  out[c] = s;
+  for (int r = 0; r < job.rows; r++) s += job.partial[(int64_t)r * job.stride + c];
+  if (job.out_dtype == LT_F32) reinterpret_cast<float*>(job.out)[c] = s;
+  else reinterpret_cast<bf16*>(job.out)[c] = (bf16)s;
 }
 
 // same, 16 row lanes x 16 column lanes of 4 columns per workgroup: short dependent chains, 16-byte loads, eight of them in flight (the
@@ -509,7 +534,8 @@ __device__ __forceinline__ void colreduce4_block(const ColReduceJob& job, unsign
 #pragma unroll
       for (int q = 0; q < 16; q++) o[e] += red[q][cl][e];
     }
-    store4(job.out + c, o);
+    if (job.out_dtype == LT_F32) store4(reinterpret_cast<float*>(job.out) + c, o);
+    else store4(reinterpret_cast<bf16*>(job.out) + c, o);
   }
 }
 __global__ __launch_bounds__(256) void colreduce4_kernel(ColReduceJob job) { colreduce4_block(job, blockIdx.x); }
@@ -563,17 +589,14 @@ __global__ __launch_bounds__(256) void deferred_sums_kernel(ColReduceQueue q, Su
 
 // out[c] = sum of `rows` rows of partial: picks the vector kernel when the layout allows; with a queue that has room, the
 // vector form waits for the queue's flush
-static void launch_colreduce(int rows, int64_t stride, int cols, const float* partial, float* out, hipStream_t stream,
-                             ColReduceQueue* defer = nullptr) {
-  const bool vec = (cols & 3) == 0 && (stride & 3) == 0 && lt_aligned(partial, 16) && lt_aligned(out, 16);
-  if (vec && defer && defer->n < ColReduceQueue::MAX) {
-    defer->job[defer->n++] = ColReduceJob{partial, out, rows, cols, stride};
-    return;
-  }
-  if (vec)
-    hipLaunchKernelGGL(colreduce4_kernel, dim3((unsigned)((cols + 63) / 64)), dim3(256), 0, stream, ColReduceJob{partial, out, rows, cols, stride});
-  else
-    hipLaunchKernelGGL(colreduce_kernel, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, stream, rows, stride, cols, partial, out);
+static bool colreduce_vec(const ColReduceJob& job) {
+  return (job.cols & 3) == 0 && (job.stride & 3) == 0 && lt_aligned(job.partial, 16) && lt_aligned(job.out, 16);
+}
+static void launch_colreduce(const ColReduceJob& job, hipStream_t stream, ColReduceQueue* defer = nullptr) {
+  const bool vec = colreduce_vec(job);
+  if (vec && defer && defer->n < ColReduceQueue::MAX) defer->job[defer->n++] = job;
+  else if (vec) hipLaunchKernelGGL(colreduce4_kernel, dim3((unsigned)((job.cols + 63) / 64)), dim3(256), 0, stream, job);
+  else hipLaunchKernelGGL(colreduce_kernel, dim3((unsigned)((job.cols + 255) / 256)), dim3(256), 0, stream, job);
 }
 
 
@@ -795,43 +818,57 @@ inline unsigned blocks_for(int64_t n, int threads) { return (unsigned)((n + thre
 // ---------------------------------------------------------------------------------------------------------------------
 // host-side launchers
 // ---------------------------------------------------------------------------------------------------------------------
-int lt_ln_forward(int64_t T, int H, float eps, int x_dtype, const void* x, const float* w, const float* b, int y_dtype,
+int lt_ln_forward(int64_t T, int H, float eps, int x_dtype, const void* x, int w_dtype, const void* w, const void* b, int y_dtype,
                   void* y, float* stats, int res_dtype, const void* residual, const DropoutParams* drop, bool tail,
-                  hipStream_t stream) {
+                  hipStream_t stream, const WidenJobs* widen) {
   LT_REQUIRE(T > 0 && H > 0 && x, LT_ERR_BAD_ARG, "layernorm: bad arguments");
   LT_REQUIRE(!y || (w && b), LT_ERR_BAD_ARG, "layernorm: weight and bias are required when an output is requested");
   // rows are held in registers and moved 4 elements at a time when the size and every pointer allow it
   int vec = (H & 3) == 0 && H <= 64 * 4 * LN_MAXV && lt_aligned(x, 16) && (!y || lt_aligned(y, 16)) &&
             (!w || lt_aligned(w, 16)) && (!b || lt_aligned(b, 16)) && (!residual || lt_aligned(residual, 16));
   if (vec && (H & 7) == 0) vec = 2;  // 8 elements per lane per piece: 16-byte stores of a bf16 output
-  dim3 grid(blocks_for(T, 4)), block(256);
+  WidenJobs jobs;
+  jobs.n = 0;
+  if (widen) jobs = *widen;
+  unsigned blocks = blocks_for(T, 4);
+  for (int i = 0; i < jobs.n; i++) blocks += blocks_for(jobs.count[i], 1024);
+  dim3 grid(blocks), block(256);
   DropoutParams d = drop ? *drop : make_dropout(0.f, 0, 0);
   LtProfileScope scope(tail ? "layernorm_fwd_tail" : (y ? "layernorm_fwd" : "layernorm_stats"), 0.0,
                        (double)T * H * (lt_dtype_size(x_dtype) + (y ? lt_dtype_size(y_dtype) : 0) +
                                         (residual ? lt_dtype_size(res_dtype) : 0)) + (stats ? 8.0 * T : 0.0),
                        stream);
   const int maxv = ln_vectors_per_lane(H);
-#define LT_LN_LAUNCH_V(TX, TY, TR, TAILV, MAXV)                                                                             \
-  hipLaunchKernelGGL((ln_fwd_kernel<TX, TY, TR, TAILV, MAXV>), grid, block, 0, stream, T, H, eps, (const TX*)x, w, b, (TY*)y, \
-                     stats, (const TR*)residual, d, vec)
-#define LT_LN_LAUNCH(TX, TY, TR, TAILV)                     \
-  do {                                                      \
-    if (maxv == 8) LT_LN_LAUNCH_V(TX, TY, TR, TAILV, 8);    \
-    else if (maxv == 16) LT_LN_LAUNCH_V(TX, TY, TR, TAILV, 16); \
-    else LT_LN_LAUNCH_V(TX, TY, TR, TAILV, 32);             \
+#define LT_LN_LAUNCH_V(TX, TY, TR, TW, TAILV, MAXV)                                                                        \
+  hipLaunchKernelGGL((ln_fwd_kernel<TX, TY, TR, TW, TAILV, MAXV>), grid, block, 0, stream, T, H, eps, (const TX*)x, (const TW*)w, \
+                     (const TW*)b, (TY*)y, stats, (const TR*)residual, d, vec, jobs)
+#define LT_LN_LAUNCH(TX, TY, TR, TW, TAILV)                         \
+  do {                                                              \
+    if (maxv == 8) LT_LN_LAUNCH_V(TX, TY, TR, TW, TAILV, 8);        \
+    else if (maxv == 16) LT_LN_LAUNCH_V(TX, TY, TR, TW, TAILV, 16); \
+    else LT_LN_LAUNCH_V(TX, TY, TR, TW, TAILV, 32);                 \
   } while (0)
+  // (16-bit parameters come with a 16-bit compute type: the type of y, after a down-projection that of x)
   if (!tail) {
-    if (x_dtype == LT_F32 && y_dtype == LT_F32) LT_LN_LAUNCH(float, float, float, false);
-    else if (x_dtype == LT_F32) LT_LN_LAUNCH(float, bf16, float, false);
-    else if (y_dtype == LT_F32) LT_LN_LAUNCH(bf16, float, float, false);
-    else LT_LN_LAUNCH(bf16, bf16, float, false);
+    if (w_dtype == LT_BF16) {
+      LT_REQUIRE(y_dtype == LT_BF16, LT_ERR_BAD_ARG, "layernorm: 16-bit parameters with an fp32 output");
+      if (x_dtype == LT_F32) LT_LN_LAUNCH(float, bf16, float, bf16, false);
+      else LT_LN_LAUNCH(bf16, bf16, float, bf16, false);
+    } else if (x_dtype == LT_F32 && y_dtype == LT_F32) LT_LN_LAUNCH(float, float, float, float, false);
+    else if (x_dtype == LT_F32) LT_LN_LAUNCH(float, bf16, float, float, false);
+    else if (y_dtype == LT_F32) LT_LN_LAUNCH(bf16, float, float, float, false);
+    else LT_LN_LAUNCH(bf16, bf16, float, float, false);
   } else {
     // post-LayerNorm tail: input in the compute dtype, output and residual in the io dtype (res_dtype == y_dtype)
     LT_REQUIRE(res_dtype == y_dtype, LT_ERR_BAD_ARG, "layernorm tail: residual and output dtypes differ");
-    if (x_dtype == LT_F32 && y_dtype == LT_F32) LT_LN_LAUNCH(float, float, float, true);
-    else if (x_dtype == LT_F32) LT_LN_LAUNCH(float, bf16, bf16, true);
-    else if (y_dtype == LT_F32) LT_LN_LAUNCH(bf16, float, float, true);
-    else LT_LN_LAUNCH(bf16, bf16, bf16, true);
+    if (w_dtype == LT_BF16) {
+      LT_REQUIRE(x_dtype == LT_BF16, LT_ERR_BAD_ARG, "layernorm tail: 16-bit parameters with an fp32 input");
+      if (y_dtype == LT_F32) LT_LN_LAUNCH(bf16, float, float, bf16, true);
+      else LT_LN_LAUNCH(bf16, bf16, bf16, bf16, true);
+    } else if (x_dtype == LT_F32 && y_dtype == LT_F32) LT_LN_LAUNCH(float, float, float, float, true);
+    else if (x_dtype == LT_F32) LT_LN_LAUNCH(float, bf16, bf16, float, true);
+    else if (y_dtype == LT_F32) LT_LN_LAUNCH(bf16, float, float, float, true);
+    else LT_LN_LAUNCH(bf16, bf16, bf16, float, true);
   }
 #undef LT_LN_LAUNCH
 #undef LT_LN_LAUNCH_V
@@ -860,10 +897,10 @@ size_t lt_ln_backward_workspace(int64_t T, int H) {
   return (size_t)rows * 2 * (size_t)H * sizeof(float);
 }
 
-int lt_ln_backward(int64_t T, int H, int x_dtype, const void* x, const float* stats, const float* w, int dy_dtype,
-                   const void* dy, int dx_dtype, const void* residual_grad, void* dx, float* dweight, float* dbias,
-                   void* workspace, size_t workspace_bytes, hipStream_t stream, ColReduceQueue* defer) {
-  LT_REQUIRE(T > 0 && H > 0 && x && stats && w && dy, LT_ERR_BAD_ARG, "layernorm backward: bad arguments");
+int lt_ln_backward(int64_t T, int H, int x_dtype, const void* x, const float* stats, int w_dtype, const void* w_any, float* w_room,
+                   int dy_dtype, const void* dy, int dx_dtype, const void* residual_grad, void* dx, int dw_dtype, void* dweight,
+                   void* dbias, void* workspace, size_t workspace_bytes, hipStream_t stream, ColReduceQueue* defer) {
+  LT_REQUIRE(T > 0 && H > 0 && x && stats && w_any && dy, LT_ERR_BAD_ARG, "layernorm backward: bad arguments");
   LT_REQUIRE((dweight == nullptr) == (dbias == nullptr), LT_ERR_BAD_ARG, "layernorm backward: pass both dweight and dbias or neither");
   float* partial = dweight ? (float*)workspace : nullptr;
   LtProfileScope scope("layernorm_bwd", 0.0,
@@ -871,7 +908,7 @@ int lt_ln_backward(int64_t T, int H, int x_dtype, const void* x, const float* st
                            (double)T * H * ((dx ? lt_dtype_size(dx_dtype) : 0) + (dx && residual_grad ? lt_dtype_size(dx_dtype) : 0)),
                        stream);
   const int key = (x_dtype == LT_BF16) * 4 + (dy_dtype == LT_BF16) * 2 + (dx_dtype == LT_BF16);
-  const bool vec = (H & 3) == 0 && H <= 64 * 4 * LN_MAXV && lt_aligned(x, 16) && lt_aligned(dy, 16) && lt_aligned(w, 16) &&
+  const bool vec = (H & 3) == 0 && H <= 64 * 4 * LN_MAXV && lt_aligned(x, 16) && lt_aligned(dy, 16) && lt_aligned(w_any, 16) &&
                    (!dx || lt_aligned(dx, 16)) && (!residual_grad || lt_aligned(residual_grad, 16)) &&
                    (!partial || lt_aligned(partial, 16));
   const bool wide = H > 256 * LNB_MAXC;  // wider than the register-resident kernels take
@@ -886,11 +923,17 @@ int lt_ln_backward(int64_t T, int H, int x_dtype, const void* x, const float* st
     LT_REQUIRE(workspace && workspace_bytes >= need, LT_ERR_WORKSPACE,
                "layernorm backward: %zu bytes of scratch needed for the parameter gradients, %zu given", need, workspace_bytes);
   }
+  const float* w = (const float*)w_any;
+  if (!one_pass && w_dtype != LT_F32) {  // the other kernels read the weight once a row: in fp32
+    LT_REQUIRE(w_room, LT_ERR_BAD_ARG, "layernorm backward: no room for the weight in fp32");
+    LT_TRY(lt_widen(WidenJobs{{w_any}, {w_room}, {H}, 1}, stream));
+    w = w_room;
+  }
   if (one_pass) {
     dim3 grid((unsigned)partial_rows), block(1024);
     const int wpr = ln_rows_wavefronts(H);
 #define LT_LNB_ROWS_W(TX, TDX, WPR)                                                                                             \
-  hipLaunchKernelGGL((ln_bwd_rows_kernel<TX, TDX, WPR>), grid, block, 0, stream, T, H, (const TX*)x, stats, w, (const bf16*)dy, \
+  hipLaunchKernelGGL((ln_bwd_rows_kernel<TX, TDX, WPR>), grid, block, 0, stream, T, H, (const TX*)x, stats, (const void*)w_any, (int)(w_dtype == LT_BF16), (const bf16*)dy, \
                      (const TDX*)residual_grad, (TDX*)dx, partial)
 #define LT_LNB_ROWS(TX, TDX)                      \
   do {                                            \
@@ -1003,8 +1046,8 @@ int lt_ln_backward(int64_t T, int H, int x_dtype, const void* x, const float* st
   }
   if (dweight) {
     // partial rows alternate (dweight, dbias): stride 2 * H between them
-    launch_colreduce(partial_rows, (int64_t)2 * H, H, partial, dweight, stream, defer);
-    launch_colreduce(partial_rows, (int64_t)2 * H, H, partial + H, dbias, stream, defer);
+    launch_colreduce(ColReduceJob{partial, dweight, partial_rows, H, (int64_t)2 * H, dw_dtype}, stream, defer);
+    launch_colreduce(ColReduceJob{partial + H, dbias, partial_rows, H, (int64_t)2 * H, dw_dtype}, stream, defer);
     LT_LAUNCH_CHECK();
   }
   return LT_OK;
@@ -1061,8 +1104,8 @@ extern "C" int lt_layernorm_backward_static(int64_t tokens, int32_t hidden, int3
                (int)LT_F32, (int)LT_BF16);
   void* ptr = nullptr;
   if (dweight) LT_TRY(static_scratch_for(stream, &ptr));
-  const int status = lt_ln_backward(tokens, hidden, x_dtype, x, stats, weight, dy_dtype, dy, dx_dtype, residual_grad, dx,
-                                    dweight, dbias, ptr, LT_LN_STATIC_SCRATCH_BYTES, stream);
+  const int status = lt_ln_backward(tokens, hidden, x_dtype, x, stats, LT_F32, weight, nullptr, dy_dtype, dy, dx_dtype, residual_grad, dx,
+                                    LT_F32, dweight, dbias, ptr, LT_LN_STATIC_SCRATCH_BYTES, stream);
   if (status == LT_ERR_WORKSPACE)
     LT_FAIL(LT_ERR_UNSUPPORTED,
             "layernorm backward (static scratch): tokens=%lld hidden=%d needs more than the %zu-byte static buffer "
@@ -1080,7 +1123,7 @@ static int colsum_slices(int64_t rows) {
 
 size_t lt_colsum_workspace(int64_t rows, int cols) { return (size_t)colsum_slices(rows) * (size_t)cols * sizeof(float); }
 
-int lt_colsum(int64_t rows, int cols, int64_t ld, int dtype, const void* in, float* out, void* workspace,
+int lt_colsum(int64_t rows, int cols, int64_t ld, int dtype, const void* in, void* out, int sum_dtype, void* workspace,
               size_t workspace_bytes, hipStream_t stream, ColReduceQueue* defer) {
   LT_REQUIRE(rows > 0 && cols > 0 && in && out, LT_ERR_BAD_ARG, "colsum: bad arguments");
   LT_REQUIRE(workspace && workspace_bytes >= lt_colsum_workspace(rows, cols), LT_ERR_WORKSPACE,
@@ -1102,7 +1145,7 @@ int lt_colsum(int64_t rows, int cols, int64_t ld, int dtype, const void* in, flo
     else
       hipLaunchKernelGGL((colsum_partial_kernel<bf16>), grid, block, 0, stream, rows, cols, ld, (const bf16*)in, rps, partial);
   }
-  launch_colreduce(slices, (int64_t)cols, cols, partial, out, stream, defer);
+  launch_colreduce(ColReduceJob{partial, out, slices, cols, (int64_t)cols, sum_dtype}, stream, defer);
   LT_LAUNCH_CHECK();
   return LT_OK;
 }
@@ -1166,14 +1209,14 @@ int lt_dropout_cast(int64_t n, int in_dtype, const void* in, int out_dtype, void
 
 // lt_dropout_cast of a [rows, cols] tensor plus colsum[c] = sum over rows of the result; workspace as for lt_colsum
 int lt_dropout_cast_colsum(int64_t rows, int cols, int in_dtype, const void* in, int out_dtype, void* out,
-                           const DropoutParams& drop, float* colsum, void* workspace, size_t workspace_bytes,
+                           const DropoutParams& drop, void* colsum, int sum_dtype, void* workspace, size_t workspace_bytes,
                            hipStream_t stream, ColReduceQueue* defer) {
   LT_REQUIRE(rows > 0 && cols > 0 && in && out && colsum, LT_ERR_BAD_ARG, "dropout + column sums: bad arguments");
   LT_REQUIRE(workspace && workspace_bytes >= lt_colsum_workspace(rows, cols), LT_ERR_WORKSPACE,
              "dropout + column sums: workspace of %zu bytes needed", lt_colsum_workspace(rows, cols));
   if ((cols & 7) != 0 || !lt_aligned(in, 16) || !lt_aligned(out, 16) || !lt_aligned(workspace, 16)) {
     LT_TRY(lt_dropout_cast(rows * cols, in_dtype, in, out_dtype, out, drop, stream));
-    return lt_colsum(rows, cols, cols, out_dtype, out, colsum, workspace, workspace_bytes, stream, defer);
+    return lt_colsum(rows, cols, cols, out_dtype, out, colsum, sum_dtype, workspace, workspace_bytes, stream, defer);
   }
   LtProfileScope scope("dropout_replay_cast", 0.0, (double)rows * cols * (lt_dtype_size(in_dtype) + lt_dtype_size(out_dtype)),
                        stream);
@@ -1188,7 +1231,7 @@ int lt_dropout_cast_colsum(int64_t rows, int cols, int in_dtype, const void* in,
     case 2: hipLaunchKernelGGL((dropout_cast_colsum_kernel<bf16, float>), grid, block, 0, stream, rows, cols, (const bf16*)in, (float*)out, drop, rps, partial); break;
     default: hipLaunchKernelGGL((dropout_cast_colsum_kernel<bf16, bf16>), grid, block, 0, stream, rows, cols, (const bf16*)in, (bf16*)out, drop, rps, partial); break;
   }
-  launch_colreduce(slices, (int64_t)cols, cols, partial, colsum, stream, defer);
+  launch_colreduce(ColReduceJob{partial, colsum, slices, cols, (int64_t)cols, sum_dtype}, stream, defer);
   LT_LAUNCH_CHECK();
   return LT_OK;
 }
@@ -1231,25 +1274,19 @@ int lt_splitk_reduce(const float* partial, int slices, int64_t stride, int64_t c
 }
 
 namespace {
-// 4 elements per thread, blockIdx.y picks the vector.  A few ten kilobytes: bound by its launch, which is why it is one
-__global__ __launch_bounds__(256) void widen_kernel(WidenJobs jobs) {
-  const int j = blockIdx.y;
-  const bf16* in = reinterpret_cast<const bf16*>(jobs.in[j]);
-  const int base = blockIdx.x * 1024 + threadIdx.x;
-#pragma unroll
-  for (int e = 0; e < 4; e++) {
-    const int i = base + e * 256;
-    if (i < jobs.count[j]) jobs.out[j][i] = (float)in[i];
-  }
-}
+__global__ __launch_bounds__(256) void widen_kernel(WidenJobs jobs) { widen_block(jobs, blockIdx.x); }
 }  // namespace
 
 int lt_widen(const WidenJobs& jobs, hipStream_t stream) {
-  if (jobs.n == 0) return LT_OK;
-  int most = 0;
-  for (int i = 0; i < jobs.n; i++) most = std::max(most, jobs.count[i]);
-  LtProfileScope scope("widen_vectors", 0.0, 6.0 * most * jobs.n, stream);
-  hipLaunchKernelGGL(widen_kernel, dim3((unsigned)((most + 1023) / 1024), (unsigned)jobs.n), dim3(256), 0, stream, jobs);
+  unsigned blocks = 0;
+  double bytes = 0.0;
+  for (int i = 0; i < jobs.n; i++) {
+    blocks += blocks_for(jobs.count[i], 1024);
+    bytes += 6.0 * jobs.count[i];
+  }
+  if (blocks == 0) return LT_OK;
+  LtProfileScope scope("widen_vectors", 0.0, bytes, stream);
+  hipLaunchKernelGGL(widen_kernel, dim3(blocks), dim3(256), 0, stream, jobs);
   LT_LAUNCH_CHECK();
   return LT_OK;
 }
@@ -1282,15 +1319,14 @@ int lt_colreduce_flush(ColReduceQueue& queue, hipStream_t stream) {
   return LT_OK;
 }
 
-int lt_colreduce(int rows, int64_t stride, int cols, const float* partial, float* out, hipStream_t stream,
-                 ColReduceQueue* defer) {
-  LT_REQUIRE(rows > 0 && cols > 0 && partial && out, LT_ERR_BAD_ARG, "colreduce: bad arguments");
-  if (defer && defer->n < ColReduceQueue::MAX && (cols & 3) == 0 && (stride & 3) == 0 && lt_aligned(partial, 16) && lt_aligned(out, 16)) {
-    launch_colreduce(rows, stride, cols, partial, out, stream, defer);
+int lt_colreduce(const ColReduceJob& job, hipStream_t stream, ColReduceQueue* defer) {
+  LT_REQUIRE(job.rows > 0 && job.cols > 0 && job.partial && job.out, LT_ERR_BAD_ARG, "colreduce: bad arguments");
+  if (defer && defer->n < ColReduceQueue::MAX && colreduce_vec(job)) {
+    launch_colreduce(job, stream, defer);
     return LT_OK;
   }
-  LtProfileScope scope("colreduce", 0.0, (double)cols * 4.0 * (rows + 1), stream);
-  launch_colreduce(rows, stride, cols, partial, out, stream);
+  LtProfileScope scope("colreduce", 0.0, (double)job.cols * 4.0 * (job.rows + 1), stream);
+  launch_colreduce(job, stream);
   LT_LAUNCH_CHECK();
   return LT_OK;
 }

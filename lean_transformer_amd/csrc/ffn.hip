@@ -286,7 +286,7 @@ size_t deferred_sum_room(const lt_linear& lin, int64_t T, int dtype) {
 int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void* x_act, const void* dy,
                          const void* lowrank_hid, int kind_dx, const EpiParams& epi_dx, const lt_linear_grads& grads,
                          int grad_dtype, const LinearBwdScratch& s, int io_dtype, hipStream_t stream, float* act_colsum = nullptr,
-                         int* act_colsum_rows = nullptr, ColReduceQueue* defer = nullptr) {
+                         int* act_colsum_rows = nullptr, ColReduceQueue* defer = nullptr, int bias_grad_dtype = LT_F32) {
   const int64_t in = lin.in_features, out = lin.out_features, r = lin.lowrank;
   const bool need_dx = kind_dx >= 0;
   if (r > 0 && (need_dx || grads.lowrank_first)) {  // g_hid = dy L2  [T, r]
@@ -326,7 +326,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
       LT_TRY(lt_launch_gemm_sparse(p, kind_dx, dtype, io_dtype, stream));
     }
   }
-  if (grads.bias) LT_TRY(lt_colsum(T, (int)out, out, dtype, dy, grads.bias, s.colsum, s.colsum_bytes, stream, defer));
+  if (grads.bias) LT_TRY(lt_colsum(T, (int)out, out, dtype, dy, grads.bias, bias_grad_dtype, s.colsum, s.colsum_bytes, stream, defer));
   if (grads.weight) {
     GemmProblem p = blank_problem();
     if (lin.block == 0) {  // dW[out, in] = dy^T x
@@ -412,7 +412,7 @@ struct FwdScratch {
   void* hid;     // [T, I] compute dtype: activation output
   void* skinny;  // split-k partial sums of the low-rank GEMMs
   size_t skinny_bytes;
-  float* vectors;  // 16-bit small vectors in fp32
+  float* vectors;  // room for 16-bit small vectors in fp32
 };
 
 // room for the small vectors of a call in fp32, where they are not (with_biases: the forward pass reads those too); each piece
@@ -424,12 +424,17 @@ float* take_vectors(const lt_ffn_desc& d, Bump& ws, bool with_biases) {
   return (float*)ws.take(elements * sizeof(float));
 }
 
-// fills that room and points the descriptor at it
-int widen_vectors(lt_ffn_desc& d, float* room, bool with_biases, hipStream_t stream) {
+// Points the descriptor's 16-bit small vectors at that room where the kernels take them in fp32: the biases (forward), which `later` lists
+// for the launch that widens them, and LayerNorm parameters that are not 16-byte aligned, widened here.  *ln_dtype: type of the latter then.
+// *spare: H floats left of the room for each LayerNorm.
+int place_vectors(lt_ffn_desc& d, float* room, bool with_biases, WidenJobs& later, int* ln_dtype, float* spare[2], hipStream_t stream) {
+  later.n = 0;
+  *ln_dtype = d.vector_dtype;
+  spare[0] = spare[1] = nullptr;
   if (d.vector_dtype == LT_F32) return LT_OK;
-  WidenJobs jobs;
-  jobs.n = 0;
-  auto widen = [&](const float*& vector, int count) {
+  WidenJobs now;
+  now.n = 0;
+  auto widen = [&](WidenJobs& jobs, const float*& vector, int count) {
     if (!vector) return;
     jobs.in[jobs.n] = vector;
     jobs.out[jobs.n] = room;
@@ -437,15 +442,23 @@ int widen_vectors(lt_ffn_desc& d, float* room, bool with_biases, hipStream_t str
     vector = room;
     room += lt_align_up(count, 64);
   };
-  widen(d.ln_weight, d.hidden);
-  widen(d.ln_bias, d.hidden);
-  widen(d.post_ln_weight, d.hidden);
-  widen(d.post_ln_bias, d.hidden);
   if (with_biases) {
-    widen(d.i2h.bias, d.i2h.out_features);
-    widen(d.h2o.bias, d.h2o.out_features);
+    widen(later, d.i2h.bias, d.i2h.out_features);
+    widen(later, d.h2o.bias, d.h2o.out_features);
   }
-  return lt_widen(jobs, stream);
+  bool aligned = true;
+  for (const float* v : {d.ln_weight, d.ln_bias, d.post_ln_weight, d.post_ln_bias}) aligned = aligned && lt_aligned(v, 16);
+  if (aligned) {
+    spare[0] = room;
+    spare[1] = room + lt_align_up(d.hidden, 64);
+    return LT_OK;
+  }
+  *ln_dtype = LT_F32;
+  widen(now, d.ln_weight, d.hidden);
+  widen(now, d.ln_bias, d.hidden);
+  widen(now, d.post_ln_weight, d.hidden);
+  widen(now, d.post_ln_bias, d.hidden);
+  return lt_widen(now, stream);
 }
 
 void plan_forward(const lt_ffn_desc& d, Bump& ws, FwdScratch& s) {
@@ -474,7 +487,7 @@ struct BwdScratch {
   void* ln_ws;
   size_t ln_ws_bytes;
   void* post_ln_ws;   // the same, post-LN only (both wait for the end of the step)
-  float* vectors;     // 16-bit LayerNorm parameters in fp32
+  float* vectors;     // room for 16-bit LayerNorm parameters in fp32
   float* act_colsum;  // [ceil(T / 64), N1]: partial column sums of dpre from the epilogue that writes it
   LinearBwdScratch h2o, i2h;
   void* sums;  // partial results of split gradients that are summed at the end of the step
@@ -537,13 +550,16 @@ extern "C" int lt_ffn_forward(const lt_ffn_desc* desc, const void* x, void* y, c
   Bump ws(workspace);
   FwdScratch s;
   plan_forward(d, ws, s);
-  LT_TRY(widen_vectors(d, s.vectors, true, stream));
+  WidenJobs biases;
+  int ln_dtype;
+  float* spare[2];
+  LT_TRY(place_vectors(d, s.vectors, true, biases, &ln_dtype, spare, stream));
   const int64_t T = d.tokens, H = d.hidden, I = d.intermediate, N1 = d.gated ? 2 * I : I;
   const int cdt = d.compute_dtype, io = d.io_dtype;
   const DropoutParams drop = make_dropout(d.dropout_p, d.dropout_seed, d.dropout_offset);
 
-  LT_TRY(lt_ln_forward(T, (int)H, d.ln_eps, io, x, d.ln_weight, d.ln_bias, cdt, s.u, saved->ln_stats, io, nullptr,
-                       nullptr, false, stream));
+  LT_TRY(lt_ln_forward(T, (int)H, d.ln_eps, io, x, ln_dtype, d.ln_weight, d.ln_bias, cdt, s.u, saved->ln_stats, io, nullptr,
+                       nullptr, false, stream, &biases));
 
   // up-projection + activation
   {
@@ -558,7 +574,7 @@ extern "C" int lt_ffn_forward(const lt_ffn_desc* desc, const void* x, void* y, c
   if (d.post_ln_weight) {
     EpiParams e = epi_store_params(saved->post_ln_input, H, cdt, d.h2o.bias);
     LT_TRY(linear_forward_impl(d.h2o, T, cdt, s.hid, EPI_STORE, e, saved->h2o_lowrank_hid, io, stream, s.skinny, s.skinny_bytes));
-    LT_TRY(lt_ln_forward(T, (int)H, d.ln_eps, cdt, saved->post_ln_input, d.post_ln_weight, d.post_ln_bias, io, y, nullptr,
+    LT_TRY(lt_ln_forward(T, (int)H, d.ln_eps, cdt, saved->post_ln_input, ln_dtype, d.post_ln_weight, d.post_ln_bias, io, y, nullptr,
                          io, d.residual ? x : nullptr, &drop, true, stream));
   } else {
     EpiParams e;
@@ -577,12 +593,20 @@ extern "C" int lt_ffn_backward(const lt_ffn_desc* desc, const void* x, const voi
 
 extern "C" int lt_ffn_backward_to(const lt_ffn_desc* desc, const void* x, const void* dy, const lt_ffn_saved* saved,
                                   const lt_ffn_grads* grads, int32_t grad_dtype, void* workspace, size_t workspace_bytes,
-                                  void* stream_) {
+                                  void* stream) {
+  return lt_ffn_backward_typed(desc, x, dy, saved, grads, grad_dtype, LT_F32, workspace, workspace_bytes, stream);
+}
+
+extern "C" int lt_ffn_backward_typed(const lt_ffn_desc* desc, const void* x, const void* dy, const lt_ffn_saved* saved,
+                                     const lt_ffn_grads* grads, int32_t grad_dtype, int32_t vector_grad_dtype, void* workspace,
+                                     size_t workspace_bytes, void* stream_) {
   LT_TRY(check_ffn_desc(desc));
   lt_ffn_desc d = *desc;
   hipStream_t stream = (hipStream_t)stream_;
   LT_REQUIRE(grad_dtype == LT_F32 || grad_dtype == d.compute_dtype, LT_ERR_BAD_ARG,
              "ffn backward: weight gradients in dtype %d, neither fp32 nor the compute dtype", grad_dtype);
+  LT_REQUIRE(vector_grad_dtype == LT_F32 || vector_grad_dtype == d.compute_dtype, LT_ERR_BAD_ARG,
+             "ffn backward: gradients of the small vectors in dtype %d, neither fp32 nor the compute dtype", vector_grad_dtype);
   LT_REQUIRE(x && dy && saved && grads && saved->pre_activation && saved->ln_stats, LT_ERR_BAD_ARG, "ffn backward: null tensor");
   LT_REQUIRE(!d.post_ln_weight || saved->post_ln_input, LT_ERR_BAD_ARG, "ffn backward: post_ln_input missing");
   LT_REQUIRE((grads->ln_weight == nullptr) == (grads->ln_bias == nullptr), LT_ERR_BAD_ARG, "ffn backward: pass both LayerNorm gradients or neither");
@@ -593,7 +617,10 @@ extern "C" int lt_ffn_backward_to(const lt_ffn_desc* desc, const void* x, const 
   Bump ws(workspace);
   BwdScratch s;
   plan_backward(d, ws, s);
-  LT_TRY(widen_vectors(d, s.vectors, false, stream));
+  WidenJobs none;
+  int ln_dtype;
+  float* spare[2];
+  LT_TRY(place_vectors(d, s.vectors, false, none, &ln_dtype, spare, stream));
   const int64_t T = d.tokens, H = d.hidden, I = d.intermediate, N1 = d.gated ? 2 * I : I;
   const int cdt = d.compute_dtype, io = d.io_dtype;
   const DropoutParams drop = make_dropout(d.dropout_p, d.dropout_seed, d.dropout_offset);
@@ -610,17 +637,18 @@ extern "C" int lt_ffn_backward_to(const lt_ffn_desc* desc, const void* x, const 
     g = dy;
   } else if (h2o_grads.bias && !d.post_ln_weight) {
     // the same pass also sums the columns of g: the down-projection's bias gradient
-    LT_TRY(lt_dropout_cast_colsum(T, (int)H, io, dy, cdt, s.g, drop, (float*)h2o_grads.bias, s.h2o.colsum, s.h2o.colsum_bytes,
-                                  stream, &reduces));
+    LT_TRY(lt_dropout_cast_colsum(T, (int)H, io, dy, cdt, s.g, drop, h2o_grads.bias, vector_grad_dtype, s.h2o.colsum,
+                                  s.h2o.colsum_bytes, stream, &reduces));
     h2o_grads.bias = nullptr;
   } else {
     LT_TRY(lt_dropout_cast(T * H, io, dy, cdt, s.g, drop, stream));
   }
   if (d.post_ln_weight) {
-    LT_TRY(lt_ln_forward(T, (int)H, d.ln_eps, cdt, saved->post_ln_input, nullptr, nullptr, cdt, nullptr, s.post_stats, cdt,
+    LT_TRY(lt_ln_forward(T, (int)H, d.ln_eps, cdt, saved->post_ln_input, LT_F32, nullptr, nullptr, cdt, nullptr, s.post_stats, cdt,
                          nullptr, nullptr, false, stream));
-    LT_TRY(lt_ln_backward(T, (int)H, cdt, saved->post_ln_input, s.post_stats, d.post_ln_weight, cdt, g, cdt, nullptr,
-                          s.g_post, grads->post_ln_weight, grads->post_ln_bias, s.post_ln_ws, s.ln_ws_bytes, stream, &reduces));
+    LT_TRY(lt_ln_backward(T, (int)H, cdt, saved->post_ln_input, s.post_stats, ln_dtype, d.post_ln_weight, spare[0], cdt, g, cdt, nullptr,
+                          s.g_post, vector_grad_dtype, grads->post_ln_weight, grads->post_ln_bias, s.post_ln_ws, s.ln_ws_bytes, stream,
+                          &reduces));
     g = s.g_post;
   }
 
@@ -632,27 +660,27 @@ extern "C" int lt_ffn_backward_to(const lt_ffn_desc* desc, const void* x, const 
     e.pre = saved->pre_activation; e.ld_pre = N1; e.dpre = s.dpre; e.hid = s.hid; e.ld_hid = I;
     e.gated = d.gated; e.act = d.act; e.inter = I;
     LT_TRY(linear_backward_impl(d.h2o, T, cdt, s.hid, g, saved->h2o_lowrank_hid, EPI_ACT_BWD, e, h2o_grads, grad_dtype, s.h2o, io,
-                                stream, grads->i2h.bias ? s.act_colsum : nullptr, &bias_rows, &reduces));
+                                stream, grads->i2h.bias ? s.act_colsum : nullptr, &bias_rows, &reduces, vector_grad_dtype));
   }
   lt_linear_grads i2h_grads = grads->i2h;
   if (bias_rows > 0) {  // db1 = column sums of dP, already reduced to one row per bias_rows tokens
-    LT_TRY(lt_colreduce((int)((T + bias_rows - 1) / bias_rows), N1, (int)N1, s.act_colsum, (float*)grads->i2h.bias, stream,
-                        &reduces));
+    LT_TRY(lt_colreduce(ColReduceJob{s.act_colsum, grads->i2h.bias, (int)((T + bias_rows - 1) / bias_rows), (int)N1, N1,
+                                     vector_grad_dtype}, stream, &reduces));
     i2h_grads.bias = nullptr;
   }
 
   // up-projection backward on the recomputed LayerNorm output; du in the compute dtype
-  LT_TRY(lt_ln_forward(T, (int)H, d.ln_eps, io, x, d.ln_weight, d.ln_bias, cdt, s.u, nullptr, io, nullptr, nullptr, false,
+  LT_TRY(lt_ln_forward(T, (int)H, d.ln_eps, io, x, ln_dtype, d.ln_weight, d.ln_bias, cdt, s.u, nullptr, io, nullptr, nullptr, false,
                        stream));
   const bool need_du = grads->dx || grads->ln_weight;
   {
     EpiParams e = epi_store_params(s.du, H, cdt, nullptr);
     LT_TRY(linear_backward_impl(d.i2h, T, cdt, s.u, s.dpre, saved->i2h_lowrank_hid, need_du ? EPI_STORE : -1, e,
-                                i2h_grads, grad_dtype, s.i2h, io, stream, nullptr, nullptr, &reduces));
+                                i2h_grads, grad_dtype, s.i2h, io, stream, nullptr, nullptr, &reduces, vector_grad_dtype));
   }
   if (need_du) {
-    LT_TRY(lt_ln_backward(T, (int)H, io, x, saved->ln_stats, d.ln_weight, cdt, s.du, io, d.residual ? dy : nullptr,
-                          grads->dx, grads->ln_weight, grads->ln_bias, s.ln_ws, s.ln_ws_bytes, stream, &reduces));
+    LT_TRY(lt_ln_backward(T, (int)H, io, x, saved->ln_stats, ln_dtype, d.ln_weight, spare[1], cdt, s.du, io, d.residual ? dy : nullptr,
+                          grads->dx, vector_grad_dtype, grads->ln_weight, grads->ln_bias, s.ln_ws, s.ln_ws_bytes, stream, &reduces));
   }
   return lt_colreduce_flush(reduces, stream);
 }
@@ -754,7 +782,7 @@ extern "C" int lt_layernorm_forward(int64_t tokens, int32_t hidden, float eps, i
                                     void* stream) {
   LT_TRY(check_dtype(x_dtype, "layernorm x"));
   LT_TRY(check_dtype(y_dtype, "layernorm y"));
-  return lt_ln_forward(tokens, hidden, eps, x_dtype, x, weight, bias, y_dtype, y, stats, y_dtype, nullptr, nullptr, false,
+  return lt_ln_forward(tokens, hidden, eps, x_dtype, x, LT_F32, weight, bias, y_dtype, y, stats, y_dtype, nullptr, nullptr, false,
                        (hipStream_t)stream);
 }
 
@@ -770,8 +798,8 @@ extern "C" int lt_layernorm_backward(int64_t tokens, int32_t hidden, int32_t x_d
   LT_TRY(check_dtype(x_dtype, "layernorm backward x"));
   LT_TRY(check_dtype(dy_dtype, "layernorm backward dy"));
   LT_TRY(check_dtype(dx_dtype, "layernorm backward dx"));
-  return lt_ln_backward(tokens, hidden, x_dtype, x, stats, weight, dy_dtype, dy, dx_dtype, residual_grad, dx, dweight,
-                        dbias, workspace, workspace_bytes, (hipStream_t)stream);
+  return lt_ln_backward(tokens, hidden, x_dtype, x, stats, LT_F32, weight, nullptr, dy_dtype, dy, dx_dtype, residual_grad, dx, LT_F32,
+                        dweight, dbias, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 extern "C" int lt_activation_forward(int64_t tokens, int32_t intermediate, int32_t gated, int32_t act, int32_t dtype,

@@ -493,10 +493,11 @@ int lt_gemm_colsum_rows(const GemmProblem& p, int dtype, int io_dtype);
 // block) hands the same queue to each of them and flushes it once: one launch for all sums instead of one each.  Partial rows and partial
 // results must stay untouched until the flush; the latter get their place from the queue's own `room`, what does not fit is summed at once.
 struct ColReduceJob {
-  const float* partial;
-  float* out;
+  const float* partial;  // row r at partial + r * stride
+  void* out;
   int rows, cols;
   int64_t stride;
+  int out_dtype;
 };
 struct SplitSumJob {
   const float* partial;  // slice s at partial + s * stride
@@ -513,9 +514,8 @@ struct ColReduceQueue {
   size_t room_bytes = 0;
 };
 int lt_colreduce_flush(ColReduceQueue& queue, hipStream_t stream);
-// out[c] = sum over `rows` partial rows of partial[r * stride + c] (now, or at the flush of `defer`)
-int lt_colreduce(int rows, int64_t stride, int cols, const float* partial, float* out, hipStream_t stream,
-                 ColReduceQueue* defer = nullptr);
+// out[c] = sum over the partial rows of partial[r * stride + c] (now, or at the flush of `defer`)
+int lt_colreduce(const ColReduceJob& job, hipStream_t stream, ColReduceQueue* defer = nullptr);
 // Where a split reduction of `bytes` leaves its partial results: in the room of `defer`, if that has it and a job left, else in
 // `workspace`; `defer` becomes null then.
 float* lt_split_partials(void* workspace, size_t bytes, ColReduceQueue*& defer);

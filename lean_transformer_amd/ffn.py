@@ -237,7 +237,7 @@ class _LeanFFN(torch.autograd.Function):
         """ctypes descriptor + the converted tensors it points into (which must outlive the call)"""
         act, gated, ln_eps, residual, cdt = ctx._cfg
         p, seed, offset = ctx._dropout
-        # the small vectors: as they are where all are in a 16-bit compute dtype (the library widens them, one launch), else fp32
+        # the small vectors: as they are where all are in a 16-bit compute dtype, else fp32
         keep = [ln_weight, ln_bias, post_ln_weight, post_ln_bias, i2h_bias, h2o_bias]
         vector_dtype = cdt
         if cdt == torch.float32 or not all(v is None or (v.dtype == cdt and v.is_contiguous()) for v in keep):
@@ -292,8 +292,8 @@ class _LeanFFN(torch.autograd.Function):
         need_ln = need[1] or need[2]
         need_post = post_ln_weight is not None and (need[17] or need[18])
         dx = new(x.shape, io, need[0])
-        # the kernels write the gradients of the small vectors in fp32: they share one buffer (256-byte aligned pieces) so
-        # that a single conversion brings them to the parameters' dtype afterwards
+        # the gradients of the small vectors share one buffer (aligned pieces of it).  The kernels write them in the parameters' dtype
+        # where that is the compute dtype for all of them, else in fp32 (a single conversion brings them to another common dtype)
         small_sizes = [hidden if need_ln else 0, hidden if need_ln else 0, hidden if need_post else 0,
                        hidden if need_post else 0, desc.i2h.out_features if i2h_bias is not None and need[4] else 0,
                        hidden if h2o_bias is not None and need[11] else 0]
@@ -301,7 +301,10 @@ class _LeanFFN(torch.autograd.Function):
         for n in small_sizes:
             small_offsets.append(total)
             total += -(-n // 64) * 64
-        small = torch.empty(total, dtype=torch.float32, device=device)
+        small_params = (ln_weight, ln_bias, post_ln_weight, post_ln_bias, i2h_bias, h2o_bias)
+        wanted = {t.dtype for t, n in zip(small_params, small_sizes) if n}
+        vector_dtype = cdt if wanted == {cdt} else torch.float32
+        small = torch.empty(total, dtype=vector_dtype, device=device)
 
         def piece(buffer, i):
             return buffer[small_offsets[i]:small_offsets[i] + small_sizes[i]] if small_sizes[i] else None
@@ -327,16 +330,15 @@ class _LeanFFN(torch.autograd.Function):
                                    nat.ptr(h2o_hid))
             lib = nat.lib(cdt)
             ws = nat.workspace(lib.lt_ffn_backward_workspace_bytes(desc), device)
-            nat.check(lib.lt_ffn_backward_to(desc, nat.ptr(x), nat.ptr(dy), saved, grads, nat.dtype_code(grad_dtype), nat.ptr(ws),
-                                             ws.numel(), nat.current_stream(device)), "lt_ffn_backward_to", lib)
+            nat.check(lib.lt_ffn_backward_typed(desc, nat.ptr(x), nat.ptr(dy), saved, grads, nat.dtype_code(grad_dtype),
+                                                nat.dtype_code(vector_dtype), nat.ptr(ws), ws.numel(), nat.current_stream(device)),
+                      "lt_ffn_backward_typed", lib)
             del ws, keep
         else:
             for g in outputs[1:]:
                 if g is not None:
                     g.zero_()
-        small_params = (ln_weight, ln_bias, post_ln_weight, post_ln_bias, i2h_bias, h2o_bias)
-        wanted = {t.dtype for t, n in zip(small_params, small_sizes) if n}
-        if len(wanted) == 1 and wanted != {torch.float32} and total:
+        if len(wanted) == 1 and wanted != {vector_dtype}:
             converted = small.to(wanted.pop())
             d_ln_w, d_ln_b, d_post_w, d_post_b, d_i2h_b, d_h2o_b = (piece(converted, i) for i in range(6))
         grad_input = None if dx is None else dx.view(*input.shape)
