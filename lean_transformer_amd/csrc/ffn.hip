@@ -518,6 +518,40 @@ void plan_backward(const lt_ffn_desc& d, Bump& ws, BwdScratch& s) {
 
 }  // namespace
 
+namespace {
+// Token-by-token generation: a forward pass of a few rows over dense projections in two launches, the LayerNorm inside the first
+// (gemm_stream.hip) and the small vectors read as they are.  *taken: whether this call is one.  (`hid`: [T, I] scratch)
+int forward_few_rows(const lt_ffn_desc& d, const void* x, void* y, const lt_ffn_saved& saved, void* hid, hipStream_t stream, bool* taken) {
+  const int64_t T = d.tokens, H = d.hidden, I = d.intermediate;
+  const int cdt = d.compute_dtype, io = d.io_dtype;
+  const bool half = d.vector_dtype != LT_F32;
+  *taken = false;
+  if (d.post_ln_weight || d.i2h.block || d.h2o.block || d.i2h.lowrank || d.h2o.lowrank ||
+      !lt_stream_ln_supported(T, H, io, cdt, half) || !lt_aligned(x, 16) || !lt_aligned(d.ln_weight, 16) || !lt_aligned(d.ln_bias, 16) ||
+      !lt_aligned(saved.ln_stats, 8))
+    return LT_OK;
+  GemmProblem up = blank_problem(), down = blank_problem();
+  up.M = T; up.N = I; up.K[0] = H;
+  up.A[0] = operand(x, H, true);
+  up.B[0] = operand(d.i2h.weight, H, true);
+  up.epi.bias = d.i2h.bias; up.epi.pre = saved.pre_activation; up.epi.ld_pre = d.gated ? 2 * I : I; up.epi.hid = hid; up.epi.ld_hid = I;
+  up.epi.gated = d.gated; up.epi.act = d.act; up.epi.inter = I;
+  down.M = T; down.N = H; down.K[0] = I;
+  down.A[0] = operand(hid, I, true);
+  down.B[0] = operand(d.h2o.weight, I, true);
+  down.epi.bias = d.h2o.bias; down.epi.x = d.residual ? x : nullptr; down.epi.y = y; down.epi.ldy = H;
+  down.epi.drop = make_dropout(d.dropout_p, d.dropout_seed, d.dropout_offset);
+  if (!lt_gemm_stream_supported(up, EPI_ACT_FWD, cdt, io) || !lt_gemm_stream_supported(down, EPI_OUT, cdt, io)) return LT_OK;
+  *taken = true;
+  FfnStream first{}, second{};
+  first.bias_half = second.bias_half = half;
+  first.ln_weight = d.ln_weight; first.ln_bias = d.ln_bias; first.ln_half = half; first.x_dtype = io; first.ln_eps = d.ln_eps;
+  first.ln_stats = saved.ln_stats;
+  LT_TRY(lt_launch_gemm_stream(up, EPI_ACT_FWD, cdt, io, stream, &first));
+  return lt_launch_gemm_stream(down, EPI_OUT, cdt, io, stream, &second);
+}
+}  // namespace
+
 // ---------------------------------------------------------------------------------------------------------------------
 // whole FFN block
 // ---------------------------------------------------------------------------------------------------------------------
@@ -550,6 +584,9 @@ extern "C" int lt_ffn_forward(const lt_ffn_desc* desc, const void* x, void* y, c
   Bump ws(workspace);
   FwdScratch s;
   plan_forward(d, ws, s);
+  bool few_rows;
+  LT_TRY(forward_few_rows(d, x, y, *saved, s.hid, stream, &few_rows));
+  if (few_rows) return LT_OK;
   WidenJobs biases;
   int ln_dtype;
   float* spare[2];

@@ -450,7 +450,19 @@ bool lt_gemm_mfma_supported(const GemmProblem& p, int kind);
 int lt_launch_gemm_mfma(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream);
 // up to 64 rows against a k-major weight matrix, forward epilogues (gemm_stream.hip)
 bool lt_gemm_stream_supported(const GemmProblem& p, int kind, int dtype, int io_dtype);
-int lt_launch_gemm_stream(const GemmProblem& p, int kind, int dtype, int io_dtype, hipStream_t stream);
+// what the block adds to them: small vectors in 16 bits, and for an up-projection of a few rows the LayerNorm in front of it (A is then the
+// block's input in x_dtype, and row statistics are stored as lt_ln_forward stores them)
+struct FfnStream {
+  int bias_half;          // the bias is in 16 bits
+  const void* ln_weight;  // null: no LayerNorm
+  const void* ln_bias;
+  int ln_half, x_dtype;
+  float ln_eps;
+  float* ln_stats;
+};
+constexpr int LT_STREAM_LN_MAX_H = 4096, LT_STREAM_LN_BYTES = 32768;  // of a row; of the normalised rows
+bool lt_stream_ln_supported(int64_t M, int64_t H, int x_dtype, int dtype, bool ln_half);
+int lt_launch_gemm_stream(const GemmProblem& p, int kind, int dtype, int io_dtype, hipStream_t stream, const FfnStream* ffn = nullptr);
 // 128 x 128 tiles for products too small to fill the chip with 256 x 256 ones (gemm_mid.hip)
 bool lt_gemm_mid_supported(const GemmProblem& p, int kind);
 int lt_launch_gemm_mid(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream);
