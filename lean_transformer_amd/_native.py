@@ -27,7 +27,7 @@ EXPORTED_SYMBOLS = (
     "lt_blocksparse_forward", "lt_blocksparse_backward",
     "lt_layernorm_forward", "lt_layernorm_backward_workspace_bytes", "lt_layernorm_backward",
     "lt_layernorm_backward_static_scratch_bytes", "lt_layernorm_backward_static",
-    "lt_activation_forward", "lt_activation_backward", "lt_dropout_mask", "lt_gemm", "lt_gemm_two_segments",
+    "lt_activation_forward", "lt_activation_backward", "lt_cast", "lt_dropout_mask", "lt_gemm", "lt_gemm_two_segments",
     "lt_profile_enable", "lt_profile_reset", "lt_profile_read",
 )
 
@@ -112,6 +112,7 @@ def _declare(lib):
     lib.lt_activation_forward.argtypes = [c_int64, c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p, c_void_p]
     lib.lt_activation_backward.argtypes = [c_int64, c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p, c_void_p,
                                            c_void_p]
+    lib.lt_cast.argtypes = [c_int32, POINTER(c_void_p), POINTER(c_void_p), POINTER(c_int64), c_int32, c_void_p]
     lib.lt_dropout_mask.argtypes = [c_int64, c_int32, c_float, c_uint64, c_uint64, c_void_p, c_void_p]
     lib.lt_gemm.argtypes = [c_int32, c_int64, c_int64, c_int64, c_void_p, c_int32, c_void_p, c_int32, c_int32, c_void_p,
                             c_int32, c_void_p]
@@ -190,6 +191,28 @@ def require_gpu(*tensors: Optional[torch.Tensor]):
 
 def current_stream(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def cast_all(tensors, dtype: torch.dtype, device: torch.device) -> list:
+    """detached, contiguous tensors of ``dtype`` with these values (None stays None); dense fp32 ones go to a 16-bit ``dtype`` in one launch"""
+    out, jobs = [], []
+    for t in tensors:
+        if t is None:
+            out.append(None)
+            continue
+        t = t.detach()
+        if t.dtype == torch.float32 and dtype != torch.float32 and t.is_contiguous() and t.numel():
+            new = torch.empty(t.shape, dtype=dtype, device=device)
+            jobs.append((t, new))
+            out.append(new)
+        else:
+            out.append(t.to(dtype).contiguous())
+    if jobs:
+        n = len(jobs)
+        library = lib(dtype)
+        check(library.lt_cast(n, (c_void_p * n)(*[t.data_ptr() for t, _ in jobs]), (c_void_p * n)(*[new.data_ptr() for _, new in jobs]),
+                              (c_int64 * n)(*[t.numel() for t, _ in jobs]), dtype_code(dtype), current_stream(device)), "lt_cast", library)
+    return out
 
 
 def workspace(nbytes: int, device: torch.device) -> torch.Tensor:

@@ -276,9 +276,8 @@ class _GeneralizedLinear(torch.autograd.Function):
             raise NotImplementedError("matmul_op plug-ins (Triton) are not supported; the block-sparse matmul is built in")
         device = nat.require_gpu(input, main_weight, bias, lowrank_first, lowrank_second, forward_indices, backward_indices)
         dtype = compute_dtype_for(main_weight)
-        x = _as(input, dtype).reshape(-1, input.shape[-1])
-        w = _as(main_weight, dtype)
-        l1, l2 = _as(lowrank_first, dtype), _as(lowrank_second, dtype)
+        x, w, l1, l2 = nat.cast_all((input, main_weight, lowrank_first, lowrank_second), dtype, device)
+        x = x.reshape(-1, input.shape[-1])
         b32 = _as(bias, torch.float32)
         fwd = None if forward_indices is None else forward_indices.to(torch.int32).contiguous()
         bwd = None if backward_indices is None else backward_indices.to(torch.int64).contiguous()
@@ -302,10 +301,9 @@ class _GeneralizedLinear(torch.autograd.Function):
         dtype = ctx._dtype
         device = grad_output.device
         need = tuple(ctx.needs_input_grad) + (False,) * 8
-        x = _as(input, dtype).reshape(-1, input.shape[-1])
-        dy = _as(grad_output, dtype).reshape(x.shape[0], -1)
-        w = _as(main_weight, dtype)
-        l1, l2 = _as(lowrank_first, dtype), _as(lowrank_second, dtype)
+        x, dy, w, l1, l2 = nat.cast_all((input, grad_output, main_weight, lowrank_first, lowrank_second), dtype, device)
+        x = x.reshape(-1, input.shape[-1])
+        dy = dy.reshape(x.shape[0], -1)
         fwd = None if forward_indices is None else forward_indices.to(torch.int32).contiguous()
         bwd = None if backward_indices is None else backward_indices.to(torch.int64).contiguous()
         desc = linear_desc(w, None, l1, l2, fwd, bwd, forward_indices, backward_indices)

@@ -853,6 +853,23 @@ extern "C" int lt_activation_backward(int64_t tokens, int32_t intermediate, int3
   return lt_act_backward(tokens, intermediate, gated, act, dtype, pre, d_hid, d_pre, (hipStream_t)stream);
 }
 
+extern "C" int lt_cast(int32_t n, const float* const* in, void* const* out, const int64_t* count, int32_t out_dtype, void* stream) {
+  LT_REQUIRE(n >= 0 && (n == 0 || (in && out && count)), LT_ERR_BAD_ARG, "cast: bad arguments");
+  LT_REQUIRE(out_dtype == LT_BF16, LT_ERR_BAD_ARG, "cast: dtype code %d is not this library's 16-bit type (" LT_HALF_NAME " = %d)", out_dtype,
+             (int)LT_BF16);
+  for (int32_t i = 0; i < n; i += CastJobs::MAX) {
+    CastJobs jobs;
+    jobs.n = std::min<int32_t>(CastJobs::MAX, n - i);
+    for (int j = 0; j < jobs.n; j++) {
+      jobs.in[j] = in[i + j];
+      jobs.out[j] = out[i + j];
+      jobs.count[j] = count[i + j];
+    }
+    LT_TRY(lt_cast_launch(jobs, (hipStream_t)stream));
+  }
+  return LT_OK;
+}
+
 extern "C" int lt_dropout_mask(int64_t tokens, int32_t hidden, float p, uint64_t seed, uint64_t offset, uint8_t* keep,
                                void* stream) {
   LT_REQUIRE(tokens > 0 && hidden > 0 && p >= 0.f && p < 1.f, LT_ERR_BAD_ARG, "dropout mask: bad arguments");

@@ -10,6 +10,17 @@ struct WidenJobs {
   int n;
 };
 int lt_widen(const WidenJobs& jobs, hipStream_t stream);
+// fp32 tensors -> 16 bits, up to MAX of them in one launch
+struct CastJobs {
+  static constexpr int MAX = 8;
+  const float* in[MAX];
+  void* out[MAX];
+  int64_t count[MAX];
+  unsigned first[MAX];  // first workgroup of each job; the number of workgroups where there is none
+  unsigned vec;         // bit j: job j moves 8 elements a lane (16-byte aligned)
+  int n;
+};
+int lt_cast_launch(CastJobs& jobs, hipStream_t stream);
 // LayerNorm forward.  y may be null (statistics only).  w, b: fp32, or 16 bits where the output (tail: the input) is.  tail: apply dropout,
 // then add `residual` (dtype res_dtype).  widen: vectors that the same launch widens for the kernels behind it.
 int lt_ln_forward(int64_t T, int H, float eps, int x_dtype, const void* x, int w_dtype, const void* w, const void* b, int y_dtype,

@@ -245,9 +245,11 @@ class _LeanFFN(torch.autograd.Function):
             keep = [_as(v, torch.float32) for v in keep]
         ln_weight, ln_bias, post_ln_weight, post_ln_bias, i2h_bias, h2o_bias = keep
         projections = []
+        i2h_weight, i2h_l1, i2h_l2, h2o_weight, h2o_l1, h2o_l2 = nat.cast_all((i2h_weight, i2h_l1, i2h_l2, h2o_weight, h2o_l1, h2o_l2),
+                                                                              cdt, i2h_weight.device)
         for w, b, l1, l2, fwd, bwd in ((i2h_weight, i2h_bias, i2h_l1, i2h_l2, i2h_fwd, i2h_bwd),
                                        (h2o_weight, h2o_bias, h2o_l1, h2o_l2, h2o_fwd, h2o_bwd)):
-            tensors = (_as(w, cdt), b, _as(l1, cdt), _as(l2, cdt),
+            tensors = (w, b, l1, l2,
                        None if fwd is None else fwd.to(torch.int32).contiguous(),
                        None if bwd is None else bwd.to(torch.int64).contiguous())
             keep.append(tensors)
