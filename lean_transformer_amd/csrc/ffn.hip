@@ -327,6 +327,8 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
     }
   }
   if (grads.bias) LT_TRY(lt_colsum(T, (int)out, out, dtype, dy, grads.bias, bias_grad_dtype, s.colsum, s.colsum_bytes, stream, defer));
+  GemmProblem dense[LT_MID_GROUP_MAX];  // dW of a dense layer, dL2, dL1
+  int n_dense = 0;
   if (grads.weight) {
     GemmProblem p = blank_problem();
     if (lin.block == 0) {  // dW[out, in] = dy^T x
@@ -334,7 +336,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
       p.A[0] = operand(dy, out, false);
       p.B[0] = operand(x_act, in, false);
       p.epi = epi_store_params(grads.weight, in, grad_dtype, nullptr);
-      LT_TRY(lt_launch_gemm_skinny(p, dtype, io_dtype, s.skinny, s.skinny_bytes, stream, defer));
+      dense[n_dense++] = p;
     } else {
       p.M = lin.block; p.N = in; p.K[0] = T;
       p.sp.mode = SPARSE_DW; p.sp.block = lin.block; p.sp.blocks_per_out = lin.blocks_per_out;
@@ -372,7 +374,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
     q.A[0] = operand(dy, out, false);
     q.B[0] = operand(lowrank_hid, r, false);
     q.epi = epi_store_params(grads.lowrank_second, r, grad_dtype, nullptr);
-    LT_TRY(lt_launch_gemm_skinny(q, dtype, io_dtype, s.skinny, s.skinny_bytes, stream, defer));
+    dense[n_dense++] = q;
   }
   if (r > 0 && grads.lowrank_first) {  // dL1[r, in] = g_hid^T x
     GemmProblem q = blank_problem();
@@ -380,9 +382,9 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
     q.A[0] = operand(s.g_hid, r, false);
     q.B[0] = operand(x_act, in, false);
     q.epi = epi_store_params(grads.lowrank_first, in, grad_dtype, nullptr);
-    LT_TRY(lt_launch_gemm_skinny(q, dtype, io_dtype, s.skinny, s.skinny_bytes, stream, defer));
+    dense[n_dense++] = q;
   }
-  return LT_OK;
+  return lt_launch_gemm_gradients(dense, n_dense, dtype, io_dtype, s.skinny, s.skinny_bytes, stream, defer);
 }
 
 int check_ffn_desc(const lt_ffn_desc* d) {

@@ -305,6 +305,81 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
   return lt_splitk_reduce(partial, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream, defer);
 }
 
+// Which of the products share a launch.  Low-rank gradients are a few tiles each, in as many slices as there are CUs: a launch of 9 - 16 us
+// that is mostly its start and its end.  With the same number of slices for all of a subset, their workgroups are equally long and at
+// most 256, one per CU, so that the launch takes as long as its longest slice; the estimate is mid_best's, and a launch costs 5 us more.
+// Launches one by one, together: qkv, rank 16, T 16384 (108 + 18 tiles, 2 slices) 63 + 16 us, 65; PixelFly of hidden 1024, rank 64, T 4000
+// (8 + 32, 6) 9 + 11, 12; (64 + 8, 3) 16 + 8, 18.
+int lt_launch_gemm_gradients(const GemmProblem* problems, int n, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
+                             hipStream_t stream, ColReduceQueue* defer) {
+  LT_REQUIRE(n <= LT_MID_GROUP_MAX, LT_ERR_BAD_ARG, "gradients: %d of them", n);
+  unsigned group = 0;
+  int slices = 1;
+  double gain = 0.0;
+  for (unsigned subset = 3; dtype == LT_BF16 && workspace && subset < 1u << n; subset++) {
+    int64_t tiles = 0;
+    size_t elements = 0;
+    double alone = 0.0;
+    int members = 0;
+    bool ok = true;
+    for (int j = 0; ok && j < n; j++) {
+      if (!(subset >> j & 1)) continue;
+      const GemmProblem& p = problems[j];
+      ok = !p.A[0].kmajor && !p.B[0].kmajor && p.K[0] == problems[0].K[0] && p.epi.ldo == p.N && !p.epi.bias &&
+           mid_selected(p, EPI_STORE, workspace_bytes);
+      if (!ok) break;
+      int s;
+      alone += mid_best(p.M, p.N, p.K[0], s) + 5.0;
+      tiles += mid_tiles(p.M, p.N);
+      elements += (size_t)p.M * (size_t)p.N;
+      members++;
+    }
+    if (!ok || members < 2 || tiles > 256) continue;
+    const int64_t stages = (problems[0].K[0] + 63) / 64;
+    const int most = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / tiles, stages / 4), SKINNY_MAX_SLICES));
+    for (int s = 1; s <= most; s++) {
+      if (s > 1 && s * elements * sizeof(float) + LT_MID_GROUP_MAX * 256 > workspace_bytes) break;
+      const double us = (double)((stages + s - 1) / s) * 0.45 + (s > 1 ? s * (double)elements * 8.0 / 5e6 + 4.0 : 0.0) + 5.0;
+      if (alone - us > gain) {
+        gain = alone - us;
+        group = subset;
+        slices = s;
+      }
+    }
+  }
+  GemmProblem together[LT_MID_GROUP_MAX];
+  ColReduceQueue* queue[LT_MID_GROUP_MAX];
+  int members = 0;
+  char* room = (char*)workspace;
+  for (int j = 0; j < n; j++) {
+    if (!(group >> j & 1)) continue;
+    GemmProblem& q = together[members] = problems[j];
+    queue[members] = defer;
+    if (slices > 1) {
+      const size_t bytes = lt_align_up(slices * (size_t)q.M * (size_t)q.N * sizeof(float), 256);
+      q.ksplit = slices;
+      q.split_stride = q.M * q.N;
+      q.epi.out = lt_split_partials(room, bytes, queue[members]);
+      q.epi.out_dtype = LT_F32;
+      if (!queue[members]) room += bytes;
+    }
+    members++;
+  }
+  if (members) LT_TRY(lt_launch_gemm_mid_group(together, members, stream));
+  members = 0;
+  for (int j = 0; j < n; j++) {  // (sums that do not wait, before their room is used again)
+    if (!(group >> j & 1)) continue;
+    const GemmProblem& p = problems[j];
+    if (slices > 1)
+      LT_TRY(lt_splitk_reduce((const float*)together[members].epi.out, slices, p.M * p.N, p.M * p.N, (int)p.N, nullptr, p.epi.out_dtype,
+                              p.epi.out, stream, queue[members]));
+    members++;
+  }
+  for (int j = 0; j < n; j++)
+    if (!(group >> j & 1)) LT_TRY(lt_launch_gemm_skinny(problems[j], dtype, io_dtype, workspace, workspace_bytes, stream, defer));
+  return LT_OK;
+}
+
 namespace {
 // sum of the split-k slices of an [M, N] result, 8 columns per thread, through the EPI_OUT epilogue (bias, dropout, residual)
 template <typename TX>

@@ -64,8 +64,9 @@ template <bool KM> struct MidOperand {
   }
 };
 
+// workgroup v of a product's tiles_m x tiles_n tiles and slices
 template <bool A_KM, bool B_KM, int KIND, typename TX, int ACT, int STAGES>
-__global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int tiles_m, int tiles_n) {
+__device__ __forceinline__ void mid_workgroup(const GemmProblem& p, const int tiles_m, const int tiles_n, const int v) {
   static_assert(STAGES == 2 || STAGES == 4, "stages");
   constexpr int ELEMS = MID * 64;
   // an array per stage and operand: the compiler can prove that copies and reads do not alias
@@ -92,7 +93,6 @@ __global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int t
 
   // each XCD takes a contiguous range of tiles, GROUP_M tile rows at a time
   const bool split = KIND == EPI_STORE && p.ksplit > 1;
-  const int v = (int)(blockIdx.y * gridDim.x + blockIdx.x);
   int pid, slice = 0, later = (v >> 3) & 7;  // (later: steps that a workgroup starts behind its neighbour on the XCD)
   if (split) {
     const bool tiles_first = A_KM && lt_split_tiles_first(p.M, p.N, p.K[0]);
@@ -187,6 +187,24 @@ __global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int t
   }
 }
 
+template <bool A_KM, bool B_KM, int KIND, typename TX, int ACT, int STAGES>
+__global__ __launch_bounds__(256) void gemm_bf16_mid_kernel(GemmProblem p, int tiles_m, int tiles_n) {
+  mid_workgroup<A_KM, B_KM, KIND, TX, ACT, STAGES>(p, tiles_m, tiles_n, (int)(blockIdx.y * gridDim.x + blockIdx.x));
+}
+
+// several weight gradients in one launch (both operands mn-major, plain store): workgroups first[j] .. first[j + 1] - 1 are product j's
+struct MidGroup {
+  GemmProblem p[LT_MID_GROUP_MAX];
+  int tiles_m[LT_MID_GROUP_MAX], tiles_n[LT_MID_GROUP_MAX];
+  unsigned first[LT_MID_GROUP_MAX];  // (the number of workgroups where there is no product)
+};
+__global__ __launch_bounds__(256) void gemm_bf16_mid_group_kernel(MidGroup g) {
+  int j = 0;
+#pragma unroll
+  for (int k = 1; k < LT_MID_GROUP_MAX; k++) j += blockIdx.x >= g.first[k];
+  mid_workgroup<false, false, EPI_STORE, float, -1, 4>(g.p[j], g.tiles_m[j], g.tiles_n[j], (int)(blockIdx.x - g.first[j]));
+}
+
 template <bool A_KM, bool B_KM, int KIND, typename TX> int launch_mid(const GemmProblem& p, hipStream_t stream) {
   const bool gated = KIND == EPI_ACT_FWD && p.epi.gated;
   const int tiles_m = (int)((p.M + MID - 1) / MID), tiles_n = (int)((p.N + (gated ? 63 : 127)) / (gated ? 64 : 128));
@@ -217,4 +235,30 @@ int lt_launch_gemm_mid(const GemmProblem& p, int kind, int io_dtype, hipStream_t
   if (kind == EPI_ACT_FWD) return launch_mid<true, true, EPI_ACT_FWD, float>(p, stream);
   if (kind == EPI_ACT_BWD) return launch_mid<true, false, EPI_ACT_BWD, float>(p, stream);
   return io_dtype == LT_BF16 ? launch_mid<true, true, EPI_OUT, bf16>(p, stream) : launch_mid<true, true, EPI_OUT, float>(p, stream);
+}
+
+int lt_launch_gemm_mid_group(const GemmProblem* problems, int n, hipStream_t stream) {
+  LT_REQUIRE(n > 0 && n <= LT_MID_GROUP_MAX, LT_ERR_BAD_ARG, "128 x 128 gemms in one launch: %d of them", n);
+  MidGroup g;
+  memset(&g, 0, sizeof(g));
+  unsigned total = 0;
+  double flops = 0.0;
+  for (int j = 0; j < LT_MID_GROUP_MAX; j++) {
+    g.first[j] = total;
+    if (j >= n) continue;
+    const GemmProblem& p = problems[j];
+    LT_REQUIRE(!p.A[0].kmajor && !p.B[0].kmajor && lt_gemm_mid_supported(p, EPI_STORE), LT_ERR_UNSUPPORTED,
+               "128 x 128 gemms in one launch: product %d is none of them", j);
+    g.p[j] = p;
+    g.tiles_m[j] = (int)((p.M + MID - 1) / MID);
+    g.tiles_n[j] = (int)((p.N + MID - 1) / MID);
+    total += (unsigned)(g.tiles_m[j] * g.tiles_n[j] * (p.ksplit > 1 ? p.ksplit : 1));
+    flops += lt_gemm_flops(p, EPI_STORE);
+  }
+  for (int j = n; j < LT_MID_GROUP_MAX; j++) g.first[j] = total;
+  LT_REQUIRE(total <= 256, LT_ERR_UNSUPPORTED, "128 x 128 gemms in one launch: %u workgroups", total);
+  LtProfileScope scope("gemm_mid_tn_store", flops, 0.0, stream);
+  hipLaunchKernelGGL(gemm_bf16_mid_group_kernel, dim3(total), dim3(256), 0, stream, g);
+  LT_LAUNCH_CHECK();
+  return LT_OK;
 }

@@ -466,6 +466,9 @@ int lt_launch_gemm_stream(const GemmProblem& p, int kind, int dtype, int io_dtyp
 // 128 x 128 tiles for products too small to fill the chip with 256 x 256 ones (gemm_mid.hip)
 bool lt_gemm_mid_supported(const GemmProblem& p, int kind);
 int lt_launch_gemm_mid(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream);
+// up to this many unfused ones of two mn-major operands in one launch, at most 256 tiles and slices together
+constexpr int LT_MID_GROUP_MAX = 3;
+int lt_launch_gemm_mid_group(const GemmProblem* problems, int n, hipStream_t stream);
 // block-sparse forward product or input gradient that lt_sparse_mfma_supported takes (gemm_walk.hip)
 int lt_launch_gemm_walk(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream);
 // algorithmic flops of a dense problem: 2 * M * N * (K0 + K1)
@@ -533,6 +536,10 @@ int lt_colreduce(const ColReduceJob& job, hipStream_t stream, ColReduceQueue* de
 float* lt_split_partials(void* workspace, size_t bytes, ColReduceQueue*& defer);
 int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
                           hipStream_t stream, ColReduceQueue* defer = nullptr);
+// Weight gradients of one layer (EPI_STORE, both operands mn-major, one reduction length, up to LT_MID_GROUP_MAX), none of which reads
+// another's result: those that 128 x 128 tiles take go in one launch where that is the shorter way, the rest through lt_launch_gemm_skinny.
+int lt_launch_gemm_gradients(const GemmProblem* problems, int n, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
+                             hipStream_t stream, ColReduceQueue* defer = nullptr);
 // EPI_OUT problems with few output tiles and a long reduction (the down-projection of a short batch): the reduction split
 // over workgroups into fp32 partial sums in `workspace`, then one pass that sums them through the same epilogue.  Takes as
 // many slices as the workspace holds; falls back to lt_launch_gemm when the shape does not fit or one slice is enough.
