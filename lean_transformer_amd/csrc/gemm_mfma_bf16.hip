@@ -214,6 +214,7 @@ size_t lt_gemm_generic_splitk_workspace(int64_t M, int64_t N, int64_t K) {
 int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
                           hipStream_t stream, ColReduceQueue* defer) {
   if (lt_gemm_stream_supported(p, EPI_STORE, dtype, io_dtype)) return lt_launch_gemm_stream(p, EPI_STORE, dtype, io_dtype, stream);
+  if (lt_gemm_thin_selected(p, dtype, workspace != nullptr)) return lt_launch_gemm_thin(p, stream);
   const bool a_km = p.A[0].kmajor, b_km = p.B[0].kmajor;
   const EpiParams& e = p.epi;
   if (e.bias) defer = nullptr;

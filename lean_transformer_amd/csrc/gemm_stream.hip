@@ -15,6 +15,11 @@
 // L2, behind its first requests for weights, and keeps them in LDS, up to 32 KiB, where the loop reads them.  A launch of its own takes 4 -
 // 9 us for a row or two: three trips to memory, one behind another.  (Rows normalised block by block on their way through the loop took more
 // registers: one workgroup on a CU where there had been two, one row, hidden 3776 79 us -> 84.)
+//
+// The same kernel computes the thin products of a low-rank term, hid = x L1^T and g L2, with the roles exchanged (THIN): the rows of the
+// activation are streamed as the weights are, once, against up to 64 rows of the factor, which comes out of L2; L2, whose rows are k, goes through
+// LDS as it is and is transposed by the reads (ds_read_b64_tr_b16).  128 x 128 tiles leave half or more of such a tile empty and most CUs
+// without one, or pay for a sum of slices.  lt_gemm_thin_selected has the line and both sides.
 #include <algorithm>
 
 #include "lt_internal.h"
@@ -47,7 +52,8 @@ template <typename T> __device__ __forceinline__ void widened(const lt_u32x4* w,
 
 // MT: 16-row tiles of A (M <= 16 MT), NT: 16-row tiles of W per workgroup, WAVES: wavefronts per workgroup
 // XT, VT: with LayerNorm, the types of its input and of its parameters (NoLn: A is used as it is)
-template <typename TI, int KIND, typename TX, int MT, int NT, int WAVES, typename XT = NoLn, typename VT = NoLn>
+// THIN: 1, 2: the result is stored transposed, out[n, m]; 2: A is mn-major, element (m, k) at ptr[k * ld + m]
+template <typename TI, int KIND, typename TX, int MT, int NT, int WAVES, typename XT = NoLn, typename VT = NoLn, int THIN = 0>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(std::is_same<XT, NoLn>::value ? 1 : WAVES / 2 < 4 ? 2 : 4)))
 void gemm_stream_kernel(GemmProblem p, FfnStream ffn) {
   constexpr bool LN = !std::is_same<XT, NoLn>::value;
@@ -81,15 +87,27 @@ void gemm_stream_kernel(GemmProblem p, FfnStream ffn) {
       const int tile = j >> 1, t = gated && tile >= NT / 2 ? tile - NT / 2 : tile;
       const int64_t n = min(n0 + t * 16 + (j & 1) * 8 + row_in, N - 1) - n0;
       off[j] = (uint32_t)(n * p.B[0].ld * (int64_t)sizeof(TI));
+    } else if constexpr (THIN == 2) {  // piece j * 64 + lane of a block's 64 k x 2 MT pieces of 8 columns; past the last column the last 8 again
+      off[j] = (uint32_t)(min((((j - 2 * NT) * 64 + lane) % (2 * MT)) * 8, M - 8) * (int)sizeof(TI));
     } else {
       off[j] = (uint32_t)(min((j - 2 * NT) * 8 + row_in, M - 1) * p.A[0].ld * (int64_t)sizeof(TI));
     }
   }
+  // (THIN == 2) k of that piece inside its block, and the piece's place in a row of LDS: 16 rows are read at once, 32 bytes of each
+  auto thin_k = [&](int j) { return ((j - 2 * NT) * 64 + lane) / (2 * MT); };
+  auto thin_slot = [](int k, int c) { return k * 2 * MT + (MT == 4 ? c ^ (((k >> 1 & 1) << 1) | ((k >> 3 & 1) << 2)) : MT == 2 ? c ^ ((k >> 3 & 1) << 1) : c); };
   const uint32_t my_k = (uint32_t)(lane & 7) * 16;
   auto fetch = [&](uint32_t block, lt_u32x4 (&r)[LOADS]) __attribute__((always_inline)) {
     const uint32_t k = min(block * 128 + my_k, k_bytes - 16);
 #pragma unroll
     for (int j = 0; j < LOADS; j++) {
+      if constexpr (THIN == 2) {
+        if (j >= 2 * NT) {
+          const uint32_t row = min(block * 64 + thin_k(j), (uint32_t)p.K[0] - 1);
+          r[j] = *reinterpret_cast<const lt_u32x4*>(a_base + (size_t)(off[j] + row * (uint32_t)(p.A[0].ld * sizeof(TI))));
+          continue;
+        }
+      }
       const char* base = j >= 2 * NT ? a_base : (NT > 1 && j >= NT) ? w_base2 : w_base;
       r[j] = *reinterpret_cast<const lt_u32x4*>(base + (size_t)(off[j] + k));
     }
@@ -110,6 +128,15 @@ void gemm_stream_kernel(GemmProblem p, FfnStream ffn) {
 #pragma unroll
     for (int j = 0; j < LOADS; j++) {
       lt_u32x4 v = r[j];
+      if constexpr (THIN == 2) {
+        if (j >= 2 * NT) {
+          const bool live = block * 64 + thin_k(j) < (uint32_t)p.K[0];
+#pragma unroll
+          for (int e = 0; e < 4; e++) v[e] = live ? v[e] : 0u;
+          stage[NT * 128 + thin_slot(thin_k(j), ((j - 2 * NT) * 64 + lane) % (2 * MT))] = v;
+          continue;
+        }
+      }
 #pragma unroll
       for (int e = 0; e < 4; e++) v[e] = inside ? v[e] : 0u;
       stage[slot(j * 8 + row_in, lane & 7)] = v;
@@ -129,6 +156,16 @@ void gemm_stream_kernel(GemmProblem p, FfnStream ffn) {
           a[j] = *reinterpret_cast<const lt_u32x4*>(rows + min(j * 16 + (lane & 15), M - 1) * row_bytes + (in_row ? k : 0));
 #pragma unroll
           for (int e = 0; e < 4; e++) a[j][e] = in_row ? a[j][e] : 0u;
+        } else if constexpr (THIN == 2) {
+          union { lt_u32x4 v; s16x4 h[2]; } u;
+          const int col = j * 16 + 4 * (lane & 3);
+#pragma unroll
+          for (int h = 0; h < 2; h++) {
+            const int k = s * 32 + 8 * (lane >> 4) + 4 * h + ((lane & 15) >> 2);
+            const bf16* src = reinterpret_cast<const bf16*>(stage + NT * 128 + thin_slot(k, col >> 3)) + (col & 7);
+            u.h[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(src));
+          }
+          a[j] = u.v;
         } else {
           a[j] = stage[slot((NT + j) * 16 + (lane & 15), c)];
         }
@@ -136,7 +173,7 @@ void gemm_stream_kernel(GemmProblem p, FfnStream ffn) {
 #pragma unroll
       for (int i = 0; i < NT; i++)
 #pragma unroll
-        for (int j = 0; j < MT; j++) acc[i][j] = StreamMfma<TI>::run(w[i], a[j], acc[i][j]);
+        for (int j = 0; j < MT; j++) acc[i][j] = THIN ? StreamMfma<TI>::run(a[j], w[i], acc[i][j]) : StreamMfma<TI>::run(w[i], a[j], acc[i][j]);
     }
     __builtin_amdgcn_wave_barrier();
   };
@@ -275,6 +312,14 @@ void gemm_stream_kernel(GemmProblem p, FfnStream ffn) {
     else load4(e.bias + i, b);
   };
   for (int q = wave; q < own * MT; q += WAVES) {
+    if constexpr (THIN) {  // the lane's four values are consecutive m
+      const int64_t m = (q % MT) * 16 + (lane >> 4) * 4, n = n0 + (q / MT) * 16 + (lane & 15);
+      if (m >= M || n >= N) continue;  // (M is a multiple of 8)
+      float v[4];
+      total(q, v);
+      store4(reinterpret_cast<bf16*>(e.out) + n * e.ldo + m, v);
+      continue;
+    }
     const int64_t m = (q % MT) * 16 + (lane & 15), n = n0 + (q / MT) * 16 + (lane >> 4) * 4;
     if (m >= M || n >= N) continue;  // (N is a multiple of 4)
     float v[4], bias[4] = {0.f, 0.f, 0.f, 0.f};
@@ -371,6 +416,16 @@ template <typename TI, int KIND, typename TX> int launch_shape(const GemmProblem
   return launch<TI, KIND, TX, 4, 2, 8>(p, ffn, gated, stream);
 }
 
+template <int MT, int NT, int WAVES> int launch_thin_shape(const GemmProblem& q, hipStream_t stream) {
+  const dim3 grid((unsigned)((q.N + 16 * NT - 1) / (16 * NT))), block(64 * WAVES);
+  if (q.A[0].kmajor)
+    hipLaunchKernelGGL((gemm_stream_kernel<bf16, EPI_STORE, float, MT, NT, WAVES, NoLn, NoLn, 1>), grid, block, 0, stream, q, FfnStream{});
+  else
+    hipLaunchKernelGGL((gemm_stream_kernel<bf16, EPI_STORE, float, MT, NT, WAVES, NoLn, NoLn, 2>), grid, block, 0, stream, q, FfnStream{});
+  LT_LAUNCH_CHECK();
+  return LT_OK;
+}
+
 template <typename TI> int launch_kind(const GemmProblem& p, const FfnStream& ffn, int kind, int io_dtype, hipStream_t stream) {
   if (kind == EPI_STORE) return launch_shape<TI, EPI_STORE, float>(p, ffn, stream);
   if (kind == EPI_ACT_FWD) return launch_shape<TI, EPI_ACT_FWD, float>(p, ffn, stream);
@@ -415,4 +470,42 @@ int lt_launch_gemm_stream(const GemmProblem& p, int kind, int dtype, int io_dtyp
              LT_ERR_UNSUPPORTED, "streaming gemm does not take this LayerNorm");
   LtProfileScope scope("gemm_stream", lt_gemm_flops(p, kind), 0.0, stream);
   return dtype == LT_F32 ? launch_kind<float>(p, ffn, kind, io_dtype, stream) : launch_kind<bf16>(p, ffn, kind, io_dtype, stream);
+}
+
+// [M, N] of up to 64 columns, a k-major A of more rows than that, 16-bit operands and result
+bool lt_gemm_thin_supported(const GemmProblem& p, int dtype) {
+  const EpiParams& e = p.epi;
+  if (dtype != LT_BF16 || p.sp.mode != SPARSE_NONE || p.nseg != 1 || p.ksplit > 1 || p.variant || e.bias || e.out_dtype != LT_BF16) return false;
+  if (p.M <= 64 || p.N < 8 || p.N > 64 || p.N % 8 || p.K[0] < 8 || p.K[0] % 8 || !p.A[0].kmajor) return false;
+  if (p.A[0].ld % 8 || p.B[0].ld % 8 || !lt_aligned(p.A[0].ptr, 16) || !lt_aligned(p.B[0].ptr, 16) || e.ldo % 4 || !lt_aligned(e.out, 8))
+    return false;
+  // 32-bit byte offsets: inside a workgroup's rows, over the whole factor
+  if (64 * p.A[0].ld * 2 >= (int64_t)1 << 31 || (p.B[0].kmajor ? p.N : p.K[0]) * p.B[0].ld * 2 >= (int64_t)1 << 31 || p.K[0] >= (int64_t)1 << 29)
+    return false;
+  return (p.M + 15) / 16 <= 0x7fffffff;
+}
+
+// 128 x 128 tiles (with the sum of their slices) and this, us, operands from memory.  Up to 16 columns: [500, 16] over 768 11.9, 8.2; over 8192
+// 18.5, 11.4; [4000, 16] over 1024 15.4, 7.7; over 4096 20.8, 13.0; [16384, 16] over 768 11.6, 11.2; over 2048 25.3, 19.8; over 4096 29.8, 30.4.  32:
+// [4000, 32] over 2304 18.2, 11.9; [8192, 32] over 4096 26.4, 22.1; [12000, 32] over 768 13.1, 13.3.  64 columns, where the factor is read from L2
+// more often: [500, 64] over 1024 15.6, 10.1; [4000, 64] over 1024 13.5, 9.8; over 2048 17.6, 13.7; over 4096 20.6, 19.0, but 17.1, 18.4 with the
+// activation still in the caches; over 8192 26.4, 29.0 (52.4 where the caller has no room for slices); [16384, 64] over 1024 16.6, 17.2.
+bool lt_gemm_thin_selected(const GemmProblem& p, int dtype, bool can_split) {
+  if (!lt_gemm_thin_supported(p, dtype)) return false;
+  if (p.N <= 16) return p.M <= 8192 || p.K[0] <= 3072;
+  return p.M <= 8192 && (p.K[0] <= (p.N <= 32 ? 4096 : 2048) || !can_split);
+}
+
+int lt_launch_gemm_thin(const GemmProblem& p, hipStream_t stream) {
+  LT_REQUIRE(lt_gemm_thin_supported(p, LT_BF16), LT_ERR_UNSUPPORTED, "thin gemm does not take this problem");
+  GemmProblem q = p;  // the factor as A, the activation as the streamed operand
+  q.M = p.N; q.N = p.M;
+  q.A[0] = p.B[0]; q.B[0] = p.A[0];
+  LtProfileScope scope("gemm_thin", lt_gemm_flops(p, EPI_STORE), 0.0, stream);
+  // One tile of rows a workgroup while its workgroups run at once, two a CU with up to 16 columns, else one ([4000, 16] over 4096 12.3 us, two
+  // tiles 14.5; [8192, 16] over 1024 11.3, 8.8; [8192, 64] over 1024 15.2, 10.2; [4000, 64] over 4096 18.8, 19.1).
+  const bool wide = p.M > (p.N <= 16 ? 8191 : 4096);
+  if (p.N <= 16) return wide ? launch_thin_shape<1, 2, 8>(q, stream) : launch_thin_shape<1, 1, 16>(q, stream);
+  if (p.N <= 32) return wide ? launch_thin_shape<2, 2, 8>(q, stream) : launch_thin_shape<2, 1, 16>(q, stream);
+  return wide ? launch_thin_shape<4, 2, 8>(q, stream) : launch_thin_shape<4, 1, 8>(q, stream);
 }

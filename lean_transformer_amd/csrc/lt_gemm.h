@@ -463,6 +463,10 @@ struct FfnStream {
 constexpr int LT_STREAM_LN_MAX_H = 4096, LT_STREAM_LN_BYTES = 32768;  // of a row; of the normalised rows
 bool lt_stream_ln_supported(int64_t M, int64_t H, int x_dtype, int dtype, bool ln_half);
 int lt_launch_gemm_stream(const GemmProblem& p, int kind, int dtype, int io_dtype, hipStream_t stream, const FfnStream* ffn = nullptr);
+// products of a large k-major operand with a factor of up to 64 columns (gemm_stream.hip)
+bool lt_gemm_thin_supported(const GemmProblem& p, int dtype);
+bool lt_gemm_thin_selected(const GemmProblem& p, int dtype, bool can_split);  // ... where they are the shorter way
+int lt_launch_gemm_thin(const GemmProblem& p, hipStream_t stream);
 // 128 x 128 tiles for products too small to fill the chip with 256 x 256 ones (gemm_mid.hip)
 bool lt_gemm_mid_supported(const GemmProblem& p, int kind);
 int lt_launch_gemm_mid(const GemmProblem& p, int kind, int io_dtype, hipStream_t stream);
