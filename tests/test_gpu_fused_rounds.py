@@ -1,0 +1,40 @@
+"""Activation epilogues on more 128 x 128 tiles than run at once: forward, input gradient and the bias gradient that the latter's epilogue
+sums, at ragged rows and columns, and the whole rounds of 256 x 256 tiles that stay with the other kernel."""
+import pytest
+import torch
+
+import lean_transformer_amd as lt
+from conftest import assert_close
+from helpers import oracle_params, run_oracle
+from lean_transformer_amd import _native as nat
+from test_gpu_ffn_bf16_paths import _randomise_small_vectors
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens,hidden,inter,gated,act,kernel", [
+    (5500, 512, 2048, False, "silu", "mid"),       # 176 tiles of 256 x 256
+    (4231, 264, 3080, False, "gelu", "mid"),       # columns off the 64-wide sub-tiles, the last row tile of seven rows
+    (1601, 392, 2568, True, "gelu_fused", "mid"),  # gated pairs off the tile
+    (8192, 2048, 2048, False, "relu", "bf16"),     # 256 tiles: one whole round
+])
+def test_activation_epilogues(dtype, tokens, hidden, inter, gated, act, kernel):
+    torch.manual_seed(tokens)
+    ffn = lt.LeanFFN(hidden, inter, activation=lt.ACT2FN[act], gated=gated, layer_norm_eps=1e-5)
+    _randomise_small_vectors(ffn)
+    ffn = ffn.to(DEV).to(dtype)
+    x, dy = torch.randn(tokens, hidden), torch.randn(tokens, hidden)
+    y_ref, dx_ref, g_ref = run_oracle(oracle_params(ffn), x, dy)
+    xd = x.to(DEV).requires_grad_(True)
+    lib = nat.lib(dtype)
+    lib.lt_profile_reset()
+    lib.lt_profile_enable(1)
+    y = ffn(xd)
+    dx, dw1, db1, dw2 = torch.autograd.grad(y, [xd, ffn.i2h_proj.weight, ffn.i2h_proj.bias, ffn.h2o_proj.weight], dy.to(DEV))
+    lib.lt_profile_enable(0)
+    tags = {e[0] for e in nat.profile_read(lib)}
+    assert f"gemm_{kernel}_nt_act_fwd" in tags and (gated or f"gemm_{kernel}_nn_act_bwd" in tags), tags
+    for name, got, ref in (("y", y, y_ref), ("dx", dx, dx_ref), ("dW1", dw1, g_ref[2]), ("db1", db1, g_ref[3]), ("dW2", dw2, g_ref[4])):
+        assert_close(got, ref, dtype, name)
