@@ -18,7 +18,7 @@ DEV = "cuda:0"
     (5500, 512, 2048, False, "silu", "mid"),       # 176 tiles of 256 x 256
     (4231, 264, 3080, False, "gelu", "mid"),       # columns off the 64-wide sub-tiles, the last row tile of seven rows
     (1601, 392, 2568, True, "gelu_fused", "mid"),  # gated pairs off the tile
-    (8192, 2048, 2048, False, "relu", "bf16"),     # 256 tiles: one whole round
+    (8192, 2048, 2048, False, "silu", "bf16"),     # 256 tiles: one whole round
 ])
 def test_activation_epilogues(dtype, tokens, hidden, inter, gated, act, kernel):
     torch.manual_seed(tokens)
