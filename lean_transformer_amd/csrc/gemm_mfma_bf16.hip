@@ -82,20 +82,26 @@ int mid_slices(int64_t M, int64_t N, int64_t K) {
   return slices;
 }
 int splitk_slices(int64_t M, int64_t N, int64_t K);
-// Activation epilogues on more 128 x 128 tiles than run at once (512): by the rounds that both kinds of tile take.  A last round that fills part of the
+// More 128 x 128 tiles than run at once (512): by the rounds that both kinds of tile take.  A last round that fills part of the
 // chip costs 256 x 256 tiles most of a whole one, one that leaves the CUs a single 128 x 128 tile half of a whole one; and the two
-// workgroups of a CU work through their epilogues beside each other's products, which is the more the shorter the reduction.  Two whole rounds
+// workgroups of a CU work through their epilogues beside each other's products, which is the more the shorter the reduction.  Activation epilogues, two whole rounds
 // of 128 x 128 tiles against one of 256 x 256, us: over 512 69, 80; over 1024 104, 103; over 2048 348, 321 (4 rounds); a gated forward
 // epilogue, which 256 x 256 tiles read back whole, 10 % worse.  360 products, T 1100 - 16384, widths 512 - 4096: where the estimate takes these tiles they
 // are 0.69 - 1.014 of the other's time, 13 % below it on average.  256 x 256 and 128 x 128 tiles, us: [3333, 6400] over 1600, SiLU 115, 98, its input
 // gradient 128, 110; [5500, 3072] over 768 84, 58; [2500, 8192] over 2048 148, 108; [4096, 2048] over 512 46.6, 40.0.
-bool mid_rounds_shorter(int64_t M, int64_t columns, int64_t K, bool gated_forward) {
+// Unfused products and down-projections have less of an epilogue to work beside: two whole rounds against one 57, 53 over 1024, 94, 79 over 2048,
+// 172, 145 over 4096.  They change where the large tiles' second round is nearly empty: [5500, 2880] over 2880 148, 113, its input gradient 137, 110;
+// over 11520 494, 397; [10000, 1600] over 1600 100, 85; [10000, 2048] over 2048 142, 120.
+bool mid_rounds_shorter(int64_t M, int64_t columns, int64_t K, int kind, bool gated_forward) {
   const double large = (double)((M + 255) / 256 * ((columns + 255) / 256)) / 256, small = (double)mid_tiles(M, columns) / 512;
   auto whole = [](double r) { return (double)(int64_t)r; };
   const double lf = large - whole(large), sf = small - whole(small);
   const double large_rounds = lf == 0.0 ? large : large < 1.0 ? 0.65 + 0.35 * lf : whole(large) + std::min(1.0, 0.58 + std::max(0.0, lf - 0.4) * 1.1);
   const double small_rounds = sf == 0.0 ? small : whole(small) + (sf <= 0.5 ? 0.5 : std::min(1.0, 0.82 + (sf - 0.5) * 0.7));
-  const double ratio = 0.92 + 0.16 * std::min(1.0, std::max(0.0, ((double)K - 512) / 1536)) + (gated_forward ? 0.1 : 0.0);
+  const bool fused = kind == EPI_ACT_FWD || kind == EPI_ACT_BWD;
+  if (!fused && (large < 1.0 || K < 768)) return false;  // (shorter reductions: not measured)
+  const double ratio = fused ? 0.92 + 0.16 * std::min(1.0, std::max(0.0, ((double)K - 512) / 1536)) + (gated_forward ? 0.1 : 0.0)
+                             : 1.0 + 0.22 * std::min(1.0, std::max(0.0, ((double)K - 768) / 2048));
   return ratio * small_rounds / 2 < 0.96 * large_rounds;
 }
 // 128 x 128 tiles where they all run at once, two workgroups per CU; 256 x 256 ones then fill half of the chip at most.  [1024, 8192]
@@ -110,7 +116,7 @@ bool mid_selected(const GemmProblem& p, int kind, size_t room = 0) {
   const int64_t columns = kind == EPI_ACT_FWD && p.epi.gated ? 2 * p.N : p.N;
   if (!lt_gemm_mid_supported(p, kind)) return false;
   if (mid_tiles(p.M, columns) > 512)
-    return (kind == EPI_ACT_FWD || kind == EPI_ACT_BWD) && mid_rounds_shorter(p.M, columns, p.K[0], kind == EPI_ACT_FWD && p.epi.gated);
+    return p.A[0].kmajor && mid_rounds_shorter(p.M, columns, p.K[0], kind, kind == EPI_ACT_FWD && p.epi.gated);
   const int64_t tiles = ((p.M + 255) / 256) * ((p.N + 255) / 256), stages = (p.K[0] + 63) / 64;
   const double partial_us = (double)p.M * p.N * 4.0 / 5e6;  // a pass over one slice's partial sums
   int slices;

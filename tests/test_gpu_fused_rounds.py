@@ -1,11 +1,11 @@
-"""Activation epilogues on more 128 x 128 tiles than run at once: forward, input gradient and the bias gradient that the latter's epilogue
+"""Products on more 128 x 128 tiles than run at once: forward, input gradient and the bias gradient that the latter's epilogue
 sums, at ragged rows and columns, and the whole rounds of 256 x 256 tiles that stay with the other kernel."""
 import pytest
 import torch
 
 import lean_transformer_amd as lt
 from conftest import assert_close
-from helpers import oracle_params, run_oracle
+from helpers import dropout_mask, generator_position, oracle_params, run_oracle
 from lean_transformer_amd import _native as nat
 from test_gpu_ffn_bf16_paths import _randomise_small_vectors
 
@@ -37,4 +37,31 @@ def test_activation_epilogues(dtype, tokens, hidden, inter, gated, act, kernel):
     tags = {e[0] for e in nat.profile_read(lib)}
     assert f"gemm_{kernel}_nt_act_fwd" in tags and (gated or f"gemm_{kernel}_nn_act_bwd" in tags), tags
     for name, got, ref in (("y", y, y_ref), ("dx", dx, dx_ref), ("dW1", dw1, g_ref[2]), ("db1", db1, g_ref[3]), ("dW2", dw2, g_ref[4])):
+        assert_close(got, ref, dtype, name)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dropout", [0.0, 0.2])
+def test_unfused_products_and_down_projection(dtype, dropout):
+    """272 tiles of 256 x 256 for 256 compute units: down-projection and du on 1139 of 128 x 128, ragged in rows and columns"""
+    tokens, hidden, inter = 8449, 2040, 776
+    torch.manual_seed(5)
+    ffn = lt.LeanFFN(hidden, inter, activation=lt.ACT2FN["silu"], layer_norm_eps=1e-5, dropout=dropout)
+    _randomise_small_vectors(ffn)
+    ffn = ffn.to(DEV).to(dtype)
+    x, dy = torch.randn(tokens, hidden), torch.randn(tokens, hidden)
+    mask = None
+    if dropout:
+        mask = dropout_mask(tokens, hidden, dropout, *generator_position(DEV), torch.device(DEV)).cpu()
+    y_ref, dx_ref, g_ref = run_oracle(oracle_params(ffn), x, dy, mask)
+    xd = x.to(DEV).requires_grad_(True)
+    lib = nat.lib(dtype)
+    lib.lt_profile_reset()
+    lib.lt_profile_enable(1)
+    y = ffn(xd)
+    dx, dw2 = torch.autograd.grad(y, [xd, ffn.h2o_proj.weight], dy.to(DEV))
+    lib.lt_profile_enable(0)
+    tags = {e[0] for e in nat.profile_read(lib)}
+    assert {"gemm_mid_nt_out", "gemm_mid_nn_store"} <= tags, tags
+    for name, got, ref in (("y", y, y_ref), ("dx", dx, dx_ref), ("dW2", dw2, g_ref[4])):
         assert_close(got, ref, dtype, name)
