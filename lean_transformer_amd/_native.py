@@ -193,25 +193,30 @@ def current_stream(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+_Pointers8, _Counts8 = c_void_p * 8, c_int64 * 8  # what one launch of lt_cast takes
+
+
 def cast_all(tensors, dtype: torch.dtype, device: torch.device) -> list:
     """detached, contiguous tensors of ``dtype`` with these values (None stays None); dense fp32 ones go to a 16-bit ``dtype`` in one launch"""
-    out, jobs = [], []
+    out, wide, narrow = [], [], []
     for t in tensors:
-        if t is None:
-            out.append(None)
-            continue
-        t = t.detach()
-        if t.dtype == torch.float32 and dtype != torch.float32 and t.is_contiguous() and t.numel():
-            new = torch.empty(t.shape, dtype=dtype, device=device)
-            jobs.append((t, new))
-            out.append(new)
-        else:
-            out.append(t.to(dtype).contiguous())
-    if jobs:
-        n = len(jobs)
+        if t is not None:
+            t = t.detach()
+            if t.dtype != dtype:
+                if t.dtype == torch.float32 and t.is_contiguous() and t.numel():
+                    wide.append(t)
+                    t = torch.empty(t.shape, dtype=dtype, device=device)
+                    narrow.append(t)
+                else:
+                    t = t.to(dtype).contiguous()
+            elif not t.is_contiguous():
+                t = t.contiguous()
+        out.append(t)
+    for i in range(0, len(wide), 8):
+        some, into = wide[i:i + 8], narrow[i:i + 8]
         library = lib(dtype)
-        check(library.lt_cast(n, (c_void_p * n)(*[t.data_ptr() for t, _ in jobs]), (c_void_p * n)(*[new.data_ptr() for _, new in jobs]),
-                              (c_int64 * n)(*[t.numel() for t, _ in jobs]), dtype_code(dtype), current_stream(device)), "lt_cast", library)
+        check(library.lt_cast(len(some), _Pointers8(*[t.data_ptr() for t in some]), _Pointers8(*[t.data_ptr() for t in into]),
+                              _Counts8(*[t.numel() for t in some]), _DTYPES[dtype], current_stream(device)), "lt_cast", library)
     return out
 
 
