@@ -82,12 +82,12 @@ int mid_slices(int64_t M, int64_t N, int64_t K) {
   return slices;
 }
 int splitk_slices(int64_t M, int64_t N, int64_t K);
-// More 128 x 128 tiles than run at once (512): by the rounds that both kinds of tile take.  A last round that fills part of the
-// chip costs 256 x 256 tiles most of a whole one, one that leaves the CUs a single 128 x 128 tile half of a whole one; and the two
-// workgroups of a CU work through their epilogues beside each other's products, which is the more the shorter the reduction.  Activation epilogues, two whole rounds
-// of 128 x 128 tiles against one of 256 x 256, us: over 512 69, 80; over 1024 104, 103; over 2048 348, 321 (4 rounds); a gated forward
-// epilogue, which 256 x 256 tiles read back whole, 10 % worse.  360 products, T 1100 - 16384, widths 512 - 4096: where the estimate takes these tiles they
-// are 0.69 - 1.014 of the other's time, 13 % below it on average.  256 x 256 and 128 x 128 tiles, us: [3333, 6400] over 1600, SiLU 115, 98, its input
+// More 128 x 128 tiles than run at once (512): by the rounds that both kinds of tile take.  A last round that fills part of the chip costs 256 x
+// 256 tiles most of a whole one, one that leaves the CUs a single 128 x 128 tile half of a whole one; and the two workgroups of a CU work
+// through their epilogues beside each other's products, which is worth the more the shorter the reduction.
+// Activation epilogues, whole rounds of 128 x 128 tiles against half as many of 256 x 256, us: over 512 69, 80; over 1024 104, 103; over 2048 348,
+// 321; a gated forward epilogue, which 256 x 256 tiles read back whole, 10 % worse.  360 products, T 1100 - 16384, widths 512 - 4096: where the
+// estimate takes these tiles they are 0.63 - 1.014 of the other's time, 15 % below it on average.  256 x 256 and 128 x 128 tiles, us: [3333, 6400] over 1600, SiLU 115, 98, its input
 // gradient 128, 110; [5500, 3072] over 768 84, 58; [2500, 8192] over 2048 148, 108; [4096, 2048] over 512 46.6, 40.0.
 // Unfused products and down-projections have less of an epilogue to work beside: two whole rounds against one 57, 53 over 1024, 94, 79 over 2048,
 // 172, 145 over 4096.  They change where the large tiles' second round is nearly empty: [5500, 2880] over 2880 148, 113, its input gradient 137, 110;

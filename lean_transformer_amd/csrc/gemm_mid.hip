@@ -3,7 +3,7 @@
 //
 // What bounds it: 256 x 256 tiles of [512, 8192] are 64 workgroups for 256 CUs, each walking the whole reduction; four times as many
 // tiles fill the chip, at the price of LDS bandwidth: a wavefront's 64 x 64 sub-tile reads as many cycles of LDS as it has of
-// matrix instructions, so a chip full of 256 x 256 tiles is faster (the line: mid_selected in gemm_mfma_bf16.hip).  A grid of at most
+// matrix instructions, so a chip full of 256 x 256 tiles is faster over a long reduction (the lines: mid_selected in gemm_mfma_bf16.hip).  A grid of at most
 // one workgroup per CU keeps four 64-k stages of both operands in LDS (128 KiB), three of them on their way; a larger one two
 // stages, and two workgroups share a CU.  Measured, 256 x 256 tiles against these: [512, 8192] over 2048 43 us, 21 (805 TFLOP/s); [1024,
 // 4096] over 16384 276, 137 (1000 TFLOP/s); [768, 3072] over 768 22, 11.
