@@ -86,9 +86,13 @@ int splitk_slices(int64_t M, int64_t N, int64_t K);
 // 256 tiles most of a whole one, one that leaves the CUs a single 128 x 128 tile half of a whole one; and the two workgroups of a CU work
 // through their epilogues beside each other's products, which is worth the more the shorter the reduction.
 // Activation epilogues, whole rounds of 128 x 128 tiles against half as many of 256 x 256, us: over 512 69, 80; over 1024 104, 103; over 2048 348,
-// 321; a gated forward epilogue, which 256 x 256 tiles read back whole, 10 % worse.  360 products, T 1100 - 16384, widths 512 - 4096: where the
-// estimate takes these tiles they are 0.63 - 1.014 of the other's time, 15 % below it on average.  256 x 256 and 128 x 128 tiles, us: [3333, 6400] over 1600, SiLU 115, 98, its input
-// gradient 128, 110; [5500, 3072] over 768 84, 58; [2500, 8192] over 2048 148, 108; [4096, 2048] over 512 46.6, 40.0.
+// 321; a gated forward epilogue, which 256 x 256 tiles read back whole, 10 % worse.  419 products, T 560 - 70000, widths 128 - 28672, reductions
+// 64 - 4096: where the estimate takes these tiles they are 0.39 - 1.06 of the other's time, 24 % below it on average.  256 x 256 and 128 x 128
+// tiles, us: [3333, 6400] over 1600, SiLU 115, 98, its input gradient 128, 110; [5500, 3072] over 768 84, 58; [2500, 8192] over 2048 148, 108;
+// [4096, 2048] over 512 46.6, 40.0.
+// A single round of 256 x 256 tiles that leaves CUs idle has the caches to itself, and over a long reduction nothing is left to work beside:
+// forward [2203, 5176] over 4096 107, 119; [563, 14776] over 3584 111, 119; [1100, 8192] over 3072 85, 91 (over 2048 65, 63); backward [2203, 5176]
+// over 4096 121, 136 (over 3584 [889, 10048] 114, 105).
 // Unfused products and down-projections have less of an epilogue to work beside: two whole rounds against one 57, 53 over 1024, 94, 79 over 2048,
 // 172, 145 over 4096.  They change where the large tiles' second round is nearly empty: [5500, 2880] over 2880 148, 113, its input gradient 137, 110;
 // over 11520 494, 397; [10000, 1600] over 1600 100, 85; [10000, 2048] over 2048 142, 120.
@@ -100,6 +104,7 @@ bool mid_rounds_shorter(int64_t M, int64_t columns, int64_t K, int kind, bool ga
   const double small_rounds = sf == 0.0 ? small : whole(small) + (sf <= 0.5 ? 0.5 : std::min(1.0, 0.82 + (sf - 0.5) * 0.7));
   const bool fused = kind == EPI_ACT_FWD || kind == EPI_ACT_BWD;
   if (!fused && (large < 1.0 || K < 768)) return false;  // (shorter reductions: not measured)
+  if (fused && large < 1.0 && K > (kind == EPI_ACT_BWD ? 3584 : 2048)) return false;
   const double ratio = fused ? 0.92 + 0.16 * std::min(1.0, std::max(0.0, ((double)K - 512) / 1536)) + (gated_forward ? 0.1 : 0.0)
                              : 1.0 + 0.22 * std::min(1.0, std::max(0.0, ((double)K - 768) / 2048));
   return ratio * small_rounds / 2 < 0.96 * large_rounds;

@@ -65,3 +65,23 @@ def test_unfused_products_and_down_projection(dtype, dropout):
     assert {"gemm_mid_nt_out", "gemm_mid_nn_store"} <= tags, tags
     for name, got, ref in (("y", y, y_ref), ("dx", dx, dx_ref), ("dW2", dw2, g_ref[4])):
         assert_close(got, ref, dtype, name)
+
+
+@pytest.mark.parametrize("tokens,hidden,inter,forward,backward", [
+    (1100, 2048, 8192, "mid", "mid"),    # 160 tiles of 256 x 256
+    (563, 2056, 14776, "bf16", "mid"),   # a longer reduction
+    (889, 3584, 10048, "bf16", "mid"),
+    (2203, 4096, 5176, "bf16", "bf16"),  # 189 tiles, the longest
+    (2203, 4096, 8200, "mid", "mid"),    # 297: more than one round
+])
+def test_long_reductions_that_leave_compute_units_idle(tokens, hidden, inter, forward, backward):
+    """which kernel takes the two activation epilogues (what it computes is the other tests' matter)"""
+    ffn = lt.LeanFFN(hidden, inter, activation=lt.ACT2FN["silu"]).to(DEV).to(torch.bfloat16)
+    x = torch.randn(tokens, hidden, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    lib = nat.lib(torch.bfloat16)
+    lib.lt_profile_reset()
+    lib.lt_profile_enable(1)
+    torch.autograd.grad(ffn(x), x, torch.randn_like(x))
+    lib.lt_profile_enable(0)
+    tags = {e[0] for e in nat.profile_read(lib)}
+    assert {f"gemm_{forward}_nt_act_fwd", f"gemm_{backward}_nn_act_bwd"} <= tags, tags
