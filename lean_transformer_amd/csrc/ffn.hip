@@ -230,10 +230,11 @@ struct LinearBwdScratch {
   void* g_hid;     // [T, r] dtype
   void* colsum;    // lt_colsum_workspace(T, out)
   size_t colsum_bytes;
-  void* skinny;    // split-k partial sums of the low-rank GEMMs
+  void* skinny;    // partial results of split products, one at a time or those that wait for one sum (ColReduceQueue::scratch)
   size_t skinny_bytes;
 };
 
+// (all but the place of `skinny`)
 void plan_linear_backward(const lt_linear& lin, int64_t T, int dtype, Bump& ws, LinearBwdScratch& s) {
   s.g_hid = lin.lowrank > 0 ? ws.take((size_t)T * lin.lowrank * lt_dtype_size(dtype)) : nullptr;
   s.colsum_bytes = lt_colsum_workspace(T, lin.out_features);
@@ -254,26 +255,6 @@ void plan_linear_backward(const lt_linear& lin, int64_t T, int dtype, Bump& ws, 
     s.skinny_bytes = std::max(s.skinny_bytes,
                               lt_sparse_dw_split_workspace(lin.in_features, lin.out_features, lin.blocks_per_in, lin.blocks_per_out,
                                                            group_length(lin.in_group), group_length(lin.out_group), T));
-  s.skinny = s.skinny_bytes ? ws.take(s.skinny_bytes) : nullptr;
-}
-
-// Room for the partial results of the split weight and low-rank gradients of a layer, to be summed with others in one launch: at most
-// 32 MiB, an upper bound (up to 16 slices) where that is less.  Larger results gain nothing by waiting and are no longer in the caches then:
-// fused qkv over 16384 tokens with room for none 346 us, 8 MiB 337, 32 MiB 332, 128 MiB 336; tiled butterfly of hidden 1024 473, -, 455,
-// 455; GPT layer (57 and 66 MiB a result) 999, -, 999, 1003.
-constexpr size_t SUM_ROOM = (size_t)32 << 20;
-size_t deferred_sum_room(const lt_linear& lin, int64_t T, int dtype) {
-  const int64_t in = lin.in_features, out = lin.out_features;
-  size_t bytes = (size_t)16 * lin.lowrank * (in + out) * sizeof(float) + 3 * 256;
-  if (lin.block == 0) {
-    size_t dw = lt_gemm_generic_splitk_workspace(out, in, T);
-    if (dtype == LT_BF16) dw = std::max({dw, lt_gemm_splitk_workspace(out, in, T), lt_gemm_mid_splitk_workspace(out, in, T)});
-    bytes += dw;
-  } else if (lin.block == 64 && dtype == LT_BF16) {
-    bytes += lt_sparse_dw_split_workspace(in, out, lin.blocks_per_in, lin.blocks_per_out, group_length(lin.in_group),
-                                          group_length(lin.out_group), T);
-  }
-  return bytes > SUM_ROOM ? SUM_ROOM : bytes;
 }
 
 // gradient side of one generalized linear layer.  The input-gradient GEMM runs FIRST, through epilogue `kind_dx`
@@ -286,7 +267,7 @@ size_t deferred_sum_room(const lt_linear& lin, int64_t T, int dtype) {
 int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void* x_act, const void* dy,
                          const void* lowrank_hid, int kind_dx, const EpiParams& epi_dx, const lt_linear_grads& grads,
                          int grad_dtype, const LinearBwdScratch& s, int io_dtype, hipStream_t stream, float* act_colsum = nullptr,
-                         int* act_colsum_rows = nullptr, ColReduceQueue* defer = nullptr, int bias_grad_dtype = LT_F32) {
+                         int* act_colsum_rows = nullptr, ColReduceQueue* queue = nullptr, int bias_grad_dtype = LT_F32) {
   const int64_t in = lin.in_features, out = lin.out_features, r = lin.lowrank;
   const bool need_dx = kind_dx >= 0;
   if (r > 0 && (need_dx || grads.lowrank_first)) {  // g_hid = dy L2  [T, r]
@@ -295,7 +276,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
     q.A[0] = operand(dy, out, true);
     q.B[0] = operand(lin.lowrank_second, r, false);
     q.epi = epi_store_params(s.g_hid, r, dtype, nullptr);
-    LT_TRY(lt_launch_gemm_skinny(q, dtype, io_dtype, s.skinny, s.skinny_bytes, stream));
+    LT_TRY(lt_launch_gemm_skinny(q, dtype, io_dtype, s.skinny, s.skinny_bytes, stream, queue));
   }
   if (need_dx) {  // dx = dy W (+ g_hid L1)
     GemmProblem p = blank_problem();
@@ -312,7 +293,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
       p.B[0] = operand(lin.weight, in, false);
       if (kind_dx == EPI_ACT_BWD && act_colsum && (*act_colsum_rows = lt_gemm_colsum_rows(p, dtype, io_dtype)) > 0)
         p.epi.colsum = act_colsum;
-      if (kind_dx == EPI_STORE && r == 0) LT_TRY(lt_launch_gemm_skinny(p, dtype, io_dtype, s.skinny, s.skinny_bytes, stream));
+      if (kind_dx == EPI_STORE && r == 0) LT_TRY(lt_launch_gemm_skinny(p, dtype, io_dtype, s.skinny, s.skinny_bytes, stream, queue));
       else LT_TRY(lt_launch_gemm(p, kind_dx, dtype, io_dtype, stream));
     } else {
       p.K[0] = lin.block;
@@ -326,7 +307,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
       LT_TRY(lt_launch_gemm_sparse(p, kind_dx, dtype, io_dtype, stream));
     }
   }
-  if (grads.bias) LT_TRY(lt_colsum(T, (int)out, out, dtype, dy, grads.bias, bias_grad_dtype, s.colsum, s.colsum_bytes, stream, defer));
+  if (grads.bias) LT_TRY(lt_colsum(T, (int)out, out, dtype, dy, grads.bias, bias_grad_dtype, s.colsum, s.colsum_bytes, stream, queue));
   GemmProblem dense[LT_MID_GROUP_MAX];  // dW of a dense layer, dL2, dL1
   int n_dense = 0;
   if (grads.weight) {
@@ -353,8 +334,9 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
         // the reduction over the tokens split over workgroups: fp32 partial gradients, summed into the parameter's dtype
         p.ksplit = slices;
         p.split_stride = (int64_t)elements;
-        ColReduceQueue* later = defer;
-        float* const partial = lt_split_partials(s.skinny, (size_t)slices * elements * sizeof(float), later);
+        ColReduceQueue* later = queue;
+        float* partial;
+        LT_TRY(lt_place_partials(s.skinny, (size_t)slices * elements * sizeof(float), 1, true, later, &partial, stream));
         p.epi.out = partial;
         p.epi.out_dtype = LT_F32;
         LT_TRY(lt_launch_gemm_sparse(p, EPI_STORE, dtype, io_dtype, stream));
@@ -384,7 +366,7 @@ int linear_backward_impl(const lt_linear& lin, int64_t T, int dtype, const void*
     q.epi = epi_store_params(grads.lowrank_first, in, grad_dtype, nullptr);
     dense[n_dense++] = q;
   }
-  return lt_launch_gemm_gradients(dense, n_dense, dtype, io_dtype, s.skinny, s.skinny_bytes, stream, defer);
+  return lt_launch_gemm_gradients(dense, n_dense, dtype, io_dtype, s.skinny, s.skinny_bytes, stream, queue);
 }
 
 int check_ffn_desc(const lt_ffn_desc* d) {
@@ -492,8 +474,8 @@ struct BwdScratch {
   float* vectors;     // room for 16-bit LayerNorm parameters in fp32
   float* act_colsum;  // [ceil(T / 64), N1]: partial column sums of dpre from the epilogue that writes it
   LinearBwdScratch h2o, i2h;
-  void* sums;  // partial results of split gradients that are summed at the end of the step
-  size_t sum_bytes;
+  size_t split_bytes;  // of both layers, one piece, in front of `hid`
+  size_t hid_bytes;
 };
 
 void plan_backward(const lt_ffn_desc& d, Bump& ws, BwdScratch& s) {
@@ -503,7 +485,6 @@ void plan_backward(const lt_ffn_desc& d, Bump& ws, BwdScratch& s) {
   s.g = ws.take((size_t)T * d.hidden * e);
   s.g_post = d.post_ln_weight ? ws.take((size_t)T * d.hidden * e) : nullptr;
   s.post_stats = d.post_ln_weight ? (float*)ws.take((size_t)T * 2 * sizeof(float)) : nullptr;
-  s.hid = ws.take((size_t)T * d.intermediate * e);
   s.dpre = ws.take((size_t)T * n1 * e);
   s.u = ws.take((size_t)T * d.hidden * e);
   s.du = ws.take((size_t)T * d.hidden * e);
@@ -514,8 +495,12 @@ void plan_backward(const lt_ffn_desc& d, Bump& ws, BwdScratch& s) {
   s.act_colsum = (float*)ws.take((size_t)((T + 63) / 64) * n1 * sizeof(float));
   plan_linear_backward(d.h2o, T, d.compute_dtype, ws, s.h2o);
   plan_linear_backward(d.i2h, T, d.compute_dtype, ws, s.i2h);
-  s.sum_bytes = std::min(SUM_ROOM, deferred_sum_room(d.h2o, T, d.compute_dtype) + deferred_sum_room(d.i2h, T, d.compute_dtype));
-  s.sums = ws.take(s.sum_bytes);
+  s.split_bytes = s.h2o.skinny_bytes + s.i2h.skinny_bytes;  // (multiples of 256)
+  s.hid_bytes = (size_t)T * d.intermediate * e;
+  char* const split = (char*)ws.take(s.split_bytes);
+  s.hid = ws.take(s.hid_bytes);
+  s.h2o.skinny = s.h2o.skinny_bytes ? split : nullptr;
+  s.i2h.skinny = s.i2h.skinny_bytes ? split : nullptr;
 }
 
 }  // namespace
@@ -667,8 +652,8 @@ extern "C" int lt_ffn_backward_typed(const lt_ffn_desc* desc, const void* x, con
   // the sums at the end of several passes (bias, LayerNorm parameter, split weight and low-rank gradients) wait for one launch at the
   // end of the step
   ColReduceQueue reduces;
-  reduces.room = (char*)s.sums;
-  reduces.room_bytes = s.sum_bytes;
+  reduces.scratch = (char*)s.hid - s.split_bytes;
+  reduces.scratch_bytes = s.split_bytes;
   // gradient entering the down-projection: dropout replayed on dy, then (optionally) back through the post-LN
   const void* g = s.g;
   lt_linear_grads h2o_grads = grads->h2o;
@@ -701,6 +686,7 @@ extern "C" int lt_ffn_backward_typed(const lt_ffn_desc* desc, const void* x, con
     LT_TRY(linear_backward_impl(d.h2o, T, cdt, s.hid, g, saved->h2o_lowrank_hid, EPI_ACT_BWD, e, h2o_grads, grad_dtype, s.h2o, io,
                                 stream, grads->i2h.bias ? s.act_colsum : nullptr, &bias_rows, &reduces, vector_grad_dtype));
   }
+  reduces.scratch_bytes += s.hid_bytes;  // (nothing launched from here on reads hid)
   lt_linear_grads i2h_grads = grads->i2h;
   if (bias_rows > 0) {  // db1 = column sums of dP, already reduced to one row per bias_rows tokens
     LT_TRY(lt_colreduce(ColReduceJob{s.act_colsum, grads->i2h.bias, (int)((T + bias_rows - 1) / bias_rows), (int)N1, N1,
@@ -732,7 +718,7 @@ extern "C" size_t lt_linear_backward_workspace_bytes(const lt_linear* lin, int64
   Bump ws(nullptr);
   LinearBwdScratch s;
   plan_linear_backward(*lin, tokens, dtype, ws, s);
-  ws.take(deferred_sum_room(*lin, tokens, dtype));
+  ws.take(s.skinny_bytes);
   return lt_align_up(ws.used, 256);
 }
 
@@ -768,8 +754,9 @@ extern "C" int lt_linear_backward_to(const lt_linear* lin, int64_t tokens, int32
   LinearBwdScratch s;
   plan_linear_backward(*lin, tokens, dtype, ws, s);
   ColReduceQueue reduces;
-  reduces.room_bytes = deferred_sum_room(*lin, tokens, dtype);
-  reduces.room = (char*)ws.take(reduces.room_bytes);
+  s.skinny = s.skinny_bytes ? ws.take(s.skinny_bytes) : nullptr;
+  reduces.scratch = (char*)s.skinny;
+  reduces.scratch_bytes = s.skinny_bytes;
   EpiParams e = epi_store_params(dx, lin->in_features, dx_dtype, nullptr);
   LT_TRY(linear_backward_impl(*lin, tokens, dtype, x, dy, lowrank_hid, dx ? EPI_STORE : -1, e, *grads, grad_dtype, s, dtype,
                               (hipStream_t)stream, nullptr, nullptr, &reduces));

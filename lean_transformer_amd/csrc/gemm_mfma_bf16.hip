@@ -241,12 +241,12 @@ size_t lt_gemm_generic_splitk_workspace(int64_t M, int64_t N, int64_t K) {
 }
 
 int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
-                          hipStream_t stream, ColReduceQueue* defer) {
+                          hipStream_t stream, ColReduceQueue* queue, bool may_wait) {
   if (lt_gemm_stream_supported(p, EPI_STORE, dtype, io_dtype)) return lt_launch_gemm_stream(p, EPI_STORE, dtype, io_dtype, stream);
   if (lt_gemm_thin_selected(p, dtype, workspace != nullptr)) return lt_launch_gemm_thin(p, stream);
   const bool a_km = p.A[0].kmajor, b_km = p.B[0].kmajor;
   const EpiParams& e = p.epi;
-  if (e.bias) defer = nullptr;
+  if (e.bias) may_wait = false;
   const size_t slice = (size_t)p.M * (size_t)p.N * sizeof(float);
   if (dtype == LT_BF16 && e.ldo == p.N && mid_selected(p, EPI_STORE, workspace ? workspace_bytes : 0)) {
     const int slices = (int)std::min<size_t>((size_t)mid_slices(p.M, p.N, p.K[0]), workspace ? workspace_bytes / slice : 0);
@@ -255,12 +255,13 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
     q.ksplit = slices;
     q.split_stride = p.M * p.N;
     q.epi = EpiParams{};
-    float* const partial = lt_split_partials(workspace, slices * slice, defer);
+    float* partial;
+    LT_TRY(lt_place_partials(workspace, slices * slice, 1, may_wait, queue, &partial, stream));
     q.epi.out = partial;
     q.epi.ldo = p.N;
     q.epi.out_dtype = LT_F32;
     LT_TRY(lt_launch_gemm(q, EPI_STORE, dtype, io_dtype, stream));
-    return lt_splitk_reduce(partial, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream, defer);
+    return lt_splitk_reduce(partial, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream, queue);
   }
   bool ok = dtype == LT_BF16 && p.nseg == 1 && p.sp.mode == SPARSE_NONE && p.M > 0 && p.N > 0 && p.N % 128 == 0 &&
             !(!a_km && b_km) && (a_km || p.M % 128 == 0) && ((!a_km && !b_km) || p.K[0] % 8 == 0) && p.K[0] > 0 &&
@@ -278,13 +279,14 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
       q.ksplit = slices;
       q.variant = 2;
       q.split_stride = p.M * p.N;
-      float* const partial = lt_split_partials(workspace, slices * slice, defer);
+      float* partial;
+      LT_TRY(lt_place_partials(workspace, slices * slice, 1, may_wait, queue, &partial, stream));
       q.epi.out = partial;
       q.epi.ldo = p.N;
       q.epi.out_dtype = LT_F32;
       q.epi.bias = nullptr;
       LT_TRY(lt_launch_gemm(q, EPI_STORE, dtype, io_dtype, stream));
-      return lt_splitk_reduce(partial, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream, defer);
+      return lt_splitk_reduce(partial, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream, queue);
     }
     if (((p.M + 255) / 256) * ((p.N + 255) / 256) >= 64 || slices == 1) ok = false;
   }
@@ -298,12 +300,13 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
       GemmProblem q = p;
       q.ksplit = slices;
       q.split_stride = p.M * p.N;
-      float* const partial = lt_split_partials(workspace, slices * slice, defer);
+      float* partial;
+      LT_TRY(lt_place_partials(workspace, slices * slice, 1, may_wait, queue, &partial, stream));
       q.epi.out = partial;
       q.epi.out_dtype = LT_F32;
       q.epi.bias = nullptr;
       LT_TRY(lt_launch_gemm_generic(q, EPI_STORE, dtype, io_dtype, stream));
-      return lt_splitk_reduce(partial, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream, defer);
+      return lt_splitk_reduce(partial, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream, queue);
     }
     return lt_launch_gemm(p, EPI_STORE, dtype, io_dtype, stream);
   }
@@ -323,7 +326,8 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
   if (slices > 1) {
     q.ksplit = slices;
     q.split_stride = p.M * p.N;
-    q.epi.out = partial = lt_split_partials(workspace, slices * slice, defer);
+    LT_TRY(lt_place_partials(workspace, slices * slice, 1, may_wait, queue, &partial, stream));
+    q.epi.out = partial;
     q.epi.out_dtype = LT_F32;
     q.epi.bias = nullptr;
   }
@@ -332,7 +336,7 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
     const int status = lt_mfma_launch_skinny(q, slices, stream);
     if (status != LT_OK || slices == 1) return status;
   }
-  return lt_splitk_reduce(partial, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream, defer);
+  return lt_splitk_reduce(partial, slices, p.M * p.N, p.M * p.N, (int)p.N, e.bias, e.out_dtype, e.out, stream, queue);
 }
 
 // Which of the products share a launch.  Low-rank gradients are a few tiles each, in as many slices as there are CUs: a launch of 9 - 16 us
@@ -341,7 +345,7 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
 // Launches one by one, together: qkv, rank 16, T 16384 (108 + 18 tiles, 2 slices) 63 + 16 us, 65; PixelFly of hidden 1024, rank 64, T 4000
 // (8 + 32, 6) 9 + 11, 12; (64 + 8, 3) 16 + 8, 18.
 int lt_launch_gemm_gradients(const GemmProblem* problems, int n, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
-                             hipStream_t stream, ColReduceQueue* defer) {
+                             hipStream_t stream, ColReduceQueue* queue) {
   LT_REQUIRE(n <= LT_MID_GROUP_MAX, LT_ERR_BAD_ARG, "gradients: %d of them", n);
   unsigned group = 0;
   int slices = 1;
@@ -378,35 +382,44 @@ int lt_launch_gemm_gradients(const GemmProblem* problems, int n, int dtype, int 
     }
   }
   GemmProblem together[LT_MID_GROUP_MAX];
-  ColReduceQueue* queue[LT_MID_GROUP_MAX];
+  ColReduceQueue* sums = queue;
+  char* place = nullptr;
   int members = 0;
-  char* room = (char*)workspace;
+  if (slices > 1) {
+    size_t bytes = 0;
+    int results = 0;
+    for (int j = 0; j < n; j++)
+      if (group >> j & 1) {
+        bytes += lt_align_up(slices * (size_t)problems[j].M * (size_t)problems[j].N * sizeof(float), 256);
+        results++;
+      }
+    float* partial;
+    LT_TRY(lt_place_partials(workspace, bytes, results, true, sums, &partial, stream));
+    place = (char*)partial;
+  }
   for (int j = 0; j < n; j++) {
     if (!(group >> j & 1)) continue;
-    GemmProblem& q = together[members] = problems[j];
-    queue[members] = defer;
+    GemmProblem& q = together[members++] = problems[j];
     if (slices > 1) {
-      const size_t bytes = lt_align_up(slices * (size_t)q.M * (size_t)q.N * sizeof(float), 256);
       q.ksplit = slices;
       q.split_stride = q.M * q.N;
-      q.epi.out = lt_split_partials(room, bytes, queue[members]);
+      q.epi.out = place;
       q.epi.out_dtype = LT_F32;
-      if (!queue[members]) room += bytes;
+      place += lt_align_up(slices * (size_t)q.M * (size_t)q.N * sizeof(float), 256);
     }
-    members++;
   }
   if (members) LT_TRY(lt_launch_gemm_mid_group(together, members, stream));
   members = 0;
-  for (int j = 0; j < n; j++) {  // (sums that do not wait, before their room is used again)
+  for (int j = 0; j < n; j++) {  // (sums that do not wait, before their place is used again)
     if (!(group >> j & 1)) continue;
     const GemmProblem& p = problems[j];
     if (slices > 1)
       LT_TRY(lt_splitk_reduce((const float*)together[members].epi.out, slices, p.M * p.N, p.M * p.N, (int)p.N, nullptr, p.epi.out_dtype,
-                              p.epi.out, stream, queue[members]));
+                              p.epi.out, stream, sums));
     members++;
   }
   for (int j = 0; j < n; j++)
-    if (!(group >> j & 1)) LT_TRY(lt_launch_gemm_skinny(problems[j], dtype, io_dtype, workspace, workspace_bytes, stream, defer));
+    if (!(group >> j & 1)) LT_TRY(lt_launch_gemm_skinny(problems[j], dtype, io_dtype, workspace, workspace_bytes, stream, queue, true));
   return LT_OK;
 }
 

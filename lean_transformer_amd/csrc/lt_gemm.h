@@ -510,7 +510,8 @@ int lt_gemm_colsum_rows(const GemmProblem& p, int dtype, int io_dtype);
 // Sums that may wait: column sums of partial rows (bias and LayerNorm parameter gradients) and the partial results of split
 // reductions (weight and low-rank gradients).  A caller that runs several passes with such a tail (the backward of a layer or of the whole
 // block) hands the same queue to each of them and flushes it once: one launch for all sums instead of one each.  Partial rows and partial
-// results must stay untouched until the flush; the latter get their place from the queue's own `room`, what does not fit is summed at once.
+// results must stay untouched until the flush.  The latter wait at the front of `scratch`, the caller's memory for split reductions, where
+// every split reduction of the pass gets its place from the queue, those that do not wait too.
 struct ColReduceJob {
   const float* partial;  // row r at partial + r * stride
   void* out;
@@ -529,21 +530,22 @@ struct ColReduceQueue {
   ColReduceJob job[MAX];
   SplitSumJob split[MAX];
   int n = 0, n_split = 0;
-  char* room = nullptr;  // 256-byte aligned
-  size_t room_bytes = 0;
+  char* scratch = nullptr;  // 256-byte aligned
+  size_t scratch_bytes = 0, waiting = 0;
 };
 int lt_colreduce_flush(ColReduceQueue& queue, hipStream_t stream);
 // out[c] = sum over the partial rows of partial[r * stride + c] (now, or at the flush of `defer`)
 int lt_colreduce(const ColReduceJob& job, hipStream_t stream, ColReduceQueue* defer = nullptr);
-// Where a split reduction of `bytes` leaves its partial results: in the room of `defer`, if that has it and a job left, else in
-// `workspace`; `defer` becomes null then.
-float* lt_split_partials(void* workspace, size_t bytes, ColReduceQueue*& defer);
+// Where split reductions of `bytes` in all (`results` of them) leave their partial results: without a queue in `workspace`, else in the queue's
+// memory, behind what waits there; that is flushed first where it leaves too little.  `queue` becomes null if their sums cannot wait.
+int lt_place_partials(void* workspace, size_t bytes, int results, bool may_wait, ColReduceQueue*& queue, float** partial, hipStream_t stream);
+// With a queue, whose memory has at least workspace_bytes, partial results go there, and their sum waits if it may.
 int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
-                          hipStream_t stream, ColReduceQueue* defer = nullptr);
+                          hipStream_t stream, ColReduceQueue* queue = nullptr, bool may_wait = false);
 // Weight gradients of one layer (EPI_STORE, both operands mn-major, one reduction length, up to LT_MID_GROUP_MAX), none of which reads
 // another's result: those that 128 x 128 tiles take go in one launch where that is the shorter way, the rest through lt_launch_gemm_skinny.
 int lt_launch_gemm_gradients(const GemmProblem* problems, int n, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
-                             hipStream_t stream, ColReduceQueue* defer = nullptr);
+                             hipStream_t stream, ColReduceQueue* queue = nullptr);
 // EPI_OUT problems with few output tiles and a long reduction (the down-projection of a short batch): the reduction split
 // over workgroups into fp32 partial sums in `workspace`, then one pass that sums them through the same epilogue.  Takes as
 // many slices as the workspace holds; falls back to lt_launch_gemm when the shape does not fit or one slice is enough.
@@ -552,7 +554,7 @@ size_t lt_gemm_out_splitk_workspace(int dtype, int64_t M, int64_t N, int64_t K, 
 int lt_launch_gemm_out(const GemmProblem& p, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
                        hipStream_t stream);
 // out[i] = sum_s partial[s * stride + i] (+ bias[i % cols]) for i < count, cast to out_dtype (now, or without a bias at the flush of
-// `defer`, which lt_split_partials took the partial results' place from)
+// `defer`, in whose memory lt_place_partials has put the partial results)
 int lt_splitk_reduce(const float* partial, int slices, int64_t stride, int64_t count, int cols, const float* bias,
                      int out_dtype, void* out, hipStream_t stream, ColReduceQueue* defer = nullptr);
 // picks the tiled kernel when it applies and dtype is bf16, else the any-shape kernel

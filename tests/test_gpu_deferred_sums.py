@@ -3,7 +3,7 @@ them, for some of them, and where nothing is split."""
 import pytest
 import torch
 
-import lean_transformer_amd as lt
+from lean_transformer_amd import _native as nat
 from lean_transformer_amd.blocksparse.linear import GeneralizedMatrix, GeneralizedLinear
 
 pytestmark = pytest.mark.gpu
@@ -49,3 +49,23 @@ def test_gradients_summed_at_the_end(tokens, fan_in, fan_out, rank, bias, comput
                 assert ((g.double() - ref).abs() <= 2.0**-8 * room + 1e-30).all(), name
                 continue
         assert ((g.double() - ref).abs() <= (tokens + fan_in + 64) * 2.0**-23 * room + 1e-30).all(), name
+
+
+def test_partial_results_that_do_not_all_fit():
+    """split results take turns in the memory that holds the largest of them: the weight gradient's four slices (8 MiB) fill it, the low-rank
+    pair's wait behind a first sum"""
+    torch.manual_seed(0)
+    layer = GeneralizedLinear(GeneralizedMatrix(512, 2048, "pixelfly(block_size=64, stretch=False)", 8)).to(DEV).bfloat16()
+    x, dy = torch.randn(4096, 512, device=DEV, dtype=torch.bfloat16), torch.randn(4096, 2048, device=DEV, dtype=torch.bfloat16)
+    y = layer(x)
+    weight, pair = layer.matrix.weight, [layer.matrix.lowrank_first, layer.matrix.lowrank_second]
+    lib = nat.lib(torch.bfloat16)
+    lib.lt_profile_reset()
+    lib.lt_profile_enable(1)
+    together = torch.autograd.grad(y, [weight, *pair, layer.bias], dy, retain_graph=True)
+    lib.lt_profile_enable(0)
+    launches = {tag: n for tag, n, *_ in nat.profile_read(lib)}
+    assert launches["splitk_reduce"] == 2, launches
+    assert torch.equal(together[0], torch.autograd.grad(y, weight, dy, retain_graph=True)[0])
+    for a, b in zip(together[1:], torch.autograd.grad(y, [*pair, layer.bias], dy)):
+        assert torch.equal(a, b)

@@ -307,3 +307,34 @@ def test_shared_list_run_of_pixelfly_layouts():
     assert shared_list_run(forward_indices, per_in) == 4
     forward_indices[1] = forward_indices[8]  # output block 1 now reads other input blocks than 0, 2 and 3
     assert shared_list_run(forward_indices, per_in) == 1
+
+
+def _linear_desc(fan_in, fan_out, rank):
+    """a dense layer's descriptor, for the calls that read nothing but its sizes"""
+    some = 1 << 20
+    lin = nat.LtLinear()
+    lin.in_features, lin.out_features, lin.weight, lin.lowrank = fan_in, fan_out, some, rank
+    if rank:
+        lin.lowrank_first = lin.lowrank_second = some
+    return lin
+
+
+@pytest.mark.parametrize("tokens,fan_in,fan_out,rank", [(4096, 4096, 32768, 128), (4096, 16384, 4096, 128), (16384, 768, 2304, 16), (1000, 640, 384, 8)])
+def test_backward_workspace_of_a_low_rank_term(tokens, fan_in, fan_out, rank):
+    """it costs its own factor and 16 slices of a product of that size, no further room for partial results"""
+    lib = nat.lib(torch.bfloat16)
+    size = [lib.lt_linear_backward_workspace_bytes(_linear_desc(fan_in, fan_out, r), tokens, nat.LT_BF16) for r in (0, rank)]
+    assert 0 < size[0] and size[1] - size[0] <= tokens * rank * (2 + 16 * 4) + 1024
+
+
+@pytest.mark.parametrize("tokens,hidden,inter,rank", [(4096, 4096, 16384, 128), (4000, 1024, 4096, 64)])
+def test_backward_workspace_of_a_block_with_low_rank_terms(tokens, hidden, inter, rank):
+    lib = nat.lib(torch.bfloat16)
+    size = []
+    for r in (0, rank):
+        desc = nat.LtFfnDesc()
+        desc.tokens, desc.hidden, desc.intermediate, desc.gated, desc.compute_dtype, desc.vector_dtype = tokens, hidden, inter, 1, nat.LT_BF16, nat.LT_F32
+        desc.ln_weight = desc.ln_bias = 1 << 20
+        desc.i2h, desc.h2o = _linear_desc(hidden, 2 * inter, r), _linear_desc(inter, hidden, r)
+        size.append(lib.lt_ffn_backward_workspace_bytes(desc))
+    assert 0 < size[0] and size[1] - size[0] <= 2 * tokens * rank * (2 + 16 * 4) + 2048
