@@ -34,6 +34,18 @@ __device__ __forceinline__ void widen_block(const WidenJobs& jobs, int block) {
   }
 }
 
+// a * b + c in the output's type.  In binary16 rounded once, by the multiply-add that does so: left to choose, the compiler took that one or an
+// fp32 multiply-add and a conversion, which rounds twice, as the type of the parameters and the unrolling suited it, and a row's bits
+// depended on whether the parameters' addresses let them be read as they are.
+template <typename T> __device__ __forceinline__ T multiply_add(float a, float b, float c) { return from_f32<T>(fmaf(a, b, c)); }
+#ifdef LT_HALF_IS_FP16
+template <> __device__ __forceinline__ bf16 multiply_add<bf16>(float a, float b, float c) {
+  uint32_t r = 0;
+  asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "+v"(r) : "v"(a), "v"(b), "v"(c));
+  return __builtin_bit_cast(bf16, (uint16_t)r);
+}
+#endif
+
 template <typename TX, typename TY, typename TR, typename TW, bool TAIL, int MAXV>
 __global__ __launch_bounds__(256) void ln_fwd_kernel(int64_t T, int H, float eps, const TX* __restrict__ x,
                                                       const TW* __restrict__ w, const TW* __restrict__ b,
@@ -135,12 +147,15 @@ __global__ __launch_bounds__(256) void ln_fwd_kernel(int64_t T, int H, float eps
     rstd = 1.0f / sqrtf(wave_sum(q) * inv_h + eps);
     if (y) {
       for (int c = lane; c < H; c += 64) {
-        float o = (ldf(xr, c) - mean) * rstd * ldf(w, c) + ldf(b, c);
+        const float u = (ldf(xr, c) - mean) * rstd, wv = ldf(w, c), bv = ldf(b, c);
         if constexpr (TAIL) {
+          float o = u * wv + bv;
           if (drop.p > 0.f) o = dropout_keep(drop, row * H + c) ? o * drop.scale : 0.f;
           if (residual) o += ldf(residual, row * H + c);
+          stf(y, row * H + c, o);
+        } else {
+          y[row * H + c] = multiply_add<TY>(u, wv, bv);
         }
-        stf(y, row * H + c, o);
       }
     }
   }
