@@ -846,17 +846,22 @@ extern "C" int lt_cast(int32_t n, const float* const* in, void* const* out, cons
   LT_REQUIRE(n >= 0 && (n == 0 || (in && out && count)), LT_ERR_BAD_ARG, "cast: bad arguments");
   LT_REQUIRE(out_dtype == LT_BF16, LT_ERR_BAD_ARG, "cast: dtype code %d is not this library's 16-bit type (" LT_HALF_NAME " = %d)", out_dtype,
              (int)LT_BF16);
-  for (int32_t i = 0; i < n; i += CastJobs::MAX) {
-    CastJobs jobs;
-    jobs.n = std::min<int32_t>(CastJobs::MAX, n - i);
-    for (int j = 0; j < jobs.n; j++) {
-      jobs.in[j] = in[i + j];
-      jobs.out[j] = out[i + j];
-      jobs.count[j] = count[i + j];
+  for (int32_t j = 0; j < n; j++)  // all of them before the first launch
+    LT_REQUIRE(count[j] == 0 || (count[j] > 0 && in[j] && out[j]), LT_ERR_BAD_ARG, "cast: tensor %d of %lld elements is null or of a negative size", j,
+               (long long)count[j]);
+  CastJobs jobs;
+  jobs.n = 0;
+  for (int32_t j = 0; j < n; j++) {
+    if (count[j] == 0) continue;
+    jobs.in[jobs.n] = in[j];
+    jobs.out[jobs.n] = out[j];
+    jobs.count[jobs.n++] = count[j];
+    if (jobs.n == CastJobs::MAX) {
+      LT_TRY(lt_cast_launch(jobs, (hipStream_t)stream));
+      jobs.n = 0;
     }
-    LT_TRY(lt_cast_launch(jobs, (hipStream_t)stream));
   }
-  return LT_OK;
+  return lt_cast_launch(jobs, (hipStream_t)stream);
 }
 
 extern "C" int lt_dropout_mask(int64_t tokens, int32_t hidden, float p, uint64_t seed, uint64_t offset, uint8_t* keep,

@@ -338,3 +338,17 @@ def test_backward_workspace_of_a_block_with_low_rank_terms(tokens, hidden, inter
         desc.i2h, desc.h2o = _linear_desc(hidden, 2 * inter, r), _linear_desc(inter, hidden, r)
         size.append(lib.lt_ffn_backward_workspace_bytes(desc))
     assert 0 < size[0] and size[1] - size[0] <= 2 * tokens * rank * (2 + 16 * 4) + 2048
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_cast_of_nothing_and_of_bad_tensors(dtype):
+    """empty tensors have no address; a bad one behind eight good ones is refused before anything is launched (here any launch would fail)"""
+    lib, code = nat.lib(dtype), nat.LT_BF16 if dtype == torch.bfloat16 else nat.LT_F16
+    nothing = (ctypes.c_void_p * 3)()
+    assert lib.lt_cast(3, nothing, nothing, (ctypes.c_int64 * 3)(), code, None) == 0
+    assert lib.lt_cast(0, None, None, None, code, None) == 0
+    good = [1 << 20] * 8
+    for bad, count in ((None, 5), (1 << 20, -1)):
+        tensors = (ctypes.c_void_p * 9)(*good, bad)
+        assert lib.lt_cast(9, tensors, tensors, (ctypes.c_int64 * 9)(*[4] * 8, count), code, None) == 1
+        assert b"tensor 8" in lib.lt_last_error()
