@@ -240,7 +240,7 @@ int lt_activation_forward(int64_t tokens, int32_t intermediate, int32_t gated, i
 int lt_activation_backward(int64_t tokens, int32_t intermediate, int32_t gated, int32_t act, int32_t dtype,
                            const void* pre, const void* d_hid, void* d_pre, void* stream);
 
-/* ---- fp32 tensors to the library's 16-bit type: in[j] -> out[j], count[j] elements, any n, one launch per eight of them ----
+/* ---- fp32 tensors to the library's 16-bit type: in[j] -> out[j], count[j] elements, any n, a launch for every eight of them (of 2^30 elements) ----
  * A count of 0 is skipped (its pointers may be null); an argument error leaves all outputs as they were. */
 int lt_cast(int32_t n, const float* const* in, void* const* out, const int64_t* count, int32_t out_dtype, void* stream);
 

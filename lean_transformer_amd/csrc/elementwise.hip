@@ -1341,7 +1341,7 @@ int lt_cast_launch(CastJobs& jobs, hipStream_t stream) {
     if (j >= jobs.n) continue;
     LT_REQUIRE(jobs.in[j] && jobs.out[j] && jobs.count[j] > 0, LT_ERR_BAD_ARG, "cast: bad arguments");
     const int64_t blocks = (jobs.count[j] + 2047) / 2048;
-    LT_REQUIRE(blocks + total <= 0x7fffffff, LT_ERR_UNSUPPORTED, "cast: %lld elements", (long long)jobs.count[j]);
+    LT_REQUIRE(blocks + total < (int64_t)1 << 24, LT_ERR_UNSUPPORTED, "cast: %lld elements in one launch", (long long)jobs.count[j]);
     total += (unsigned)blocks;
     bytes += 6.0 * jobs.count[j];
     if (lt_aligned(jobs.in[j], 16) && lt_aligned(jobs.out[j], 16)) jobs.vec |= 1u << j;

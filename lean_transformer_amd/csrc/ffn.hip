@@ -849,18 +849,19 @@ extern "C" int lt_cast(int32_t n, const float* const* in, void* const* out, cons
   for (int32_t j = 0; j < n; j++)  // all of them before the first launch
     LT_REQUIRE(count[j] == 0 || (count[j] > 0 && in[j] && out[j]), LT_ERR_BAD_ARG, "cast: tensor %d of %lld elements is null or of a negative size", j,
                (long long)count[j]);
+  constexpr int64_t PIECE = (int64_t)1 << 30;  // (a launch holds fewer than 2^32 threads of 8 elements)
   CastJobs jobs;
   jobs.n = 0;
-  for (int32_t j = 0; j < n; j++) {
-    if (count[j] == 0) continue;
-    jobs.in[jobs.n] = in[j];
-    jobs.out[jobs.n] = out[j];
-    jobs.count[jobs.n++] = count[j];
-    if (jobs.n == CastJobs::MAX) {
-      LT_TRY(lt_cast_launch(jobs, (hipStream_t)stream));
-      jobs.n = 0;
+  for (int32_t j = 0; j < n; j++)
+    for (int64_t at = 0; at < count[j]; at += PIECE) {
+      jobs.in[jobs.n] = in[j] + at;
+      jobs.out[jobs.n] = (char*)out[j] + at * 2;
+      jobs.count[jobs.n++] = std::min(PIECE, count[j] - at);
+      if (jobs.n == CastJobs::MAX) {
+        LT_TRY(lt_cast_launch(jobs, (hipStream_t)stream));
+        jobs.n = 0;
+      }
     }
-  }
   return lt_cast_launch(jobs, (hipStream_t)stream);
 }
 

@@ -36,3 +36,13 @@ def test_others_are_left_to_torch():
     assert torch.equal(out[0], a.t().contiguous().bfloat16()) and out[0].is_contiguous()
     assert out[1].data_ptr() == half.data_ptr() and out[2].shape == (0, 10)
     assert nat.cast_all([a], torch.float32, DEV)[0].data_ptr() == a.data_ptr()
+
+
+def test_a_tensor_in_pieces():
+    """2^30 elements are one piece of a launch"""
+    n = (1 << 30) + 2051
+    t = torch.arange(n, device=DEV, dtype=torch.int32).bitwise_and_(0xffff).float()
+    out, = nat.cast_all([t], torch.bfloat16, DEV)
+    for part in (slice(0, 4096), slice((1 << 30) - 4096, n)):
+        assert torch.equal(out[part], t[part].bfloat16())
+    assert torch.equal(out[::4097], t[::4097].bfloat16())
