@@ -203,7 +203,7 @@ def cast_all(tensors, dtype: torch.dtype, device: torch.device) -> list:
         if t is not None:
             t = t.detach()
             if t.dtype != dtype:
-                if t.dtype == torch.float32 and t.is_contiguous() and t.numel():
+                if t.dtype == torch.float32 and t.is_contiguous() and t.numel() and not t.is_neg():  # (a negated view's memory holds the other sign)
                     wide.append(t)
                     t = torch.empty(t.shape, dtype=dtype, device=device)
                     narrow.append(t)

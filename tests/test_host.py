@@ -352,3 +352,10 @@ def test_cast_of_nothing_and_of_bad_tensors(dtype):
         tensors = (ctypes.c_void_p * 9)(*good, bad)
         assert lib.lt_cast(9, tensors, tensors, (ctypes.c_int64 * 9)(*[4] * 8, count), code, None) == 1
         assert b"tensor 8" in lib.lt_last_error()
+
+
+def test_cast_of_a_negated_view():
+    """a tensor whose sign is a flag beside its memory is torch's to convert"""
+    a = torch.randn(3, 8)
+    out, = nat.cast_all([torch._neg_view(a)], torch.bfloat16, torch.device("cpu"))
+    assert torch.equal(out, (-a).bfloat16()) and not out.is_neg()
