@@ -482,7 +482,7 @@ bool lt_gemm_thin_supported(const GemmProblem& p, int dtype) {
   // 32-bit byte offsets: inside a workgroup's rows, over the whole factor
   if (64 * p.A[0].ld * 2 >= (int64_t)1 << 31 || (p.B[0].kmajor ? p.N : p.K[0]) * p.B[0].ld * 2 >= (int64_t)1 << 31 || p.K[0] >= (int64_t)1 << 29)
     return false;
-  return (p.M + 15) / 16 <= 0x7fffffff;
+  return p.M < (int64_t)1 << 28;  // 16 threads a row (8 wavefronts on 32 rows), less than 2^32 a launch
 }
 
 // 128 x 128 tiles (with the sum of their slices) and this, us, operands from memory.  Up to 16 columns: [500, 16] over 768 11.9, 8.2; over 8192
