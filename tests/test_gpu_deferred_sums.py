@@ -10,14 +10,17 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("tokens,fan_in,fan_out,rank,bias", [
+CASES = [
     (1, 8, 8, 0, True),          # nothing split, one column sum
     (257, 64, 72, 8, True),      # one tile a product
-    (4099, 768, 320, 16, True),  # every gradient split, all in the room
+    (4099, 768, 320, 16, True),  # every gradient split, all of them wait
     (4099, 768, 320, 16, False),
-    (4096, 1536, 2048, 64, True),   # a weight gradient of more than the room, summed at once, beside low-rank ones that wait
+    (4096, 1536, 2048, 64, True),   # a weight gradient too large to wait, summed at once, beside low-rank ones that wait
     (2051, 1003, 517, 5, True),     # sizes off every tile: the any-shape kernel's splits
-])
+]
+
+
+@pytest.mark.parametrize("tokens,fan_in,fan_out,rank,bias", CASES)
 @pytest.mark.parametrize("compute", ["autocast", "fp32"])
 def test_gradients_summed_at_the_end(tokens, fan_in, fan_out, rank, bias, compute):
     torch.manual_seed(tokens + fan_in)
@@ -49,6 +52,43 @@ def test_gradients_summed_at_the_end(tokens, fan_in, fan_out, rank, bias, comput
                 assert ((g.double() - ref).abs() <= 2.0**-8 * room + 1e-30).all(), name
                 continue
         assert ((g.double() - ref).abs() <= (tokens + fan_in + 64) * 2.0**-23 * room + 1e-30).all(), name
+
+
+def check_whole_numbers(tokens, fan_in, fan_out, rank, bias, compute):
+    """Gradients of whole numbers, and one-hot low-rank factors, whose products are columns of x and dy: every sum is
+    exact (below 2^24), in any order, and none may lack a token.  Returns the launches of the backward pass by their tags."""
+    torch.manual_seed(tokens + fan_out)
+    layer = GeneralizedLinear(GeneralizedMatrix(fan_in, fan_out), adapter_dim=rank, bias=bias).to(DEV)
+    x = torch.randint(-3, 4, (tokens, fan_in), device=DEV).float()
+    dy = torch.randint(-3, 4, (tokens, fan_out), device=DEV).float()
+    x[-1].abs_().add_(1.0)  # (the last token is in every sum)
+    dy[-1].abs_().add_(1.0)
+    expected = {"weight": dy.double().t() @ x.double(), "bias": dy.double().sum(0)}
+    if rank:
+        of_x, of_dy = torch.randperm(fan_in, device=DEV)[:rank], torch.randperm(fan_out, device=DEV)[:rank]
+        one_hot = torch.nn.functional.one_hot
+        with torch.no_grad():
+            layer.adapter_first.copy_(one_hot(of_x, fan_in))
+            layer.adapter_second.copy_(one_hot(of_dy, fan_out).t())
+        expected["adapter_second"] = dy.double().t() @ x.double()[:, of_x]
+        expected["adapter_first"] = dy.double()[:, of_dy].t() @ x.double()
+    with torch.autocast("cuda", torch.bfloat16, enabled=compute == "autocast"):
+        y = layer(x)
+    names, params = zip(*layer.named_parameters())
+    lib = nat.lib(torch.bfloat16)
+    lib.lt_profile_reset()
+    lib.lt_profile_enable(1)
+    grads = torch.autograd.grad(y, params, dy.to(y.dtype))
+    lib.lt_profile_enable(0)
+    for name, g in zip(names, grads):
+        assert g.dtype == torch.float32 and torch.equal(g.double(), expected[name.split(".")[-1]]), name
+    return {tag: n for tag, n, *_ in nat.profile_read(lib)}
+
+
+@pytest.mark.parametrize("tokens,fan_in,fan_out,rank,bias", CASES)
+@pytest.mark.parametrize("compute", ["autocast", "fp32"])
+def test_no_token_is_lost(tokens, fan_in, fan_out, rank, bias, compute):
+    check_whole_numbers(tokens, fan_in, fan_out, rank, bias, compute)
 
 
 def test_partial_results_that_do_not_all_fit():

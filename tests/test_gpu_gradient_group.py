@@ -5,23 +5,27 @@ import torch
 
 from lean_transformer_amd import _native as nat
 from lean_transformer_amd.blocksparse.linear import GeneralizedLinear, GeneralizedMatrix
-from test_gpu_deferred_sums import test_gradients_summed_at_the_end as check
+from test_gpu_deferred_sums import check_whole_numbers, test_gradients_summed_at_the_end as check
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("tokens,fan_in,fan_out,rank", [
-    (65, 128, 128, 8),        # three products of a tile each, one slice
-    (1000, 136, 264, 128),    # edges of tiles
-    (4001, 640, 136, 136),    # a rank over one tile
-    (2049, 768, 2304, 16),    # with the weight gradient where both fit 256 workgroups, the third alone
-    (300, 2048, 2048, 24),    # 256 tiles of the weight gradient
-    (300, 2176, 2048, 24),    # more: the low-rank pair alone
-    (8200, 64, 64, 8),        # many slices
+# launches: of 128 x 128 tiles, for the weight gradient and the low-rank pair
+@pytest.mark.parametrize("tokens,fan_in,fan_out,rank,launches", [
+    (65, 128, 128, 8, 1),        # three products of a tile each, one slice
+    (1000, 136, 264, 128, 1),    # edges of tiles
+    (4001, 640, 136, 136, 1),    # a rank over one tile
+    (2049, 768, 2304, 16, 1),    # 132 tiles, one slice
+    (8200, 768, 2304, 16, 2),    # two slices: the weight gradient with the one that fits 256 workgroups beside it, the third alone
+    (300, 2048, 2048, 24, 2),    # 256 tiles of the weight gradient: the low-rank pair alone
+    (300, 2176, 2048, 24, 2),    # more
+    (8200, 64, 64, 8, 1),        # many slices
 ])
-def test_gradients(tokens, fan_in, fan_out, rank):
+def test_gradients(tokens, fan_in, fan_out, rank, launches):
     check(tokens, fan_in, fan_out, rank, True, "autocast")
+    seen = check_whole_numbers(tokens, fan_in, fan_out, rank, True, "autocast")
+    assert seen["gemm_mid_tn_store"] == launches, seen
 
 
 def test_they_share_a_launch():

@@ -1,5 +1,5 @@
 """Blocks of a few rows, whose LayerNorm is part of the up-projection: against the oracle, gradients (which read the statistics it leaves)
-among them, at the edges of rows, widths and the three workgroup shapes, and rows alone against rows in a larger batch."""
+among them, at the edges of rows, widths and the three workgroup shapes, and rows alone against the same rows in larger batches."""
 import pytest
 import torch
 
@@ -80,3 +80,17 @@ def test_rows_with_infinities(dtype):
     assert torch.equal(few.isnan(), many.isnan()) and few[2:4].isnan().all() and not few[[0, 1, 4]].isnan().any()
     keep = [0, 1, 4]
     assert_close(few[keep], many[keep].float().cpu(), dtype, "y")
+
+
+@pytest.mark.parametrize("hidden,inter,gated", [(104, 1000, False), (520, 2056, True), (64, 32768, False)])
+@pytest.mark.parametrize("dtype,most", [(torch.float32, 4), (torch.bfloat16, 8), (torch.float16, 8)])
+def test_rows_alone_and_in_larger_batches(hidden, inter, gated, dtype, most):
+    """the same bits for a row in every batch that is taken; above, its LayerNorm is summed in another order (one wavefront a row)"""
+    ffn = _ffn(hidden, inter, gated, dtype)
+    x = (3 * torch.randn(24, hidden) + 1).to(dtype).to(DEV)
+    with torch.no_grad():
+        rows = torch.cat([ffn(x[i:i + 1]) for i in range(most)])
+        for tokens in (2, 3, most):
+            assert torch.equal(ffn(x[:tokens]), rows[:tokens]), tokens
+        for tokens in (most + 1, 24):
+            assert_close(ffn(x[:tokens])[:most], rows.cpu(), dtype, "y")
