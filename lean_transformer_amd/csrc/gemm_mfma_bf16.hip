@@ -95,7 +95,10 @@ int splitk_slices(int64_t M, int64_t N, int64_t K);
 // over 4096 121, 136 (over 3584 [889, 10048] 114, 105).
 // Unfused products and down-projections have less of an epilogue to work beside: two whole rounds against one 57, 53 over 1024, 94, 79 over 2048,
 // 172, 145 over 4096.  They change where the large tiles' second round is nearly empty: [5500, 2880] over 2880 148, 113, its input gradient 137, 110;
-// over 11520 494, 397; [10000, 1600] over 1600 100, 85; [10000, 2048] over 2048 142, 120.
+// over 11520 494, 397; [10000, 1600] over 1600 100, 85; a down-projection, whose dropout and residual are some work, also where it is half
+// full ([11376, 2080] over 784 90, 81) or one of several ([31229, 3616] over 848 410, 371), where an unfused product keeps the large tiles: input
+// gradient [19957, 1392] over 1104 102, 117; [16748, 3408] over 1048 151, 168; [11462, 2832] over 1424 145, 161.  T 2000 - 40000, widths 512 - 4096,
+// reductions 768 - 16384, of the other's time: 102 down-projections 0.54 - 1.04, 13 % below it on average, 41 input gradients 0.69 - 1.00, 14 %.
 bool mid_rounds_shorter(int64_t M, int64_t columns, int64_t K, int kind, bool gated_forward) {
   const double large = (double)((M + 255) / 256 * ((columns + 255) / 256)) / 256, small = (double)mid_tiles(M, columns) / 512;
   auto whole = [](double r) { return (double)(int64_t)r; };
@@ -106,7 +109,7 @@ bool mid_rounds_shorter(int64_t M, int64_t columns, int64_t K, int kind, bool ga
   if (!fused && (large < 1.0 || K < 768)) return false;  // (shorter reductions: not measured)
   if (fused && large < 1.0 && K > (kind == EPI_ACT_BWD ? 3584 : 2048)) return false;
   const double ratio = fused ? 0.92 + 0.16 * std::min(1.0, std::max(0.0, ((double)K - 512) / 1536)) + (gated_forward ? 0.1 : 0.0)
-                             : 1.0 + 0.22 * std::min(1.0, std::max(0.0, ((double)K - 768) / 2048));
+                             : (kind == EPI_OUT ? 1.0 : 1.16) + 0.26 * std::min(1.0, std::max(0.0, ((double)K - 768) / 1600));
   return ratio * small_rounds / 2 < 0.96 * large_rounds;
 }
 // 128 x 128 tiles where they all run at once, two workgroups per CU; 256 x 256 ones then fill half of the chip at most.  [1024, 8192]

@@ -85,3 +85,21 @@ def test_long_reductions_that_leave_compute_units_idle(tokens, hidden, inter, fo
     lib.lt_profile_enable(0)
     tags = {e[0] for e in nat.profile_read(lib)}
     assert {f"gemm_{forward}_nt_act_fwd", f"gemm_{backward}_nn_act_bwd"} <= tags, tags
+
+
+@pytest.mark.parametrize("tokens,hidden,inter,out,input_gradient", [
+    (9528, 1600, 792, "mid", "mid"),    # 266 tiles of 256 x 256: a second round of ten
+    (8541, 2376, 1208, "mid", "bf16"),  # a third of a second round
+    (16384, 2048, 1024, "bf16", "bf16"),  # two whole rounds
+])
+def test_unfused_products_by_rounds(tokens, hidden, inter, out, input_gradient):
+    """which kernel takes the down-projection and the up-projection's input gradient"""
+    ffn = lt.LeanFFN(hidden, inter, activation=lt.ACT2FN["silu"]).to(DEV).to(torch.bfloat16)
+    x = torch.randn(tokens, hidden, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    lib = nat.lib(torch.bfloat16)
+    lib.lt_profile_reset()
+    lib.lt_profile_enable(1)
+    torch.autograd.grad(ffn(x), x, torch.randn_like(x))
+    lib.lt_profile_enable(0)
+    tags = {e[0] for e in nat.profile_read(lib)}
+    assert {f"gemm_{out}_nt_out", f"gemm_{input_gradient}_nn_store"} <= tags, tags
