@@ -486,13 +486,15 @@ bool lt_gemm_thin_supported(const GemmProblem& p, int dtype) {
 }
 
 // 128 x 128 tiles (with the sum of their slices) and this, us, operands from memory.  Up to 16 columns: [500, 16] over 768 11.9, 8.2; over 8192
-// 18.5, 11.4; [4000, 16] over 1024 15.4, 7.7; over 4096 20.8, 13.0; [16384, 16] over 768 11.6, 11.2; over 2048 25.3, 19.8; over 4096 29.8, 30.4.  32:
+// 18.5, 11.4; [4000, 16] over 1024 15.4, 7.7; over 4096 20.8, 13.0; [16384, 16] over 768 11.6, 11.2; over 2048 25.3, 19.8; over 4096 29.8, 30.4.  More
+// rows are several rounds of short workgroups: [24000, 16] over 512 12.0, 13.1; [50000, 16] over 256 13.1, 15.4; [65000, 16] over 64 9.1, 11.5, over
+// 1024 29.8, 31.9; from 65537 on the other side is 256 x 256 tiles: [66000, 16] over 256 33, 17; [131072, 16] over 256 35, 25, over 1024 71, 44.  32:
 // [4000, 32] over 2304 18.2, 11.9; [8192, 32] over 4096 26.4, 22.1; [12000, 32] over 768 13.1, 13.3.  64 columns, where the factor is read from L2
 // more often: [500, 64] over 1024 15.6, 10.1; [4000, 64] over 1024 13.5, 9.8; over 2048 17.6, 13.7; over 4096 20.6, 19.0, but 17.1, 18.4 with the
 // activation still in the caches; over 8192 26.4, 29.0 (52.4 where the caller has no room for slices); [16384, 64] over 1024 16.6, 17.2.
 bool lt_gemm_thin_selected(const GemmProblem& p, int dtype, bool can_split) {
   if (!lt_gemm_thin_supported(p, dtype)) return false;
-  if (p.N <= 16) return p.M <= 8192 || p.K[0] <= 3072;
+  if (p.N <= 16) return p.M <= 8192 || (p.K[0] <= 3072 && (p.M <= 16384 || p.M > 65536));
   return p.M <= 8192 && (p.K[0] <= (p.N <= 32 ? 4096 : 2048) || !can_split);
 }
 

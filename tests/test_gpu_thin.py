@@ -78,6 +78,22 @@ def test_neighbours_of_the_rule(tokens, k, rank):
     _check(g_hid, long, factor, torch.bfloat16)
 
 
+@pytest.mark.parametrize("tokens,thin", [(16384, True), (16385, False), (65536, False), (65537, True)])
+def test_rows_of_the_rule(tokens, thin):
+    """up to 16 columns: rows of one launch's workgroups, and more than 128 x 128 tiles run at once"""
+    layer = _layer(64, 8, 16, torch.bfloat16)
+    x = torch.randint(-2, 3, (tokens, 64), device=DEV).bfloat16()
+    with torch.no_grad():
+        layer.adapter_first.copy_(torch.eye(16, 64))
+        layer.adapter_second.copy_(torch.eye(8, 16))
+        lib = nat.lib(torch.bfloat16)
+        lib.lt_profile_reset()
+        lib.lt_profile_enable(1)
+        y = layer(x)
+        lib.lt_profile_enable(0)
+    assert ("gemm_thin" in {e[0] for e in nat.profile_read(lib)}) == thin and torch.equal(y, x[:, :8])
+
+
 def test_values_past_the_end_are_not_read_into_the_sums():
     """rows of the factor and of the activation behind the last one hold NaN in memory"""
     tokens, k, rank = 100, 72, 24
