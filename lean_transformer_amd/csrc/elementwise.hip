@@ -16,7 +16,7 @@ static int ln_vectors_per_lane(int H) { return H <= 2048 ? 8 : H <= 4096 ? 16 : 
 // mean and the centred second moment are reduced across the 64 lanes with shuffles, and the normalised row is written in
 // the GEMM operand dtype.  TAIL fuses what follows a post-LayerNorm: dropout, then the residual add.  Weight and bias come in TW, as the
 // module holds them, and workgroups behind those of the rows widen the biases of the products to come: a launch of their own for these few
-// kilobytes took 2.5 - 4 us and the host's time for it (with the trips to memory overlapped: eight tokens, hidden 768 44.6 us, 42.0; a prompt of 512, hidden 2048 63.5, 60.9).
+// kilobytes took 2.5 - 4 us and the host's time for it (a prompt of 512, hidden 2048 63.5 us, 60.9).  Blocks of up to eight rows have theirs elsewhere (gemm_stream.hip).
 // ---------------------------------------------------------------------------------------------------------------------
 __device__ __forceinline__ void widen_block(const WidenJobs& jobs, int block) {
   for (int j = 0; j < jobs.n; j++) {

@@ -113,7 +113,7 @@ bool mid_rounds_shorter(int64_t M, int64_t columns, int64_t K, int kind, bool ga
   return ratio * small_rounds / 2 < 0.96 * large_rounds;
 }
 // 128 x 128 tiles where they all run at once, two workgroups per CU; 256 x 256 ones then fill half of the chip at most.  [1024, 8192]
-// over 2048 (512 of them): 37 us against 47; [1536, 6400] over 1600 (600): 51 against 44.  Where the product is unfused, the 256 x 256
+// over 2048 (512 of them): 37 us against 47.  Where the product is unfused, the 256 x 256
 // kernel can split its reduction into as many slices as `room` (bytes of workspace) holds, and the estimates are compared:
 //   k-major A: 64 k take 0.58 us (two workgroups on a CU 1.04) against 1.45, and a start and an end of 15 us.  Down-projection of hidden
 //     4096 over 16384, T 1025 and 1790: 260 and 269 us against 209 and 238 in two slices; its input gradient, T 1024 and 1200: 170 and
@@ -345,8 +345,9 @@ int lt_launch_gemm_skinny(const GemmProblem& p, int dtype, int io_dtype, void* w
 // Which of the products share a launch.  Low-rank gradients are a few tiles each, in as many slices as there are CUs: a launch of 9 - 16 us
 // that is mostly its start and its end.  With the same number of slices for all of a subset, their workgroups are equally long and at
 // most 256, one per CU, so that the launch takes as long as its longest slice; the estimate is mid_best's, and a launch costs 5 us more.
-// Launches one by one, together: qkv, rank 16, T 16384 (108 + 18 tiles, 2 slices) 63 + 16 us, 65; PixelFly of hidden 1024, rank 64, T 4000
-// (8 + 32, 6) 9 + 11, 12; (64 + 8, 3) 16 + 8, 18.
+// Launches one by one, together: qkv, rank 16, T 16384 (108 + 18 tiles, 2 slices) 63 + 16 us, 67; PixelFly of hidden 1024, rank 64, T 4000
+// (8 + 32, 6) 9 + 11, 13.5; (64 + 8, 3) 16 + 8, 17.5.  108 layers, T 64 - 20000, widths 64 - 6144, ranks 8 - 136: where the estimate puts products
+// together, all take 0.46 - 0.96 of the launches one by one with their sums, the older loop's stage time notwithstanding.
 int lt_launch_gemm_gradients(const GemmProblem* problems, int n, int dtype, int io_dtype, void* workspace, size_t workspace_bytes,
                              hipStream_t stream, ColReduceQueue* queue) {
   LT_REQUIRE(n <= LT_MID_GROUP_MAX, LT_ERR_BAD_ARG, "gradients: %d of them", n);

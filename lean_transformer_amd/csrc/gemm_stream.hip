@@ -2,8 +2,8 @@
 // fp32 or 16-bit, with the forward epilogues fused.
 //
 // What bounds it: the weights, which are read once (403 MB per token at hidden 4096, gated: 70 us at 5.8 TB/s); a 256 x 256 tile
-// spends all its time on a few rows, and leaves most CUs without a tile (hidden 4096, one token: 220 us for the block; 101 now, its two
-// products 53 and 31 us = 5.1 and 4.4 TB/s).  So the reduction
+// spends all its time on a few rows, and leaves most CUs without a tile (hidden 4096, one token: 220 us for the block; 88 now, its two
+// launches 55 and 31 us = 4.9 and 4.4 TB/s).  So the reduction
 // is split over the wavefronts of a workgroup: a workgroup owns 16 NT rows of W (gated up-projection: half of them gate rows, half
 // the matching linear rows), wavefront w takes the 128-byte k-blocks w, w + W, ... of all of them, and the partial sums meet in
 // LDS at the end, in wavefront order, so that a result is the same at every run.  A block is fetched 128 contiguous bytes per 8 lanes
